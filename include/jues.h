@@ -131,9 +131,10 @@ jues_status jues_create(jues_ctx** ctx, int device);
 void jues_destroy(jues_ctx* ctx);
 const char* jues_last_error(const jues_ctx* ctx);
 void jues_cc_default_opts(jues_cc_opts* opts);
-/* Bytes of device memory currently held by the context (integrals, scratch). */
+/* Bytes of device memory currently held by the library: integrals, scratch, and the blocks that
+ * each context keeps for its next buffers (at most a sixteenth of the device's memory). */
 size_t jues_device_bytes(const jues_ctx* ctx);
-/* Release all device buffers held by the context (keeps the stream). */
+/* Release all device buffers held by the context, kept blocks included (keeps the stream). */
 jues_status jues_release(jues_ctx* ctx);
 
 /* ---- AO integrals (the Wfn.ao_eri carrier, Backend/Wavefunction.jl:87) ------

@@ -23,6 +23,7 @@ jues_status jues_create(jues_ctx** out, int device) {
   }
   jues_ctx* c = new jues_ctx();
   c->device = device;
+  c->pool = std::make_shared<BlockPool>(device);
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
     delete c;
     return JUES_HIP_ERROR;
@@ -35,6 +36,7 @@ void jues_destroy(jues_ctx* ctx) {
   if (!ctx) return;
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
+  ctx->pool->close();
   ctx->cc.reset();
   release_scratch(ctx);
   for (auto& p : ctx->pending) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
@@ -57,6 +59,7 @@ jues_status jues_release(jues_ctx* ctx) {
   ctx->Bfac.release();
   ctx->Bfac32.release();
   ctx->n = ctx->naux = 0;
+  ctx->pool->trim();
   JUES_API_END(ctx)
 }
 

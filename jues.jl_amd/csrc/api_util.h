@@ -9,7 +9,8 @@
   if (!(ctx)) return JUES_BAD_ARG;                  \
   try {                                             \
     if (hipSetDevice((ctx)->device) != hipSuccess)  \
-      throw ::jues::Error(JUES_HIP_ERROR, "hipSetDevice failed");
+      throw ::jues::Error(JUES_HIP_ERROR, "hipSetDevice failed"); \
+    ::jues::PoolScope pool_scope_((ctx)->pool);
 
 #define JUES_API_END(ctx)                                 \
   }                                                       \

@@ -106,7 +106,7 @@ bool ladder_recompute_mode(jues_ctx* ctx, const CCState& S, int mode, int prec) 
   }
   if (!factors) return false;
   size_t free_b = 0, total_b = 0;
-  JUES_HIP(hipMemGetInfo(&free_b, &total_b));
+  device_memory(ctx, &free_b, &total_b);
   const double N2 = (double)S.o * S.o * S.v * S.v;
   const double vv = (double)S.P.npv * S.P.npv + (double)S.P.nmv * S.P.nmv;
   const int dm = S.opts.diis ? S.opts.diis_max : 1;
@@ -1095,7 +1095,7 @@ double cc_energy(jues_ctx* ctx, CCState& S) {
 static void thin_fp64_ints(jues_ctx* ctx, CCState& S) {
   if (S.i64_thin) return;
   size_t free_b = 0, total_b = 0;
-  JUES_HIP(hipMemGetInfo(&free_b, &total_b));
+  device_memory(ctx, &free_b, &total_b);
   const char* env = std::getenv("JUES_THIN_FP64_INTS");
   const bool force = env && std::atoi(env) != 0;
   if (!force && (double)free_b >= 0.15 * (double)total_b) return;

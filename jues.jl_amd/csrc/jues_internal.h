@@ -4,10 +4,13 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <list>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/jues.h"
@@ -33,6 +36,45 @@ struct Error : std::exception {
     if (!(cond)) throw ::jues::Error(JUES_BAD_ARG, std::string(msg));    \
   } while (0)
 
+// Device blocks that a context's buffers released and may use again.  A solve, a gradient or a transform
+// allocates and frees tens of buffers of up to hundreds of megabytes, and hipMalloc / hipFree cost from
+// tens of microseconds to several milliseconds each (the driver maps and clears the memory, and hipFree waits
+// for the device): at n = 256 they took 2.2 of the 8.7 ms of a factor-route MP2 gradient, and 40 ms of it when
+// three contexts took turns.
+// One pool per context, so every block is reused in the order of that context's stream.  Kept are at most a
+// sixteenth of the device's memory and 256 blocks, the least recently released going first; jues_release
+// and jues_destroy give all of them back, and an allocation that the device refuses is tried again after
+// every pool of the process has given its blocks back.
+class BlockPool {
+ public:
+  explicit BlockPool(int device);
+  ~BlockPool();
+  void* take(size_t bytes, size_t& capacity);  // a kept block of at least `bytes`, or null
+  void give(void* p, size_t capacity);         // keeps or frees the block
+  void trim();                                 // frees every kept block
+  void close();                                // trim, and free what is given from now on
+  size_t kept();
+  int device() const { return device_; }
+
+ private:
+  struct Block {
+    void* p;
+    size_t capacity;
+  };
+  std::mutex mu_;
+  std::list<Block> blocks_;  // oldest first
+  size_t kept_ = 0, limit_ = 0;
+  int device_;
+  bool open_ = true;
+};
+
+// While one is active on the calling thread, DevBuf::alloc uses the given pool.
+struct PoolScope {
+  std::shared_ptr<BlockPool> prev;
+  explicit PoolScope(const std::shared_ptr<BlockPool>& pool);
+  ~PoolScope();
+};
+
 // Owning device allocation.  Allocation failure raises JUES_OOM.
 struct DevBuf {
   void* p = nullptr;
@@ -41,18 +83,31 @@ struct DevBuf {
   explicit DevBuf(size_t nbytes) { alloc(nbytes); }
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
-  DevBuf(DevBuf&& o) noexcept : p(o.p), bytes(o.bytes) { o.p = nullptr; o.bytes = 0; }
+  DevBuf(DevBuf&& o) noexcept { swap(o); }
   DevBuf& operator=(DevBuf&& o) noexcept {
-    if (this != &o) { release(); p = o.p; bytes = o.bytes; o.p = nullptr; o.bytes = 0; }
+    if (this != &o) { release(); swap(o); }
     return *this;
   }
   ~DevBuf() { release(); }
   void alloc(size_t nbytes);
   void release();
   template <typename T> T* as() const { return static_cast<T*>(p); }
+
+ private:
+  void swap(DevBuf& o) noexcept {
+    std::swap(p, o.p);
+    std::swap(bytes, o.bytes);
+    std::swap(capacity, o.capacity);
+    pool.swap(o.pool);
+  }
+  size_t capacity = 0;              // of the block, at least `bytes`
+  std::shared_ptr<BlockPool> pool;  // where the block goes on release
 };
 
+// Device memory allocated by the process (buffers in use and kept blocks)
 size_t device_bytes_in_use();
+// Free and total memory of the context's device; kept blocks, which the next allocation may take, count as free
+void device_memory(jues_ctx* ctx, size_t* free_bytes, size_t* total_bytes);
 
 // Allocation-free scope: while one is active on the calling thread, DevBuf::alloc and
 // scratch() raise instead of allocating, and gemm() avoids its workspace paths (split-K,
@@ -82,6 +137,8 @@ struct jues_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   std::string err;
+  std::shared_ptr<jues::BlockPool> pool;
+  jues::DevBuf scratch[20];  // temporaries, grown on demand (jues::scratch)
   // AO integrals: exactly one of gao (n^4) / Bfac (n*n*naux) is set.
   int n = 0, naux = 0;
   jues::DevBuf gao;

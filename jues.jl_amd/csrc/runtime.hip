@@ -13,44 +13,155 @@ NoAllocScope::NoAllocScope() : prev(tl_no_alloc) { tl_no_alloc = true; }
 NoAllocScope::~NoAllocScope() { tl_no_alloc = prev; }
 bool no_alloc_active() { return tl_no_alloc; }
 
+// ---- kept blocks ----------------------------------------------------------------------
+namespace {
+constexpr size_t kMaxBlocks = 256;
+
+void device_free(void* p, size_t bytes) {
+  (void)hipFree(p);
+  g_bytes -= bytes;
+}
+
+// every open pool of the process
+std::mutex g_pools_mu;
+std::list<BlockPool*>& all_pools() {
+  static std::list<BlockPool*> l;
+  return l;
+}
+thread_local std::shared_ptr<BlockPool> tl_pool;
+}  // namespace
+
+BlockPool::BlockPool(int device) : device_(device) {
+  size_t free_b = 0, total_b = 0;
+  if (hipMemGetInfo(&free_b, &total_b) == hipSuccess) limit_ = total_b / 16;
+  std::lock_guard<std::mutex> l(g_pools_mu);
+  all_pools().push_back(this);
+}
+
+BlockPool::~BlockPool() {
+  {
+    std::lock_guard<std::mutex> l(g_pools_mu);
+    all_pools().remove(this);
+  }
+  trim();
+}
+
+// The smallest kept block that holds `bytes` with at most an eighth (and 256 bytes) to spare, so that a
+// pool serves the same sizes again without tying up large blocks under small buffers.
+void* BlockPool::take(size_t bytes, size_t& capacity) {
+  std::lock_guard<std::mutex> l(mu_);
+  auto best = blocks_.end();
+  for (auto it = blocks_.begin(); it != blocks_.end(); ++it)
+    if (it->capacity >= bytes && it->capacity <= bytes + bytes / 8 + 256 &&
+        (best == blocks_.end() || it->capacity < best->capacity))
+      best = it;
+  if (best == blocks_.end()) return nullptr;
+  void* p = best->p;
+  capacity = best->capacity;
+  kept_ -= capacity;
+  blocks_.erase(best);
+  return p;
+}
+
+void BlockPool::give(void* p, size_t capacity) {
+  std::list<Block> out;  // freed outside the lock (hipFree waits for the device)
+  {
+    std::lock_guard<std::mutex> l(mu_);
+    bool keep = open_ && capacity <= limit_;
+    if (keep) {
+      try {
+        blocks_.push_back({p, capacity});
+      } catch (...) {  // no host memory for the list node: called from destructors, so nothing may leave
+        keep = false;
+      }
+    }
+    if (keep) {
+      p = nullptr;
+      kept_ += capacity;
+      while (kept_ > limit_ || blocks_.size() > kMaxBlocks) {
+        kept_ -= blocks_.front().capacity;
+        out.splice(out.end(), blocks_, blocks_.begin());
+      }
+    }
+  }
+  if (p) device_free(p, capacity);
+  for (const Block& b : out) device_free(b.p, b.capacity);
+}
+
+void BlockPool::trim() {
+  std::list<Block> out;
+  {
+    std::lock_guard<std::mutex> l(mu_);
+    out.swap(blocks_);
+    kept_ = 0;
+  }
+  for (const Block& b : out) device_free(b.p, b.capacity);
+}
+
+void BlockPool::close() {
+  {
+    std::lock_guard<std::mutex> l(mu_);
+    open_ = false;
+  }
+  trim();
+}
+
+size_t BlockPool::kept() {
+  std::lock_guard<std::mutex> l(mu_);
+  return kept_;
+}
+
+PoolScope::PoolScope(const std::shared_ptr<BlockPool>& pool) : prev(std::move(tl_pool)) { tl_pool = pool; }
+PoolScope::~PoolScope() { tl_pool = std::move(prev); }
+
 void DevBuf::alloc(size_t nbytes) {
   release();
   if (nbytes == 0) return;
   if (tl_no_alloc) throw Error(JUES_BAD_ARG, "device allocation inside an allocation-free entry point");
-  void* q = nullptr;
-  const hipError_t e = hipMalloc(&q, nbytes);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    throw Error(e == hipErrorOutOfMemory ? JUES_OOM : JUES_HIP_ERROR,
-                "hipMalloc(" + std::to_string(nbytes) + " bytes): " + hipGetErrorString(e));
+  void* q = tl_pool ? tl_pool->take(nbytes, capacity) : nullptr;
+  if (!q) {
+    hipError_t e = hipMalloc(&q, nbytes);
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();
+      {
+        std::lock_guard<std::mutex> l(g_pools_mu);
+        for (BlockPool* b : all_pools()) b->trim();
+      }
+      e = hipMalloc(&q, nbytes);
+    }
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      throw Error(e == hipErrorOutOfMemory ? JUES_OOM : JUES_HIP_ERROR,
+                  "hipMalloc(" + std::to_string(nbytes) + " bytes): " + hipGetErrorString(e));
+    }
+    capacity = nbytes;
+    g_bytes += nbytes;
   }
   p = q;
   bytes = nbytes;
-  g_bytes += nbytes;
+  pool = tl_pool;
 }
 
 void DevBuf::release() {
   if (p) {
-    (void)hipFree(p);
-    g_bytes -= bytes;
+    if (pool) pool->give(p, capacity);
+    else device_free(p, capacity);
   }
   p = nullptr;
-  bytes = 0;
+  bytes = capacity = 0;
+  pool.reset();
 }
 
-namespace {
-struct ScratchPool {
-  DevBuf slot[20];
-};
-std::map<const jues_ctx*, ScratchPool>& pools() {
-  static std::map<const jues_ctx*, ScratchPool> m;
-  return m;
+void device_memory(jues_ctx* ctx, size_t* free_bytes, size_t* total_bytes) {
+  JUES_HIP(hipMemGetInfo(free_bytes, total_bytes));
+  std::lock_guard<std::mutex> l(g_pools_mu);
+  for (BlockPool* b : all_pools())
+    if (b->device() == ctx->device) *free_bytes += b->kept();
 }
-}  // namespace
 
 void* scratch(jues_ctx* ctx, int slot, size_t bytes) {
   if (tl_no_alloc) throw Error(JUES_BAD_ARG, "context scratch inside an allocation-free entry point");
-  DevBuf& b = pools()[ctx].slot[slot];
+  DevBuf& b = ctx->scratch[slot];
   if (b.bytes < bytes) {
     if (b.p) JUES_HIP(hipStreamSynchronize(ctx->stream));
     b.alloc(bytes + bytes / 8 + 256);
@@ -58,7 +169,9 @@ void* scratch(jues_ctx* ctx, int slot, size_t bytes) {
   return b.p;
 }
 
-void release_scratch(jues_ctx* ctx) { pools().erase(ctx); }
+void release_scratch(jues_ctx* ctx) {
+  for (DevBuf& b : ctx->scratch) b.release();
+}
 
 void h2d(jues_ctx* ctx, void* dst, const void* src, size_t bytes) {
   if (bytes == 0) return;
