@@ -1,17 +1,14 @@
-// LDS-tiled MFMA GEMM for gfx950 (FP64 and FP32), column-major, batched.
+// MFMA GEMM for gfx950 (FP64 and FP32), column-major, batched: LDS-staged kernels with 128x128, 64x64
+// and 48 / 64 x 256 tiles, a direct kernel for products with few output tiles, and the dispatch
+// between them.
 //
-// One 256-thread workgroup (4 wavefronts of 64) computes a 128x128 tile of C.
-// Each wavefront owns a 64x64 sub-tile as a 4x4 grid of 16x16 MFMA blocks
-// (v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32).  The MFMA is issued with the
-// operands swapped (B^T * A^T) so that each lane's accumulator column is an m
-// index: lanes 0..15 then hold 16 consecutive rows of C and the epilogue stores
-// are 16-element contiguous runs along the leading dimension.
+// Every kernel works in 16x16 MFMA blocks (v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32), issued with
+// the operands swapped (B^T * A^T) so that each lane's accumulator column is an m index: lanes 0..15
+// then hold 16 consecutive rows of C and the epilogue stores are 16-element contiguous runs along the
+// leading dimension.
 //
-// The K loop stages BK-deep slices of A and B through LDS; the next slice's
-// global loads are issued before the MFMAs of the current one so the load
-// latency overlaps the matrix work.  Workgroup ids are remapped so that each of
-// the 8 XCDs (each with its own L2) receives a contiguous range of tiles, and
-// tiles are walked in groups of 8 tile-rows to reuse B columns within an L2.
+// Workgroup ids are remapped so that each of the 8 XCDs (each with its own L2) receives a contiguous
+// range of tiles, and tiles are walked in groups of 8 tile-rows to reuse B columns within an L2.
 #include "jues_internal.h"
 
 #include <algorithm>
@@ -26,7 +23,6 @@ typedef float fvec4 __attribute__((ext_vector_type(4)));
 template <typename T> struct Mfma;
 template <> struct Mfma<double> {
   typedef dvec4 acc;
-  static constexpr int BK = 16;
   // accumulator element r of lane l is row (l/16) + 4r of the 16x16 block
   __device__ static inline int row(int lane, int r) { return (lane >> 4) + 4 * r; }
   __device__ static inline acc op(double a, double b, acc c) {
@@ -35,7 +31,6 @@ template <> struct Mfma<double> {
 };
 template <> struct Mfma<float> {
   typedef fvec4 acc;
-  static constexpr int BK = 32;
   // accumulator element r of lane l is row 4(l/16) + r of the 16x16 block
   __device__ static inline int row(int lane, int r) { return 4 * (lane >> 4) + r; }
   __device__ static inline acc op(float a, float b, acc c) {
@@ -60,33 +55,18 @@ template <> __device__ inline float bload<float>(__amdgpu_buffer_rsrc_t r, int v
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
 }
 
-__device__ inline void tile_coords(int pid, int nwg, int tiles_m, int tiles_n, int& tm, int& tn) {
-  // XCD-aware remap (bijective for any nwg): consecutive hardware ids go to
-  // different XCDs; give each XCD a contiguous block of logical tile ids.
-  const int per = (nwg + NXCD - 1) / NXCD;
-  int tall = nwg % NXCD;
-  if (tall == 0) tall = NXCD;
-  const int xcd = pid % NXCD, loc = pid / NXCD;
-  const int p2 = xcd < tall ? xcd * per + loc : tall * per + (xcd - tall) * (per - 1) + loc;
-  // grouped ordering: GROUP_M tile-rows share each sweep over tile-columns
-  const int group_size = GROUP_M * tiles_n;
-  const int gid = p2 / group_size;
-  const int first_m = gid * GROUP_M;
-  const int gsz = min(tiles_m - first_m, GROUP_M);
-  const int r = p2 - gid * group_size;
-  tm = first_m + r % gsz;
-  tn = r / gsz;
-}
-
-// As tile_coords over nwg workgroup ids of which only the first tiles_m * tiles_n carry a
-// tile (a launch padded to a multiple of NXCD); false for the padding ids.
+// Tile of workgroup pid of nwg, of which only the first tiles_m * tiles_n carry a tile (a launch
+// padded to a multiple of NXCD); false for the padding ids.
 __device__ inline bool tile_coords_bounded(int pid, int nwg, int tiles_m, int tiles_n, int& tm, int& tn) {
+  // XCD-aware remap (bijective for any nwg): consecutive hardware ids go to different XCDs; give
+  // each XCD a contiguous block of logical tile ids
   const int per = (nwg + NXCD - 1) / NXCD;
   int tall = nwg % NXCD;
   if (tall == 0) tall = NXCD;
   const int xcd = pid % NXCD, loc = pid / NXCD;
   const int p2 = xcd < tall ? xcd * per + loc : tall * per + (xcd - tall) * (per - 1) + loc;
   if (p2 >= tiles_m * tiles_n) return false;
+  // grouped ordering: GROUP_M tile-rows share each sweep over tile-columns
   const int group_size = GROUP_M * tiles_n;
   const int gid = p2 / group_size;
   const int first_m = gid * GROUP_M;
@@ -117,188 +97,6 @@ struct GemmSide {
   double* C64 = nullptr;
 };
 
-// Shared-memory layout of one operand slice.  When the operand's contiguous
-// global dimension is the row index (m, or n for B) the slice is stored k-major,
-// [k][m], padded so that the four k rows an MFMA fragment read touches start 16
-// (FP32) / 32 (FP64) banks apart; when k is contiguous it is stored m-major,
-// [m][k] with an odd padded row, so that both the coalesced stores and the
-// fragment reads are bank-conflict free.
-template <typename T, bool KMAJOR, int ROWS, int BK>
-struct Slice {
-  static constexpr int PADR = sizeof(T) == 8 ? 16 : 16;  // k-major row padding (elements)
-  static constexpr int PADK = 1;                          // m-major row padding (elements)
-  static constexpr int SIZE = KMAJOR ? BK * (ROWS + PADR) : ROWS * (BK + PADK);
-  __device__ static inline int idx(int r, int k) { return KMAJOR ? k * (ROWS + PADR) + r : r * (BK + PADK) + k; }
-};
-
-// KIND only separates kernel symbols (0 generic, 1 CC ring, 2 CC pp-ladder) so that
-// profiles attribute time to the coupled-cluster hot spots.
-// BM x BN workgroup tile over WM x (4/WM) wavefronts of 64x64: 128x128 (2x2) in general; 64x256
-// (1x4) and 256x64 (4x1) for skinny products (M or N <= 64 against a long other side), where a
-// 128-wide tile would compute mostly padding.
-template <typename T, bool TA, bool TB, int KIND, int BM = 128, int BN = 128, int WM = 2>
-__global__ __launch_bounds__(256, (BM == 128 && BN == 128) ? 2 : 1) void gemm_kernel(int M, int N, int K, T alpha,
-                                                      const T* __restrict__ A, long lda, long sA,
-                                                      const T* __restrict__ B, long ldb, long sB,
-                                                      T beta, T* __restrict__ C, long ldc, long sC,
-                                                      int tiles_m, int tiles_n, int fast_ok) {
-  constexpr int BK = Mfma<T>::BK;
-  constexpr int LA = BM * BK / NT;  // A elements loaded per thread per slice
-  constexpr int LB = BN * BK / NT;
-  // A is m-contiguous unless transposed; B is k-contiguous unless transposed.
-  using SA = Slice<T, !TA, BM, BK>;
-  using SB = Slice<T, TB, BN, BK>;
-  __shared__ T As[2][SA::SIZE];
-  __shared__ T Bs[2][SB::SIZE];
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  static_assert(BM == 64 * WM && BN == 64 * (4 / WM), "tile does not match the wave layout");
-  const int wm = wave % WM, wn = wave / WM;
-  A += (long)blockIdx.z * sA;
-  B += (long)blockIdx.z * sB;
-  C += (long)blockIdx.z * sC;
-
-  int tm, tn;
-  tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
-
-  // element e of a thread's share: the contiguous global dimension varies fastest
-  auto a_rk = [](int e, int& m, int& k) {
-    if (TA) { k = e % BK; m = e / BK; } else { m = e % BM; k = e / BM; }
-  };
-  auto b_rk = [](int e, int& n, int& k) {
-    if (TB) { n = e % BN; k = e / BN; } else { k = e % BK; n = e / BK; }
-  };
-
-  T ra[LA], rb[LB];
-  // Interior tiles and full k-slices load without any bounds logic: element r of
-  // a thread's share sits at p0 + k0*kstride + r*rstride.  Edge tiles and the
-  // last partial k-slice clamp rows/columns into the matrix (those values only
-  // reach output elements that are never stored) and zero k >= K with a select,
-  // so no load is ever predicated by a branch.
-  // per-lane byte offsets inside a tile's k-slice and per-element scalar strides
-  const int a_lane = (int)(sizeof(T) * (TA ? (tid % BK) + (long)(tid / BK) * lda : (tid % BM) + (long)(tid / BM) * lda));
-  const int b_lane = (int)(sizeof(T) * (TB ? (tid % BN) + (long)(tid / BN) * ldb : (tid % BK) + (long)(tid / BK) * ldb));
-  const int a_rs = (int)(sizeof(T) * (TA ? (long)(NT / BK) * lda : (long)(NT / BM) * lda));
-  const int b_rs = (int)(sizeof(T) * (TB ? (long)(NT / BN) * ldb : (long)(NT / BK) * ldb));
-  const bool interior = fast_ok && (m0 + BM <= M) && (n0 + BN <= N);
-  auto load = [&](int k0) {
-    if (interior && k0 + BK <= K) {
-      const auto rA = make_rsrc(TA ? A + k0 + (long)m0 * lda : A + m0 + (long)k0 * lda);
-      const auto rB = make_rsrc(TB ? B + n0 + (long)k0 * ldb : B + k0 + (long)n0 * ldb);
-#pragma unroll
-      for (int r = 0; r < LA; ++r) ra[r] = bload<T>(rA, a_lane, r * a_rs);
-#pragma unroll
-      for (int r = 0; r < LB; ++r) rb[r] = bload<T>(rB, b_lane, r * b_rs);
-    } else {
-#pragma unroll
-      for (int r = 0; r < LA; ++r) {
-        int m, k;
-        a_rk(tid + NT * r, m, k);
-        const int gm = min(m0 + m, M - 1), gk = k0 + k, gkc = min(gk, K - 1);
-        const T val = TA ? A[(long)gkc + (long)gm * lda] : A[(long)gm + (long)gkc * lda];
-        ra[r] = gk < K ? val : T(0);
-      }
-#pragma unroll
-      for (int r = 0; r < LB; ++r) {
-        int n, k;
-        b_rk(tid + NT * r, n, k);
-        const int gn = min(n0 + n, N - 1), gk = k0 + k, gkc = min(gk, K - 1);
-        const T val = TB ? B[(long)gn + (long)gkc * ldb] : B[(long)gkc + (long)gn * ldb];
-        rb[r] = gk < K ? val : T(0);
-      }
-    }
-  };
-  auto store = [&](int buf) {
-#pragma unroll
-    for (int r = 0; r < LA; ++r) {
-      int m, k;
-      a_rk(tid + NT * r, m, k);
-      As[buf][SA::idx(m, k)] = ra[r];
-    }
-#pragma unroll
-    for (int r = 0; r < LB; ++r) {
-      int n, k;
-      b_rk(tid + NT * r, n, k);
-      Bs[buf][SB::idx(n, k)] = rb[r];
-    }
-  };
-
-  typename Mfma<T>::acc acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = typename Mfma<T>::acc{0, 0, 0, 0};
-
-  const int fr = lane & 15, fk = lane >> 4;
-  T af[2][4], bf[2][4];
-  auto frags = [&](int buf, int kk, int slot) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) af[slot][i] = As[buf][SA::idx(wm * 64 + i * 16 + fr, kk + fk)];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) bf[slot][j] = Bs[buf][SB::idx(wn * 64 + j * 16 + fr, kk + fk)];
-  };
-
-  const int nk = (K + BK - 1) / BK;
-  load(0);
-  store(0);
-  __syncthreads();
-  // the last slice is peeled off, so that the loop body is one block without conditions
-  auto compute = [&](int cur) {
-    if constexpr (sizeof(T) == 4) {
-      // FP32: the 32-cycle MFMAs cannot hide a fragment read, so fragments for
-      // step s+1 are fetched while the MFMAs of step s issue
-      frags(cur, 0, 0);
-#pragma unroll
-      for (int s = 0; s < BK / 4; ++s) {
-        if (s + 1 < BK / 4) frags(cur, (s + 1) * 4, (s + 1) & 1);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc[i][j] = Mfma<T>::op(bf[s & 1][j], af[s & 1][i], acc[i][j]);
-      }
-    } else {
-      // FP64: sixteen 64-cycle MFMAs per step cover the fragment latency
-#pragma unroll
-      for (int s = 0; s < BK / 4; ++s) {
-        frags(cur, s * 4, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc[i][j] = Mfma<T>::op(bf[0][j], af[0][i], acc[i][j]);
-      }
-    }
-  };
-  for (int kt = 0; kt + 1 < nk; ++kt) {
-    const int cur = kt & 1;
-    load((kt + 1) * BK);
-    compute(cur);
-    store(cur ^ 1);
-    __syncthreads();
-  }
-  compute((nk - 1) & 1);
-
-  // acc[i][j][r] holds C(m, n) with m = lane%16 of block i, n = Mfma<T>::row(lane, r) of block j.
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + wm * 64 + i * 16 + (lane & 15);
-    if (m >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int n = n0 + wn * 64 + j * 16 + Mfma<T>::row(lane, r);
-        if (n < N) {
-          const long off = (long)m + (long)n * ldc;
-          T v = alpha * acc[i][j][r];
-          if (beta != T(0)) v += beta * C[off];
-          C[off] = v;
-        }
-      }
-    }
-  }
-}
-
 // FP32 C = alpha A op(B) + beta C with A m-contiguous and B k-contiguous (NN) or
 // n-contiguous (NT), 128x128 tile, 4 wavefronts of 64x64.
 // The K slice is 16 deep, so a workgroup needs 32 KB of LDS and at most 128 VGPRs per
@@ -322,10 +120,12 @@ __device__ inline int g32_chunk(int q, int r) { return q ^ ((r >> 2) & 3); }
 // Workgroups [0, nt0) run product p0 (nt0 padded up to a multiple of NXCD when a second
 // product follows), the rest p1.  OUT64: C = alpha A op(B) is written to the FP64 array C64
 // (beta = 0).
-template <int KIND, bool TB, bool TA = false, bool SEG = false, bool OUT64 = false>
+template <int KIND, bool TB, bool TA = false, bool SEG = false, bool OUT64 = false, int BT = 128>
 __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, GemmSide<float> p1, int nt0,
                                                            float alpha, float beta) {
-  constexpr int BM = 128, BN = 128, BK = 16;
+  constexpr int BM = BT, BN = BT, BK = 16;
+  // 64-row shares per thread, 16-row MFMA blocks per wavefront side, wavefront tile edge
+  constexpr int NJ = BT / 64, NB = BT / 32, WT = BT / 2;
   __shared__ __attribute__((aligned(16))) float As[2][BM * BK];
   __shared__ __attribute__((aligned(16))) float Bs[2][BN * BK];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -349,11 +149,11 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
 
   // A share: row am, 4-k chunks ac0 and ac0 + 2; B share: rows bn and bn + 64, chunk bc
   // (ac0 is uniform within a wavefront: in a scalar register the per-k offsets are scalar too)
-  const int am = tid & 127, ac0 = __builtin_amdgcn_readfirstlane(tid >> 7);
+  const int am = tid & (BT - 1), ac0 = __builtin_amdgcn_readfirstlane(tid / BT);
   const int bn = tid >> 2, bc = tid & 3;
-  float ra[8];
-  f4v rat[2];  // TA (A k-contiguous): shared like a k-contiguous B, rows bn and bn + 64, chunk bc
-  f4v rb[2];
+  float ra[4 * NJ];
+  f4v rat[NJ];  // TA (A k-contiguous): shared like a k-contiguous B, rows bn and bn + 64, chunk bc
+  f4v rb[NJ];
   // rows past the edge of M or N load the last row instead (their results are not stored).
   // B k-contiguous (TB false): 16-byte loads of 4 k; B n-contiguous (TB true, op(B) = B^T):
   // loaded like A, one dword per k with row n = am of the tile.
@@ -372,11 +172,11 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
       const auto rA0 = make_rsrc(Ab + k0 + (long)m0 * lda);
       const auto rA1 = make_rsrc(Ab + k0 + (long)m1 * lda);
       rat[0] = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(rA0, at_voff0, 0, 0));
-      rat[1] = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(rA1, at_voff1, 0, 0));
+      if constexpr (NJ == 2) rat[1] = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(rA1, at_voff1, 0, 0));
     } else {
       const auto rA = make_rsrc(Ab + m0 + (long)k0 * lda);
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < NJ; ++j)
 #pragma unroll
         for (int u = 0; u < 4; ++u)
           ra[4 * j + u] = bload<float>(rA, a_voff, 4 * (4 * (ac0 + 2 * j) + u) * (int)lda);
@@ -384,7 +184,7 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
     if constexpr (TB) {
       const auto rB = make_rsrc(Bb + n0 + (long)k0 * ldb);
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < NJ; ++j)
 #pragma unroll
         for (int u = 0; u < 4; ++u)
           rb[j][u] = bload<float>(rB, bt_voff, 4 * (4 * (ac0 + 2 * j) + u) * (int)ldb);
@@ -392,11 +192,11 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
       const auto rB0 = make_rsrc(Bb + k0 + (long)n0 * ldb);
       const auto rB1 = make_rsrc(Bb + k0 + (long)n1 * ldb);
       rb[0] = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(rB0, b_voff0, 0, 0));
-      rb[1] = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(rB1, b2_voff1, 0, 0));
+      if constexpr (NJ == 2) rb[1] = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(rB1, b2_voff1, 0, 0));
     } else {
       const auto rB = make_rsrc(Bb + k0 + (long)n0 * ldb);
       rb[0] = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(rB, b_voff0, 0, 0));
-      rb[1] = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(rB, b_voff1, 0, 0));
+      if constexpr (NJ == 2) rb[1] = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(rB, b_voff1, 0, 0));
     }
   };
   // full slice s of the contraction: segment 0's K / BK slices, then segment 1's
@@ -411,7 +211,7 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
   };
   auto store = [&](int buf) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < NJ; ++j) {
       if constexpr (TA) {
         const int m = bn + 64 * j;
         *reinterpret_cast<f4v*>(&As[buf][m * BK + 4 * g32_chunk(bc, m)]) = rat[j];
@@ -422,7 +222,7 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
       }
     }
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < NJ; ++j) {
       if constexpr (TB) {
         const int c = ac0 + 2 * j;
         *reinterpret_cast<f4v*>(&Bs[buf][am * BK + 4 * g32_chunk(c, am)]) = rb[j];
@@ -433,11 +233,11 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
     }
   };
 
-  fvec4 acc[4][4];
+  fvec4 acc[NB][NB];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NB; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = fvec4{0, 0, 0, 0};
+    for (int j = 0; j < NB; ++j) acc[i][j] = fvec4{0, 0, 0, 0};
 
   const int fr = lane & 15, fk = lane >> 4;
   // slices: the K tail (columns 16 floor(K/16) .. K-1, zero-padded) first when there is one, then the
@@ -447,7 +247,7 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
   if (tail) {
     if constexpr (TA) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < NJ; ++j)
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const int gk = K16 + 4 * bc + u;
@@ -458,7 +258,7 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
     } else {
       const float* Ar = A + m0 + (a_voff >> 2);
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < NJ; ++j)
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const int gk = K16 + 4 * (ac0 + 2 * j) + u;
@@ -467,7 +267,7 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
         }
     }
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         float val;
@@ -487,26 +287,26 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
   store(0);
   __syncthreads();
   auto compute = [&](int cur) {
-    f4v bf[4];
+    f4v bf[NB];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int r = wn * 64 + j * 16 + fr;
+    for (int j = 0; j < NB; ++j) {
+      const int r = wn * WT + j * 16 + fr;
       bf[j] = *reinterpret_cast<const f4v*>(&Bs[cur][r * BK + 4 * g32_chunk(fk, r)]);
     }
-    f4v a0 = *reinterpret_cast<const f4v*>(&As[cur][(wm * 64 + fr) * BK + 4 * g32_chunk(fk, wm * 64 + fr)]);
+    f4v a0 = *reinterpret_cast<const f4v*>(&As[cur][(wm * WT + fr) * BK + 4 * g32_chunk(fk, wm * WT + fr)]);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NB; ++i) {
       f4v a1;
-      if (i + 1 < 4) {
-        const int r = wm * 64 + (i + 1) * 16 + fr;
+      if (i + 1 < NB) {
+        const int r = wm * WT + (i + 1) * 16 + fr;
         a1 = *reinterpret_cast<const f4v*>(&As[cur][r * BK + 4 * g32_chunk(fk, r)]);
       }
 #pragma unroll
       for (int s2 = 0; s2 < 4; ++s2)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < NB; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j][s2], a0[s2], acc[i][j], 0, 0, 0);
-      if (i + 1 < 4) a0 = a1;
+      if (i + 1 < NB) a0 = a1;
     }
   };
   // the last slice is peeled off, so that the loop body is one block without conditions (a schedule
@@ -523,14 +323,14 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
   if constexpr (OUT64) {
     double* __restrict__ C64 = g.C64 + (long)blockIdx.z * g.sC;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = m0 + wm * 64 + i * 16 + (lane & 15);
+    for (int i = 0; i < NB; ++i) {
+      const int m = m0 + wm * WT + i * 16 + (lane & 15);
       if (m >= M) continue;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < NB; ++j) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int n = n0 + wn * 64 + j * 16 + 4 * (lane >> 4) + r;
+          const int n = n0 + wn * WT + j * 16 + 4 * (lane >> 4) + r;
           if (n < N) C64[(long)m + (long)n * ldc] = (double)(alpha * acc[i][j][r]);
         }
       }
@@ -541,30 +341,30 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
     // interior tile accumulating into C: per 16-row block, all of the lane's C loads before
     // its stores (an element-wise load -> store round trip would serialise the epilogue)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const long m = m0 + wm * 64 + i * 16 + (lane & 15);
-      float cv[4][4];
+    for (int i = 0; i < NB; ++i) {
+      const long m = m0 + wm * WT + i * 16 + (lane & 15);
+      float cv[NB][4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < NB; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) cv[j][r] = C[m + (long)(n0 + wn * 64 + j * 16 + 4 * (lane >> 4) + r) * ldc];
+        for (int r = 0; r < 4; ++r) cv[j][r] = C[m + (long)(n0 + wn * WT + j * 16 + 4 * (lane >> 4) + r) * ldc];
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < NB; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          C[m + (long)(n0 + wn * 64 + j * 16 + 4 * (lane >> 4) + r) * ldc] = alpha * acc[i][j][r] + beta * cv[j][r];
+          C[m + (long)(n0 + wn * WT + j * 16 + 4 * (lane >> 4) + r) * ldc] = alpha * acc[i][j][r] + beta * cv[j][r];
     }
     return;
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + wm * 64 + i * 16 + (lane & 15);
+  for (int i = 0; i < NB; ++i) {
+    const int m = m0 + wm * WT + i * 16 + (lane & 15);
     if (m >= M) continue;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < NB; ++j) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int n = n0 + wn * 64 + j * 16 + 4 * (lane >> 4) + r;
+        const int n = n0 + wn * WT + j * 16 + 4 * (lane >> 4) + r;
         if (n < N) {
           const long off = (long)m + (long)n * ldc;
           float v = alpha * acc[i][j][r];
@@ -588,14 +388,15 @@ typedef double d2v __attribute__((ext_vector_type(2)));
 
 __device__ inline int g64_chunk(int q, int r) { return q ^ (r & 7); }
 
-template <int KIND, bool TB, bool TA = false, bool SEG = false>
-__global__ __launch_bounds__(512, 4) void gemm64_kernel(GemmSide<double> p0, GemmSide<double> p1, int nt0,
+template <int KIND, bool TB, bool TA = false, bool SEG = false, int BT = 128>
+__global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, GemmSide<double> p1, int nt0,
                                                         double alpha, double beta) {
-  constexpr int BM = 128, BN = 128, BK = 16;
+  constexpr int BM = BT, BN = BT, BK = 16;
+  constexpr int HT = BT / 2, IB = BT / 32;  // half tile; 16-row MFMA blocks of a wavefront (HT rows)
   __shared__ __attribute__((aligned(16))) double As[2][BM * BK];
   __shared__ __attribute__((aligned(16))) double Bs[2][BN * BK];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave & 1, wn = wave >> 1;  // 2 x 4 wavefronts of 64 x 32
+  const int wm = wave & 1, wn = wave >> 1;  // 2 x (BT / 32) wavefronts of HT x 32
   const bool second = (int)blockIdx.x >= nt0;
   const GemmSide<double> g = second ? p1 : p0;
   const int M = g.M, N = g.N, K = (int)blockIdx.z == (int)gridDim.z - 1 ? g.Klast : g.K;
@@ -612,9 +413,9 @@ __global__ __launch_bounds__(512, 4) void gemm64_kernel(GemmSide<double> p0, Gem
                            g.tiles_m, g.tiles_n, tm, tn))
     return;
   const int m0 = tm * BM, n0 = tn * BN;
-  // A (and n-contiguous B) share: row am, k = 4 kq + u; k-contiguous B share: rows bn, bn + 64, chunk bc
+  // A (and n-contiguous B) share: row am, k = 4 kq + u; k-contiguous B share: rows bn, bn + HT, chunk bc
   // (a k-contiguous A, TA, is shared like a k-contiguous B)
-  const int am = tid & 127, kq = __builtin_amdgcn_readfirstlane(tid >> 7);
+  const int am = tid & (BT - 1), kq = __builtin_amdgcn_readfirstlane(tid / BT);
   const int bn = tid >> 3, bc = tid & 7;
   double ra[4];
   d2v rat[2];
@@ -622,13 +423,13 @@ __global__ __launch_bounds__(512, 4) void gemm64_kernel(GemmSide<double> p0, Gem
   const int a_voff = 8 * (min(m0 + am, M - 1) - m0);
   const int bt_voff = 8 * (min(n0 + am, N - 1) - n0);
   const int b_voff0 = 8 * (2 * bc + (min(n0 + bn, N - 1) - n0) * (int)ldb);
-  const int b_voff1 = 8 * (2 * bc + (min(n0 + bn + 64, N - 1) - n0) * (int)ldb);
-  // TA: k-contiguous rows addressed from two bases, rows m0.. and m1 = min(m0 + 64, M - 1).., so that a
+  const int b_voff1 = 8 * (2 * bc + (min(n0 + bn + HT, N - 1) - n0) * (int)ldb);
+  // TA: k-contiguous rows addressed from two bases, rows m0.. and m1 = min(m0 + HT, M - 1).., so that a
   // byte offset spans at most 63 rows (the same for B in the TA instantiations)
-  const int m1 = min(m0 + 64, M - 1), n1 = min(n0 + 64, N - 1);
+  const int m1 = min(m0 + HT, M - 1), n1 = min(n0 + HT, N - 1);
   const int at_voff0 = 8 * (2 * bc + (min(m0 + bn, M - 1) - m0) * (int)lda);
-  const int at_voff1 = 8 * (2 * bc + (min(m0 + bn + 64, M - 1) - m1) * (int)lda);
-  const int b2_voff1 = 8 * (2 * bc + (min(n0 + bn + 64, N - 1) - n1) * (int)ldb);
+  const int at_voff1 = 8 * (2 * bc + (min(m0 + bn + HT, M - 1) - m1) * (int)lda);
+  const int b2_voff1 = 8 * (2 * bc + (min(n0 + bn + HT, N - 1) - n1) * (int)ldb);
   auto load_seg = [&](const double* Ab, const double* Bb, int k0) {
     if constexpr (TA) {
       const auto rA0 = make_rsrc(Ab + k0 + (long)m0 * lda);
@@ -669,7 +470,7 @@ __global__ __launch_bounds__(512, 4) void gemm64_kernel(GemmSide<double> p0, Gem
     if constexpr (TA) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const int m = bn + 64 * j;
+        const int m = bn + HT * j;
         *reinterpret_cast<d2v*>(&As[buf][m * BK + 2 * g64_chunk(bc, m)]) = rat[j];
       }
     } else {
@@ -682,15 +483,15 @@ __global__ __launch_bounds__(512, 4) void gemm64_kernel(GemmSide<double> p0, Gem
     } else {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const int n = bn + 64 * j;
+        const int n = bn + HT * j;
         *reinterpret_cast<d2v*>(&Bs[buf][n * BK + 2 * g64_chunk(bc, n)]) = rb[j];
       }
     }
   };
 
-  dvec4 acc[4][2];
+  dvec4 acc[IB][2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < IB; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = dvec4{0, 0, 0, 0};
   const int fr = lane & 15, fk = lane >> 4;
@@ -704,7 +505,7 @@ __global__ __launch_bounds__(512, 4) void gemm64_kernel(GemmSide<double> p0, Gem
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           const int gk = K16 + 2 * bc + u;
-          const int m = min(m0 + bn + 64 * j, M - 1);
+          const int m = min(m0 + bn + HT * j, M - 1);
           const double val = A[(long)min(gk, K - 1) + (long)m * lda];
           rat[j][u] = gk < K ? val : 0.0;
         }
@@ -730,7 +531,7 @@ __global__ __launch_bounds__(512, 4) void gemm64_kernel(GemmSide<double> p0, Gem
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           const int gk = K16 + 2 * bc + u;
-          const int n = min(n0 + bn + 64 * j, N - 1);
+          const int n = min(n0 + bn + HT * j, N - 1);
           const double val = B[(long)min(gk, K - 1) + (long)n * ldb];
           rb[j][u] = gk < K ? val : 0.0;
         }
@@ -750,14 +551,14 @@ __global__ __launch_bounds__(512, 4) void gemm64_kernel(GemmSide<double> p0, Gem
     }
     d2v a0[2], a1[2];
     {
-      const int r = wm * 64 + fr;
+      const int r = wm * HT + fr;
       a0[0] = *reinterpret_cast<const d2v*>(&As[cur][r * BK + 2 * g64_chunk(2 * fk, r)]);
       a0[1] = *reinterpret_cast<const d2v*>(&As[cur][r * BK + 2 * g64_chunk(2 * fk + 1, r)]);
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (i + 1 < 4) {
-        const int r = wm * 64 + (i + 1) * 16 + fr;
+    for (int i = 0; i < IB; ++i) {
+      if (i + 1 < IB) {
+        const int r = wm * HT + (i + 1) * 16 + fr;
         a1[0] = *reinterpret_cast<const d2v*>(&As[cur][r * BK + 2 * g64_chunk(2 * fk, r)]);
         a1[1] = *reinterpret_cast<const d2v*>(&As[cur][r * BK + 2 * g64_chunk(2 * fk + 1, r)]);
       }
@@ -767,7 +568,7 @@ __global__ __launch_bounds__(512, 4) void gemm64_kernel(GemmSide<double> p0, Gem
         for (int j = 0; j < 2; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bf[j][s2 >> 1][s2 & 1], a0[s2 >> 1][s2 & 1], acc[i][j],
                                                            0, 0, 0);
-      if (i + 1 < 4) { a0[0] = a1[0]; a0[1] = a1[1]; }
+      if (i + 1 < IB) { a0[0] = a1[0]; a0[1] = a1[1]; }
     }
   };
   // the last slice is peeled off, so that the loop body is one block without conditions
@@ -784,8 +585,8 @@ __global__ __launch_bounds__(512, 4) void gemm64_kernel(GemmSide<double> p0, Gem
   if (beta != 0.0 && m0 + BM <= M && n0 + BN <= N) {
     // interior tile accumulating into C: per 16-row block, the loads before the stores
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const long m = m0 + wm * 64 + i * 16 + (lane & 15);
+    for (int i = 0; i < IB; ++i) {
+      const long m = m0 + wm * HT + i * 16 + (lane & 15);
       double cv[2][4];
 #pragma unroll
       for (int j = 0; j < 2; ++j)
@@ -800,8 +601,8 @@ __global__ __launch_bounds__(512, 4) void gemm64_kernel(GemmSide<double> p0, Gem
     return;
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + wm * 64 + i * 16 + (lane & 15);
+  for (int i = 0; i < IB; ++i) {
+    const int m = m0 + wm * HT + i * 16 + (lane & 15);
     if (m >= M) continue;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -819,6 +620,130 @@ __global__ __launch_bounds__(512, 4) void gemm64_kernel(GemmSide<double> p0, Gem
   }
 }
 
+// C = alpha op(A) op(B) + beta C for products with few output tiles (M = 1 vectors, o x o and o x v
+// blocks, the (ov) x (ov) products of a small basis): a (16 IM) x (16 JN) tile per workgroup, whose NW
+// wavefronts share the contraction instead of the tile.  Wavefront w takes the 16-deep k-slabs w, w + NW,
+// ...: it loads their fragments from global memory straight into registers (nothing is shared between
+// wavefronts, so nothing is staged in LDS and the loop has no barrier), two slabs in flight, and the
+// NW partial tiles are added in a fixed order through LDS at the end.  Lane l supplies
+// k = 4 (l / 16) + s at MFMA step s, so a k-contiguous operand is read 4 consecutive k per lane and an
+// m-contiguous one in runs of 16 rows.  Rows past M or N load a clamped row and are not stored; the K
+// tail is a predicated slab after the full ones.
+template <typename T, bool TA, bool TB, int NW, int IM, int JN>
+__global__ __launch_bounds__(64 * NW) void gemm_direct_kernel(GemmSide<T> g, T alpha, T beta) {
+  constexpr int BM = 16 * IM, BN = 16 * JN;
+  typedef T t4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+  __shared__ T red[NW][BN * BM];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int M = g.M, N = g.N, K = (int)blockIdx.z == (int)gridDim.z - 1 ? g.Klast : g.K;
+  const long lda = g.lda, ldb = g.ldb;
+  const T* __restrict__ A = g.A + (long)blockIdx.z * g.sA;
+  const T* __restrict__ B = g.B + (long)blockIdx.z * g.sB;
+  T* __restrict__ C = g.C + (long)blockIdx.z * g.sC;
+  int tm, tn;
+  if (!tile_coords_bounded((int)blockIdx.x, (int)gridDim.x, g.tiles_m, g.tiles_n, tm, tn)) return;
+  const int m0 = tm * BM, n0 = tn * BN, fr = lane & 15, fk = lane >> 4;
+  const T *Ap[IM], *Bp[JN];
+#pragma unroll
+  for (int i = 0; i < IM; ++i) Ap[i] = A + (long)min(m0 + 16 * i + fr, M - 1) * (TA ? lda : 1L);
+#pragma unroll
+  for (int j = 0; j < JN; ++j) Bp[j] = B + (long)min(n0 + 16 * j + fr, N - 1) * (TB ? 1L : ldb);
+  T ra[2][IM][4], rb[2][JN][4];
+  auto load = [&](int slot, int s) {
+    const long k = 16L * s + 4 * fk;
+#pragma unroll
+    for (int i = 0; i < IM; ++i) {
+      if constexpr (TA) {
+        const t4 x = *reinterpret_cast<const t4*>(Ap[i] + k);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) ra[slot][i][u] = x[u];
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) ra[slot][i][u] = Ap[i][(k + u) * lda];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < JN; ++j) {
+      if constexpr (TB) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) rb[slot][j][u] = Bp[j][(k + u) * ldb];
+      } else {
+        const t4 x = *reinterpret_cast<const t4*>(Bp[j] + k);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) rb[slot][j][u] = x[u];
+      }
+    }
+  };
+  typename Mfma<T>::acc acc[IM][JN];
+#pragma unroll
+  for (int i = 0; i < IM; ++i)
+#pragma unroll
+    for (int j = 0; j < JN; ++j) acc[i][j] = typename Mfma<T>::acc{0, 0, 0, 0};
+  auto mma = [&](int slot) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int i = 0; i < IM; ++i)
+#pragma unroll
+        for (int j = 0; j < JN; ++j) acc[i][j] = Mfma<T>::op(rb[slot][j][u], ra[slot][i][u], acc[i][j]);
+  };
+  // this wavefront's full slabs: wave, wave + NW, ... below K / 16
+  const int full = K / 16, mine = full > wave ? (full - wave + NW - 1) / NW : 0;
+  if (mine > 0) load(0, wave);
+  int it = 0;
+  for (; it + 2 < mine; it += 2) {
+    load(1, wave + (it + 1) * NW);
+    mma(0);
+    load(0, wave + (it + 2) * NW);
+    mma(1);
+  }
+  if (mine - it == 2) {
+    load(1, wave + (it + 1) * NW);
+    mma(0);
+    mma(1);
+  } else if (mine - it == 1) {
+    mma(0);
+  }
+  if (K > 16 * full && full % NW == wave) {  // the K tail, zero-padded
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int gk = 16 * full + 4 * fk + u;
+      const long kc = min(gk, K - 1);
+#pragma unroll
+      for (int i = 0; i < IM; ++i) {
+        const T x = Ap[i][TA ? kc : kc * lda];
+        ra[0][i][u] = gk < K ? x : T(0);
+      }
+#pragma unroll
+      for (int j = 0; j < JN; ++j) {
+        const T x = Bp[j][TB ? kc * ldb : kc];
+        rb[0][j][u] = gk < K ? x : T(0);
+      }
+    }
+    mma(0);
+  }
+#pragma unroll
+  for (int i = 0; i < IM; ++i)
+#pragma unroll
+    for (int j = 0; j < JN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        red[wave][(16 * j + Mfma<T>::row(lane, r)) * BM + 16 * i + fr] = acc[i][j][r];
+  __syncthreads();
+  for (int e = tid; e < BM * BN; e += 64 * NW) {
+    T v = red[0][e];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) v += red[w][e];
+    const int m = m0 + e % BM, n = n0 + e / BM;
+    if (m < M && n < N) {
+      const long off = (long)m + (long)n * g.ldc;
+      v *= alpha;
+      if (beta != T(0)) v += beta * C[off];
+      C[off] = v;
+    }
+  }
+}
+
 template <typename T>
 __global__ void scale_kernel(T* C, long M, long N, long ldc, T beta) {
   const long total = M * N;
@@ -828,14 +753,24 @@ __global__ void scale_kernel(T* C, long M, long N, long ldc, T beta) {
   }
 }
 
-// C = beta*C + sum_s W[s] (fixed order), W[s] is M x N with leading dimension M.
+// C = beta*C + sum_s W[s] (fixed order), W[s] is M x N with leading dimension M.  Eight loads are in
+// flight per thread: with one element per thread and a few hundred partial products (a 20 x 20 result
+// of K = 200000) the sum is otherwise a chain of as many memory latencies.
 template <typename T>
-__global__ void splitk_reduce_kernel(const T* __restrict__ W, int S, long M, long N, T* __restrict__ C, long ldc,
-                                     T beta) {
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(const T* __restrict__ W, int S, long M, long N,
+                                                            T* __restrict__ C, long ldc, T beta) {
   const long total = M * N;
   for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < total; e += (long)gridDim.x * blockDim.x) {
     double acc = 0.0;
-    for (int q = 0; q < S; ++q) acc += (double)W[(long)q * total + e];
+    int q = 0;
+    for (; q + 8 <= S; q += 8) {
+      T w[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) w[u] = W[(long)(q + u) * total + e];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc += (double)w[u];
+    }
+    for (; q < S; ++q) acc += (double)W[(long)q * total + e];
     const long m = e % M, n = e / M;
     const long off = m + n * ldc;
     if (beta != T(0)) acc += (double)beta * (double)C[off];
@@ -1393,33 +1328,137 @@ __global__ __launch_bounds__(256, 4) void gemm32_tall_kernel(GemmSide<float> g, 
   }
 }
 
-static inline long tiles_m128(long x) { return (x + 127) / 128; }
+// ---------------------------------------------------------------------------
+// dispatch
+// ---------------------------------------------------------------------------
+// Kernel forms of one product.  TILE128 / TILE64: the LDS-staged kernels with 128x128 / 64x64 tiles;
+// SHORT / TALL: their 48 or 64 by 256 tiles for M <= 64 / N <= 64 (NN only); the DIRECT forms:
+// gemm_direct_kernel with 32x32, 32x16, 16x32 (four wavefronts) and 16x16 tiles (eight).
+enum GemmForm { TILE128, TILE64, SHORT, TALL, DIRECT22, DIRECT21, DIRECT12, DIRECT11, GEMM_FORMS };
 
-// Whether a product can run on the high-occupancy kernels: 128x128 tiles, at least one full
-// k-slice, and a tile's k-slice addressable with 32-bit byte offsets from one buffer base:
-// an m-contiguous A (n-contiguous B) spans 16 columns of lda (ldb); a k-contiguous B spans 128 rows of
-// ldb; in the TN / TT instantiations a k-contiguous A, and its k-contiguous B, span 64 rows of lda /
-// ldb from each of two bases.
+struct GemmPlan {
+  int form = DIRECT22;
+  long split = 1;   // chunks of the contraction, each a launch-z entry with its own partial product
+  double us = 1e300;
+};
+
+static inline long cdiv(long a, long b) { return (a + b - 1) / b; }
+
+static void form_tile(int form, long M, long N, long& bm, long& bn) {
+  switch (form) {
+    case TILE128: bm = bn = 128; break;
+    case TILE64: bm = bn = 64; break;
+    case SHORT: bm = M <= 48 ? 48 : 64; bn = 256; break;
+    case TALL: bm = 256; bn = N <= 48 ? 48 : 64; break;
+    case DIRECT22: bm = bn = 32; break;
+    case DIRECT21: bm = 32; bn = 16; break;
+    case DIRECT12: bm = 16; bn = 32; break;
+    default: bm = bn = 16; break;
+  }
+}
+
+// Whether a form takes the product.  The LDS-staged kernels address a tile's k-slice with 32-bit byte
+// offsets from one buffer base: an m-contiguous A (n-contiguous B) spans 16 columns of lda (ldb), a
+// k-contiguous operand the tile's rows of it (in the 128-row TN / TT instantiations 64 rows from each
+// of two bases).  The direct kernel addresses with 64 bits and takes everything.
 template <typename T>
-static bool occ_kernel_ok(bool ta, bool tb, long K, long lda, long ldb) {
-  if (K < 16) return false;
+static bool form_ok(int form, bool ta, bool tb, long M, long N, long K, long lda, long ldb) {
   const auto fits = [](long rows, long ld) { return (long)sizeof(T) * rows * (ld + 1) < (1L << 31); };
-  const bool a_ok = ta ? fits(64, lda) : fits(16, lda);
-  const bool b_ok = tb ? fits(16, ldb) : fits(ta ? 64 : 128, ldb);
-  return a_ok && b_ok;
+  switch (form) {
+    case TILE128:
+    case TILE64: {
+      const long rows = form == TILE128 && !ta ? 128 : 64;
+      return fits(ta ? rows : 16, lda) && fits(tb ? 16 : rows, ldb);
+    }
+    case SHORT: return M <= 64 && !ta && !tb && K % 16 == 0 && fits(256 + 64, std::max(lda, ldb));
+    case TALL: return N <= 64 && !ta && !tb && K % 16 == 0 && fits(16, lda) && fits(64, ldb);
+    default: return true;
+  }
+}
+
+// Estimated time (us) of `products` tiles-sets sharing one launch: tiles workgroups in all, each
+// walking `slabs` 16-deep k-slabs.  Per compute unit the larger of three times: the workgroups' k-loops one
+// after another at the kernel's reach of the MFMA rate (a 16x16 block of a slab is 0.107 us of one SIMD's
+// FP64 pipe, half that in FP32), one workgroup's own latency-bound loop, and for the direct kernel, whose
+// wavefronts share nothing, the cache traffic of its fragments; over the chip the traffic from HBM
+// (`bytes`).  The constants are fitted to measurements of all forms over 62 shapes (95^3 to 8640^2 x 768,
+// M = 1 vectors, 34 x 34 x 1227400, batches of 20 x 108 x 128; FP64 and FP32): the form picked is on
+// average 2% from the best measured one.
+template <typename T>
+static double form_us(int form, long tiles, long slabs, double bytes) {
+  const double f = sizeof(T) == 8 ? 1.0 : 0.5;
+  const double cu = (double)cdiv(tiles, 256);  // workgroups per compute unit
+  const double hbm = bytes / 5.6e6;
+  switch (form) {
+    case TILE128: return 8.5 + std::max(hbm, (slabs + 1) * std::max(f == 1.0 ? 2.5 : 1.4, cu * 1.71 * f / 0.86));
+    case TILE64: return 7.0 + std::max(hbm, (slabs + 1) * std::max(f == 1.0 ? 0.8 : 0.72, cu * 0.427 * f / 0.8));
+    case SHORT:
+    case TALL: return 8.0 + std::max(hbm, (slabs + 1) * std::max(1.6 * f, cu * 1.28 * f / 0.75));
+    default: {
+      const int nw = form == DIRECT11 ? 8 : 4, blocks = form == DIRECT22 ? 4 : form == DIRECT11 ? 1 : 2;
+      const int sides = form == DIRECT22 ? 4 : form == DIRECT11 ? 2 : 3;
+      const double L = (double)cdiv(slabs, nw), m = 0.107 * blocks * f;
+      const double resident = (form == DIRECT22 ? 3.0 : 4.0) * 4 / nw;
+      const double own = L * (0.2 + 0.025 * sides + m) * std::max(1.0, cu / resident);
+      const double mfma = cu * nw * L * m / 4 / 0.55;
+      const double cache = (double)tiles * nw * L * 256.0 * sides * sizeof(T) / 9.0e6;
+      return 3.0 + std::max(std::max(own, hbm), std::max(mfma, cache));
+    }
+  }
+}
+
+// time of adding S partial products of `elems` elements (splitk_reduce_kernel)
+template <typename T>
+static double reduce_us(long S, double elems) {
+  return S > 1 ? 2.0 + (S + 1) * elems * sizeof(T) / 4.5e6 + 0.18 * S : 0.0;
+}
+
+static const long kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128};
+
+// The form and split with the smallest estimated time.  A split product's partial results take at most
+// 256 MiB of workspace, 2 GiB when K >= 32768 (RCCSD's o^2 x v.m x v^2 products over (ia|bc)).
+template <typename T>
+static GemmPlan gemm_plan(bool ta, bool tb, long M, long N, long K, long lda, long ldb, long sA, long sB, int batch,
+                          bool allow_split) {
+  GemmPlan best;
+  const double bytes = (double)sizeof(T) * ((double)M * K * (sA || batch == 1 ? batch : 1) +
+                                            (double)N * K * (sB || batch == 1 ? batch : 1) + (double)M * N * batch);
+  const double room = K >= 32768 ? 2147483648.0 : 268435456.0;
+  for (int form = 0; form < GEMM_FORMS; ++form) {
+    // a transposed short A (the transform's orbital block) is transposed first for SHORT
+    const bool copy_a = form == SHORT && ta && !tb && lda == K && batch == 1 && allow_split;
+    if (!form_ok<T>(form, copy_a ? false : ta, tb, M, N, K, copy_a ? M : lda, ldb)) continue;
+    long bm, bn;
+    form_tile(form, M, N, bm, bn);
+    const long tiles = cdiv(M, bm) * cdiv(N, bn);
+    if (tiles >= (1L << 31)) continue;
+    for (const long s : kSplits) {
+      if (s > 1 && (!allow_split || batch > 1 || K < 64 * s || tiles * s > 8192 || form == SHORT || form == TALL ||
+                    (double)s * M * N * sizeof(T) > room))
+        break;
+      const long slabs = cdiv(cdiv(K, s), 16);
+      const double us = form_us<T>(form, tiles * s * batch, slabs, bytes) + reduce_us<T>(s, (double)M * N) +
+                        (copy_a ? 6.0 : 0.0);
+      if (us < best.us) best = GemmPlan{form, s, us};
+    }
+  }
+  return best;
 }
 
 template <typename T>
 static GemmSide<T> make_side(long M, long N, long K, const T* A, long lda, long sA, const T* B, long ldb, long sB,
-                             T* C, long ldc, long sC) {
-  return GemmSide<T>{A, B, C, lda, ldb, ldc, sA, sB, sC, (int)M, (int)N, (int)K, (int)tiles_m128(M),
-                     (int)tiles_m128(N), (int)K, nullptr, nullptr, 0};
+                             T* C, long ldc, long sC, int form = TILE128) {
+  long bm, bn;
+  form_tile(form, M, N, bm, bn);
+  return GemmSide<T>{A, B, C, lda, ldb, ldc, sA, sB, sC, (int)M, (int)N, (int)K, (int)cdiv(M, bm),
+                     (int)cdiv(N, bn), (int)K, nullptr, nullptr, 0};
 }
 
-// One launch of the high-occupancy kernel over p0 (and p1 when `two`), nb batch entries.
+// One launch of the LDS-staged kernel with 128x128 or 64x64 tiles over p0 (and p1 when `two`), nb batch
+// entries.  The ring and ladder symbols (kind 1 and 2) exist for the 128x128 NN kernels.
 template <typename T>
-static void occ_launch(jues_ctx* ctx, bool tb, int kind, GemmSide<T> p0, GemmSide<T> p1, bool two, int nb, T alpha,
-                       T beta, bool ta = false, bool seg = false) {
+static void tile_launch(jues_ctx* ctx, int form, bool tb, int kind, GemmSide<T> p0, GemmSide<T> p1, bool two, int nb,
+                        T alpha, T beta, bool ta = false, bool seg = false) {
   const long t0 = (long)p0.tiles_m * p0.tiles_n;
   const long nt0 = two ? (t0 + NXCD - 1) / NXCD * NXCD : t0;
   const long total = two ? nt0 + (long)p1.tiles_m * p1.tiles_n : t0;
@@ -1427,37 +1466,122 @@ static void occ_launch(jues_ctx* ctx, bool tb, int kind, GemmSide<T> p0, GemmSid
   if (!two) p1 = p0;
   const dim3 grid((unsigned)total, 1, nb);
   if constexpr (sizeof(T) == 4) {
-#define JUES_GEMM32(K_, TB_, TA_, SEG_)                                                                 \
-  hipLaunchKernelGGL((gemm32_nn_kernel<K_, TB_, TA_, SEG_>), grid, dim3(NT), 0, ctx->stream, p0, p1, (int)nt0, \
-                     (float)alpha, (float)beta)
-    if (seg) {
-      if (tb) JUES_GEMM32(0, true, false, true);
-      else JUES_GEMM32(0, false, false, true);
-    } else if (ta) {
-      if (tb) JUES_GEMM32(0, true, true, false);
-      else JUES_GEMM32(0, false, true, false);
-    } else if (tb) JUES_GEMM32(0, true, false, false);
-    else if (kind == 1) JUES_GEMM32(1, false, false, false);
-    else if (kind == 2) JUES_GEMM32(2, false, false, false);
-    else JUES_GEMM32(0, false, false, false);
+#define JUES_GEMM32(K_, TB_, TA_, SEG_, BT_)                                                                        \
+  hipLaunchKernelGGL((gemm32_nn_kernel<K_, TB_, TA_, SEG_, false, BT_>), grid, dim3(NT), 0, ctx->stream, p0, p1,    \
+                     (int)nt0, (float)alpha, (float)beta)
+#define JUES_GEMM32_SHAPES(BT_)                      \
+  if (seg) {                                         \
+    if (tb) JUES_GEMM32(0, true, false, true, BT_);  \
+    else JUES_GEMM32(0, false, false, true, BT_);    \
+  } else if (ta) {                                   \
+    if (tb) JUES_GEMM32(0, true, true, false, BT_);  \
+    else JUES_GEMM32(0, false, true, false, BT_);    \
+  } else if (tb) JUES_GEMM32(0, true, false, false, BT_)
+    if (form == TILE64) {
+      JUES_GEMM32_SHAPES(64);
+      else JUES_GEMM32(0, false, false, false, 64);
+    } else {
+      JUES_GEMM32_SHAPES(128);
+      else if (kind == 1) JUES_GEMM32(1, false, false, false, 128);
+      else if (kind == 2) JUES_GEMM32(2, false, false, false, 128);
+      else JUES_GEMM32(0, false, false, false, 128);
+    }
+#undef JUES_GEMM32_SHAPES
 #undef JUES_GEMM32
   } else {
-#define JUES_GEMM64(K_, TB_, TA_, SEG_)                                                               \
-  hipLaunchKernelGGL((gemm64_kernel<K_, TB_, TA_, SEG_>), grid, dim3(512), 0, ctx->stream, p0, p1, (int)nt0, \
+#define JUES_GEMM64(K_, TB_, TA_, SEG_, BT_)                                                                     \
+  hipLaunchKernelGGL((gemm64_kernel<K_, TB_, TA_, SEG_, BT_>), grid, dim3(4 * BT_), 0, ctx->stream, p0, p1, (int)nt0, \
                      (double)alpha, (double)beta)
-    if (seg) {
-      if (tb) JUES_GEMM64(0, true, false, true);
-      else JUES_GEMM64(0, false, false, true);
-    } else if (ta) {
-      if (tb) JUES_GEMM64(0, true, true, false);
-      else JUES_GEMM64(0, false, true, false);
-    } else if (tb) JUES_GEMM64(0, true, false, false);
-    else if (kind == 1) JUES_GEMM64(1, false, false, false);
-    else if (kind == 2) JUES_GEMM64(2, false, false, false);
-    else JUES_GEMM64(0, false, false, false);
+#define JUES_GEMM64_SHAPES(BT_)                      \
+  if (seg) {                                         \
+    if (tb) JUES_GEMM64(0, true, false, true, BT_);  \
+    else JUES_GEMM64(0, false, false, true, BT_);    \
+  } else if (ta) {                                   \
+    if (tb) JUES_GEMM64(0, true, true, false, BT_);  \
+    else JUES_GEMM64(0, false, true, false, BT_);    \
+  } else if (tb) JUES_GEMM64(0, true, false, false, BT_)
+    if (form == TILE64) {
+      JUES_GEMM64_SHAPES(64);
+      else JUES_GEMM64(0, false, false, false, 64);
+    } else {
+      JUES_GEMM64_SHAPES(128);
+      else if (kind == 1) JUES_GEMM64(1, false, false, false, 128);
+      else if (kind == 2) JUES_GEMM64(2, false, false, false, 128);
+      else JUES_GEMM64(0, false, false, false, 128);
+    }
+#undef JUES_GEMM64_SHAPES
 #undef JUES_GEMM64
   }
   JUES_HIP(hipGetLastError());
+}
+
+template <typename T>
+static void short_launch(jues_ctx* ctx, bool tall, GemmSide<T> p, int nb, T alpha, T beta) {
+  const dim3 grid((unsigned)((long)p.tiles_m * p.tiles_n), 1, nb);
+  const bool three = (tall ? p.N : p.M) <= 48;  // 16-row (16-column) blocks: 3 or 4
+#define JUES_SHORT(KERNEL_, THREADS_)                                                                      \
+  do {                                                                                                     \
+    if (three) hipLaunchKernelGGL(KERNEL_<3>, grid, dim3(THREADS_), 0, ctx->stream, p, alpha, beta);       \
+    else hipLaunchKernelGGL(KERNEL_<4>, grid, dim3(THREADS_), 0, ctx->stream, p, alpha, beta);             \
+  } while (0)
+  if constexpr (sizeof(T) == 4) {
+    if (tall) JUES_SHORT(gemm32_tall_kernel, 256);
+    else JUES_SHORT(gemm32_sk_kernel, 256);
+  } else {
+    if (tall) JUES_SHORT(gemm64_tall_kernel, 512);
+    else JUES_SHORT(gemm64_sk_kernel, 512);
+  }
+#undef JUES_SHORT
+  JUES_HIP(hipGetLastError());
+}
+
+template <typename T, bool TA, bool TB>
+static void direct_launch_ab(jues_ctx* ctx, int form, GemmSide<T> p, int nb, T alpha, T beta) {
+  const dim3 grid((unsigned)((long)p.tiles_m * p.tiles_n), 1, nb);
+#define JUES_DIRECT(NW_, IM_, JN_)                                                                            \
+  hipLaunchKernelGGL((gemm_direct_kernel<T, TA, TB, NW_, IM_, JN_>), grid, dim3(64 * NW_), 0, ctx->stream, p, \
+                     alpha, beta)
+  if (form == DIRECT22) JUES_DIRECT(4, 2, 2);
+  else if (form == DIRECT21) JUES_DIRECT(4, 2, 1);
+  else if (form == DIRECT12) JUES_DIRECT(4, 1, 2);
+  else JUES_DIRECT(8, 1, 1);
+#undef JUES_DIRECT
+  JUES_HIP(hipGetLastError());
+}
+
+// One launch of `form` over nb batch entries of p (made for that form).
+template <typename T>
+static void form_launch(jues_ctx* ctx, int form, bool ta, bool tb, int kind, const GemmSide<T>& p, int nb, T alpha,
+                        T beta) {
+  if (form == TILE128 || form == TILE64) tile_launch<T>(ctx, form, tb, kind, p, p, false, nb, alpha, beta, ta);
+  else if (form == SHORT || form == TALL) short_launch<T>(ctx, form == TALL, p, nb, alpha, beta);
+  else if (ta && tb) direct_launch_ab<T, true, true>(ctx, form, p, nb, alpha, beta);
+  else if (ta) direct_launch_ab<T, true, false>(ctx, form, p, nb, alpha, beta);
+  else if (tb) direct_launch_ab<T, false, true>(ctx, form, p, nb, alpha, beta);
+  else direct_launch_ab<T, false, false>(ctx, form, p, nb, alpha, beta);
+}
+
+template <typename T>
+static void reduce_launch(jues_ctx* ctx, const T* W, long S, long M, long N, T* C, long ldc, T beta) {
+  const unsigned nb = (unsigned)std::max(1L, std::min(cdiv(M * N, 256), 65536L));
+  hipLaunchKernelGGL((splitk_reduce_kernel<T>), dim3(nb), dim3(256), 0, ctx->stream, W, (int)S, M, N, C, ldc, beta);
+  JUES_HIP(hipGetLastError());
+}
+
+// Workspace for partial products, or null when the device has no room for it (the product then runs
+// unsplit, which needs none).
+template <typename T>
+static T* split_work(jues_ctx* ctx, int slot, size_t elems) {
+  try {
+    return static_cast<T*>(scratch(ctx, slot, sizeof(T) * elems));
+  } catch (const Error& e) {
+    if (e.st != JUES_OOM) throw;
+    return nullptr;
+  }
+}
+
+static int symbol_kind(const char* tag) {
+  return !tag ? 0 : (std::strcmp(tag, "cc_ring") == 0 ? 1 : (std::strcmp(tag, "cc_pp_ladder") == 0 ? 2 : 0));
 }
 
 template <typename T>
@@ -1470,7 +1594,7 @@ static void gemm_impl(jues_ctx* ctx, bool ta, bool tb, long M, long N, long K, T
   JUES_REQUIRE(lda >= (ta ? K : M) || K == 0, "gemm: lda too small");
   JUES_REQUIRE(ldb >= (tb ? N : K) || K == 0, "gemm: ldb too small");
   const char* name = tag ? tag : (sizeof(T) == 8 ? "gemm_f64" : "gemm_f32");
-  const int kind = !tag ? 0 : (std::strcmp(tag, "cc_ring") == 0 ? 1 : (std::strcmp(tag, "cc_pp_ladder") == 0 ? 2 : 0));
+  const int kind = symbol_kind(tag);
   if (K <= 0) {
     KTimer t(ctx, name, 0, 0);
     for (int b = 0; b < batch; ++b)
@@ -1479,208 +1603,41 @@ static void gemm_impl(jues_ctx* ctx, bool ta, bool tb, long M, long N, long K, T
     JUES_HIP(hipGetLastError());
     return;
   }
-  // tile shape: 0 = 128x128, 1 = 64x256 (skinny M), 2 = 256x64 (skinny N)
-  // (the ring and ladder kernel symbols, KIND 1 and 2, exist in the 128x128 shape only: a skinny
-  // product under those tags runs on the KIND 0 kernel of its shape)
-  // (a skinny product with K <= 128 is bound by streaming op(B) and C: the 128x128 kernel, whose
-  // extra MFMA work on the clamped rows costs nothing there, serves it)
-  // (a batched short product, M <= 64 with at least 1024 workgroups of 256 columns -- 256 when K is
-  // long -- such as the 40 x 216 blocks of the MP2 adjoint's second half-transform, takes the
-  // skinny-M tile too: its 16-row blocks waste less of the MFMA work than a 128-row tile)
-  const bool short_batched = M <= 64 && !ta && !tb && K > 128 && K % 16 == 0 && N >= 128 &&
-                             (long)batch * ((N + 255) / 256) >= (K >= 2048 ? 256 : 1024);
-  const int shape = (M <= 64 && N >= 8192 && (ta || K > 128)) || short_batched ? 1
-                    : (N <= 64 && M >= 8192 && (ta || K > 128)) ? 2
-                                                                 : 0;
-  const long BM = shape == 1 ? 64 : shape == 2 ? 256 : 128, BN = shape == 1 ? 256 : shape == 2 ? 64 : 128;
-  const long tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  JUES_REQUIRE(tiles_m * tiles_n < (1L << 31), "gemm: too many tiles");
-  // Few output tiles and a long K (the Fock-like terms): split K over workgroups,
-  // write partial products to a workspace and reduce them in a fixed order.  The chunks fill
-  // the chip's resident workgroup slots (four FP32 or two FP64 high-occupancy workgroups per CU).
-  // A long-K product whose tiles fill their last round of slots poorly (under 80% overall, such as
-  // the o^2 x v.m x v^2 products of RCCSD's (ia|bc) terms) is split into the fewest chunks that
-  // fill the rounds, when the partial products fit in 2 GiB.
-  const long slots = sizeof(T) == 4 ? 1024 : 512;
-  const long tiles = tiles_m * tiles_n;
-  auto round_fill = [&](long s) {
-    const long t = tiles * s;
-    return (double)t / (double)(((t + slots - 1) / slots) * slots);
-  };
-  long s_fill = 1;
-  if (allow_split && batch == 1 && shape == 0 && tiles >= 128 && K >= 32768 && !no_alloc_active() &&
-      round_fill(1) < 0.8) {
-    for (long s = 2; s <= 16; ++s)
-      if (round_fill(s) > round_fill(s_fill) + 0.02 && (double)s * M * N * sizeof(T) <= double(2L << 30)) s_fill = s;
+  const bool split_ok = allow_split && !no_alloc_active();
+  GemmPlan plan = gemm_plan<T>(ta, tb, M, N, K, lda, ldb, sA, sB, batch, split_ok);
+  if (plan.form == SHORT && ta) {
+    // the transposed copy of A that the SHORT form of a TN product reads
+    T* At = static_cast<T*>(scratch(ctx, 18, sizeof(T) * (size_t)(M * K)));
+    permute<T, T>(ctx, A, {K, M}, {1, 0}, At, 1.0, 0.0, name);
+    A = At;
+    lda = M;
+    ta = false;
   }
-  if (allow_split && batch == 1 && (tiles < 128 || s_fill > 1) && K >= 4096 && !no_alloc_active()) {
-    const long want = s_fill > 1 ? s_fill : std::max(2L, std::min(K / 1024, slots / tiles));
-    const int BKs = sizeof(T) == 8 ? 16 : 32;
-    long kc = (K + want - 1) / want;
-    kc = (kc + BKs - 1) / BKs * BKs;
-    const int S = (int)((K + kc - 1) / kc);
-    T* Wk = static_cast<T*>(scratch(ctx, 9, sizeof(T) * (size_t)S * M * N));
-    const long sa = ta ? kc : kc * lda, sb = tb ? kc * ldb : kc;
-    const long klast = K - (long)(S - 1) * kc;
-    if (shape == 0 && occ_kernel_ok<T>(ta, tb, std::min(kc, klast), lda, ldb)) {
-      // all chunks in one launch, the last one shorter
-      KTimer t1(ctx, name, 2.0 * M * N * K, (double)sizeof(T) * ((double)M * K + (double)K * N + (double)S * M * N));
-      GemmSide<T> p = make_side<T>(M, N, kc, A, lda, sa, B, ldb, sb, Wk, M, M * N);
-      p.Klast = (int)klast;
-      occ_launch<T>(ctx, tb, kind, p, p, false, S, alpha, T(0), ta);
-    } else {
-      if (S > 1)
-        gemm_impl<T>(ctx, ta, tb, M, N, kc, alpha, A, lda, sa, B, ldb, sb, T(0), Wk, M, M * N, S - 1, tag, false);
-      gemm_impl<T>(ctx, ta, tb, M, N, klast, alpha, A + (long)(S - 1) * sa, lda, 0, B + (long)(S - 1) * sb, ldb, 0,
-                   T(0), Wk + (long)(S - 1) * M * N, M, 0, 1, tag, false);
+  if (plan.split > 1) {
+    // chunks of K in one launch, the last one shorter; the partial products are added in a fixed order
+    const long kc = cdiv(cdiv(K, plan.split), 16) * 16, S = cdiv(K, kc);
+    T* Wk = S > 1 ? split_work<T>(ctx, 9, (size_t)S * M * N) : nullptr;
+    if (Wk) {
+      {
+        KTimer t1(ctx, name, 2.0 * M * N * K, (double)sizeof(T) * ((double)M * K + (double)K * N + (double)S * M * N));
+        GemmSide<T> p = make_side<T>(M, N, kc, A, lda, ta ? kc : kc * lda, B, ldb, tb ? kc * ldb : kc, Wk, M, M * N,
+                                     plan.form);
+        p.Klast = (int)(K - (S - 1) * kc);
+        form_launch<T>(ctx, plan.form, ta, tb, kind, p, (int)S, alpha, T(0));
+      }
+      KTimer t(ctx, name, 0.0, (double)sizeof(T) * S * M * N);
+      reduce_launch<T>(ctx, Wk, S, M, N, C, ldc, beta);
+      return;
     }
-    KTimer t(ctx, name, 0.0, (double)sizeof(T) * S * M * N);
-    const long tot = M * N;
-    const int nb = (int)std::max(1L, std::min((tot + 255) / 256, 65536L));
-    hipLaunchKernelGGL((splitk_reduce_kernel<T>), dim3(nb), dim3(256), 0, ctx->stream, Wk, S, M, N, C, ldc, beta);
-    JUES_HIP(hipGetLastError());
-    return;
+    plan = gemm_plan<T>(ta, tb, M, N, K, lda, ldb, sA, sB, batch, false);
   }
   const double flops = 2.0 * M * N * K * batch;
   const double bytes = (double)sizeof(T) * ((double)M * K + (double)K * N + (beta != T(0) ? 2.0 : 1.0) * M * N) * batch;
-  // Short, wide NN products (M <= 64): gemm32_sk_kernel / gemm64_sk_kernel, 64x256 tiles; a
-  // transposed A (at most 64 x K, the transform's orbital block) is transposed first
-  if (shape == 1 && ta && !tb && lda == K && batch == 1 && K % 16 == 0 && !no_alloc_active() &&
-      (long)sizeof(T) * (256 + 64) * (std::max(M, ldb) + 1) < (1L << 31)) {
-    T* At = static_cast<T*>(scratch(ctx, 18, sizeof(T) * (size_t)(M * K)));
-    permute<T, T>(ctx, A, {K, M}, {1, 0}, At, 1.0, 0.0, name);
-    gemm_impl<T>(ctx, false, tb, M, N, K, alpha, At, M, 0, B, ldb, sB, beta, C, ldc, sC, 1, tag, allow_split);
-    return;
-  }
-  if constexpr (sizeof(T) == 4) {
-    if (shape == 1 && !ta && !tb && K % 16 == 0 && 4L * (256 + 64) * (std::max(lda, ldb) + 1) < (1L << 31)) {
-      KTimer timer(ctx, name, flops, bytes);
-      for (int b0 = 0; b0 < batch; b0 += 65535) {
-        const int nb = std::min(batch - b0, 65535);
-        GemmSide<float> p = make_side<float>(M, N, K, reinterpret_cast<const float*>(A + (long)b0 * sA), lda, sA,
-                                             reinterpret_cast<const float*>(B + (long)b0 * sB), ldb, sB,
-                                             reinterpret_cast<float*>(C + (long)b0 * sC), ldc, sC);
-        const int bm = M <= 48 ? 48 : 64;  // 16-row blocks: 3 or 4
-        p.tiles_m = (int)((M + bm - 1) / bm);
-        p.tiles_n = (int)((N + 255) / 256);
-        const dim3 grid((unsigned)((long)p.tiles_m * p.tiles_n), 1, nb);
-        if (bm == 48)
-          hipLaunchKernelGGL(gemm32_sk_kernel<3>, grid, dim3(256), 0, ctx->stream, p, (float)alpha, (float)beta);
-        else
-          hipLaunchKernelGGL(gemm32_sk_kernel<4>, grid, dim3(256), 0, ctx->stream, p, (float)alpha, (float)beta);
-        JUES_HIP(hipGetLastError());
-      }
-      return;
-    }
-  }
-  if constexpr (sizeof(T) == 8) {
-    if (shape == 1 && !ta && !tb && K % 16 == 0 && 8L * (256 + 64) * (std::max(lda, ldb) + 1) < (1L << 31)) {
-      KTimer timer(ctx, name, flops, bytes);
-      for (int b0 = 0; b0 < batch; b0 += 65535) {
-        const int nb = std::min(batch - b0, 65535);
-        GemmSide<double> p = make_side<double>(M, N, K, reinterpret_cast<const double*>(A + (long)b0 * sA), lda, sA,
-                                               reinterpret_cast<const double*>(B + (long)b0 * sB), ldb, sB,
-                                               reinterpret_cast<double*>(C + (long)b0 * sC), ldc, sC);
-        const int bm = M <= 48 ? 48 : 64;  // 16-row blocks: 3 or 4
-        p.tiles_m = (int)((M + bm - 1) / bm);
-        p.tiles_n = (int)((N + 255) / 256);
-        const dim3 grid((unsigned)((long)p.tiles_m * p.tiles_n), 1, nb);
-        if (bm == 48)
-          hipLaunchKernelGGL(gemm64_sk_kernel<3>, grid, dim3(512), 0, ctx->stream, p, (double)alpha, (double)beta);
-        else
-          hipLaunchKernelGGL(gemm64_sk_kernel<4>, grid, dim3(512), 0, ctx->stream, p, (double)alpha, (double)beta);
-        JUES_HIP(hipGetLastError());
-      }
-      return;
-    }
-  }
-  // Tall, narrow NN products (N <= 64): gemm64_tall_kernel / gemm32_tall_kernel, 256x48 or 256x64
-  // tiles (a k-slice of A spans 16 lda, B's 64 rows 64 ldb, within 32-bit byte offsets)
-  if constexpr (sizeof(T) == 4) {
-    if (shape == 2 && !ta && !tb && K % 16 == 0 && 4L * 16 * (lda + 1) < (1L << 31) &&
-        4L * 64 * (ldb + 1) < (1L << 31)) {
-      KTimer timer(ctx, name, flops, bytes);
-      for (int b0 = 0; b0 < batch; b0 += 65535) {
-        const int nb = std::min(batch - b0, 65535);
-        GemmSide<float> p = make_side<float>(M, N, K, reinterpret_cast<const float*>(A + (long)b0 * sA), lda, sA,
-                                             reinterpret_cast<const float*>(B + (long)b0 * sB), ldb, sB,
-                                             reinterpret_cast<float*>(C + (long)b0 * sC), ldc, sC);
-        const int bn = N <= 48 ? 48 : 64;  // 16-column blocks: 3 or 4
-        p.tiles_m = (int)((M + 255) / 256);
-        p.tiles_n = (int)((N + bn - 1) / bn);
-        const dim3 grid((unsigned)((long)p.tiles_m * p.tiles_n), 1, nb);
-        if (bn == 48)
-          hipLaunchKernelGGL(gemm32_tall_kernel<3>, grid, dim3(256), 0, ctx->stream, p, (float)alpha, (float)beta);
-        else
-          hipLaunchKernelGGL(gemm32_tall_kernel<4>, grid, dim3(256), 0, ctx->stream, p, (float)alpha, (float)beta);
-        JUES_HIP(hipGetLastError());
-      }
-      return;
-    }
-  }
-  if constexpr (sizeof(T) == 8) {
-    if (shape == 2 && !ta && !tb && K % 16 == 0 && 8L * 16 * (lda + 1) < (1L << 31) &&
-        8L * 64 * (ldb + 1) < (1L << 31)) {
-      KTimer timer(ctx, name, flops, bytes);
-      for (int b0 = 0; b0 < batch; b0 += 65535) {
-        const int nb = std::min(batch - b0, 65535);
-        GemmSide<double> p = make_side<double>(M, N, K, reinterpret_cast<const double*>(A + (long)b0 * sA), lda, sA,
-                                               reinterpret_cast<const double*>(B + (long)b0 * sB), ldb, sB,
-                                               reinterpret_cast<double*>(C + (long)b0 * sC), ldc, sC);
-        const int bn = N <= 48 ? 48 : 64;  // 16-column blocks: 3 or 4
-        p.tiles_m = (int)((M + 255) / 256);
-        p.tiles_n = (int)((N + bn - 1) / bn);
-        const dim3 grid((unsigned)((long)p.tiles_m * p.tiles_n), 1, nb);
-        if (bn == 48)
-          hipLaunchKernelGGL(gemm64_tall_kernel<3>, grid, dim3(512), 0, ctx->stream, p, (double)alpha, (double)beta);
-        else
-          hipLaunchKernelGGL(gemm64_tall_kernel<4>, grid, dim3(512), 0, ctx->stream, p, (double)alpha, (double)beta);
-        JUES_HIP(hipGetLastError());
-      }
-      return;
-    }
-  }
-  // FP32 NN and NT: gemm32_nn_kernel (four workgroups per CU); FP64: gemm64_kernel (two
-  // 512-thread workgroups per CU)
-  if (shape == 0 && occ_kernel_ok<T>(ta, tb, K, lda, ldb)) {
-    KTimer timer(ctx, name, flops, bytes);
-    for (int b0 = 0; b0 < batch; b0 += 65535) {
-      const int nb = std::min(batch - b0, 65535);
-      const GemmSide<T> p = make_side<T>(M, N, K, A + (long)b0 * sA, lda, sA, B + (long)b0 * sB, ldb, sB,
-                                         C + (long)b0 * sC, ldc, sC);
-      occ_launch<T>(ctx, tb, kind, p, p, false, nb, alpha, beta, ta);
-    }
-    return;
-  }
   KTimer timer(ctx, name, flops, bytes);
-  // the buffer-load path addresses a tile's k-slice with 32-bit byte offsets
-  const long span = (long)sizeof(T) * (std::max<long>(BM, BN) + 64) * (std::max(lda, ldb) + 1);
-  const int fast_ok = span < (1L << 31) ? 1 : 0;
   for (int b0 = 0; b0 < batch; b0 += 65535) {
-    const int nb = std::min(batch - b0, 65535);
-    dim3 grid((unsigned)(tiles_m * tiles_n), 1, nb);
-    const T* Ab = A + (long)b0 * sA;
-    const T* Bb = B + (long)b0 * sB;
-    T* Cb = C + (long)b0 * sC;
-#define JUES_GEMM_LAUNCH_S(TA_, TB_, K_, BM_, BN_, WM_)                                                  \
-  hipLaunchKernelGGL((gemm_kernel<T, TA_, TB_, K_, BM_, BN_, WM_>), grid, dim3(NT), 0, ctx->stream, (int)M, (int)N, \
-                     (int)K, alpha, Ab, lda, sA, Bb, ldb, sB, beta, Cb, ldc, sC, (int)tiles_m, (int)tiles_n, fast_ok)
-#define JUES_GEMM_LAUNCH(TA_, TB_, K_)                                          \
-  do {                                                                          \
-    if (shape == 1) JUES_GEMM_LAUNCH_S(TA_, TB_, K_, 64, 256, 1);               \
-    else if (shape == 2) JUES_GEMM_LAUNCH_S(TA_, TB_, K_, 256, 64, 4);          \
-    else JUES_GEMM_LAUNCH_S(TA_, TB_, K_, 128, 128, 2);                         \
-  } while (0)
-    if (!ta && !tb) {
-      if (kind == 1 && shape == 0) JUES_GEMM_LAUNCH_S(false, false, 1, 128, 128, 2);
-      else if (kind == 2 && shape == 0) JUES_GEMM_LAUNCH_S(false, false, 2, 128, 128, 2);
-      else JUES_GEMM_LAUNCH(false, false, 0);
-    } else if (!ta && tb) JUES_GEMM_LAUNCH(false, true, 0);
-    else if (ta && !tb) JUES_GEMM_LAUNCH(true, false, 0);
-    else JUES_GEMM_LAUNCH(true, true, 0);
-#undef JUES_GEMM_LAUNCH
-#undef JUES_GEMM_LAUNCH_S
-    JUES_HIP(hipGetLastError());
+    const GemmSide<T> p = make_side<T>(M, N, K, A + (long)b0 * sA, lda, sA, B + (long)b0 * sB, ldb, sB,
+                                       C + (long)b0 * sC, ldc, sC, plan.form);
+    form_launch<T>(ctx, plan.form, ta, tb, kind, p, std::min(batch - b0, 65535), alpha, beta);
   }
 }
 
@@ -1692,7 +1649,7 @@ void gemm(jues_ctx* ctx, bool ta, bool tb, long M, long N, long K, T alpha, cons
 
 bool gemm32_out64(jues_ctx* ctx, long M, long N, long K, const float* A, long lda, const float* B, long ldb,
                   double* C, long ldc, const char* tag) {
-  if (M <= 0 || N <= 0 || K <= 0 || !occ_kernel_ok<float>(false, false, K, lda, ldb)) return false;
+  if (M <= 0 || N <= 0 || K < 16 || !form_ok<float>(TILE128, false, false, M, N, K, lda, ldb)) return false;
   JUES_REQUIRE(lda >= M && ldb >= K && ldc >= M, "gemm32_out64: leading dimension too small");
   GemmSide<float> p = make_side<float>(M, N, K, A, lda, 0, B, ldb, 0, nullptr, ldc, 0);
   p.C64 = C;
@@ -1712,21 +1669,46 @@ void gemm_batch_sum(jues_ctx* ctx, bool ta, bool tb, long M, long N, long K, T a
   const char* name = tag ? tag : (sizeof(T) == 8 ? "gemm_f64" : "gemm_f32");
   gemm_impl<T>(ctx, ta, tb, M, N, K, alpha, A, lda, sA, B, ldb, sB, T(0), work, M, M * N, batch, tag, false);
   KTimer t(ctx, name, 0.0, (double)sizeof(T) * ((double)batch + (beta != T(0) ? 2.0 : 1.0)) * M * N);
-  const long tot = M * N;
-  hipLaunchKernelGGL((splitk_reduce_kernel<T>), dim3((unsigned)std::max(1L, std::min((tot + 255) / 256, 65536L))),
-                     dim3(256), 0, ctx->stream, work, batch, M, N, C, ldc, beta);
-  JUES_HIP(hipGetLastError());
+  reduce_launch<T>(ctx, work, batch, M, N, C, ldc, beta);
 }
 
 template <typename T>
 void gemm_pair(jues_ctx* ctx, bool tb, long M0, long N0, long K0, const T* A0, long lda0, const T* B0, long ldb0,
                T* C0, long ldc0, long M1, long N1, long K1, const T* A1, long lda1, const T* B1, long ldb1, T* C1,
                long ldc1, T alpha, T beta, const char* tag) {
-  const bool skinny0 = (M0 <= 64 && N0 >= 8192) || (N0 <= 64 && M0 >= 8192);
-  const bool skinny1 = (M1 <= 64 && N1 >= 8192) || (N1 <= 64 && M1 >= 8192);
   const bool empty0 = M0 <= 0 || N0 <= 0, empty1 = M1 <= 0 || N1 <= 0;
-  if (empty0 || empty1 || skinny0 || skinny1 || !occ_kernel_ok<T>(false, tb, K0, lda0, ldb0) ||
-      !occ_kernel_ok<T>(false, tb, K1, lda1, ldb1)) {
+  // One launch of 64x64 or 128x128 tiles, its contractions split over S chunks, against two planned
+  // products, by the same estimate.
+  GemmPlan best;
+  if (!empty0 && !empty1 && K0 >= 16 && K1 >= 16) {
+    const double bytes = (double)sizeof(T) * ((double)M0 * K0 + (double)K0 * N0 + (double)M0 * N0 + (double)M1 * K1 +
+                                              (double)K1 * N1 + (double)M1 * N1);
+    for (const int form : {(int)TILE128, (int)TILE64}) {
+      if (!form_ok<T>(form, false, tb, M0, N0, K0, lda0, ldb0) || !form_ok<T>(form, false, tb, M1, N1, K1, lda1, ldb1))
+        continue;
+      const long bt = form == TILE128 ? 128 : 64;
+      const long tiles = cdiv(M0, bt) * cdiv(N0, bt) + cdiv(M1, bt) * cdiv(N1, bt);
+      const double elems = (double)M0 * N0 + (double)M1 * N1;
+      for (const long s : kSplits) {
+        if (s > 1 && (no_alloc_active() || s > 16 || std::min(K0, K1) < 64 * s || tiles * s > 8192 ||
+                      (double)s * elems * sizeof(T) > 268435456.0))
+          break;
+        const double us = form_us<T>(form, tiles * s, cdiv(cdiv(std::max(K0, K1), s), 16), bytes) +
+                          (s > 1 ? 2.0 : 0.0) + reduce_us<T>(s, elems);
+        if (us < best.us) best = GemmPlan{form, s, us};
+      }
+    }
+    const double apart = gemm_plan<T>(false, tb, M0, N0, K0, lda0, ldb0, 0, 0, 1, !no_alloc_active()).us +
+                         gemm_plan<T>(false, tb, M1, N1, K1, lda1, ldb1, 0, 0, 1, !no_alloc_active()).us;
+    if (apart <= best.us) best.us = 1e300;
+  }
+  T* Wk = nullptr;
+  long S = best.split;
+  if (best.us < 1e300 && S > 1) {
+    Wk = split_work<T>(ctx, 16, (size_t)S * (M0 * N0 + M1 * N1));
+    if (!Wk) best.us = 1e300;
+  }
+  if (best.us >= 1e300) {
     gemm<T>(ctx, false, tb, M0, N0, K0, alpha, A0, lda0, 0, B0, ldb0, 0, beta, C0, ldc0, 0, 1, tag);
     gemm<T>(ctx, false, tb, M1, N1, K1, alpha, A1, lda1, 0, B1, ldb1, 0, beta, C1, ldc1, 0, 1, tag);
     return;
@@ -1738,67 +1720,71 @@ void gemm_pair(jues_ctx* ctx, bool tb, long M0, long N0, long K0, const T* A0, l
   JUES_REQUIRE(lda0 >= M0 && lda1 >= M1, "gemm: lda too small");
   JUES_REQUIRE(ldb0 >= (tb ? N0 : K0) && ldb1 >= (tb ? N1 : K1), "gemm: ldb too small");
   const char* name = tag ? tag : (sizeof(T) == 8 ? "gemm_f64" : "gemm_f32");
-  const int kind = !tag ? 0 : (std::strcmp(tag, "cc_ring") == 0 ? 1 : (std::strcmp(tag, "cc_pp_ladder") == 0 ? 2 : 0));
+  const int kind = symbol_kind(tag);
   const double sz = sizeof(T), bf = beta != T(0) ? 2.0 : 1.0;
   const double flops = 2.0 * M0 * N0 * K0 + 2.0 * M1 * N1 * K1;
-  GemmSide<T> p0 = make_side<T>(M0, N0, K0, A0, lda0, 0, B0, ldb0, 0, C0, ldc0, 0);
-  GemmSide<T> p1 = make_side<T>(M1, N1, K1, A1, lda1, 0, B1, ldb1, 0, C1, ldc1, 0);
-  // Fewer tiles than about two rounds of resident workgroups (1024 FP32, 512 FP64) and long
-  // K: split both K ranges into S chunks (one launch; the last chunk of each shorter), write
-  // the partial products to a workspace and add them to C0 / C1 in a fixed order.
-  const long tiles = (long)p0.tiles_m * p0.tiles_n + (long)p1.tiles_m * p1.tiles_n;
-  const long slots = sizeof(T) == 4 ? 1024 : 512;
-  const long S = std::min(std::min(K0, K1) / 1024, (2 * slots + tiles - 1) / tiles);
-  if (tiles < slots && S >= 2) {
-    const long kc0 = (K0 + S - 1) / S, kc1 = (K1 + S - 1) / S;
-    const long n0 = M0 * N0, n1 = M1 * N1;
-    T* Wk = static_cast<T*>(scratch(ctx, 16, sizeof(T) * (size_t)S * (n0 + n1)));
+  const long n0 = M0 * N0, n1 = M1 * N1;
+  const double in = sz * ((double)M0 * K0 + (double)K0 * N0 + (double)M1 * K1 + (double)K1 * N1);
+  if (Wk) {
+    // both K ranges in S chunks (the last chunk of each shorter): the partial products go to the
+    // workspace and are added to C0 / C1 in a fixed order
+    const long kc0 = cdiv(K0, S), kc1 = cdiv(K1, S);
     {
-      KTimer timer(ctx, name, flops, sz * ((double)M0 * K0 + (double)K0 * N0 + (double)M1 * K1 + (double)K1 * N1 +
-                                           (double)S * (n0 + n1)));
-      p0 = make_side<T>(M0, N0, kc0, A0, lda0, kc0 * lda0, B0, ldb0, tb ? kc0 * ldb0 : kc0, Wk, M0, n0);
-      p1 = make_side<T>(M1, N1, kc1, A1, lda1, kc1 * lda1, B1, ldb1, tb ? kc1 * ldb1 : kc1, Wk + S * n0, M1, n1);
+      KTimer timer(ctx, name, flops, in + sz * S * (n0 + n1));
+      GemmSide<T> p0 = make_side<T>(M0, N0, kc0, A0, lda0, kc0 * lda0, B0, ldb0, tb ? kc0 * ldb0 : kc0, Wk, M0, n0,
+                                    best.form);
+      GemmSide<T> p1 = make_side<T>(M1, N1, kc1, A1, lda1, kc1 * lda1, B1, ldb1, tb ? kc1 * ldb1 : kc1, Wk + S * n0,
+                                    M1, n1, best.form);
       p0.Klast = (int)(K0 - (S - 1) * kc0);
       p1.Klast = (int)(K1 - (S - 1) * kc1);
-      occ_launch<T>(ctx, tb, kind, p0, p1, true, (int)S, alpha, T(0));
+      tile_launch<T>(ctx, best.form, tb, kind, p0, p1, true, (int)S, alpha, T(0));
     }
     KTimer t(ctx, name, 0.0, sz * (S + bf) * (n0 + n1));
-    hipLaunchKernelGGL((splitk_reduce_kernel<T>), dim3((unsigned)std::min((n0 + 255) / 256, 65536L)), dim3(256), 0,
-                       ctx->stream, Wk, (int)S, M0, N0, C0, ldc0, beta);
-    hipLaunchKernelGGL((splitk_reduce_kernel<T>), dim3((unsigned)std::min((n1 + 255) / 256, 65536L)), dim3(256), 0,
-                       ctx->stream, Wk + S * n0, (int)S, M1, N1, C1, ldc1, beta);
-    JUES_HIP(hipGetLastError());
+    reduce_launch<T>(ctx, Wk, S, M0, N0, C0, ldc0, beta);
+    reduce_launch<T>(ctx, Wk + S * n0, S, M1, N1, C1, ldc1, beta);
     return;
   }
-  const double bytes = sz * ((double)M0 * K0 + (double)K0 * N0 + bf * M0 * N0 + (double)M1 * K1 + (double)K1 * N1 +
-                             bf * M1 * N1);
-  KTimer timer(ctx, name, flops, bytes);
-  occ_launch<T>(ctx, tb, kind, p0, p1, true, 1, alpha, beta);
+  KTimer timer(ctx, name, flops, in + sz * bf * (n0 + n1));
+  tile_launch<T>(ctx, best.form, tb, kind,
+                 make_side<T>(M0, N0, K0, A0, lda0, 0, B0, ldb0, 0, C0, ldc0, 0, best.form),
+                 make_side<T>(M1, N1, K1, A1, lda1, 0, B1, ldb1, 0, C1, ldc1, 0, best.form), true, 1, alpha, beta);
 }
 
 template <typename T>
 void gemm_ksum(jues_ctx* ctx, bool tb, long M, long N, long K0, const T* A0, const T* B0, long K1, const T* A1,
                const T* B1, long lda, long ldb, long sA, long sB, T alpha, T beta, T* C, long ldc, long sC, int batch,
                const char* tag) {
-  const bool skinny = (M <= 64 && N >= 8192) || (N <= 64 && M >= 8192);
   if (M <= 0 || N <= 0 || batch <= 0) return;
-  if (skinny || K0 < 16 || K1 < 16 || K0 % 16 != 0 || K1 % 16 != 0 || batch > 65535 ||
-      !occ_kernel_ok<T>(false, tb, std::max(K0, K1), lda, ldb)) {
+  const long Kmax = std::max(K0, K1);
+  GemmPlan best;
+  if (K0 >= 16 && K1 >= 16 && K0 % 16 == 0 && K1 % 16 == 0 && batch <= 65535) {
+    const double bytes = (double)sizeof(T) * batch * ((double)M * (K0 + K1) + (double)N * (K0 + K1) + (double)M * N);
+    for (const int form : {(int)TILE128, (int)TILE64}) {
+      if (!form_ok<T>(form, false, tb, M, N, Kmax, lda, ldb)) continue;
+      const long bt = form == TILE128 ? 128 : 64;
+      const double us = form_us<T>(form, cdiv(M, bt) * cdiv(N, bt) * batch, (K0 + K1) / 16, bytes);
+      if (us < best.us) best = GemmPlan{form, 1, us};
+    }
+    const double apart = gemm_plan<T>(false, tb, M, N, K0, lda, ldb, sA, sB, batch, false).us +
+                         gemm_plan<T>(false, tb, M, N, K1, lda, ldb, sA, sB, batch, false).us;
+    if (apart <= best.us) best.us = 1e300;
+  }
+  if (best.us >= 1e300) {
     gemm<T>(ctx, false, tb, M, N, K0, alpha, A0, lda, sA, B0, ldb, sB, beta, C, ldc, sC, batch, tag);
     gemm<T>(ctx, false, tb, M, N, K1, alpha, A1, lda, sA, B1, ldb, sB, T(1), C, ldc, sC, batch, tag);
     return;
   }
   JUES_REQUIRE(M < (1L << 31) && N < (1L << 31) && K0 + K1 < (1L << 31), "gemm: dimension too large");
-  JUES_REQUIRE(ldc >= M && lda >= M && ldb >= (tb ? N : std::max(K0, K1)), "gemm: leading dimension too small");
+  JUES_REQUIRE(ldc >= M && lda >= M && ldb >= (tb ? N : Kmax), "gemm: leading dimension too small");
   const char* name = tag ? tag : (sizeof(T) == 8 ? "gemm_f64" : "gemm_f32");
   const double K = (double)(K0 + K1);
   KTimer timer(ctx, name, 2.0 * M * N * K * batch,
                (double)sizeof(T) * ((double)M * K + K * N + (beta != T(0) ? 2.0 : 1.0) * M * N) * batch);
-  GemmSide<T> p = make_side<T>(M, N, K0, A0, lda, sA, B0, ldb, sB, C, ldc, sC);
+  GemmSide<T> p = make_side<T>(M, N, K0, A0, lda, sA, B0, ldb, sB, C, ldc, sC, best.form);
   p.A1 = A1;
   p.B1 = B1;
   p.K1 = (int)K1;
-  occ_launch<T>(ctx, tb, 0, p, p, false, batch, alpha, beta, false, true);
+  tile_launch<T>(ctx, best.form, tb, 0, p, p, false, batch, alpha, beta, false, true);
 }
 
 template void gemm_ksum<double>(jues_ctx*, bool, long, long, long, const double*, const double*, long, const double*,
