@@ -93,6 +93,11 @@ struct GemmSide {
   const T* A1;
   const T* B1;
   int K1;
+  // SEG launches: batch entry z is entry z % inner of group z / inner, whose operands A, B, A1, B1 are offset
+  // by tab[4 group + 0..3] elements and whose C by group * sG
+  const long* tab = nullptr;
+  int inner = 1;
+  long sG = 0;
   // FP32 products that write an FP64 result (the OUT64 instantiation; C is not used there)
   double* C64 = nullptr;
 };
@@ -134,13 +139,16 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
   const GemmSide<float> g = second ? p1 : p0;
   const int M = g.M, N = g.N, K = (int)blockIdx.z == (int)gridDim.z - 1 ? g.Klast : g.K;
   const long lda = g.lda, ldb = g.ldb, ldc = g.ldc;
-  const float* __restrict__ A = g.A + (long)blockIdx.z * g.sA;
-  const float* __restrict__ B = g.B + (long)blockIdx.z * g.sB;
-  float* __restrict__ C = OUT64 ? nullptr : g.C + (long)blockIdx.z * g.sC;
+  const int grp = SEG ? (int)blockIdx.z / g.inner : 0;  // the table only in the SEG instantiations
+  const long zb = (long)blockIdx.z - (SEG ? (long)grp * g.inner : 0L);
+  const long* tab = SEG ? g.tab + 4L * grp : nullptr;
+  const float* __restrict__ A = g.A + zb * g.sA + (SEG ? tab[0] : 0L);
+  const float* __restrict__ B = g.B + zb * g.sB + (SEG ? tab[1] : 0L);
+  float* __restrict__ C = OUT64 ? nullptr : g.C + zb * g.sC + (SEG ? grp * g.sG : 0L);
   // a second contraction segment (A1, B1 over K1 columns) only in the SEG instantiations
   const int K1 = SEG ? g.K1 : 0;
-  const float* A1 = K1 > 0 ? g.A1 + (long)blockIdx.z * g.sA : A;
-  const float* B1 = K1 > 0 ? g.B1 + (long)blockIdx.z * g.sB : B;
+  const float* A1 = SEG ? g.A1 + zb * g.sA + tab[2] : A;
+  const float* B1 = SEG ? g.B1 + zb * g.sB + tab[3] : B;
   int tm, tn;
   if (!tile_coords_bounded(second ? (int)blockIdx.x - nt0 : (int)blockIdx.x, second ? (int)gridDim.x - nt0 : nt0,
                            g.tiles_m, g.tiles_n, tm, tn))
@@ -401,13 +409,16 @@ __global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, 
   const GemmSide<double> g = second ? p1 : p0;
   const int M = g.M, N = g.N, K = (int)blockIdx.z == (int)gridDim.z - 1 ? g.Klast : g.K;
   const long lda = g.lda, ldb = g.ldb, ldc = g.ldc;
-  const double* __restrict__ A = g.A + (long)blockIdx.z * g.sA;
-  const double* __restrict__ B = g.B + (long)blockIdx.z * g.sB;
-  double* __restrict__ C = g.C + (long)blockIdx.z * g.sC;
+  const int grp = SEG ? (int)blockIdx.z / g.inner : 0;  // the table only in the SEG instantiations
+  const long zb = (long)blockIdx.z - (SEG ? (long)grp * g.inner : 0L);
+  const long* tab = SEG ? g.tab + 4L * grp : nullptr;
+  const double* __restrict__ A = g.A + zb * g.sA + (SEG ? tab[0] : 0L);
+  const double* __restrict__ B = g.B + zb * g.sB + (SEG ? tab[1] : 0L);
+  double* __restrict__ C = g.C + zb * g.sC + (SEG ? grp * g.sG : 0L);
   // a second contraction segment (A1, B1 over K1 columns) only in the SEG instantiations
   const int K1 = SEG ? g.K1 : 0;
-  const double* A1 = K1 > 0 ? g.A1 + (long)blockIdx.z * g.sA : A;
-  const double* B1 = K1 > 0 ? g.B1 + (long)blockIdx.z * g.sB : B;
+  const double* A1 = SEG ? g.A1 + zb * g.sA + tab[2] : A;
+  const double* B1 = SEG ? g.B1 + zb * g.sB + tab[3] : B;
   int tm, tn;
   if (!tile_coords_bounded(second ? (int)blockIdx.x - nt0 : (int)blockIdx.x, second ? (int)gridDim.x - nt0 : nt0,
                            g.tiles_m, g.tiles_n, tm, tn))
@@ -1751,48 +1762,41 @@ void gemm_pair(jues_ctx* ctx, bool tb, long M0, long N0, long K0, const T* A0, l
 }
 
 template <typename T>
-void gemm_ksum(jues_ctx* ctx, bool tb, long M, long N, long K0, const T* A0, const T* B0, long K1, const T* A1,
-               const T* B1, long lda, long ldb, long sA, long sB, T alpha, T beta, T* C, long ldc, long sC, int batch,
-               const char* tag) {
-  if (M <= 0 || N <= 0 || batch <= 0) return;
-  const long Kmax = std::max(K0, K1);
+void gemm_ksum(jues_ctx* ctx, bool tb, long M, long N, long K, const T* A0, const T* B0, const T* A1, const T* B1,
+               const long* tab, int groups, int inner, long lda, long ldb, long sA, long sB, T alpha, T beta, T* C,
+               long ldc, long sC, long sG, const char* tag) {
+  if (M <= 0 || N <= 0 || groups <= 0 || inner <= 0) return;
+  JUES_REQUIRE(M < (1L << 31) && N < (1L << 31) && 2 * K < (1L << 31), "gemm: dimension too large");
+  JUES_REQUIRE(K >= 16 && K % 16 == 0 && (long)groups * inner <= 65535, "gemm_ksum: bad contraction or batch");
+  JUES_REQUIRE(ldc >= M && lda >= M && ldb >= (tb ? N : K), "gemm: leading dimension too small");
+  const long batch = (long)groups * inner;
+  const double bytes = (double)sizeof(T) * batch * (2.0 * M * K + 2.0 * N * K + (beta != T(0) ? 2.0 : 1.0) * M * N);
   GemmPlan best;
-  if (K0 >= 16 && K1 >= 16 && K0 % 16 == 0 && K1 % 16 == 0 && batch <= 65535) {
-    const double bytes = (double)sizeof(T) * batch * ((double)M * (K0 + K1) + (double)N * (K0 + K1) + (double)M * N);
-    for (const int form : {(int)TILE128, (int)TILE64}) {
-      if (!form_ok<T>(form, false, tb, M, N, Kmax, lda, ldb)) continue;
-      const long bt = form == TILE128 ? 128 : 64;
-      const double us = form_us<T>(form, cdiv(M, bt) * cdiv(N, bt) * batch, (K0 + K1) / 16, bytes);
-      if (us < best.us) best = GemmPlan{form, 1, us};
-    }
-    const double apart = gemm_plan<T>(false, tb, M, N, K0, lda, ldb, sA, sB, batch, false).us +
-                         gemm_plan<T>(false, tb, M, N, K1, lda, ldb, sA, sB, batch, false).us;
-    if (apart <= best.us) best.us = 1e300;
+  for (const int form : {(int)TILE128, (int)TILE64}) {
+    if (!form_ok<T>(form, false, tb, M, N, K, lda, ldb)) continue;
+    const long bt = form == TILE128 ? 128 : 64;
+    const double us = form_us<T>(form, cdiv(M, bt) * cdiv(N, bt) * batch, 2 * K / 16, 0.0);
+    if (us < best.us) best = GemmPlan{form, 1, us};
   }
-  if (best.us >= 1e300) {
-    gemm<T>(ctx, false, tb, M, N, K0, alpha, A0, lda, sA, B0, ldb, sB, beta, C, ldc, sC, batch, tag);
-    gemm<T>(ctx, false, tb, M, N, K1, alpha, A1, lda, sA, B1, ldb, sB, T(1), C, ldc, sC, batch, tag);
-    return;
-  }
-  JUES_REQUIRE(M < (1L << 31) && N < (1L << 31) && K0 + K1 < (1L << 31), "gemm: dimension too large");
-  JUES_REQUIRE(ldc >= M && lda >= M && ldb >= (tb ? N : Kmax), "gemm: leading dimension too small");
+  JUES_REQUIRE(best.us < 1e300, "gemm_ksum: leading dimension too large");
   const char* name = tag ? tag : (sizeof(T) == 8 ? "gemm_f64" : "gemm_f32");
-  const double K = (double)(K0 + K1);
-  KTimer timer(ctx, name, 2.0 * M * N * K * batch,
-               (double)sizeof(T) * ((double)M * K + K * N + (beta != T(0) ? 2.0 : 1.0) * M * N) * batch);
-  GemmSide<T> p = make_side<T>(M, N, K0, A0, lda, sA, B0, ldb, sB, C, ldc, sC, best.form);
+  KTimer timer(ctx, name, 4.0 * M * N * K * batch, bytes);
+  GemmSide<T> p = make_side<T>(M, N, K, A0, lda, sA, B0, ldb, sB, C, ldc, sC, best.form);
   p.A1 = A1;
   p.B1 = B1;
-  p.K1 = (int)K1;
-  tile_launch<T>(ctx, best.form, tb, 0, p, p, false, batch, alpha, beta, false, true);
+  p.K1 = (int)K;
+  p.tab = tab;
+  p.inner = inner;
+  p.sG = sG;
+  tile_launch<T>(ctx, best.form, tb, 0, p, p, false, (int)batch, alpha, beta, false, true);
 }
 
-template void gemm_ksum<double>(jues_ctx*, bool, long, long, long, const double*, const double*, long, const double*,
-                                const double*, long, long, long, long, double, double, double*, long, long, int,
-                                const char*);
-template void gemm_ksum<float>(jues_ctx*, bool, long, long, long, const float*, const float*, long, const float*,
-                               const float*, long, long, long, long, float, float, float*, long, long, int,
-                               const char*);
+template void gemm_ksum<double>(jues_ctx*, bool, long, long, long, const double*, const double*, const double*,
+                                const double*, const long*, int, int, long, long, long, long, double, double, double*,
+                                long, long, long, const char*);
+template void gemm_ksum<float>(jues_ctx*, bool, long, long, long, const float*, const float*, const float*,
+                               const float*, const long*, int, int, long, long, long, long, float, float, float*, long,
+                               long, long, const char*);
 
 template void gemm_pair<double>(jues_ctx*, bool, long, long, long, const double*, long, const double*, long, double*,
                                 long, long, long, long, const double*, long, const double*, long, double*, long,

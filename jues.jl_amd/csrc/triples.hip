@@ -10,6 +10,13 @@
 // over c with its output in W[a,b,c] order (a fastest): W is accumulated in place
 // with coalesced stores and no permutation pass.
 //
+// Triples are taken in groups whose W fit together in 192 MB (pt_group): one launch of
+// each product, of the energy kernel and of the reduction serves the group, through a table of the
+// triples' operand offsets.  One triple at a time, a basis of v = 51 leaves a product 82 workgroups and a few
+// microseconds of work, and the launches' latency sets the time (21.1 ms for the 220 triples of o = 10; the
+// 6 flop of v^3 (v + o) work are 0.3 ms); the group's W still fits in the last-level cache (256 MB), which
+// holds it between the product that writes it and the ones that update and read it.
+//
 // The energy kernel then visits ordered 8x8x8 virtual blocks A >= B >= C.  A
 // workgroup stages the six permuted blocks of W (and V = W + T1 x Vvovo terms,
 // PerturbativeTriples.jl:112) in LDS, evaluates the bracket of :118-125 for
@@ -38,7 +45,8 @@ __global__ __launch_bounds__(512) void pt_energy_kernel(const T* __restrict__ W,
                                                         const double* __restrict__ Kc,
                                                         const double* __restrict__ t1t, int o,
                                                         const double* __restrict__ fo,
-                                                        const double* __restrict__ fv, int i, int j, int k,
+                                                        const double* __restrict__ fv,
+                                                        const int* __restrict__ triples,
                                                         const int* __restrict__ blocks,
                                                         double* __restrict__ part) {
   __shared__ double Ws[6][512];
@@ -46,6 +54,10 @@ __global__ __launch_bounds__(512) void pt_energy_kernel(const T* __restrict__ W,
   __shared__ double red[8];
   const int t = threadIdx.x;
   const int x = t & 7, y = (t >> 3) & 7, z = t >> 6;
+  // triple blockIdx.y of the group, virtual block blockIdx.x
+  const int i = triples[3 * blockIdx.y], j = triples[3 * blockIdx.y + 1], k = triples[3 * blockIdx.y + 2];
+  W += (long)blockIdx.y * v * v * v;
+  part += (long)blockIdx.y * gridDim.x;
   const int A = blocks[3 * blockIdx.x], B = blocks[3 * blockIdx.x + 1], C = blocks[3 * blockIdx.x + 2];
   // tiles in the order (A,B,C) (A,C,B) (B,A,C) (B,C,A) (C,A,B) (C,B,A)
   const int P1[6] = {A, A, B, B, C, C}, P2[6] = {B, C, A, C, A, B}, P3[6] = {C, B, C, A, B, A};
@@ -99,10 +111,14 @@ __global__ __launch_bounds__(512) void pt_energy_kernel(const T* __restrict__ W,
   }
 }
 
-// et[0] = weight * sum(part[0..n)), summed in a fixed order by one workgroup
-__global__ __launch_bounds__(256) void pt_reduce_kernel(const double* __restrict__ part, int n, double weight,
-                                                        double* __restrict__ et) {
+// et[g] = (2 - d_ij - d_jk) * sum(part[g][0..n)) for triple g of the group, summed in a fixed order by one
+// workgroup
+__global__ __launch_bounds__(256) void pt_reduce_kernel(const double* __restrict__ part, int n,
+                                                        const int* __restrict__ triples, double* __restrict__ et) {
   __shared__ double sh[256];
+  part += (long)blockIdx.x * n;
+  const int* ijk = triples + 3 * blockIdx.x;
+  const double weight = 2.0 - (ijk[0] == ijk[1]) - (ijk[1] == ijk[2]);
   double s = 0.0;
   for (int q = threadIdx.x; q < n; q += 256) s += part[q];
   sh[threadIdx.x] = s;
@@ -111,7 +127,7 @@ __global__ __launch_bounds__(256) void pt_reduce_kernel(const double* __restrict
     if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) et[0] = weight * sh[0];
+  if (threadIdx.x == 0) et[blockIdx.x] = weight * sh[0];
 }
 
 // Operands of the (T) kernels in precision T (FP64 or FP32); K, T1 and the orbital
@@ -161,26 +177,44 @@ static void copy2d(jues_ctx* ctx, void* dst, size_t dpitch, const void* src, siz
 // contraction length of the packed (T) operands: v + o rounded up to a multiple of 16
 static inline long pt_ve(int o, int v) { return ((long)v + o + 15) / 16 * 16; }
 
-// W[a,b,c] (PerturbativeTriples.jl:105-111) for one triple (i, j, k): six terms, each a
-// Vvvvo term plus the Vvooo term with the same output layout, as three products of two
-// contraction segments each (W written once and updated twice).
+// W[a,b,c] (PerturbativeTriples.jl:105-111) for a group of `count` triples, one v^3 block each: six terms,
+// each a Vvvvo term plus the Vvooo term with the same output layout, as three products of two contraction
+// segments each (W written once and updated twice).  tab: the triples' operand offsets (pt_offsets), 12 each
+// in three planes of `planes` triples.
 template <typename T>
-void pt_build_W(jues_ctx* ctx, const PTOperands<T>& S, int o, int v, int i, int j, int k) {
-  const long vv = (long)v * v, ve = pt_ve(o, v), blkP = vv * ve, blkT = (long)v * ve;
+void pt_build_W(jues_ctx* ctx, const PTOperands<T>& S, int o, int v, const long* tab, long planes, int count) {
+  const long vv = (long)v * v, ve = pt_ve(o, v);
   const T* Pe = S.Pe.template as<T>();
   const T* P2e = S.P2e.template as<T>();
   const T* Te = S.Te.template as<T>();
   T* W = S.W.template as<T>();
-  auto P = [&](int x) { return Pe + x * blkP; };
-  auto P2 = [&](int x) { return P2e + x * blkP; };
-  auto Tq = [&](int p, int q) { return Te + (long)(p + (long)o * q) * blkT; };
   const T one = T(1);
+  const long* t1 = tab + 4 * planes;
+  const long* t2 = tab + 8 * planes;
   // ijk abc + jik bac: W[(a,b),c] = Pe_i[(a,b),d'] Te_kj[c,d'] + P2e_j[(a,b),d'] Te_ki[c,d']
-  gemm_ksum<T>(ctx, true, vv, v, ve, P(i), Tq(k, j), ve, P2(j), Tq(k, i), vv, v, 0, 0, one, T(0), W, vv, 0, 1, "pt_w");
+  gemm_ksum<T>(ctx, true, vv, v, ve, Pe, Te, P2e, Te, tab, count, 1, vv, v, 0, 0, one, T(0), W, vv, 0, vv * v, "pt_w");
   // ikj acb + kij cab: W[a,b,c] += Pe_i[a,c,d'] Te_jk[b,d'] + P2e_k[a,c,d'] Te_ji[b,d']  (batched over c)
-  gemm_ksum<T>(ctx, true, v, v, ve, P(i), Tq(j, k), ve, P2(k), Tq(j, i), vv, v, v, 0, one, one, W, v, vv, v, "pt_w");
+  gemm_ksum<T>(ctx, true, v, v, ve, Pe, Te, P2e, Te, t1, count, v, vv, v, v, 0, one, one, W, v, vv, vv * v, "pt_w");
   // kji cba + jki bca: W[a,(b,c)] += Te_ij[a,d'] P2e_k[(b,c),d'] + Te_ik[a,d'] Pe_j[(b,c),d']
-  gemm_ksum<T>(ctx, true, v, vv, ve, Tq(i, j), P2(k), ve, Tq(i, k), P(j), v, vv, 0, 0, one, one, W, v, 0, 1, "pt_w");
+  gemm_ksum<T>(ctx, true, v, vv, ve, Te, P2e, Te, Pe, t2, count, 1, v, vv, 0, 0, one, one, W, v, 0, vv * v, "pt_w");
+}
+
+// The operand offsets of triple (i, j, k) in the three products of pt_build_W: A0, B0, A1, B1 of each
+void pt_offsets(int o, int v, int i, int j, int k, long* first, long* second, long* third) {
+  const long blkP = (long)v * v * pt_ve(o, v), blkT = (long)v * pt_ve(o, v);
+  auto Tq = [&](int p, int q) { return (p + (long)o * q) * blkT; };
+  const long x[3][4] = {{i * blkP, Tq(k, j), j * blkP, Tq(k, i)},
+                        {i * blkP, Tq(j, k), k * blkP, Tq(j, i)},
+                        {Tq(i, j), k * blkP, Tq(i, k), j * blkP}};
+  std::copy(x[0], x[0] + 4, first);
+  std::copy(x[1], x[1] + 4, second);
+  std::copy(x[2], x[2] + 4, third);
+}
+
+// Triples per group: as many as their W fit in 192 MB, at most 65535 / v (the products' launch grid)
+static inline long pt_group(long ntrip, int v, size_t elem) {
+  const long fit = (192L << 20) / ((long)v * v * v * (long)elem);
+  return std::max(1L, std::min(std::min(ntrip, fit), 65535L / v));
 }
 
 // The amplitude columns of Pe/P2e and the amplitude half of Te, from T2 (device FP64).
@@ -205,7 +239,6 @@ template <typename T>
 double pt_run(jues_ctx* ctx, PTOperands<T>& S, const double* T2d, int o, int v, int verbose) {
   const long vv = (long)v * v;
   pt_pack_amplitudes<T>(ctx, S, T2d, o, v);
-  S.W.alloc(sizeof(T) * (size_t)vv * v);
   // ordered virtual blocks A >= B >= C
   const int nbk = (v + TE - 1) / TE;
   std::vector<int> hb;
@@ -215,26 +248,47 @@ double pt_run(jues_ctx* ctx, PTOperands<T>& S, const double* T2d, int o, int v, 
   const int nblk = (int)(hb.size() / 3);
   DevBuf blocks(hb.size() * sizeof(int));
   h2d(ctx, blocks.p, hb.data(), hb.size() * sizeof(int));
+  // occupied triples i >= j >= k and their operand offsets
   const long ntrip = (long)o * (o + 1) * (o + 2) / 6;
-  DevBuf part(sizeof(double) * (size_t)nblk), et(sizeof(double) * (size_t)ntrip);
-  long tix = 0;
-  for (int i = 0; i < o; ++i) {
-    if (verbose) {  // PerturbativeTriples.jl:81
-      sync(ctx);
-      std::fprintf(stderr, "  (T) occupied orbital %d of %d\n", i + 1, o);
-    }
+  std::vector<int> ht;
+  std::vector<long> hoff((size_t)(12 * ntrip));
+  ht.reserve((size_t)(3 * ntrip));
+  for (int i = 0; i < o; ++i)
     for (int j = 0; j <= i; ++j)
-      for (int k = 0; k <= j; ++k, ++tix) {
-        pt_build_W<T>(ctx, S, o, v, i, j, k);
-        const double weight = 2.0 - (i == j) - (j == k);
-        KTimer tm(ctx, "pt_energy", 0.0, (double)sizeof(T) * vv * v);
-        hipLaunchKernelGGL((pt_energy_kernel<T>), dim3(nblk), dim3(512), 0, ctx->stream, S.W.template as<T>(), v,
-                           S.Kc.template as<double>(), S.t1t.template as<double>(), o, S.fo, S.fv, i, j, k,
-                           blocks.as<int>(), part.as<double>());
-        hipLaunchKernelGGL(pt_reduce_kernel, dim3(1), dim3(256), 0, ctx->stream, part.as<double>(), nblk, weight,
-                           et.as<double>() + tix);
-        JUES_HIP(hipGetLastError());
+      for (int k = 0; k <= j; ++k) {
+        const long x = (long)ht.size() / 3;
+        pt_offsets(o, v, i, j, k, &hoff[4 * x], &hoff[4 * (ntrip + x)], &hoff[4 * (2 * ntrip + x)]);
+        ht.insert(ht.end(), {i, j, k});
       }
+  DevBuf triples(ht.size() * sizeof(int)), offsets(hoff.size() * sizeof(long));
+  h2d(ctx, triples.p, ht.data(), ht.size() * sizeof(int));
+  h2d(ctx, offsets.p, hoff.data(), hoff.size() * sizeof(long));
+  long group = pt_group(ntrip, v, sizeof(T));
+  try {
+    S.W.alloc(sizeof(T) * (size_t)(vv * v * group));
+  } catch (const Error& e) {  // no room for a group: one triple at a time
+    if (e.st != JUES_OOM || group == 1) throw;
+    group = 1;
+    S.W.alloc(sizeof(T) * (size_t)(vv * v));
+  }
+  DevBuf part(sizeof(double) * (size_t)(nblk * group)), et(sizeof(double) * (size_t)ntrip);
+  for (long x = 0; x < ntrip; x += group) {
+    const int count = (int)std::min(group, ntrip - x);
+    if (verbose)  // PerturbativeTriples.jl:81: a line per occupied orbital i, before its first triple
+      for (long y = x; y < x + count; ++y)
+        if (ht[3 * y + 1] == 0 && ht[3 * y + 2] == 0) {
+          sync(ctx);
+          std::fprintf(stderr, "  (T) occupied orbital %d of %d\n", ht[3 * y] + 1, o);
+        }
+    pt_build_W<T>(ctx, S, o, v, offsets.as<long>() + 4 * x, ntrip, count);
+    KTimer tm(ctx, "pt_energy", 0.0, (double)sizeof(T) * vv * v * count);
+    const int* tr = triples.as<int>() + 3 * x;
+    hipLaunchKernelGGL((pt_energy_kernel<T>), dim3(nblk, count), dim3(512), 0, ctx->stream, S.W.template as<T>(), v,
+                       S.Kc.template as<double>(), S.t1t.template as<double>(), o, S.fo, S.fv, tr, blocks.as<int>(),
+                       part.as<double>());
+    hipLaunchKernelGGL(pt_reduce_kernel, dim3(count), dim3(256), 0, ctx->stream, part.as<double>(), nblk, tr,
+                       et.as<double>() + x);
+    JUES_HIP(hipGetLastError());
   }
   std::vector<double> het((size_t)ntrip);
   d2h(ctx, het.data(), et.p, het.size() * sizeof(double));
