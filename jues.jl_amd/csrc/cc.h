@@ -38,8 +38,8 @@ struct CCWork {
   // RCCSD
   DevBuf t1, Fme, X2, Z, Q, n1, U2, Tau, FmiT;
   // RCCSD o v^3 terms through the factors: B1[m,P,e] / Y2[m,e,P] = sum_f t1[m,f] Lvv[e,f,P],
-  // Y3[m,j,P] = sum_f Lov[m,f,P] t1[j,f], W1[i,e,P], W2[i,f,P], g[P]; Zs / Zsp: slabs of (mf|ae)
-  DevBuf B1, Y2, Y3, W1, W2, gP, Zs, Zsp;
+  // Y3[m,j,P] = sum_f Lov[m,f,P] t1[j,f], W1[i,e,P], g[P]; Zs / Zsp: slabs of (mf|ae)
+  DevBuf B1, Y2, Y3, W1, gP, Zs, Zsp;
   DevBuf UL;  // U Lov (ov x naux): the factored K U ring product
   // where the last residual evaluation left H, Y (ov layout) and, when the update kernel does
   // not symmetrise them itself, S = H + Y^x + (H + Y^x)^T (the buffers may be shared)
@@ -179,10 +179,10 @@ void rccd_delta_contractions(jues_ctx* ctx, CCState& S, const double* t2);
 template <typename T>
 void ovvv_z_slab(jues_ctx* ctx, CCState& S, int m0, int cnt, const T* LovT, const T* Lvv, const T* Tpp, T* Zs,
                  T* Zsp, T* Z);
-// RCCSD's (ia|bc) factor products (split-FP16 in the split stage): W1 = Tov Lov (ov x naux);
+// RCCSD's (ia|bc) factor products (split-FP16 in the split stage): W1 = Uov Lov (ov x naux);
 // C += Lov Y2^T (y2_right) or C += Y2 Lov^T (Y2: ov x naux); Q = Y3 Lvv^T (Y3: o^2 x naux)
 template <typename T>
-void fac_tov_lov(jues_ctx* ctx, CCState& S, const T* Tov, T* W1);
+void fac_uov_lov(jues_ctx* ctx, CCState& S, const T* Uov, T* W1);
 template <typename T>
 void fac_lov_y2(jues_ctx* ctx, CCState& S, const T* Y2, bool y2_right, T* C);
 template <typename T>

@@ -378,18 +378,18 @@ template void ovvv_z_slab<double>(jues_ctx*, CCState&, int, int, const double*, 
                                   double*, double*, double*);
 
 template <typename T>
-void fac_tov_lov(jues_ctx* ctx, CCState& S, const T* Tov, T* W1) {
+void fac_uov_lov(jues_ctx* ctx, CCState& S, const T* Uov, T* W1) {
   const long ov = (long)S.o * S.v, naux = ctx->naux;
   if constexpr (sizeof(T) == 4) {
     if (S.split_on) {
-      // Tov is symmetric: its ring planes serve as the TN kernel's left operand
-      const Split16& t = split_operand<float>(ctx, S, SP_TOV, Tov, ov, ov);
+      // Uov is symmetric: its ring planes serve as the TN kernel's left operand
+      const Split16& t = split_operand<float>(ctx, S, SP_UOV, Uov, ov, ov);
       const Split16& l = split_operand<double>(ctx, S, SP_LOV, S.i64->Lov.as<double>(), ov, naux);
       gemm16_tn(ctx, ov, naux, 1.0f, t, l, 0.0f, W1, ov, "cc_ovvv_fac");
       return;
     }
   }
-  gemm<T>(ctx, false, false, ov, naux, ov, T(1), Tov, ov, 0, ints<T>(S).Lov.template as<T>(), ov, 0, T(0), W1, ov,
+  gemm<T>(ctx, false, false, ov, naux, ov, T(1), Uov, ov, 0, ints<T>(S).Lov.template as<T>(), ov, 0, T(0), W1, ov,
           0, 1, "cc_ovvv_fac");
 }
 
@@ -431,8 +431,8 @@ void fac_y3_lvv(jues_ctx* ctx, CCState& S, const T* Y3, T* Q) {
           1, "cc_ovvv_fac");
 }
 
-template void fac_tov_lov<double>(jues_ctx*, CCState&, const double*, double*);
-template void fac_tov_lov<float>(jues_ctx*, CCState&, const float*, float*);
+template void fac_uov_lov<double>(jues_ctx*, CCState&, const double*, double*);
+template void fac_uov_lov<float>(jues_ctx*, CCState&, const float*, float*);
 template void fac_lov_y2<double>(jues_ctx*, CCState&, const double*, bool, double*);
 template void fac_lov_y2<float>(jues_ctx*, CCState&, const float*, bool, float*);
 template void fac_y3_lvv<double>(jues_ctx*, CCState&, const double*, double*);

@@ -204,7 +204,7 @@ __device__ inline double block_sum256(double v, double* sh) {
   return (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
-// One block per (a,b): assemble R[ijab] = K[ijab] + S[ia,jb] + L+ + L- (both ladders),
+// One block per (a,b): assemble R[ijab] = K[ijab] + S[ia,jb] + L+ + L- (both ladders) + X[ijab] + X[jiba] (extra),
 // t_new = R/D, e = t_new - t_old; write t_new and e into the DIIS slot; block
 // partial sums of E = sum Lener*t_new, e.e and e.e_k for the stored errors.
 template <typename TR>
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(256) void t2_update_kernel(UpdateArgs<TR> A) {
         R += (double)(sij * sab) * (double)A.Lm[pm + A.nmo * qm];
       }
     }
-    if (A.extra) R += (double)A.extra[x];
+    if (A.extra) R += (double)A.extra[x] + (double)A.extra[j + (long)o * i + oo * (b + (long)v * a)];
     if (A.R_out) A.R_out[x] = R;
     const double tn = A.lambda * R / (A.eps[i] + A.eps[j] + dab);
     const double e = tn - A.t_old[x];
@@ -325,66 +325,73 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(const double* __restri
 // Store the new B row/column and solve the bordered Pulay system (mRCCD.jl:185-198)
 // in FP64 with partial pivoting.  small layout: [0]=E, [1]=ee, [2..2+nold)=dots,
 // B at SMALL_B (MAX_DIIS^2, by slot), coefficients at SMALL_C (MAX_DIIS, by order).
-__global__ void diis_solve_kernel(double* small, DiisOrder ord) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  double* B = small + SMALL_B;
+// One wavefront with the augmented matrix (at most 9 x 10) in LDS: the elements of an elimination step are
+// independent, so they are updated together.  (One thread on arrays that the compiler put in scratch memory
+// took 24 us at five vectors and 37 us behind a larger solve, of an iteration of 150 us at n = 24.)
+__global__ __launch_bounds__(64) void diis_solve_kernel(double* small, DiisOrder ord) {
+  constexpr int NMAX = MAX_DIIS + 1;
+  __shared__ double M[NMAX][NMAX + 1];  // column N: the right-hand side, then the solution
+  __shared__ double B[MAX_DIIS][MAX_DIIS];
+  const int t = threadIdx.x;
+  for (int e = t; e < MAX_DIIS * MAX_DIIS; e += 64) B[e / MAX_DIIS][e % MAX_DIIS] = small[SMALL_B + e];
+  __syncthreads();
   const int s = ord.newest;
-  B[s * MAX_DIIS + s] = small[1];
-  for (int k = 0; k < ord.nold; ++k) {
-    const int sk = ord.old_slots[k];
-    B[s * MAX_DIIS + sk] = small[2 + k];
-    B[sk * MAX_DIIS + s] = small[2 + k];
+  if (t <= ord.nold) {
+    const int sk = t < ord.nold ? ord.old_slots[t] : s;
+    const double d = t < ord.nold ? small[2 + t] : small[1];
+    B[s][sk] = B[sk][s] = d;
+    small[SMALL_B + s * MAX_DIIS + sk] = small[SMALL_B + sk * MAX_DIIS + s] = d;
   }
-  const int m = ord.m;
+  const int m = ord.m, N = m + 1;
   double* c = small + SMALL_C;
-  if (m == 1) { c[0] = 1.0; small[SMALL_FLAG] = 0.0; return; }
-  double M[(MAX_DIIS + 1) * (MAX_DIIS + 1)];
-  double r[MAX_DIIS + 1];
-  const int N = m + 1;
+  if (m == 1) {
+    if (t == 0) { c[0] = 1.0; small[SMALL_FLAG] = 0.0; }
+    return;
+  }
+  __syncthreads();
   double mx = 0.0;
   for (int p = 0; p < m; ++p)
-    for (int q = 0; q < m; ++q) mx = fmax(mx, fabs(B[ord.slots[p] * MAX_DIIS + ord.slots[q]]));
+    for (int q = 0; q < m; ++q) mx = fmax(mx, fabs(B[ord.slots[p]][ord.slots[q]]));
   if (!(mx > 0.0)) mx = 1.0;
-  for (int p = 0; p < N; ++p) {
-    for (int q = 0; q < N; ++q) {
-      double val;
-      if (p < m && q < m) val = B[ord.slots[p] * MAX_DIIS + ord.slots[q]] / mx;
-      else if (p == m && q == m) val = 0.0;
-      else val = -1.0;
-      M[p * N + q] = val;
-    }
-    r[p] = p == m ? -1.0 : 0.0;
+  for (int e = t; e < N * (N + 1); e += 64) {
+    const int p = e / (N + 1), q = e % (N + 1);
+    double val;
+    if (q == N) val = p == m ? -1.0 : 0.0;
+    else if (p < m && q < m) val = B[ord.slots[p]][ord.slots[q]] / mx;
+    else val = p == m && q == m ? 0.0 : -1.0;
+    M[p][q] = val;
   }
+  __syncthreads();
   bool ok = true;
   for (int k = 0; k < N; ++k) {
     int piv = k;
     for (int p = k + 1; p < N; ++p)
-      if (fabs(M[p * N + k]) > fabs(M[piv * N + k])) piv = p;
-    if (!(fabs(M[piv * N + k]) > 1e-300)) { ok = false; break; }
-    if (piv != k) {
-      for (int q = 0; q < N; ++q) { const double tmp = M[k * N + q]; M[k * N + q] = M[piv * N + q]; M[piv * N + q] = tmp; }
-      const double tmp = r[k]; r[k] = r[piv]; r[piv] = tmp;
+      if (fabs(M[p][k]) > fabs(M[piv][k])) piv = p;
+    if (!(fabs(M[piv][k]) > 1e-300)) { ok = false; break; }
+    __syncthreads();
+    if (piv != k && t <= N) { const double tmp = M[k][t]; M[k][t] = M[piv][t]; M[piv][t] = tmp; }
+    __syncthreads();
+    // rows below k; column k itself is not read again
+    const int rows = N - 1 - k, cols = N - k;
+    for (int e = t; e < rows * cols; e += 64) {
+      const int p = k + 1 + e / cols, q = k + 1 + e % cols;
+      const double f = M[p][k] / M[k][k];
+      M[p][q] -= f * M[k][q];
     }
-    for (int p = k + 1; p < N; ++p) {
-      const double f = M[p * N + k] / M[k * N + k];
-      for (int q = k; q < N; ++q) M[p * N + q] -= f * M[k * N + q];
-      r[p] -= f * r[k];
-    }
+    __syncthreads();
   }
-  if (ok) {
-    for (int k = N - 1; k >= 0; --k) {
-      double acc = r[k];
-      for (int q = k + 1; q < N; ++q) acc -= M[k * N + q] * r[q];
-      r[k] = acc / M[k * N + k];
+  if (t == 0) {
+    if (ok) {
+      for (int k = N - 1; k >= 0; --k) {
+        double acc = M[k][N];
+        for (int q = k + 1; q < N; ++q) acc -= M[k][q] * M[q][N];
+        M[k][N] = acc / M[k][k];
+      }
+      for (int p = 0; p < m; ++p) ok = ok && isfinite(M[p][N]);
     }
-    for (int p = 0; p < m; ++p) ok = ok && isfinite(r[p]);
-  }
-  if (ok) {
-    for (int p = 0; p < m; ++p) c[p] = r[p];
-    small[SMALL_FLAG] = 0.0;
-  } else {  // singular subspace: take the newest vector (a plain Jacobi step)
-    for (int p = 0; p < m; ++p) c[p] = p == m - 1 ? 1.0 : 0.0;
-    small[SMALL_FLAG] = 1.0;
+    // a singular subspace: take the newest vector (a plain Jacobi step)
+    for (int p = 0; p < m; ++p) c[p] = ok ? M[p][N] : (p == m - 1 ? 1.0 : 0.0);
+    small[SMALL_FLAG] = ok ? 0.0 : 1.0;
   }
 }
 

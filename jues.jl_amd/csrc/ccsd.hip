@@ -27,22 +27,53 @@
 namespace jues {
 namespace {
 
-// tau = t2 + t1 t1 into Tpp, 2 tau' - tau'^(ij) (tau' = t2 + t1 t1 / 2) into Upp, both [i,j,a,b],
-// and tt^x[i,a,j,b] = t1[i,b] t1[j,a] (ov layout) into ttx, in the compute type
+// The amplitude layouts of the CCSD residual in the compute type, all from one read of t2 and t1:
+//   Tpp = tau = t2 + t1 t1, Upp = 2 tau' - tau'^(ij) (tau' = t2 + t1 t1 / 2)          [i,j,a,b]
+//   Tov = t2, Ttov[i,a,j,b] = t2[i,j,b,a], Uov = 2 t2 - t2^(ij)                        [i,a,j,b]
+//   U2 = Uov - 2 tt^x, Q = Ttov + 2 tt^x with tt^x[i,a,j,b] = t1[i,b] t1[j,a]           [i,a,j,b]
 template <typename T>
-__global__ __launch_bounds__(256) void ccsd_amps_kernel(const double* __restrict__ t2, const double* __restrict__ t1,
-                                                        int o, int v, T* __restrict__ Tpp, T* __restrict__ Upp,
-                                                        T* __restrict__ ttx) {
-  const long oo = (long)o * o, ov = (long)o * v, n = oo * v * v;
-  for (long x = blockIdx.x * 256L + threadIdx.x; x < n; x += (long)gridDim.x * 256L) {
-    const long ij = x % oo, ab = x / oo;
-    const int i = (int)(ij % o), j = (int)(ij / o), a = (int)(ab % v), b = (int)(ab / v);
-    const double tt = t1[i + (long)o * a] * t1[j + (long)o * b];
-    const double tt_ji = t1[j + (long)o * a] * t1[i + (long)o * b];
-    const double t2ji = t2[j + (long)o * i + oo * ab];
-    Tpp[x] = (T)(t2[x] + tt);
-    Upp[x] = (T)(2.0 * (t2[x] + 0.5 * tt) - (t2ji + 0.5 * tt_ji));
-    ttx[i + (long)o * a + ov * (j + (long)o * b)] = (T)tt_ji;
+struct CcsdLayouts {
+  int o, v;
+  T *Tpp, *Upp, *Tov, *Ttov, *Uov, *U2, *Q;
+  // element (i,j,a,b) from t2 = t2[ijab], t2x = t2[jiab]
+  __device__ inline void put(const double* __restrict__ t1, int i, int j, int a, int b, double t2, double t2x) const {
+    const long oo = (long)o * o, ov = (long)o * v, x = i + (long)o * j + oo * (a + (long)v * b);
+    const double tt = t1[i + (long)o * a] * t1[j + (long)o * b], ttx = t1[i + (long)o * b] * t1[j + (long)o * a];
+    const long y = i + (long)o * a + ov * (j + (long)o * b), yx = i + (long)o * b + ov * (j + (long)o * a);
+    Tpp[x] = (T)(t2 + tt);
+    Upp[x] = (T)(2.0 * (t2 + 0.5 * tt) - (t2x + 0.5 * ttx));
+    const T u = (T)(2.0 * t2 - t2x);
+    Tov[y] = (T)t2;
+    Uov[y] = u;
+    U2[y] = (T)((double)u - 2.0 * (double)(T)ttx);
+    Ttov[yx] = (T)t2;                                  // Ttov[i,b,j,a] = t2[i,j,a,b]
+    Q[yx] = (T)((double)(T)t2 + 2.0 * (double)(T)tt);  // tt^x[i,b,j,a] = t1[i,a] t1[j,b]
+  }
+};
+
+// One workgroup per (a,b) pair, whose o x o slab of t2 is staged in LDS (rows padded to o + 1) so that the
+// exchanged read t2[j,i,a,b] comes from LDS: t2 is read once and each of the seven layouts written once, in
+// runs of o.  Dynamic LDS: o (o + 1) doubles; without it (o too large) the exchanged element is read from memory.
+// Bound by the writes; it replaces five launches that made 14 passes over o^2 v^2 elements between them, and the
+// three passes that built U2 and Q later.
+template <typename T>
+__global__ __launch_bounds__(256) void ccsd_layouts_kernel(const double* __restrict__ t2, const double* __restrict__ t1,
+                                                           CcsdLayouts<T> L, int staged) {
+  extern __shared__ double slab[];
+  const int o = L.o, oo = o * o, ld = o + 1;
+  const long vv = (long)L.v * L.v;
+  for (long ab = blockIdx.x; ab < vv; ab += gridDim.x) {
+    const int a = (int)(ab % L.v), b = (int)(ab / L.v);
+    const double* src = t2 + ab * oo;
+    if (staged) {
+      __syncthreads();  // the previous pair's readers are done with the slab
+      for (int q = threadIdx.x; q < oo; q += 256) slab[q % o + ld * (q / o)] = src[q];
+      __syncthreads();
+    }
+    for (int q = threadIdx.x; q < oo; q += 256) {
+      const int i = q % o, j = q / o;
+      L.put(t1, i, j, a, b, staged ? slab[i + ld * j] : src[q], staged ? slab[j + ld * i] : src[j + (long)o * i]);
+    }
   }
 }
 
@@ -149,19 +180,17 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
   const long naux = ctx->naux;
 
   // ---- amplitudes in the compute type -------------------------------------------
-  T* ttx = U2;  // tt^x [i,a,j,b] (overwritten below once used)
   convert<double, T>(ctx, t1_64, t1, ov);
   {
-    KTimer k(ctx, "cc_prep", 0.0, (double)N2 * (16.0 + 3.0 * sizeof(T)));
-    hipLaunchKernelGGL((ccsd_amps_kernel<T>), dim3(g256(N2)), dim3(256), 0, ctx->stream, t2, t1_64, o, v, Tpp, Upp,
-                       ttx);
+    const size_t slab = (size_t)o * (o + 1) * sizeof(double);
+    const bool staged = slab <= 65536;
+    KTimer k(ctx, "cc_prep", 0.0, (double)N2 * ((staged ? 8.0 : 16.0) + 7.0 * sizeof(T)));
+    hipLaunchKernelGGL((ccsd_layouts_kernel<T>), dim3((unsigned)std::min(vv, 1L << 20)), dim3(256),
+                       staged ? slab : 0, ctx->stream, t2, t1_64, CcsdLayouts<T>{o, v, Tpp, Upp, Tov, Ttov, Uov, U2, Q},
+                       staged ? 1 : 0);
     JUES_HIP(hipGetLastError());
   }
   permute<T, T>(ctx, Upp, d4, {2, 0, 1, 3}, Ua, 1.0, 0.0, "cc_prep");
-  permute<double, T>(ctx, t2, d4, {0, 2, 1, 3}, Tov, 1.0, 0.0, "cc_prep");
-  permute<double, T>(ctx, t2, d4, {0, 3, 1, 2}, Ttov, 1.0, 0.0, "cc_prep");
-  permute<T, T>(ctx, Tov, {ov, ov}, {0, 1}, Uov, 2.0, 0.0, "cc_prep");
-  permute<T, T>(ctx, Ttov, {ov, ov}, {0, 1}, Uov, -1.0, 1.0, "cc_prep");
 
   // factors of (ia|bc) and their contractions with t1
   const T* Lov = fac ? I.Lov.template as<T>() : nullptr;    // [m,e,P]
@@ -232,15 +261,11 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
   contract<T>(ctx, -2.0, TN(Tov, "nema"), TN(ooov, "mine"), 1.0, TN(n1, "ia"), "cc_t1");
   contract<T>(ctx, 1.0, TN(Tov, "nema"), TN(ooov, "nime"), 1.0, TN(n1, "ia"), "cc_t1");
   if (fac) {
-    // 2 sum_emf T[ie,mf] (mf|ae): W1[(ie),P] = T[(ie),(mf)] Lov[(mf),P], n1 += 2 W1[i,(eP)] Lvv[a,(eP)];
-    // - sum_emf T[ie,mf] (me|af): W2[i,f,P] = sum_(em) T[i,(em),f] LovT[(em),P] (batched over f and
-    // written straight into [i,f,P]), n1 -= W2[i,(fP)] Lvv[a,(fP)]
+    // sum_emf (2 T[ie,mf] - T[me,if]) (mf|ae) = sum_(eP) W1[i,(eP)] Lvv[a,(eP)] with
+    // W1[(ie),P] = sum_(mf) U[(ie),(mf)] Lov[(mf),P], U = 2 T - T^x: both terms in one (ov)^2 naux product
     T* W1 = bufp_t<T>(W.W1, ov * naux);
-    T* W2 = bufp_t<T>(W.W2, ov * naux);
-    fac_tov_lov<T>(ctx, S, Tov, W1);
-    gemm<T>(ctx, false, true, o, v, v * naux, T(2), W1, o, 0, Lvv, v, 0, one, n1, o, 0, 1, "cc_ovvv_fac");
-    gemm<T>(ctx, false, false, o, naux, ov, one, Tov, o, oo * v, LovT, ov, 0, zero, W2, ov, o, v, "cc_ovvv_fac");
-    gemm<T>(ctx, false, true, o, v, v * naux, T(-1), W2, o, 0, Lvv, v, 0, one, n1, o, 0, 1, "cc_ovvv_fac");
+    fac_uov_lov<T>(ctx, S, Uov, W1);
+    gemm<T>(ctx, false, true, o, v, v * naux, one, W1, o, 0, Lvv, v, 0, one, n1, o, 0, 1, "cc_ovvv_fac");
   } else {
     contract<T>(ctx, 2.0, TN(Tov, "iemf"), TN(ovvv, "mfae"), 1.0, TN(n1, "ia"), "cc_t1");
     contract<T>(ctx, -1.0, TN(Tov, "iemf"), TN(ovvv, "meaf"), 1.0, TN(n1, "ia"), "cc_t1");
@@ -259,7 +284,8 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
   contract<T>(ctx, 1.0, TN(t1, "je"), TN(ooov, "mine"), 1.0, TN(Wp, "mnij"), "cc_t1");
   contract<T>(ctx, 1.0, TN(t1, "ie"), TN(ooov, "njme"), 1.0, TN(Wp, "mnij"), "cc_t1");
   hh_mm<T>(ctx, S, Wp, Tp, Tm, Lp, Lm);
-  // Wabef's T1 part: X2 = Lz + Lz^P,  Lz[ijab] = -sum_m t1[mb] Z[ij,ma],  Z = tau . (mf|ae)
+  // Wabef's T1 part: X2 = Lz[ijab] = -sum_m t1[mb] Z[ij,ma],  Z = tau . (mf|ae); the update kernel adds
+  // Lz[ijab] + Lz[jiba]
   if (fac) {
     // Z[i,j,a,m] over slabs of m: Zs[(f,m'),(a,e)] = sum_P LovT[(f,m),P] Lvv[(ae),P] = (mf|ae),
     // Zsp[(e,f),(a,m')] its permutation, Z[(ij),(a,m)] = Tpp[(ij),(ef)] Zsp; then
@@ -272,19 +298,13 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
       const int cnt = (int)std::min<long>(ms, o - m0);
       ovvv_z_slab<T>(ctx, S, m0, cnt, LovT, Lvv, Tpp, Zs, Zsp, Z);
     }
-    gemm<T>(ctx, false, false, oo * v, v, o, T(-1), Z, oo * v, 0, t1, o, 0, zero, Q, oo * v, 0, 1, "cc_t1");
+    gemm<T>(ctx, false, false, oo * v, v, o, T(-1), Z, oo * v, 0, t1, o, 0, zero, X2, oo * v, 0, 1, "cc_t1");
   } else {
     contract<T>(ctx, 1.0, TN(Tpp, "ijef"), TN(ovvv, "mfae"), 0.0, TN(Z, "ijma"), "cc_ovvv");
-    contract<T>(ctx, -1.0, TN(t1, "mb"), TN(Z, "ijma"), 0.0, TN(Q, "ijab"), "cc_t1");
+    contract<T>(ctx, -1.0, TN(t1, "mb"), TN(Z, "ijma"), 0.0, TN(X2, "ijab"), "cc_t1");
   }
-  permute<T, T>(ctx, Q, d4, {0, 1, 2, 3}, X2, 1.0, 0.0, "cc_sym");
-  permute<T, T>(ctx, Q, d4, {1, 0, 3, 2}, X2, 1.0, 1.0, "cc_sym");
 
   // ---- ring terms -----------------------------------------------------------------------
-  // U2 = U - 2 tt^x (U2 holds tt^x on entry); Q = Tx + 2 tt^x
-  permute<T, T>(ctx, Ttov, {ov, ov}, {0, 1}, Q, 1.0, 0.0, "cc_prep");
-  permute<T, T>(ctx, U2, {ov, ov}, {0, 1}, Q, 2.0, 1.0, "cc_prep");
-  permute<T, T>(ctx, Uov, {ov, ov}, {0, 1}, U2, 1.0, -2.0, "cc_prep");
   JUES_HIP(hipMemcpyAsync(WJ, Kov, N2 * sizeof(T), hipMemcpyDeviceToDevice, ctx->stream));
   // every left operand of the ring products is a symmetric (ov) x (ov) matrix
   ring_k_mm<T>(ctx, S, half, U2, SP_U2, WJ);
