@@ -30,6 +30,20 @@ struct CCInts {
   DevBuf fOO, fVV, fOV;
 };
 
+// The launches of a small system's residual (cc_small.hip): `count` outputs from `first`, `tiles` workgroups
+struct SmallGroup {
+  int first, count, tiles;
+};
+struct CCState;
+// Their descriptors on the device, over the buffers of one stage's work set and integrals (owned by that work set)
+template <typename T>
+struct SmallPlan {
+  DevBuf desc;  // outputs, terms from term_at, points from point_at (bytes)
+  size_t term_at = 0, point_at = 0;
+  std::vector<SmallGroup> groups;
+  void build(jues_ctx* ctx, CCState& S);
+};
+
 template <typename T>
 struct CCWork {
   DevBuf Tpp, Upp, Tov, Ttov, Uov, Ua, Tp, Tm, WJ, WE, Y, H, Wp, Fae, Fmi, Lp, Lm;
@@ -46,6 +60,8 @@ struct CCWork {
   T* out_H = nullptr;
   T* out_Y = nullptr;
   T* out_S = nullptr;
+  T* out_X = nullptr;  // further terms X[i,j,a,b] of which the update kernel adds X[ijab] + X[jiba], or null
+  std::unique_ptr<SmallPlan<T>> small;
 };
 
 // Split-FP16 operand planes of the fast stage.  Slots below SPLIT_CONST hold
@@ -187,6 +203,13 @@ template <typename T>
 void fac_lov_y2(jues_ctx* ctx, CCState& S, const T* Y2, bool y2_right, T* C);
 template <typename T>
 void fac_y3_lvv(jues_ctx* ctx, CCState& S, const T* Y3, T* Q);
+// Whether the residual may be evaluated by the small system's launches (cc_small.hip), where they are faster than
+// the general form's in every precision.  FP64 iterations, general / small form: RCCD 111 / 67 us at ov = 192,
+// 136 / 128 at 336, 169 / 186 at 400; RCCSD 333 / 102 at 192, 387 / 176 at 336, 470 / 372 at 504.
+inline bool small_system(const CCState& S) { return (long)S.o * S.v <= (S.method == 1 ? 504 : 336); }
+// the residual of the resident amplitudes through the small system's launches (out_H, out_Y, out_X, Lp, Lm, R1)
+template <typename T>
+void small_contractions(jues_ctx* ctx, CCState& S);
 // the anchor's intermediates, in the inner stage's type (called by the FP64 contractions)
 void dc_capture(jues_ctx* ctx, CCState& S, const double* WJ, const double* WE, const double* Wpt,
                 const double* Wmt);

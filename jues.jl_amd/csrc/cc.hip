@@ -149,7 +149,13 @@ void cc_build_ints(jues_ctx* ctx, CCState& S, const double* Co, const double* Cv
     gemm<double>(ctx, false, true, oo, oo, naux, 1.0, Loo.as<double>(), oo, 0, Loo.as<double>(), oo, 0, 0.0, Oc, oo,
                  0, 1, "setup_ints");
     S.k_factored = true;
-    if (S.method == 1) {
+    if (S.method == 1 && small_system(S)) {
+      // the small system's residual reads the whole blocks
+      gemm<double>(ctx, false, true, oo, ov, naux, 1.0, Loo.as<double>(), oo, 0, Lov.as<double>(), ov, 0, 0.0,
+                   bufp<double>(I.ooov_c, oo * ov), oo, 0, 1, "setup_ints");
+      gemm<double>(ctx, false, true, ov, (long)v * v, naux, 1.0, Lov.as<double>(), ov, 0, Lvv.as<double>(),
+                   (long)v * v, 0, 0.0, bufp<double>(I.ovvv_c, ov * v * v), ov, 0, 1, "setup_ints");
+    } else if (S.method == 1) {
       // (ij|ka) -> ooov chem [i,j,k,a]; (ia|bc) stays factored: Lov, its two permutations and Lvv
       double* ooov = bufp<double>(I.ooov_c, oo * ov);
       gemm<double>(ctx, false, true, oo, ov, naux, 1.0, Loo.as<double>(), oo, 0, Lov.as<double>(), ov, 0, 0.0, ooov,
@@ -862,20 +868,20 @@ void cc_iteration(jues_ctx* ctx, CCState& S, jues_iter_info* info) {
   const long PB = v2 + nb1;
   double* part = static_cast<double*>(scratch(ctx, 13, sizeof(double) * (size_t)(PB * (2 + MAX_DIIS))));
 
-  const T* R1extra = nullptr;
   DCState* dc = S.dc.get();
   const bool dc_on = dc && dc->on && S.method == 0;
   const bool dc_cap = dc && dc->capture && S.method == 0 && sizeof(T) == 8;
   if (dc_cap)
     JUES_HIP(hipMemcpyAsync(bufp<double>(dc->t0, N2), t, N2 * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
-  if (S.method == 0) {
+  CCWork<T>& W = work<T>(S);
+  W.out_X = nullptr;
+  if (small_system(S) && !S.dc && !S.fock_on) small_contractions<T>(ctx, S);
+  else if (S.method == 0) {
     if (dc_on) rccd_delta_contractions<T>(ctx, S, t);
     else rccd_contractions<T>(ctx, S, t);
   } else {
     rccsd_contractions<T>(ctx, S, t, t + N2);
-    R1extra = nullptr;
   }
-  CCWork<T>& W = work<T>(S);
   UpdateArgs<T> A{};
   A.o = o;
   A.v = v;
@@ -892,7 +898,7 @@ void cc_iteration(jues_ctx* ctx, CCState& S, jues_iter_info* info) {
   }
   A.Lp = W.Lp.template as<T>();
   A.Lm = W.Lm.template as<T>();
-  A.extra = S.method == 1 ? W.X2.template as<T>() : nullptr;
+  A.extra = W.out_X;
   A.t1n = nullptr;
   A.lambda = S.lambda;
   A.npo = S.P.npo;
@@ -927,18 +933,16 @@ void cc_iteration(jues_ctx* ctx, CCState& S, jues_iter_info* info) {
   }
   t2_update<T>(ctx, A);
   double* small = S.small.as<double>();
-  reduce_rows(ctx, part, PB, PB, 2 + ord.nold, small);
   S.active.push_back(slot);
   ord.m = (int)S.active.size();
   for (int k = 0; k < ord.m; ++k) ord.slots[k] = S.active[k];
-  diis_solve(ctx, small, ord);
+  diis_solve(ctx, small, ord, part, PB);
   diis_extrap(ctx, vals, Nd, ord, small, Nd, t);
   JUES_HIP(hipEventRecord(e1, ctx->stream));
   double h[2];
   d2h(ctx, h, small, sizeof(h));
   float ms = 0.f;
   JUES_HIP(hipEventElapsedTime(&ms, e0, e1));
-  (void)R1extra;
 
   S.iter += 1;
   info->iter = S.iter;

@@ -99,7 +99,8 @@ void t2_update(jues_ctx* ctx, const UpdateArgs<TR>& A);
 inline bool fused_sym(int o, size_t elem) { return (size_t)o * (o + 1) * elem <= 48 * 1024; }
 void t1_update(jues_ctx* ctx, const T1UpdateArgs& A, int nblocks);
 void reduce_rows(jues_ctx* ctx, const double* part, long PB, long count, int nq, double* out);
-void diis_solve(jues_ctx* ctx, double* small, const DiisOrder& ord);
+// the sums of the 2 + nold rows of partial sums (PB each) into small, then the DIIS coefficients
+void diis_solve(jues_ctx* ctx, double* small, const DiisOrder& ord, const double* part, long PB);
 void diis_extrap(jues_ctx* ctx, const double* vals, long stride, const DiisOrder& ord, const double* small, long n,
                  double* t);
 void divide_d2(jues_ctx* ctx, double* t, const double* eps, int o, int v, double scale);

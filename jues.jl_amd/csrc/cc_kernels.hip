@@ -328,17 +328,35 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(const double* __restri
 // One wavefront with the augmented matrix (at most 9 x 10) in LDS: the elements of an elimination step are
 // independent, so they are updated together.  (One thread on arrays that the compiler put in scratch memory
 // took 24 us at five vectors and 37 us behind a larger solve, of an iteration of 150 us at n = 24.)
-__global__ __launch_bounds__(64) void diis_solve_kernel(double* small, DiisOrder ord) {
+// With `part` the sums small[0 .. 2 + nold) are formed here first, each over PB partial sums by one
+// wavefront in a fixed order: one launch less where there are few of them.
+__global__ __launch_bounds__(256) void diis_solve_kernel(double* small, DiisOrder ord, const double* __restrict__ part,
+                                                         long PB) {
   constexpr int NMAX = MAX_DIIS + 1;
   __shared__ double M[NMAX][NMAX + 1];  // column N: the right-hand side, then the solution
   __shared__ double B[MAX_DIIS][MAX_DIIS];
+  __shared__ double sums[2 + MAX_DIIS];
   const int t = threadIdx.x;
-  for (int e = t; e < MAX_DIIS * MAX_DIIS; e += 64) B[e / MAX_DIIS][e % MAX_DIIS] = small[SMALL_B + e];
+  for (int q = t >> 6; q < 2 + ord.nold; q += blockDim.x >> 6) {
+    double s = 0.0;
+    if (part) {
+      for (long x = t & 63; x < PB; x += 64) s += part[q * PB + x];
+      for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+    } else {
+      s = small[q];
+    }
+    if ((t & 63) == 0) {
+      sums[q] = s;
+      if (part) small[q] = s;
+    }
+  }
+  for (int e = t; e < MAX_DIIS * MAX_DIIS; e += blockDim.x) B[e / MAX_DIIS][e % MAX_DIIS] = small[SMALL_B + e];
   __syncthreads();
+  if (t >= 64) return;
   const int s = ord.newest;
   if (t <= ord.nold) {
     const int sk = t < ord.nold ? ord.old_slots[t] : s;
-    const double d = t < ord.nold ? small[2 + t] : small[1];
+    const double d = t < ord.nold ? sums[2 + t] : sums[1];
     B[s][sk] = B[sk][s] = d;
     small[SMALL_B + s * MAX_DIIS + sk] = small[SMALL_B + sk * MAX_DIIS + s] = d;
   }
@@ -349,9 +367,8 @@ __global__ __launch_bounds__(64) void diis_solve_kernel(double* small, DiisOrder
     return;
   }
   __syncthreads();
-  double mx = 0.0;
-  for (int p = 0; p < m; ++p)
-    for (int q = 0; q < m; ++q) mx = fmax(mx, fabs(B[ord.slots[p]][ord.slots[q]]));
+  double mx = t < m * m ? fabs(B[ord.slots[t / m]][ord.slots[t % m]]) : 0.0;  // m * m <= 64
+  for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
   if (!(mx > 0.0)) mx = 1.0;
   for (int e = t; e < N * (N + 1); e += 64) {
     const int p = e / (N + 1), q = e % (N + 1);
@@ -364,11 +381,17 @@ __global__ __launch_bounds__(64) void diis_solve_kernel(double* small, DiisOrder
   __syncthreads();
   bool ok = true;
   for (int k = 0; k < N; ++k) {
-    int piv = k;
-    for (int p = k + 1; p < N; ++p)
-      if (fabs(M[p][k]) > fabs(M[piv][k])) piv = p;
-    if (!(fabs(M[piv][k]) > 1e-300)) { ok = false; break; }
-    __syncthreads();
+    // the first row of the largest |M[p][k]|, p >= k
+    double best = t >= k && t < N ? fabs(M[t][k]) : -1.0;
+    int piv = t;
+    for (int off = 8; off > 0; off >>= 1) {
+      const double ob = __shfl_xor(best, off, 64);
+      const int op = __shfl_xor(piv, off, 64);
+      if (ob > best || (ob == best && op < piv)) { best = ob; piv = op; }
+    }
+    best = __shfl(best, 0, 64);
+    piv = __shfl(piv, 0, 64);
+    if (!(best > 1e-300)) { ok = false; break; }
     if (piv != k && t <= N) { const double tmp = M[k][t]; M[k][t] = M[piv][t]; M[piv][t] = tmp; }
     __syncthreads();
     // rows below k; column k itself is not read again
@@ -380,19 +403,19 @@ __global__ __launch_bounds__(64) void diis_solve_kernel(double* small, DiisOrder
     }
     __syncthreads();
   }
-  if (t == 0) {
-    if (ok) {
-      for (int k = N - 1; k >= 0; --k) {
-        double acc = M[k][N];
-        for (int q = k + 1; q < N; ++q) acc -= M[k][q] * M[q][N];
-        M[k][N] = acc / M[k][k];
-      }
-      for (int p = 0; p < m; ++p) ok = ok && isfinite(M[p][N]);
+  if (ok) {
+    for (int k = N - 1; k >= 0; --k) {
+      const double xk = M[k][N] / M[k][k];
+      __syncthreads();
+      if (t < k) M[t][N] -= M[t][k] * xk;
+      else if (t == k) M[k][N] = xk;
+      __syncthreads();
     }
-    // a singular subspace: take the newest vector (a plain Jacobi step)
-    for (int p = 0; p < m; ++p) c[p] = ok ? M[p][N] : (p == m - 1 ? 1.0 : 0.0);
-    small[SMALL_FLAG] = ok ? 0.0 : 1.0;
+    for (int p = 0; p < m; ++p) ok = ok && isfinite(M[p][N]);
   }
+  // a singular subspace: take the newest vector (a plain Jacobi step)
+  if (t < m) c[t] = ok ? M[t][N] : (t == m - 1 ? 1.0 : 0.0);
+  if (t == 0) small[SMALL_FLAG] = ok ? 0.0 : 1.0;
 }
 
 // t[x] = sum_k c_k vals[slot_k][x]
@@ -557,8 +580,12 @@ void reduce_rows(jues_ctx* ctx, const double* part, long PB, long count, int nq,
   JUES_HIP(hipGetLastError());
 }
 
-void diis_solve(jues_ctx* ctx, double* small, const DiisOrder& ord) {
-  hipLaunchKernelGGL(diis_solve_kernel, dim3(1), dim3(64), 0, ctx->stream, small, ord);
+void diis_solve(jues_ctx* ctx, double* small, const DiisOrder& ord, const double* part, long PB) {
+  // up to 8192 partial sums take the solve's own workgroup under 2 us; more are spread over a launch of their own
+  const bool fused = PB * (2 + ord.nold) <= 8192;
+  if (!fused) reduce_rows(ctx, part, PB, PB, 2 + ord.nold, small);
+  hipLaunchKernelGGL(diis_solve_kernel, dim3(1), dim3(fused ? 256 : 64), 0, ctx->stream, small, ord,
+                     fused ? part : nullptr, PB);
   JUES_HIP(hipGetLastError());
 }
 

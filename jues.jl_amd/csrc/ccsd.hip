@@ -354,6 +354,7 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
   W.out_H = H;
   W.out_Y = Y;
   W.out_S = WJ;
+  W.out_X = X2;
 }
 
 template void rccsd_contractions<double>(jues_ctx*, CCState&, const double*, const double*);
