@@ -139,7 +139,8 @@ struct CCState {
   std::unique_ptr<CCWork<float>> w32;
   std::unique_ptr<SplitState> sp;
   std::unique_ptr<DCState> dc;
-  bool split_on = false;  // the FP32 stage runs its ring / pp-ladder products on split-FP16 MFMA
+  bool fast16 = false;    // the fast stage is the split-FP16 one
+  bool split_on = false;  // ... and its ring / pp-ladder products run on split-FP16 MFMA
   bool ladder_recompute = false;  // <ab|ef> rebuilt from factors every iteration instead of stored
   hipEvent_t ev[2] = {nullptr, nullptr};
   double lambda = 1.0;  // coupling of the equations being iterated
@@ -203,6 +204,12 @@ template <typename T>
 void fac_lov_y2(jues_ctx* ctx, CCState& S, const T* Y2, bool y2_right, T* C);
 template <typename T>
 void fac_y3_lvv(jues_ctx* ctx, CCState& S, const T* Y3, T* Q);
+// The split-FP16 stage runs its products on split planes from this ov on, below it in FP32 MFMA, which is the
+// more precise form: a product's operands have to be scaled and split first (a dozen extra launches and
+// 256-column padding).  Iterations, FP32 / split: RCCD 519 / 1005 us at ov = 1200, 1270 / 1197 at 1920,
+// 2837 / 1864 at 2700; RCCSD 1011 / 1662, 2071 / 2111, 4347 / 3196.
+constexpr long SPLIT_MIN_OV = 1900;
+
 // Whether the residual may be evaluated by the small system's launches (cc_small.hip), where they are faster than
 // the general form's in every precision.  FP64 iterations, general / small form: RCCD 111 / 67 us at ov = 192,
 // 136 / 128 at 336, 169 / 186 at 400; RCCSD 333 / 102 at 192, 387 / 176 at 336, 470 / 372 at 504.

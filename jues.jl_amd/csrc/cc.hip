@@ -946,7 +946,7 @@ void cc_iteration(jues_ctx* ctx, CCState& S, jues_iter_info* info) {
 
   S.iter += 1;
   info->iter = S.iter;
-  info->stage = sizeof(T) == 4 ? (S.split_on ? 2 : 1) : 0;
+  info->stage = sizeof(T) == 4 ? (S.fast16 ? 2 : 1) : 0;
   info->energy = h[0];
   info->delta_e = S.have_prev ? h[0] - S.E_prev : h[0];
   info->rnorm = std::sqrt(std::max(0.0, h[1]));
@@ -1141,7 +1141,8 @@ void cc_run(jues_ctx* ctx, CCState& S, int stage_prec, int nsteps, bool stop_on_
   if (stage_prec != S.last_stage) ensure_fp64_ints(ctx, S);
   S.last_stage = stage_prec;
   if (stage_prec != JUES_FP64) cc_make_ints32(ctx, S);
-  S.split_on = stage_prec == JUES_FP16X3_MIXED;
+  S.fast16 = stage_prec == JUES_FP16X3_MIXED;
+  S.split_on = S.fast16 && (long)S.o * S.v >= SPLIT_MIN_OV;
   int stall = 0;
   double best = 1e300;
   static const char* stage_name[3] = {"fp64", "fp32", "fp16x3"};
