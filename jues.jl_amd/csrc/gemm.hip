@@ -55,16 +55,32 @@ template <> __device__ inline float bload<float>(__amdgpu_buffer_rsrc_t r, int v
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
 }
 
+// Place of a workgroup in a launch of many batch entries or K chunks: x among an entry's gridDim.x workgroups and
+// the entry z.  Workgroups go to the 8 XCDs in turn, so a launch whose gridDim.z is a multiple of 8 (padded to
+// it by the host; entries past the last one return) is dealt so that an entry's workgroups stay on one XCD, whose L2
+// then holds the entry's operands once.  Dealt in turn, each L2 fetched nearly all of them: FP32 34 x 34 x 1227400
+// in 128 chunks took 357 us, 142 this way (60 at the copy rate).  Returns whether it was.
+__device__ inline bool entry_place(int& x, int& z) {
+  x = (int)blockIdx.x;
+  z = (int)blockIdx.z;
+  if (gridDim.z == 1 || gridDim.z % NXCD != 0) return false;
+  const long id = x + (long)gridDim.x * z, slot = id / NXCD;
+  x = (int)(slot % gridDim.x);
+  z = (int)(slot / gridDim.x) * NXCD + (int)(id % NXCD);
+  return true;
+}
+
 // Tile of workgroup pid of nwg, of which only the first tiles_m * tiles_n carry a tile (a launch
-// padded to a multiple of NXCD); false for the padding ids.
-__device__ inline bool tile_coords_bounded(int pid, int nwg, int tiles_m, int tiles_n, int& tm, int& tn) {
+// padded to a multiple of NXCD); false for the padding ids.  plain: the workgroups are on one XCD already.
+__device__ inline bool tile_coords_bounded(int pid, int nwg, int tiles_m, int tiles_n, int& tm, int& tn,
+                                           bool plain = false) {
   // XCD-aware remap (bijective for any nwg): consecutive hardware ids go to different XCDs; give
   // each XCD a contiguous block of logical tile ids
   const int per = (nwg + NXCD - 1) / NXCD;
   int tall = nwg % NXCD;
   if (tall == 0) tall = NXCD;
   const int xcd = pid % NXCD, loc = pid / NXCD;
-  const int p2 = xcd < tall ? xcd * per + loc : tall * per + (xcd - tall) * (per - 1) + loc;
+  const int p2 = plain ? pid : xcd < tall ? xcd * per + loc : tall * per + (xcd - tall) * (per - 1) + loc;
   if (p2 >= tiles_m * tiles_n) return false;
   // grouped ordering: GROUP_M tile-rows share each sweep over tile-columns
   const int group_size = GROUP_M * tiles_n;
@@ -98,6 +114,7 @@ struct GemmSide {
   const long* tab = nullptr;
   int inner = 1;
   long sG = 0;
+  int nz = 1;  // batch entries or K chunks of the launch
   // FP32 products that write an FP64 result (the OUT64 instantiation; C is not used there)
   double* C64 = nullptr;
 };
@@ -135,12 +152,14 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
   __shared__ __attribute__((aligned(16))) float Bs[2][BN * BK];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
-  const bool second = (int)blockIdx.x >= nt0;
+  int bx, bz;
+  const bool placed = entry_place(bx, bz), second = bx >= nt0;
   const GemmSide<float> g = second ? p1 : p0;
-  const int M = g.M, N = g.N, K = (int)blockIdx.z == (int)gridDim.z - 1 ? g.Klast : g.K;
+  const int M = g.M, N = g.N, K = bz == g.nz - 1 ? g.Klast : g.K;
+  if (bz >= g.nz) return;
   const long lda = g.lda, ldb = g.ldb, ldc = g.ldc;
-  const int grp = SEG ? (int)blockIdx.z / g.inner : 0;  // the table only in the SEG instantiations
-  const long zb = (long)blockIdx.z - (SEG ? (long)grp * g.inner : 0L);
+  const int grp = SEG ? bz / g.inner : 0;  // the table only in the SEG instantiations
+  const long zb = (long)bz - (SEG ? (long)grp * g.inner : 0L);
   const long* tab = SEG ? g.tab + 4L * grp : nullptr;
   const float* __restrict__ A = g.A + zb * g.sA + (SEG ? tab[0] : 0L);
   const float* __restrict__ B = g.B + zb * g.sB + (SEG ? tab[1] : 0L);
@@ -150,8 +169,8 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
   const float* A1 = SEG ? g.A1 + zb * g.sA + tab[2] : A;
   const float* B1 = SEG ? g.B1 + zb * g.sB + tab[3] : B;
   int tm, tn;
-  if (!tile_coords_bounded(second ? (int)blockIdx.x - nt0 : (int)blockIdx.x, second ? (int)gridDim.x - nt0 : nt0,
-                           g.tiles_m, g.tiles_n, tm, tn))
+  if (!tile_coords_bounded(second ? bx - nt0 : bx, second ? (int)gridDim.x - nt0 : nt0,
+                           g.tiles_m, g.tiles_n, tm, tn, placed))
     return;
   const int m0 = tm * BM, n0 = tn * BN;
 
@@ -329,7 +348,7 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
   compute((nk - 1) & 1);
 
   if constexpr (OUT64) {
-    double* __restrict__ C64 = g.C64 + (long)blockIdx.z * g.sC;
+    double* __restrict__ C64 = g.C64 + (long)bz * g.sC;
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
       const int m = m0 + wm * WT + i * 16 + (lane & 15);
@@ -405,12 +424,14 @@ __global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, 
   __shared__ __attribute__((aligned(16))) double Bs[2][BN * BK];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;  // 2 x (BT / 32) wavefronts of HT x 32
-  const bool second = (int)blockIdx.x >= nt0;
+  int bx, bz;
+  const bool placed = entry_place(bx, bz), second = bx >= nt0;
   const GemmSide<double> g = second ? p1 : p0;
-  const int M = g.M, N = g.N, K = (int)blockIdx.z == (int)gridDim.z - 1 ? g.Klast : g.K;
+  const int M = g.M, N = g.N, K = bz == g.nz - 1 ? g.Klast : g.K;
+  if (bz >= g.nz) return;
   const long lda = g.lda, ldb = g.ldb, ldc = g.ldc;
-  const int grp = SEG ? (int)blockIdx.z / g.inner : 0;  // the table only in the SEG instantiations
-  const long zb = (long)blockIdx.z - (SEG ? (long)grp * g.inner : 0L);
+  const int grp = SEG ? bz / g.inner : 0;  // the table only in the SEG instantiations
+  const long zb = (long)bz - (SEG ? (long)grp * g.inner : 0L);
   const long* tab = SEG ? g.tab + 4L * grp : nullptr;
   const double* __restrict__ A = g.A + zb * g.sA + (SEG ? tab[0] : 0L);
   const double* __restrict__ B = g.B + zb * g.sB + (SEG ? tab[1] : 0L);
@@ -420,8 +441,8 @@ __global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, 
   const double* A1 = SEG ? g.A1 + zb * g.sA + tab[2] : A;
   const double* B1 = SEG ? g.B1 + zb * g.sB + tab[3] : B;
   int tm, tn;
-  if (!tile_coords_bounded(second ? (int)blockIdx.x - nt0 : (int)blockIdx.x, second ? (int)gridDim.x - nt0 : nt0,
-                           g.tiles_m, g.tiles_n, tm, tn))
+  if (!tile_coords_bounded(second ? bx - nt0 : bx, second ? (int)gridDim.x - nt0 : nt0,
+                           g.tiles_m, g.tiles_n, tm, tn, placed))
     return;
   const int m0 = tm * BM, n0 = tn * BN;
   // A (and n-contiguous B) share: row am, k = 4 kq + u; k-contiguous B share: rows bn, bn + HT, chunk bc
@@ -646,13 +667,16 @@ __global__ __launch_bounds__(64 * NW) void gemm_direct_kernel(GemmSide<T> g, T a
   typedef T t4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
   __shared__ T red[NW][BN * BM];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int M = g.M, N = g.N, K = (int)blockIdx.z == (int)gridDim.z - 1 ? g.Klast : g.K;
+  int bx, bz;
+  const bool placed = entry_place(bx, bz);
+  if (bz >= g.nz) return;
+  const int M = g.M, N = g.N, K = bz == g.nz - 1 ? g.Klast : g.K;
   const long lda = g.lda, ldb = g.ldb;
-  const T* __restrict__ A = g.A + (long)blockIdx.z * g.sA;
-  const T* __restrict__ B = g.B + (long)blockIdx.z * g.sB;
-  T* __restrict__ C = g.C + (long)blockIdx.z * g.sC;
+  const T* __restrict__ A = g.A + (long)bz * g.sA;
+  const T* __restrict__ B = g.B + (long)bz * g.sB;
+  T* __restrict__ C = g.C + (long)bz * g.sC;
   int tm, tn;
-  if (!tile_coords_bounded((int)blockIdx.x, (int)gridDim.x, g.tiles_m, g.tiles_n, tm, tn)) return;
+  if (!tile_coords_bounded(bx, (int)gridDim.x, g.tiles_m, g.tiles_n, tm, tn, placed)) return;
   const int m0 = tm * BM, n0 = tn * BN, fr = lane & 15, fk = lane >> 4;
   const T *Ap[IM], *Bp[JN];
 #pragma unroll
@@ -1355,6 +1379,9 @@ struct GemmPlan {
 
 static inline long cdiv(long a, long b) { return (a + b - 1) / b; }
 
+// gridDim.z of a launch of nz entries (entry_place); at most 65528 entries
+static inline unsigned grid_z(int nz) { return (unsigned)(nz >= NXCD ? cdiv(nz, NXCD) * NXCD : nz); }
+
 static void form_tile(int form, long M, long N, long& bm, long& bn) {
   switch (form) {
     case TILE128: bm = bn = 128; break;
@@ -1402,7 +1429,12 @@ static double form_us(int form, long tiles, long slabs, double bytes) {
   const double hbm = bytes / 5.6e6;
   switch (form) {
     case TILE128: return 8.5 + std::max(hbm, (slabs + 1) * std::max(f == 1.0 ? 2.5 : 1.4, cu * 1.71 * f / 0.86));
-    case TILE64: return 7.0 + std::max(hbm, (slabs + 1) * std::max(f == 1.0 ? 0.8 : 0.72, cu * 0.427 * f / 0.8));
+    case TILE64: {
+      // twice TILE128's operand traffic: at 7.2 TB/s from the L2s it is what bounds a 6460^3 FP64 product
+      // (9.5 ms; 8.6 with 128x128 tiles)
+      const double cache = (double)tiles * slabs * 2048.0 * sizeof(T) / 7.2e6;
+      return 7.0 + std::max(std::max(hbm, cache), (slabs + 1) * std::max(f == 1.0 ? 0.8 : 0.72, cu * 0.427 * f / 0.8));
+    }
     case SHORT:
     case TALL: return 8.0 + std::max(hbm, (slabs + 1) * std::max(1.6 * f, cu * 1.28 * f / 0.75));
     default: {
@@ -1474,8 +1506,9 @@ static void tile_launch(jues_ctx* ctx, int form, bool tb, int kind, GemmSide<T> 
   const long nt0 = two ? (t0 + NXCD - 1) / NXCD * NXCD : t0;
   const long total = two ? nt0 + (long)p1.tiles_m * p1.tiles_n : t0;
   JUES_REQUIRE(total < (1L << 31), "gemm: too many tiles");
+  p0.nz = p1.nz = nb;
   if (!two) p1 = p0;
-  const dim3 grid((unsigned)total, 1, nb);
+  const dim3 grid((unsigned)total, 1, grid_z(nb));
   if constexpr (sizeof(T) == 4) {
 #define JUES_GEMM32(K_, TB_, TA_, SEG_, BT_)                                                                        \
   hipLaunchKernelGGL((gemm32_nn_kernel<K_, TB_, TA_, SEG_, false, BT_>), grid, dim3(NT), 0, ctx->stream, p0, p1,    \
@@ -1548,7 +1581,8 @@ static void short_launch(jues_ctx* ctx, bool tall, GemmSide<T> p, int nb, T alph
 
 template <typename T, bool TA, bool TB>
 static void direct_launch_ab(jues_ctx* ctx, int form, GemmSide<T> p, int nb, T alpha, T beta) {
-  const dim3 grid((unsigned)((long)p.tiles_m * p.tiles_n), 1, nb);
+  p.nz = nb;
+  const dim3 grid((unsigned)((long)p.tiles_m * p.tiles_n), 1, grid_z(nb));
 #define JUES_DIRECT(NW_, IM_, JN_)                                                                            \
   hipLaunchKernelGGL((gemm_direct_kernel<T, TA, TB, NW_, IM_, JN_>), grid, dim3(64 * NW_), 0, ctx->stream, p, \
                      alpha, beta)
@@ -1645,10 +1679,10 @@ static void gemm_impl(jues_ctx* ctx, bool ta, bool tb, long M, long N, long K, T
   const double flops = 2.0 * M * N * K * batch;
   const double bytes = (double)sizeof(T) * ((double)M * K + (double)K * N + (beta != T(0) ? 2.0 : 1.0) * M * N) * batch;
   KTimer timer(ctx, name, flops, bytes);
-  for (int b0 = 0; b0 < batch; b0 += 65535) {
+  for (int b0 = 0; b0 < batch; b0 += 65528) {
     const GemmSide<T> p = make_side<T>(M, N, K, A + (long)b0 * sA, lda, sA, B + (long)b0 * sB, ldb, sB,
                                        C + (long)b0 * sC, ldc, sC, plan.form);
-    form_launch<T>(ctx, plan.form, ta, tb, kind, p, std::min(batch - b0, 65535), alpha, beta);
+    form_launch<T>(ctx, plan.form, ta, tb, kind, p, std::min(batch - b0, 65528), alpha, beta);
   }
 }
 
@@ -1767,7 +1801,7 @@ void gemm_ksum(jues_ctx* ctx, bool tb, long M, long N, long K, const T* A0, cons
                long ldc, long sC, long sG, const char* tag) {
   if (M <= 0 || N <= 0 || groups <= 0 || inner <= 0) return;
   JUES_REQUIRE(M < (1L << 31) && N < (1L << 31) && 2 * K < (1L << 31), "gemm: dimension too large");
-  JUES_REQUIRE(K >= 16 && K % 16 == 0 && (long)groups * inner <= 65535, "gemm_ksum: bad contraction or batch");
+  JUES_REQUIRE(K >= 16 && K % 16 == 0 && (long)groups * inner <= 65528, "gemm_ksum: bad contraction or batch");
   JUES_REQUIRE(ldc >= M && lda >= M && ldb >= (tb ? N : K), "gemm: leading dimension too small");
   const long batch = (long)groups * inner;
   const double bytes = (double)sizeof(T) * batch * (2.0 * M * K + 2.0 * N * K + (beta != T(0) ? 2.0 : 1.0) * M * N);

@@ -211,10 +211,10 @@ void pt_offsets(int o, int v, int i, int j, int k, long* first, long* second, lo
   std::copy(x[2], x[2] + 4, third);
 }
 
-// Triples per group: as many as their W fit in 192 MB, at most 65535 / v (the products' launch grid)
+// Triples per group: as many as their W fit in 192 MB, at most 65528 / v (the products' launch grid)
 static inline long pt_group(long ntrip, int v, size_t elem) {
   const long fit = (192L << 20) / ((long)v * v * v * (long)elem);
-  return std::max(1L, std::min(std::min(ntrip, fit), 65535L / v));
+  return std::max(1L, std::min(std::min(ntrip, fit), 65528L / v));
 }
 
 // The amplitude columns of Pe/P2e and the amplitude half of Te, from T2 (device FP64).
