@@ -13,6 +13,7 @@ struct CCInts {
   DevBuf Kov;     // (ia|jb) at [i,a,j,b]
   DevBuf Ktov;    // (ib|ja) at [i,a,j,b]
   DevBuf Jov;     // (ij|ab) at [i,a,j,b]
+  DevBuf Lx;      // (ia|jb) - (ib|ja)/2 at [i,a,j,b], by its first use (ring_lx)
   DevBuf Kpp;     // <ij|ab> = (ia|jb) at [i,j,a,b]
   DevBuf Ka;      // <mn|ef> at [e,m,n,f]
   DevBuf oooo;    // <mn|ij> at [m,n,i,j]
@@ -54,9 +55,9 @@ struct CCWork {
   // RCCSD o v^3 terms through the factors: B1[m,P,e] / Y2[m,e,P] = sum_f t1[m,f] Lvv[e,f,P],
   // Y3[m,j,P] = sum_f Lov[m,f,P] t1[j,f], W1[i,e,P], g[P]; Zs / Zsp: slabs of (mf|ae)
   DevBuf B1, Y2, Y3, W1, gP, Zs, Zsp;
-  DevBuf UL;  // U Lov (ov x naux): the factored K U ring product
   // where the last residual evaluation left H, Y (ov layout) and, when the update kernel does
-  // not symmetrise them itself, S = H + Y^x + (H + Y^x)^T (the buffers may be shared)
+  // not symmetrise them itself, S = G + G^T of G = H + y_direct Y + Y^x (the buffers may be shared)
+  double y_direct = 0.0;
   T* out_H = nullptr;
   T* out_Y = nullptr;
   T* out_S = nullptr;
@@ -69,12 +70,11 @@ struct CCWork {
 // others hold integral matrices, split once.
 // The _T slots hold the full amplitudes' layouts beside those of the correction d in a
 // defect-correction iteration; SP_WE0 / SP_WJ0 hold the anchor's intermediates.
-// SP_LOV / SP_LOVT hold the ov x naux factor Lov and its transpose (the factored K U product);
-// SP_LOVAT the transpose of LovT[(a,i),P] (RCCSD's (mf|ae) slabs).
+// SP_LOV / SP_LOVT hold RCCSD's ov x naux factor Lov and its transpose, SP_LOVAT the transpose of LovT[(a,i),P] (RCCSD's (mf|ae) slabs).
 enum SplitSlot {
-  SP_TOV, SP_UOV, SP_TTOV, SP_WE, SP_WJ, SP_U2, SP_Q, SP_TPT, SP_TMT, SP_TQ, SP_TM, SP_WPT, SP_WMT,
-  SP_TOV_T, SP_UOV_T, SP_TTOV_T,
-  SPLIT_CONST = 16, SP_K = SPLIT_CONST, SP_KX, SP_VP, SP_VM, SP_KPT, SP_KMT, SP_LVVT, SP_LVVTT, SP_WE0, SP_WJ0,
+  SP_UOV, SP_TTOV, SP_WE, SP_WJ, SP_U2, SP_Q, SP_TPT, SP_TMT, SP_TQ, SP_TM, SP_WPT, SP_WMT,
+  SP_UOV_T, SP_TTOV_T,
+  SPLIT_CONST = 16, SP_LX = SPLIT_CONST, SP_KX, SP_VP, SP_VM, SP_KPT, SP_KMT, SP_LVVT, SP_LVVTT, SP_WE0, SP_WJ0,
   SP_LOV, SP_LOVT, SP_LOVAT, SPLIT_SLOTS
 };
 struct SplitState {
@@ -85,7 +85,6 @@ struct SplitState {
   };
   Entry e[SPLIT_SLOTS];
   Split16Buf vps, vms, tpc, tmc;  // per-slab planes of the recomputed ladder (never cached)
-  Split16Buf ult;                 // (U Lov)^T of the factored K U product (never cached)
   Split16Buf tppt, zsp;           // RCCSD's tau^T (once per iteration) and one (ef) x (a m) slab
   const void* tppt_src = nullptr;
   long tppt_stamp = -2;
@@ -95,17 +94,17 @@ struct SplitState {
 };
 
 // Defect-correction refinement of RCCD.  An FP64 iteration at the anchor t0 keeps its numerator
-// R0 = <ij|ab> + S(t0) + L(t0) and its intermediates WJ0, WE0 and the packed hole-hole W'0; the
+// R0 = <ij|ab> + S(t0) + L(t0) and its ring intermediates W0 (held as WJ0), WE0 and the packed hole-hole W'0; the
 // iterations in between solve D t = lambda (R0 + [R(t) - R(t0)]) with the bracket formed from
 // d = t - t0 (every product has d, or a difference linear in d, as one factor):
-//   dWJ = K U(d)/2 - Kx T(d)/2,  dWE = Kx Tx(d)/2 + D(Fae(d), Fmi(d))/2
-//   dH = T(d) WE0 + T(t) dWE + U(d) WJ0 + U(t) dWJ,   dY = Tx(d) WE0 + Tx(t) dWE
+//   dW = Lx U(d)/2 + D(Fae(d), Fmi(d))/4,  dWE = Kx Tx(d)/2 + D(Fae(d), Fmi(d))/2
+//   dH = U(d) W0 + U(t) dW (+ dY/2),       dY = Tx(d) WE0 + Tx(t) dWE
 //   dL = pp-ladder(d) + W'0 d + dW' t,  dW'[kl,ij] = sum_cd <kl|cd> d[ij,cd]
 // so that rounding in the inner stage's type scales with |d| rather than |t|.
 struct DCState {
   DevBuf t0, R0, d;             // FP64: anchor amplitudes, its numerator, t - t0
   DevBuf WJ0, WE0, Wpt0, Wmt0;  // anchor intermediates in the inner stage's type
-  DevBuf Tt, Ttt, Ut;           // ov layouts of the full amplitudes t
+  DevBuf Ttt, Ut;               // ov layouts of the full amplitudes t
   DevBuf Tpt, Tmt, Tqt;         // packed pairs of t (Tqt: Tpt with the (a,a) columns doubled)
   int inner_prec = -1;          // the type the anchor was captured in
   bool capture = false;         // the next FP64 iteration records an anchor
@@ -129,7 +128,6 @@ struct CCState {
   std::vector<int> active;   // DIIS slots, oldest first
   DevBuf R1;       // FP64 T1 residual numerator (RCCSD)
   bool ovvv_factored = false;  // RCCSD: the (ia|bc) terms through the factors (no o v^3 block)
-  bool k_factored = false;     // K = (ia|jb) = Lov Lov^T with Lov kept: K U as two naux-wide products
   DevBuf Co, Cv;               // device orbitals (frozen core removed), to rebuild FP64 blocks
   bool i64_thin = false;       // FP64 blocks other than <ij|ab> released during a fast stage
   int last_stage = -1;         // precision of the last cc_run stage
@@ -169,11 +167,8 @@ T* bufp_t(DevBuf& b, size_t n) {
 // operand is symmetric; slotA/slotB name the operands for the split-FP16 stage.
 template <typename T>
 void ring_mm(jues_ctx* ctx, CCState& S, T alpha, const T* A, int slotA, const T* B, int slotB, T beta, T* C);
-// C += alpha K B with K = (ia|jb) at [i,a,j,b] and B a symmetric (ov) x (ov) matrix: the full
-// ring product, or with factored integrals (K = Lov Lov^T) C += alpha Lov (B Lov)^T, two
-// products of 2 (ov)^2 naux flops instead of one of 2 (ov)^3
 template <typename T>
-void ring_k_mm(jues_ctx* ctx, CCState& S, T alpha, const T* B, int slotB, T* C);
+const T* ring_lx(jues_ctx* ctx, CCState& S);
 // Hole-hole ladder sum_kl W'[kl,ij] t[kl,ab], W' = Wp + <kl|cd> t[ij,cd], on packed pairs,
 // added into the pp-ladder's Lp / Lm (run after ladder_mm, whose Tp / Tm it reads).
 // Wp: [m,n,i,j], oooo plus any T1 terms.

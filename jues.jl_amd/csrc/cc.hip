@@ -111,7 +111,7 @@ bool ladder_recompute_mode(jues_ctx* ctx, const CCState& S, int mode, int prec) 
   const double vv = (double)S.P.npv * S.P.npv + (double)S.P.nmv * S.P.nmv;
   const int dm = S.opts.diis ? S.opts.diis_max : 1;
   const double stored = 8.0 * vv * (prec == JUES_FP64 ? 1.0 : 1.5);
-  const double other = 8.0 * N2 * (10 + 2 * dm) + (prec == JUES_FP64 ? 8.0 : 4.0) * N2 * 16 +
+  const double other = 8.0 * N2 * (10 + (S.method == 1 ? 1 : 0) + 2 * dm) + (prec == JUES_FP64 ? 8.0 : 4.0) * N2 * 16 +
                        (prec == JUES_FP16X3_MIXED ? 4.0 * N2 * 9 : 0.0);
   return stored + other > 0.85 * (double)free_b;
 }
@@ -148,7 +148,6 @@ void cc_build_ints(jues_ctx* ctx, CCState& S, const double* Co, const double* Cv
                  (long)v * v, 0, 0.0, Jc, oo, 0, 1, "setup_ints");
     gemm<double>(ctx, false, true, oo, oo, naux, 1.0, Loo.as<double>(), oo, 0, Loo.as<double>(), oo, 0, 0.0, Oc, oo,
                  0, 1, "setup_ints");
-    S.k_factored = true;
     if (S.method == 1 && small_system(S)) {
       // the small system's residual reads the whole blocks
       gemm<double>(ctx, false, true, oo, ov, naux, 1.0, Loo.as<double>(), oo, 0, Lov.as<double>(), ov, 0, 0.0,
@@ -169,7 +168,7 @@ void cc_build_ints(jues_ctx* ctx, CCState& S, const double* Co, const double* Cv
       if (!S.ladder_recompute) I.Lvv = std::move(Lvv);
     }
     sync(ctx);
-    I.Lov = std::move(Lov);
+    if (S.ovvv_factored) I.Lov = std::move(Lov);
   }
   if (ctx->gao.p && S.method == 1) {
     tei_transform_dev<double>(ctx, Co, o, Co, o, Co, o, Cv, v, bufp<double>(I.ooov_c, oo * ov));
@@ -268,8 +267,6 @@ SplitState& split_state(CCState& S) {
 // planes of operand X (rows x cols, leading dimension rows; with `trans`, of X^T
 // for X stored cols x rows) in `slot`.  Per-iteration slots are split on their
 // first use in an iteration, constant slots once.
-// Ttov holds the same values as Tov (a permutation of t), so its planes take Tov's scale when
-// Tov was split earlier in the same iteration.
 template <typename Ti>
 const Split16& split_operand(jues_ctx* ctx, CCState& S, int slot, const Ti* X, long rows, long cols,
                              bool trans = false) {
@@ -280,10 +277,8 @@ const Split16& split_operand(jues_ctx* ctx, CCState& S, int slot, const Ti* X, l
   // been released to make room)
   if (stamp == -1 && e.stamp == -1 && e.src) return e.buf.s;
   if (e.src != static_cast<const void*>(X) || e.stamp != stamp) {
-    const SplitState::Entry& tov = Z.e[SP_TOV];
-    const int* same = slot == SP_TTOV && !trans && tov.stamp == stamp && tov.src ? tov.buf.s.sexp : nullptr;
     if (trans) split16t<Ti>(ctx, X, rows, cols, cols, e.buf, "cc_split");
-    else split16<Ti>(ctx, X, rows, cols, rows, e.buf, "cc_split", same);
+    else split16<Ti>(ctx, X, rows, cols, rows, e.buf, "cc_split");
     e.src = X;
     e.stamp = stamp;
   }
@@ -313,35 +308,21 @@ void ring_mm<float>(jues_ctx* ctx, CCState& S, float alpha, const float* A, int 
   gemm16_tn(ctx, ov, ov, alpha, a, b, beta, C, ov, "cc_ring");
 }
 
+// Lx = K - Kx/2 of the ring products, made by their first use (a small system's launches do without)
 template <typename T>
-void ring_k_mm(jues_ctx* ctx, CCState& S, T alpha, const T* B, int slotB, T* C) {
-  if (!S.k_factored) {
-    ring_mm<T>(ctx, S, alpha, ints<T>(S).Kov.template as<T>(), SP_K, B, slotB, T(1), C);
-    return;
+const T* ring_lx(jues_ctx* ctx, CCState& S) {
+  CCInts<T>& I = ints<T>(S);
+  const long ov = (long)S.o * S.v, N2 = ov * ov;
+  if (!I.Lx.p) {
+    T* L = bufp<T>(I.Lx, N2);
+    JUES_HIP(hipMemcpyAsync(L, I.Kov.template as<T>(), N2 * sizeof(T), hipMemcpyDeviceToDevice, ctx->stream));
+    axpby<T>(ctx, N2, -0.5, I.Ktov.template as<T>(), 1.0, L);
   }
-  const long ov = (long)S.o * S.v, naux = ctx->naux;
-  const T* L = ints<T>(S).Lov.template as<T>();
-  T* UL = bufp<T>(work<T>(S).UL, (size_t)(ov * naux));
-  if constexpr (sizeof(T) == 4) {
-    if (S.split_on) {
-      // UL = B^T Lov (B symmetric: its planes are the TN kernel's left operand, shared with the
-      // later B WJ product); then C += alpha (Lov^T)^T (UL^T), both k = naux operands transposed
-      SplitState& Z = split_state(S);
-      const Split16& b = split_operand<float>(ctx, S, slotB, B, ov, ov);
-      const Split16& l = split_operand<double>(ctx, S, SP_LOV, S.i64->Lov.as<double>(), ov, naux);
-      gemm16_tn(ctx, ov, naux, 1.0f, b, l, 0.0f, UL, ov, "cc_ring_lr");
-      const Split16& lt = split_operand<double>(ctx, S, SP_LOVT, S.i64->Lov.as<double>(), naux, ov, true);
-      split16t<float>(ctx, UL, naux, ov, ov, Z.ult, "cc_split");
-      gemm16_tn(ctx, ov, ov, alpha, lt, Z.ult.s, 1.0f, C, ov, "cc_ring_lr");
-      return;
-    }
-  }
-  gemm<T>(ctx, false, false, ov, naux, ov, T(1), B, ov, 0, L, ov, 0, T(0), UL, ov, 0, 1, "cc_ring_lr");
-  gemm<T>(ctx, false, true, ov, ov, naux, alpha, L, ov, 0, UL, ov, 0, T(1), C, ov, 0, 1, "cc_ring_lr");
+  return I.Lx.template as<T>();
 }
 
-template void ring_k_mm<double>(jues_ctx*, CCState&, double, const double*, int, double*);
-template void ring_k_mm<float>(jues_ctx*, CCState&, float, const float*, int, float*);
+template const double* ring_lx<double>(jues_ctx*, CCState&);
+template const float* ring_lx<float>(jues_ctx*, CCState&);
 
 template <typename T>
 void ovvv_z_slab(jues_ctx* ctx, CCState& S, int m0, int cnt, const T* LovT, const T* Lvv, const T* Tpp, T* Zs,
@@ -626,7 +607,6 @@ void rccd_contractions(jues_ctx* ctx, CCState& S, const double* t2) {
   const std::vector<long> d4 = {o, o, v, v};
   T* Tpp = bufp<T>(W.Tpp, N2);
   T* Upp = bufp<T>(W.Upp, N2);
-  T* Tov = bufp<T>(W.Tov, N2);
   T* Ttov = bufp<T>(W.Ttov, N2);
   T* Uov = bufp<T>(W.Uov, N2);
   T* Ua = bufp<T>(W.Ua, N2);
@@ -644,8 +624,8 @@ void rccd_contractions(jues_ctx* ctx, CCState& S, const double* t2) {
   const T one = T(1), zero = T(0), half = T(0.5);
 
   // amplitudes in the compute type and the layouts the GEMMs read
-  // Tpp = t, Upp = 2t - t^(ij), Tov = T[i,a,j,b], Ttov = t[i,j,b,a] at [i,a,j,b], Uov = U[i,a,j,b]
-  rccd_layouts<T>(ctx, t2, o, v, Tpp, Upp, Tov, Ttov, Uov);
+  // Tpp = t, Upp = 2t - t^(ij), Ttov = t[i,j,b,a] at [i,a,j,b], Uov = U[i,a,j,b]
+  rccd_layouts<T>(ctx, t2, o, v, Tpp, Upp, Ttov, Uov);
   permute<T, T>(ctx, Upp, d4, {2, 0, 1, 3}, Ua, 1.0, 0.0, "cc_prep");     // U[a,m,n,f]
 
   // Fae[a,e] = -sum U[a,(mnf)] K[e,(mnf)];  Fmi[m,i] = sum K[m,(nef)] U[i,(nef)], kept transposed
@@ -657,32 +637,33 @@ void rccd_contractions(jues_ctx* ctx, CCState& S, const double* t2) {
   ladder_mm<T>(ctx, S, t2, Tp, Tm, Lp, Lm);
   JUES_HIP(hipMemcpyAsync(Wp, I.oooo.p, oo * oo * sizeof(T), hipMemcpyDeviceToDevice, ctx->stream));
   hh_mm<T>(ctx, S, Wp, Tp, Tm, Lp, Lm);
-  // ring terms (every left operand is a symmetric (ov) x (ov) matrix)
-  const T* K = I.Kov.template as<T>();
-  const T* Kx = I.Ktov.template as<T>();
-  JUES_HIP(hipMemcpyAsync(WJ, K, N2 * sizeof(T), hipMemcpyDeviceToDevice, ctx->stream));
-  ring_k_mm<T>(ctx, S, half, Uov, SP_UOV, WJ);
-  ring_mm<T>(ctx, S, -half, Kx, SP_KX, Tov, SP_TOV, one, WJ);
-  permute<T, T>(ctx, I.Jov.template as<T>(), {ov, ov}, {0, 1}, WE, -1.0, 0.0, "cc_prep");
-  ring_mm<T>(ctx, S, half, Kx, SP_KX, Ttov, SP_TTOV, one, WE);
+  // Ring terms in four products (every left operand is a symmetric (ov) x (ov) matrix).  With T = (U + Tx)/2,
+  // U = 2T - Tx, the terms T WE + U WJ, WE = -J + Kx Tx/2, WJ = K + K U/2 - Kx T/2, are U W + Tx WE/2 with
+  // W = WJ + WE/2 = K - J/2 + (K - Kx/2) U/2, and Tx WE is the exchange ring term's product Y.  Written out they
+  // are six products, or five and two naux-wide ones with K U from the factors: FP64 1540 us at ov = 2000 and
+  // naux = 360, where these four take 1125.
   // Fock-like terms t.Fae^T - Fmi^T.t, carried by WE: with D[kc,jb] = delta_kj Fae[b,c] -
   // delta_cb Fmi[k,j], T D and (Tx D)^x each give half of them, up to a transpose that
-  // S = H + H^T absorbs
-  fock_dress<T>(ctx, WE, Fae, Fmi, o, v, half);
-  ring_mm<T>(ctx, S, one, Tov, SP_TOV, WE, SP_WE, zero, H);
-  ring_mm<T>(ctx, S, one, Uov, SP_UOV, WJ, SP_WJ, one, H);
-  // exchange ring term t[m,i,b,e] WmBEj[m,a,e,j] = (Tx WE)[ib,ja]
+  // S = G + G^T absorbs
+  const T* Kx = I.Ktov.template as<T>();
+  ring_start<T>(ctx, I.Kov.template as<T>(), T(-1), I.Jov.template as<T>(), Fae, Fmi, o, v, WE, WJ);
+  ring_mm<T>(ctx, S, half, ring_lx<T>(ctx, S), SP_LX, Uov, SP_UOV, one, WJ);
+  ring_mm<T>(ctx, S, half, Kx, SP_KX, Ttov, SP_TTOV, one, WE);
+  ring_mm<T>(ctx, S, one, Uov, SP_UOV, WJ, SP_WJ, zero, H);
+  // exchange ring term t[m,i,b,e] WmBEj[m,a,e,j] = (Tx WE)[ib,ja], and half the direct one
   ring_mm<T>(ctx, S, one, Ttov, SP_TTOV, WE, SP_WE, zero, Y);
   // an FP64 iteration that anchors a defect correction keeps WJ, WE and W' (before WJ is reused)
   if constexpr (sizeof(T) == 8)
     if (S.dc && S.dc->capture) dc_capture(ctx, S, WJ, WE, W.Wpt.template as<T>(), W.Wmt.template as<T>());
-  // S = H + Y^x + (H + Y^x)^T: summed by the update kernel, or here (into WJ) when its LDS slab
+  // S = G + G^T, G = H + Y/2 + Y^x: summed by the update kernel, or here (into WJ) when its LDS slab
   // would not fit
   if (!fused_sym(o, sizeof(T))) {
+    axpby<T>(ctx, N2, 0.5, Y, 1.0, H);
     permute<T, T>(ctx, Y, {o, v, o, v}, {0, 3, 2, 1}, H, 1.0, 1.0, "cc_sym");
     JUES_HIP(hipMemcpyAsync(WJ, H, N2 * sizeof(T), hipMemcpyDeviceToDevice, ctx->stream));
     permute<T, T>(ctx, H, {ov, ov}, {1, 0}, WJ, 1.0, 1.0, "cc_sym");
   }
+  W.y_direct = 0.5;
   W.out_H = H;
   W.out_Y = Y;
   W.out_S = WJ;
@@ -773,7 +754,6 @@ void rccd_delta_contractions(jues_ctx* ctx, CCState& S, const double* t2) {
   axpby<double>(ctx, N2, -1.0, D.t0.as<double>(), 1.0, d);
   T* Tpp = bufp<T>(W.Tpp, N2);
   T* Upp = bufp<T>(W.Upp, N2);
-  T* Tov = bufp<T>(W.Tov, N2);
   T* Ttov = bufp<T>(W.Ttov, N2);
   T* Uov = bufp<T>(W.Uov, N2);
   T* Ua = bufp<T>(W.Ua, N2);
@@ -787,7 +767,6 @@ void rccd_delta_contractions(jues_ctx* ctx, CCState& S, const double* t2) {
   T* Tm = bufp<T>(W.Tm, std::max(1L, S.P.nmo * S.P.nmv));
   T* Lp = bufp<T>(W.Lp, S.P.npo * S.P.npv);
   T* Lm = bufp<T>(W.Lm, std::max(1L, S.P.nmo * S.P.nmv));
-  T* Tt = bufp<T>(D.Tt, N2);
   T* Ttt = bufp<T>(D.Ttt, N2);
   T* Ut = bufp<T>(D.Ut, N2);
   const T* WJ0 = D.WJ0.as<T>();
@@ -795,8 +774,8 @@ void rccd_delta_contractions(jues_ctx* ctx, CCState& S, const double* t2) {
   const T one = T(1), zero = T(0), half = T(0.5);
 
   // layouts of d (as rccd_contractions makes those of t) and the ring layouts of t
-  rccd_layouts<T>(ctx, d, o, v, Tpp, Upp, Tov, Ttov, Uov);
-  rccd_layouts<T>(ctx, t2, o, v, nullptr, nullptr, Tt, Ttt, Ut);
+  rccd_layouts<T>(ctx, d, o, v, Tpp, Upp, Ttov, Uov);
+  rccd_layouts<T>(ctx, t2, o, v, nullptr, nullptr, Ttt, Ut);
   permute<T, T>(ctx, Upp, d4, {2, 0, 1, 3}, Ua, 1.0, 0.0, "cc_prep");
   // Fae, Fmi are linear in t: their values at d
   gemm<T>(ctx, false, true, v, v, oo * v, T(-1), Ua, v, 0, I.Ka.template as<T>(), v, 0, zero, Fae, v, 0, 1, "cc_fock");
@@ -804,24 +783,23 @@ void rccd_delta_contractions(jues_ctx* ctx, CCState& S, const double* t2) {
   // ladders: pp-ladder of d (linear), hole-hole W'0 d + dW' t
   ladder_mm<T>(ctx, S, d, Tp, Tm, Lp, Lm);
   hh_delta_mm<T>(ctx, S, Tp, Tm, t2, Lp, Lm);
-  // dWJ = K U(d)/2 - Kx T(d)/2,  dWE = Kx Tx(d)/2 + D(Fae(d), Fmi(d))/2
-  const T* Kx = I.Ktov.template as<T>();
-  ring_mm<T>(ctx, S, -half, Kx, SP_KX, Tov, SP_TOV, zero, WJ);
-  ring_k_mm<T>(ctx, S, half, Uov, SP_UOV, WJ);
-  ring_mm<T>(ctx, S, half, Kx, SP_KX, Ttov, SP_TTOV, zero, WE);
+  // dW = Lx U(d)/2 + D(Fae(d), Fmi(d))/4,  dWE = Kx Tx(d)/2 + D(Fae(d), Fmi(d))/2
+  ring_mm<T>(ctx, S, half, ring_lx<T>(ctx, S), SP_LX, Uov, SP_UOV, zero, WJ);
+  fock_dress<T>(ctx, WJ, Fae, Fmi, o, v, T(0.25));
+  ring_mm<T>(ctx, S, half, I.Ktov.template as<T>(), SP_KX, Ttov, SP_TTOV, zero, WE);
   fock_dress<T>(ctx, WE, Fae, Fmi, o, v, half);
-  // dH = T(d) WE0 + U(d) WJ0 + T(t) dWE + U(t) dWJ,  dY = Tx(d) WE0 + Tx(t) dWE
-  ring_mm<T>(ctx, S, one, Tov, SP_TOV, WE0, SP_WE0, zero, H);
-  ring_mm<T>(ctx, S, one, Uov, SP_UOV, WJ0, SP_WJ0, one, H);
-  ring_mm<T>(ctx, S, one, Tt, SP_TOV_T, WE, SP_WE, one, H);
+  // dH = U(d) W0 + U(t) dW,  dY = Tx(d) WE0 + Tx(t) dWE
+  ring_mm<T>(ctx, S, one, Uov, SP_UOV, WJ0, SP_WJ0, zero, H);
   ring_mm<T>(ctx, S, one, Ut, SP_UOV_T, WJ, SP_WJ, one, H);
   ring_mm<T>(ctx, S, one, Ttov, SP_TTOV, WE0, SP_WE0, zero, Y);
   ring_mm<T>(ctx, S, one, Ttt, SP_TTOV_T, WE, SP_WE, one, Y);
   if (!fused_sym(o, sizeof(T))) {
+    axpby<T>(ctx, N2, 0.5, Y, 1.0, H);
     permute<T, T>(ctx, Y, {o, v, o, v}, {0, 3, 2, 1}, H, 1.0, 1.0, "cc_sym");
     JUES_HIP(hipMemcpyAsync(WJ, H, N2 * sizeof(T), hipMemcpyDeviceToDevice, ctx->stream));
     permute<T, T>(ctx, H, {ov, ov}, {1, 0}, WJ, 1.0, 1.0, "cc_sym");
   }
+  W.y_direct = 0.5;
   W.out_H = H;
   W.out_Y = Y;
   W.out_S = WJ;
@@ -875,6 +853,7 @@ void cc_iteration(jues_ctx* ctx, CCState& S, jues_iter_info* info) {
     JUES_HIP(hipMemcpyAsync(bufp<double>(dc->t0, N2), t, N2 * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
   CCWork<T>& W = work<T>(S);
   W.out_X = nullptr;
+  W.y_direct = 0.0;
   if (small_system(S) && !S.dc && !S.fock_on) small_contractions<T>(ctx, S);
   else if (S.method == 0) {
     if (dc_on) rccd_delta_contractions<T>(ctx, S, t);
@@ -893,6 +872,7 @@ void cc_iteration(jues_ctx* ctx, CCState& S, jues_iter_info* info) {
   if (fused_sym(o, sizeof(T))) {
     A.H = W.out_H;
     A.Y = W.out_Y;
+    A.y_direct = W.y_direct;
   } else {
     A.S = W.out_S;
   }
@@ -1105,7 +1085,7 @@ static void thin_fp64_ints(jues_ctx* ctx, CCState& S) {
   if (!force && (double)free_b >= 0.15 * (double)total_b) return;
   sync(ctx);
   CCInts<double>& I = *S.i64;
-  for (DevBuf* b : {&I.Kov, &I.Ktov, &I.Jov, &I.Ka, &I.oooo, &I.Vp, &I.Vm, &I.KP, &I.KM, &I.ooov_c, &I.ovvv_c,
+  for (DevBuf* b : {&I.Kov, &I.Ktov, &I.Jov, &I.Lx, &I.Ka, &I.oooo, &I.Vp, &I.Vm, &I.KP, &I.KM, &I.ooov_c, &I.ovvv_c,
                     &I.Lov, &I.LovT, &I.Lovp, &I.Lvv, &I.Lvvt})
     b->release();
   S.i64_thin = true;

@@ -27,7 +27,8 @@ struct UpdateArgs {
   const double* Lener;  // 2<ij|ab> - <ji|ab> (FP64, ijab)
   const TR* S;          // ring + Fock-like terms, symmetrised, ov layout [i,a,j,b]; or null with:
   const TR* H;          //   H and Y (ov layout): S[ia,jb] = H[ia,jb] + Y[ib,ja] + H[jb,ia] + Y[ja,ib],
-  const TR* Y;          //   summed by the update kernel itself (fused_sym)
+  const TR* Y;          //   summed by the update kernel itself (fused_sym), with
+  double y_direct;      //   y_direct (Y[ia,jb] + Y[jb,ia]) added
   const TR* Lp;         // packed ladders (pp + hh), symmetric part
   const TR* Lm;         // packed ladders (pp + hh), antisymmetric part
   const TR* extra;      // any further ijab-ordered residual terms (RCCSD), may be null
@@ -79,13 +80,15 @@ void pack_khh(jues_ctx* ctx, const PairTables& P, const double* K, int o, int v,
 // W[m,n,i,j] -> WPT[(i<=j),(k<=l)], WMT[(i<j),(k<l)] (the kl-pair sum / difference, transposed)
 template <typename T>
 void pack_whh(jues_ctx* ctx, const PairTables& P, const T* W, int o, T* WPT, T* WMT);
-// RCCD amplitude layouts from FP64 t2 [i,j,a,b]: Tpp = t, Upp = 2t - t^(ij), Tov[i,a,j,b] = t,
-// Ttov[i,a,j,b] = t[i,j,b,a], Uov[i,a,j,b] = U[i,j,a,b]; Tpp and Upp may be null
+// RCCD amplitude layouts from FP64 t2 [i,j,a,b]: Tpp = t, Upp = 2t - t^(ij), Ttov[i,a,j,b] = t[i,j,b,a], Uov[i,a,j,b] = U[i,j,a,b]; Tpp and Upp may be null
 template <typename T>
-void rccd_layouts(jues_ctx* ctx, const double* t, int o, int v, T* Tpp, T* Upp, T* Tov, T* Ttov, T* Uov);
+void rccd_layouts(jues_ctx* ctx, const double* t, int o, int v, T* Tpp, T* Upp, T* Ttov, T* Uov);
 // WE[(k,c),(j,b)] += s (delta_kj Fae[b,c] - delta_cb Fmi[k,j]) (ov layout; FmiT[j,k] = Fmi[k,j])
 template <typename T>
 void fock_dress(jues_ctx* ctx, T* WE, const T* Fae, const T* FmiT, int o, int v, T s);
+// WE = s X + D/2 and W = K + WE/2 with D[(k,c),(j,b)] = delta_kj Fae[b,c] - delta_cb Fmi[k,j]; X may be WE
+template <typename T>
+void ring_start(jues_ctx* ctx, const T* K, T s, const T* X, const T* Fae, const T* FmiT, int o, int v, T* WE, T* W);
 // Tq = Tp with its (a,a) columns doubled
 template <typename T>
 void pair_diag2(jues_ctx* ctx, const PairTables& P, const T* Tp, T* Tq);

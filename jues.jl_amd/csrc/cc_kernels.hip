@@ -140,15 +140,35 @@ __global__ __launch_bounds__(256) void fock_dress_kernel(T* __restrict__ WE, con
   }
 }
 
+// Start of the ring intermediates: WE = s X + D/2 and W = K + WE/2, D as in fock_dress_kernel (X may be WE).
+// One pass at the copy rate in place of a copy, a scaled copy and the two dressings.
+template <typename T>
+__global__ __launch_bounds__(256) void ring_start_kernel(const T* __restrict__ K, T s, const T* X,
+                                                         const T* __restrict__ Fae, const T* __restrict__ FmiT, int o,
+                                                         int v, T* WE, T* __restrict__ W) {
+  const int ov = o * v;
+  for (int jb = blockIdx.x; jb < ov; jb += gridDim.x) {
+    const int j = jb % o, b = jb / o;
+    for (int kc = threadIdx.x; kc < ov; kc += 256) {
+      const int k = kc % o, c = kc / o;
+      const long x = kc + (long)ov * jb;
+      T w = s * X[x];
+      if (k == j) w += T(0.5) * Fae[b + (long)v * c];
+      if (c == b) w -= T(0.5) * FmiT[j + (long)o * k];
+      WE[x] = w;
+      W[x] = K[x] + T(0.5) * w;
+    }
+  }
+}
+
 // The RCCD residual's amplitude layouts from t2 (FP64, [i,j,a,b]) in one pass:
-// Tpp = t, Upp = 2t - t^(ij) ([i,j,a,b]); Tov[i,a,j,b] = t[ijab]; Uov[i,a,j,b] = U[ijab];
+// Tpp = t, Upp = 2t - t^(ij) ([i,j,a,b]); Uov[i,a,j,b] = U[ijab];
 // Ttov[i,b,j,a] = t[ijab] (that is t[i,j,b,a] at [i,a,j,b]).  Threads run i fastest, so
 // every write is a contiguous run of o; the exchanged read t[jiab] stays in one o x o slab.
 template <typename T>
 __global__ __launch_bounds__(256) void rccd_layouts_kernel(const double* __restrict__ t, int o, int v,
                                                            T* __restrict__ Tpp, T* __restrict__ Upp,
-                                                           T* __restrict__ Tov, T* __restrict__ Ttov,
-                                                           T* __restrict__ Uov) {
+                                                           T* __restrict__ Ttov, T* __restrict__ Uov) {
   const long oo = (long)o * o, ov = (long)o * v, n = oo * v * v;
   for (long x = blockIdx.x * 256L + threadIdx.x; x < n; x += (long)gridDim.x * 256L) {
     const long ij = x % oo, ab = x / oo;
@@ -159,7 +179,6 @@ __global__ __launch_bounds__(256) void rccd_layouts_kernel(const double* __restr
     if (Tpp) Tpp[x] = (T)tv;
     if (Upp) Upp[x] = (T)u;
     const long y = i + (long)o * a + ov * (j + (long)o * b);
-    Tov[y] = (T)tv;
     Uov[y] = (T)u;
     Ttov[i + (long)o * b + ov * (j + (long)o * a)] = (T)tv;
   }
@@ -171,8 +190,7 @@ __global__ __launch_bounds__(256) void rccd_layouts_kernel(const double* __restr
 template <typename T>
 __global__ __launch_bounds__(256) void rccd_layouts_slab_kernel(const double* __restrict__ t, int o, int v,
                                                                 T* __restrict__ Tpp, T* __restrict__ Upp,
-                                                                T* __restrict__ Tov, T* __restrict__ Ttov,
-                                                                T* __restrict__ Uov) {
+                                                                T* __restrict__ Ttov, T* __restrict__ Uov) {
   extern __shared__ double slab[];  // slab[i + (o + 1) j] = t[i,j,a,b]
   const int oo = o * o, ld = o + 1;
   const long ov = (long)o * v, vv = (long)v * v;
@@ -189,7 +207,6 @@ __global__ __launch_bounds__(256) void rccd_layouts_slab_kernel(const double* __
       if (Tpp) Tpp[ab * oo + q] = (T)tv;
       if (Upp) Upp[ab * oo + q] = (T)u;
       const long y = i + (long)o * a + ov * (j + (long)o * b);
-      Tov[y] = (T)tv;
       Uov[y] = (T)u;
       Ttov[i + (long)o * b + ov * (j + (long)o * a)] = (T)tv;
     }
@@ -227,11 +244,13 @@ __global__ __launch_bounds__(256) void t2_update_kernel(UpdateArgs<TR> A) {
   extern __shared__ __attribute__((aligned(16))) unsigned char dyn_lds[];
   TR* slab = reinterpret_cast<TR*>(dyn_lds);
   const int ld = o + 1;
+  // (each of Y's two o x o blocks serves an exchanged and a direct term)
+  const TR yd = (TR)A.y_direct;
   if (A.H) {
     for (int q = threadIdx.x; q < (int)oo; q += 256) {
       const int j = q % o, i = q / o;
-      slab[j + ld * i] = A.H[(long)j + (long)o * b + ov * ((long)i + (long)o * a)] +
-                         A.Y[(long)j + (long)o * a + ov * ((long)i + (long)o * b)];
+      const long ba = (long)j + (long)o * b + ov * ((long)i + (long)o * a);
+      slab[j + ld * i] = A.H[ba] + A.Y[(long)j + (long)o * a + ov * ((long)i + (long)o * b)] + yd * A.Y[ba];
     }
     __syncthreads();
   }
@@ -240,9 +259,11 @@ __global__ __launch_bounds__(256) void t2_update_kernel(UpdateArgs<TR> A) {
     const long x = (long)ij + oo * ab;
     double R = A.Kpp[x];
     if (A.S) R += (double)A.S[(long)i + (long)o * a + ov * ((long)j + (long)o * b)];
-    if (A.H)
-      R += (double)A.H[(long)i + (long)o * a + ov * ((long)j + (long)o * b)] +
-           (double)A.Y[(long)i + (long)o * b + ov * ((long)j + (long)o * a)] + (double)slab[j + ld * i];
+    if (A.H) {
+      const long iajb = (long)i + (long)o * a + ov * ((long)j + (long)o * b);
+      R += (double)A.H[iajb] + (double)A.Y[(long)i + (long)o * b + ov * ((long)j + (long)o * a)] +
+           A.y_direct * (double)A.Y[iajb] + (double)slab[j + ld * i];
+    }
     if (A.Lp) {
       const long pp = i <= j ? (long)i + (long)j * (j + 1) / 2 : (long)j + (long)i * (i + 1) / 2;
       R += (double)A.Lp[pp + A.npo * qp];
@@ -525,19 +546,28 @@ void fock_dress(jues_ctx* ctx, T* WE, const T* Fae, const T* FmiT, int o, int v,
 }
 
 template <typename T>
-void rccd_layouts(jues_ctx* ctx, const double* t, int o, int v, T* Tpp, T* Upp, T* Tov, T* Ttov, T* Uov) {
+void ring_start(jues_ctx* ctx, const T* K, T s, const T* X, const T* Fae, const T* FmiT, int o, int v, T* WE, T* W) {
+  const long n = (long)o * v * o * v;
+  KTimer k(ctx, "cc_prep", 0.0, (double)n * 4.0 * sizeof(T));
+  hipLaunchKernelGGL((ring_start_kernel<T>), dim3((unsigned)std::min((long)o * v, 1L << 20)), dim3(256), 0, ctx->stream, K, s, X, Fae, FmiT, o, v,
+                     WE, W);
+  JUES_HIP(hipGetLastError());
+}
+
+template <typename T>
+void rccd_layouts(jues_ctx* ctx, const double* t, int o, int v, T* Tpp, T* Upp, T* Ttov, T* Uov) {
   const long n = (long)o * o * v * v;
   const size_t slab = (size_t)o * (o + 1) * sizeof(double);
   // t is read once through the LDS slab, twice (direct and exchanged) otherwise
-  const double outs = 3.0 + (Tpp ? 1.0 : 0.0) + (Upp ? 1.0 : 0.0);
+  const double outs = 2.0 + (Tpp ? 1.0 : 0.0) + (Upp ? 1.0 : 0.0);
   KTimer k(ctx, "cc_prep", 0.0, (double)n * ((slab <= 65536 ? 8.0 : 16.0) + outs * sizeof(T)));
   if (slab <= 65536) {
     const long vv = (long)v * v;
     hipLaunchKernelGGL((rccd_layouts_slab_kernel<T>), dim3((unsigned)std::min(vv, 1L << 20)), dim3(256), slab,
-                       ctx->stream, t, o, v, Tpp, Upp, Tov, Ttov, Uov);
+                       ctx->stream, t, o, v, Tpp, Upp, Ttov, Uov);
   } else {
-    hipLaunchKernelGGL((rccd_layouts_kernel<T>), dim3(grid256(n)), dim3(256), 0, ctx->stream, t, o, v, Tpp, Upp, Tov,
-                       Ttov, Uov);
+    hipLaunchKernelGGL((rccd_layouts_kernel<T>), dim3(grid256(n)), dim3(256), 0, ctx->stream, t, o, v, Tpp, Upp, Ttov,
+                       Uov);
   }
   JUES_HIP(hipGetLastError());
 }
@@ -604,8 +634,12 @@ void divide_d2(jues_ctx* ctx, double* t, const double* eps, int o, int v, double
 
 template void fock_dress<double>(jues_ctx*, double*, const double*, const double*, int, int, double);
 template void fock_dress<float>(jues_ctx*, float*, const float*, const float*, int, int, float);
-template void rccd_layouts<double>(jues_ctx*, const double*, int, int, double*, double*, double*, double*, double*);
-template void rccd_layouts<float>(jues_ctx*, const double*, int, int, float*, float*, float*, float*, float*);
+template void ring_start<double>(jues_ctx*, const double*, double, const double*, const double*, const double*, int,
+                                 int, double*, double*);
+template void ring_start<float>(jues_ctx*, const float*, float, const float*, const float*, const float*, int, int,
+                                float*, float*);
+template void rccd_layouts<double>(jues_ctx*, const double*, int, int, double*, double*, double*, double*);
+template void rccd_layouts<float>(jues_ctx*, const double*, int, int, float*, float*, float*, float*);
 template void pack_whh<double>(jues_ctx*, const PairTables&, const double*, int, double*, double*);
 template void pack_whh<float>(jues_ctx*, const PairTables&, const float*, int, float*, float*);
 template void pair_diag2<double>(jues_ctx*, const PairTables&, const double*, double*);

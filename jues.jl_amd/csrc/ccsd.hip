@@ -305,22 +305,14 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
   }
 
   // ---- ring terms -----------------------------------------------------------------------
-  JUES_HIP(hipMemcpyAsync(WJ, Kov, N2 * sizeof(T), hipMemcpyDeviceToDevice, ctx->stream));
-  // every left operand of the ring products is a symmetric (ov) x (ov) matrix
-  ring_k_mm<T>(ctx, S, half, U2, SP_U2, WJ);
-  ring_mm<T>(ctx, S, -half, Kx, SP_KX, Tov, SP_TOV, one, WJ);
-  // WJ[me,jb] += sum_f t1[jf] (me|bf)
-  if (fac) fac_lov_y2<T>(ctx, S, Y2, true, WJ);
-  else contract<T>(ctx, 1.0, TN(t1, "jf"), TN(ovvv, "mebf"), 1.0, TN(WJ, "mejb"), "cc_t1");
-  // (H is free until the ring products: the [b,j,m,e] product of the ooov terms goes there)
-  contract<T>(ctx, -1.0, TN(t1, "nb"), TN(ooov, "njme"), 1.0, TN(WJ, "mejb"), "cc_t1", H, N2);
+  // (as in RCCD, with U2 = 2 T - Q: W = WJ + WE/2 = K - J/2 + (K - Kx/2) U2/2 and the T1 terms of WJ and half of
+  // WE's, H = U W + Y/2; every left operand of the ring products is a symmetric (ov) x (ov) matrix)
   permute<T, T>(ctx, Jov, {ov, ov}, {0, 1}, WE, -1.0, 0.0, "cc_prep");
-  ring_mm<T>(ctx, S, half, Kx, SP_KX, Q, SP_Q, one, WE);
-  // WE[me,jb] -= sum_f t1[jf] (mf|be): with factors, Q[(mj),(be)] = sum_P Y3[(mj),P] Lvv[(be),P]
-  // (Q is free once the ring product above has read it) permuted into WE
+  // WE[me,jb] -= sum_f t1[jf] (mf|be): with factors, H[(mj),(be)] = sum_P Y3[(mj),P] Lvv[(be),P]
+  // (H is free until the ring products) permuted into WE
   if (fac) {
-    fac_y3_lvv<T>(ctx, S, Y3, Q);
-    permute<T, T>(ctx, Q, d4, {0, 3, 1, 2}, WE, -1.0, 1.0, "cc_ovvv_fac");
+    fac_y3_lvv<T>(ctx, S, Y3, H);
+    permute<T, T>(ctx, H, d4, {0, 3, 1, 2}, WE, -1.0, 1.0, "cc_ovvv_fac");
   } else {
     contract<T>(ctx, -1.0, TN(t1, "jf"), TN(ovvv, "mfbe"), 1.0, TN(WE, "mejb"), "cc_t1");
   }
@@ -329,10 +321,15 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
   // D[kc,jb] = delta_kj Fb[b,c] - delta_cb Fj[k,j]
   T* FmiT = bufp_t<T>(W.FmiT, oo);
   permute<T, T>(ctx, Fmi, {o, o}, {1, 0}, FmiT, 1.0, 0.0, "cc_fock");
-  fock_dress<T>(ctx, WE, Fae, FmiT, o, v, half);
-  ring_mm<T>(ctx, S, one, Tov, SP_TOV, WE, SP_WE, zero, H);
-  ring_mm<T>(ctx, S, one, Uov, SP_UOV, WJ, SP_WJ, one, H);
-  // exchange ring term t[m,i,b,e] WmBEj[m,a,e,j] = (Tx WE)[ib,ja]
+  ring_start<T>(ctx, Kov, one, WE, Fae, FmiT, o, v, WE, WJ);
+  // WJ's T1 terms: sum_f t1[jf] (me|bf) - sum_n t1[nb] (nj|me)
+  if (fac) fac_lov_y2<T>(ctx, S, Y2, true, WJ);
+  else contract<T>(ctx, 1.0, TN(t1, "jf"), TN(ovvv, "mebf"), 1.0, TN(WJ, "mejb"), "cc_t1");
+  contract<T>(ctx, -1.0, TN(t1, "nb"), TN(ooov, "njme"), 1.0, TN(WJ, "mejb"), "cc_t1", H, N2);
+  ring_mm<T>(ctx, S, half, ring_lx<T>(ctx, S), SP_LX, U2, SP_U2, one, WJ);
+  ring_mm<T>(ctx, S, half, Kx, SP_KX, Q, SP_Q, one, WE);
+  ring_mm<T>(ctx, S, one, Uov, SP_UOV, WJ, SP_WJ, zero, H);
+  // exchange ring term t[m,i,b,e] WmBEj[m,a,e,j] = (Tx WE)[ib,ja], and half the direct one
   ring_mm<T>(ctx, S, one, Ttov, SP_TTOV, WE, SP_WE, zero, Y);
   // T1^2 terms: -t1[ie] t1[ma] (me|jb) and -t1[ie] t1[mb] (mj|ae); (me|jb) = K[j,b,m,e] is read
   // in place, and the products permuted into H go through U2, free once WJ is built
@@ -344,13 +341,15 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
   if (fac) fac_lov_y2<T>(ctx, S, Y2, false, H);
   else contract<T>(ctx, 1.0, TN(t1, "ie"), TN(ovvv, "jbae"), 1.0, TN(H, "iajb"), "cc_t1");
   contract<T>(ctx, -1.0, TN(t1, "ma"), TN(ooov, "mijb"), 1.0, TN(H, "iajb"), "cc_t1", U2, N2);
-  // S = H + Y^x + (H + Y^x)^T: summed by the update kernel, or here (into WJ) when its LDS slab
+  // S = G + G^T, G = H + Y/2 + Y^x: summed by the update kernel, or here (into WJ) when its LDS slab
   // would not fit
   if (!fused_sym(o, sizeof(T))) {
+    axpby<T>(ctx, N2, 0.5, Y, 1.0, H);
     permute<T, T>(ctx, Y, {o, v, o, v}, {0, 3, 2, 1}, H, 1.0, 1.0, "cc_sym");
     JUES_HIP(hipMemcpyAsync(WJ, H, N2 * sizeof(T), hipMemcpyDeviceToDevice, ctx->stream));
     permute<T, T>(ctx, H, {ov, ov}, {1, 0}, WJ, 1.0, 1.0, "cc_sym");
   }
+  W.y_direct = 0.5;
   W.out_H = H;
   W.out_Y = Y;
   W.out_S = WJ;

@@ -1,0 +1,34 @@
+"""The four-product form of the ring terms against the six products they are written with, in NumPy."""
+import numpy as np
+import pytest
+
+
+def _x(M, o, v):  # M[ib,ja] at [ia,jb]
+    return M.reshape(o, v, o, v).transpose(0, 3, 2, 1).reshape(o * v, o * v)
+
+
+@pytest.mark.parametrize("o,v", [(1, 1), (1, 4), (3, 1), (2, 5), (4, 7)])
+@pytest.mark.parametrize("singles", [False, True])
+def test_four_ring_products_equal_six(o, v, singles):
+    """With symmetric T and Tx (its exchanged form), U = 2T - Tx and, in RCCSD, Q = Tx + 2 tt^x, U2 = 2T - Q,
+    E the T1 and Fock-like parts of WE and J1 those of WJ:
+    WJ = K + K U2/2 - Kx T/2 + J1 (+ none of E), WE = -J + Kx Q/2 + E, G = T WE + U WJ + (Tx WE)^x equals
+    U W + Y/2 + Y^x with W = K - J/2 + (K - Kx/2) U2/2 + J1 + E/2 and Y = Tx WE."""
+    rng = np.random.default_rng(100 * o + v)
+    n = o * v
+    sym = lambda: (lambda A: A + A.T)(rng.normal(size=(n, n)))
+    K, J, T = sym(), sym(), sym()
+    Kx, Tx = _x(K, o, v), _x(T, o, v)
+    assert np.array_equal(Kx, Kx.T) and np.array_equal(Tx, Tx.T)
+    E, J1 = rng.normal(size=(n, n)), rng.normal(size=(n, n)) * singles
+    t1 = rng.normal(size=(o, v)) * singles
+    Q = Tx + 2 * np.einsum("ib,ja->iajb", t1, t1).reshape(n, n)
+    U, U2 = 2 * T - Tx, 2 * T - Q
+    WE = -J + 0.5 * Kx @ Q + E
+    WJ = K + 0.5 * K @ U2 - 0.5 * Kx @ T + J1
+    ref = T @ WE + U @ WJ + _x(Tx @ WE, o, v)
+    W = K - 0.5 * J + 0.5 * (K - 0.5 * Kx) @ U2 + J1 + 0.5 * E
+    Y = Tx @ WE
+    got = U @ W + 0.5 * Y + _x(Y, o, v)
+    # rounding only: a few products of n terms
+    assert np.max(np.abs(got - ref)) < 64 * n * 2.3e-16 * np.max(np.abs(ref) + 10)
