@@ -70,6 +70,17 @@ __device__ inline bool entry_place(int& x, int& z) {
   return true;
 }
 
+// Tile p2 of tiles_m x tiles_n in grouped order: GROUP_M tile-rows share each sweep over tile-columns
+__device__ inline void grouped_tile(int p2, int tiles_m, int tiles_n, int& tm, int& tn) {
+  const int group_size = GROUP_M * tiles_n;
+  const int gid = p2 / group_size;
+  const int first_m = gid * GROUP_M;
+  const int gsz = min(tiles_m - first_m, GROUP_M);
+  const int r = p2 - gid * group_size;
+  tm = first_m + r % gsz;
+  tn = r / gsz;
+}
+
 // Tile of workgroup pid of nwg, of which only the first tiles_m * tiles_n carry a tile (a launch
 // padded to a multiple of NXCD); false for the padding ids.  plain: the workgroups are on one XCD already.
 __device__ inline bool tile_coords_bounded(int pid, int nwg, int tiles_m, int tiles_n, int& tm, int& tn,
@@ -82,16 +93,44 @@ __device__ inline bool tile_coords_bounded(int pid, int nwg, int tiles_m, int ti
   const int xcd = pid % NXCD, loc = pid / NXCD;
   const int p2 = plain ? pid : xcd < tall ? xcd * per + loc : tall * per + (xcd - tall) * (per - 1) + loc;
   if (p2 >= tiles_m * tiles_n) return false;
-  // grouped ordering: GROUP_M tile-rows share each sweep over tile-columns
-  const int group_size = GROUP_M * tiles_n;
-  const int gid = p2 / group_size;
-  const int first_m = gid * GROUP_M;
-  const int gsz = min(tiles_m - first_m, GROUP_M);
-  const int r = p2 - gid * group_size;
-  tm = first_m + r % gsz;
-  tn = r / gsz;
+  grouped_tile(p2, tiles_m, tiles_n, tm, tn);
   return true;
 }
+
+// A TAIL launch of a product: `whole` workgroups have a tile each, and the other tiles' 16-deep k-slabs are shared by
+// several workgroups a tile, whose parts of it gemm_tail_kernel adds.  Tiles are taken full ones first (grouped),
+// then those past the edge of N, of M and of both: four runs of n[] tiles left to the tail, in s[] chunks each.
+// Within a run, workgroups (and their parts) are ordered chunk by chunk: neighbours read the same k-slabs.
+// 256 compute units leave much of a last round of tiles idle otherwise, and split whole products write more parts
+// (and round no better): 3082^3 took 980 us in two chunks, 878 this way, 6460^3 8.6 and 7.7 ms (73 TFLOP/s would be 7.4),
+// 253 x 8911 x 8911 855 and 652 us, 8640 x 768 x 8640 1790 and 1660.
+struct TailMap {
+  int whole = 0, wgs = 0, nk = 0, full_m = 0, full_n = 0;
+  int n[4] = {}, s[4] = {};
+
+  __device__ void coords(int p2, int& tm, int& tn) const {
+    const int full = full_m * full_n;
+    if (p2 < full) grouped_tile(p2, full_m, full_n, tm, tn);
+    else if ((p2 -= full) < n[1]) tm = p2, tn = full_n;
+    else if ((p2 -= n[1]) < n[2]) tm = full_m, tn = p2;
+    else tm = full_m, tn = full_n;
+  }
+  // tile of the tail and chunk of it (of `chunks`) of workgroup x
+  __device__ void part(int x, int& tile, int& chunk, int& chunks) const {
+    int base = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (x < n[q] * s[q]) {
+        chunk = x / n[q];
+        tile = base + x - chunk * n[q];
+        chunks = s[q];
+        return;
+      }
+      x -= n[q] * s[q];
+      base += n[q];
+    }
+  }
+};
 
 // One product of a high-occupancy kernel launch: C = alpha A op(B) + beta C, batched over
 // blockIdx.z with strides sA, sB, sC.  A launch carries one or two of them (two
@@ -115,6 +154,8 @@ struct GemmSide {
   int inner = 1;
   long sG = 0;
   int nz = 1;  // batch entries or K chunks of the launch
+  TailMap tail;      // TAIL launches
+  T* part = nullptr;
   // FP32 products that write an FP64 result (the OUT64 instantiation; C is not used there)
   double* C64 = nullptr;
 };
@@ -147,11 +188,15 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
                                                            float alpha, float beta) {
   constexpr int BM = BT, BN = BT, BK = 16;
   // 64-row shares per thread, 16-row MFMA blocks per wavefront side, wavefront tile edge
-  constexpr int NJ = BT / 64, NB = BT / 32, WT = BT / 2;
+  constexpr int NJ = BT / 64, NB = BT / 32;
   __shared__ __attribute__((aligned(16))) float As[2][BM * BK];
   __shared__ __attribute__((aligned(16))) float Bs[2][BN * BK];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wn = wave >> 1;
+  // a wavefront's 16-row and 16-column blocks alternate with its neighbour's, so that a tile at the edge of M
+  // or N keeps all of them at work on the blocks it has
+  const auto mrow = [&](int i) { return (2 * i + wm) * 16; };
+  const auto ncol = [&](int j) { return (2 * j + wn) * 16; };
   int bx, bz;
   const bool placed = entry_place(bx, bz), second = bx >= nt0;
   const GemmSide<float> g = second ? p1 : p0;
@@ -168,9 +213,13 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
   const int K1 = SEG ? g.K1 : 0;
   const float* A1 = SEG ? g.A1 + zb * g.sA + tab[2] : A;
   const float* B1 = SEG ? g.B1 + zb * g.sB + tab[3] : B;
+  // slices: the K tail (columns 16 floor(K/16) .. K-1, zero-padded) first when there is one, then the full
+  // slices from k = 0; the tail is loaded in the prologue
+  const int K16 = K / BK * BK, tail = K > K16 ? 1 : 0;
+  const int nk = K16 / BK + tail + K1 / BK;
   int tm, tn;
-  if (!tile_coords_bounded(second ? bx - nt0 : bx, second ? (int)gridDim.x - nt0 : nt0,
-                           g.tiles_m, g.tiles_n, tm, tn, placed))
+  if (!tile_coords_bounded(second ? bx - nt0 : bx, second ? (int)gridDim.x - nt0 : nt0, g.tiles_m, g.tiles_n, tm, tn,
+                           placed))
     return;
   const int m0 = tm * BM, n0 = tn * BN;
 
@@ -267,10 +316,6 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
     for (int j = 0; j < NB; ++j) acc[i][j] = fvec4{0, 0, 0, 0};
 
   const int fr = lane & 15, fk = lane >> 4;
-  // slices: the K tail (columns 16 floor(K/16) .. K-1, zero-padded) first when there is one, then the
-  // full slices from k = 0; the tail is loaded once, in the prologue
-  const int K16 = K / BK * BK, tail = K > K16 ? 1 : 0;
-  const int nk = K16 / BK + tail + K1 / BK;
   if (tail) {
     if constexpr (TA) {
 #pragma unroll
@@ -317,15 +362,15 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
     f4v bf[NB];
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-      const int r = wn * WT + j * 16 + fr;
+      const int r = ncol(j) + fr;
       bf[j] = *reinterpret_cast<const f4v*>(&Bs[cur][r * BK + 4 * g32_chunk(fk, r)]);
     }
-    f4v a0 = *reinterpret_cast<const f4v*>(&As[cur][(wm * WT + fr) * BK + 4 * g32_chunk(fk, wm * WT + fr)]);
+    f4v a0 = *reinterpret_cast<const f4v*>(&As[cur][(mrow(0) + fr) * BK + 4 * g32_chunk(fk, mrow(0) + fr)]);
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
       f4v a1;
       if (i + 1 < NB) {
-        const int r = wm * WT + (i + 1) * 16 + fr;
+        const int r = mrow(i + 1) + fr;
         a1 = *reinterpret_cast<const f4v*>(&As[cur][r * BK + 4 * g32_chunk(fk, r)]);
       }
 #pragma unroll
@@ -338,26 +383,53 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
   };
   // the last slice is peeled off, so that the loop body is one block without conditions (a schedule
   // that keeps the matrix pipe about 5% busier on the ring products than the conditional form)
-  for (int kt = 0; kt + 1 < nk; ++kt) {
-    const int cur = kt & 1;
-    load(kt + 1 - tail);
-    compute(cur);
-    store(cur ^ 1);
-    __syncthreads();
-  }
-  compute((nk - 1) & 1);
+  // a tile past the edge of M or N: only the blocks that hold results
+  const int ilim = min(NB, (M - m0 - 16 * wm + 31) / 32), jlim = min(NB, (N - n0 - 16 * wn + 31) / 32);
+  auto compute_edge = [&](int cur) {
+    if (ilim <= 0 || jlim <= 0) return;
+    f4v bf[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int r = ncol(j) + fr;
+      bf[j] = *reinterpret_cast<const f4v*>(&Bs[cur][r * BK + 4 * g32_chunk(fk, r)]);
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      if (i >= ilim) break;
+      const int r = mrow(i) + fr;
+      const f4v a = *reinterpret_cast<const f4v*>(&As[cur][r * BK + 4 * g32_chunk(fk, r)]);
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+        if (j < jlim)
+#pragma unroll
+          for (int s2 = 0; s2 < 4; ++s2)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j][s2], a[s2], acc[i][j], 0, 0, 0);
+    }
+  };
+  const auto loop = [&](auto slice) {
+    for (int kt = 0; kt + 1 < nk; ++kt) {
+      const int cur = kt & 1;
+      load(kt + 1 - tail);
+      slice(cur);
+      store(cur ^ 1);
+      __syncthreads();
+    }
+    slice((nk - 1) & 1);
+  };
+  if (ilim == NB && jlim == NB) loop(compute);
+  else loop(compute_edge);
 
   if constexpr (OUT64) {
     double* __restrict__ C64 = g.C64 + (long)bz * g.sC;
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-      const int m = m0 + wm * WT + i * 16 + (lane & 15);
+      const int m = m0 + mrow(i) + (lane & 15);
       if (m >= M) continue;
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int n = n0 + wn * WT + j * 16 + 4 * (lane >> 4) + r;
+          const int n = n0 + ncol(j) + 4 * (lane >> 4) + r;
           if (n < N) C64[(long)m + (long)n * ldc] = (double)(alpha * acc[i][j][r]);
         }
       }
@@ -369,29 +441,29 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
     // its stores (an element-wise load -> store round trip would serialise the epilogue)
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-      const long m = m0 + wm * WT + i * 16 + (lane & 15);
+      const long m = m0 + mrow(i) + (lane & 15);
       float cv[NB][4];
 #pragma unroll
       for (int j = 0; j < NB; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) cv[j][r] = C[m + (long)(n0 + wn * WT + j * 16 + 4 * (lane >> 4) + r) * ldc];
+        for (int r = 0; r < 4; ++r) cv[j][r] = C[m + (long)(n0 + ncol(j) + 4 * (lane >> 4) + r) * ldc];
 #pragma unroll
       for (int j = 0; j < NB; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          C[m + (long)(n0 + wn * WT + j * 16 + 4 * (lane >> 4) + r) * ldc] = alpha * acc[i][j][r] + beta * cv[j][r];
+          C[m + (long)(n0 + ncol(j) + 4 * (lane >> 4) + r) * ldc] = alpha * acc[i][j][r] + beta * cv[j][r];
     }
     return;
   }
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
-    const int m = m0 + wm * WT + i * 16 + (lane & 15);
+    const int m = m0 + mrow(i) + (lane & 15);
     if (m >= M) continue;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int n = n0 + wn * WT + j * 16 + 4 * (lane >> 4) + r;
+        const int n = n0 + ncol(j) + 4 * (lane >> 4) + r;
         if (n < N) {
           const long off = (long)m + (long)n * ldc;
           float v = alpha * acc[i][j][r];
@@ -415,17 +487,21 @@ typedef double d2v __attribute__((ext_vector_type(2)));
 
 __device__ inline int g64_chunk(int q, int r) { return q ^ (r & 7); }
 
-template <int KIND, bool TB, bool TA = false, bool SEG = false, int BT = 128>
+template <int KIND, bool TB, bool TA = false, bool SEG = false, int BT = 128, bool TAIL = false>
 __global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, GemmSide<double> p1, int nt0,
                                                         double alpha, double beta) {
   constexpr int BM = BT, BN = BT, BK = 16;
   constexpr int HT = BT / 2, IB = BT / 32;  // half tile; 16-row MFMA blocks of a wavefront (HT rows)
   __shared__ __attribute__((aligned(16))) double As[2][BM * BK];
   __shared__ __attribute__((aligned(16))) double Bs[2][BN * BK];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wn = wave >> 1;  // 2 x (BT / 32) wavefronts of HT x 32
+  // a wavefront's 16-row and 16-column blocks alternate with its neighbours', so that a tile at the edge of M
+  // or N keeps all of them at work on the blocks it has
+  const auto mrow = [&](int i) { return (2 * i + wm) * 16; };
+  const auto ncol = [&](int j) { return (BT / 32 * j + wn) * 16; };
   int bx, bz;
-  const bool placed = entry_place(bx, bz), second = bx >= nt0;
+  const bool placed = entry_place(bx, bz), second = !TAIL && bx >= nt0;
   const GemmSide<double> g = second ? p1 : p0;
   const int M = g.M, N = g.N, K = bz == g.nz - 1 ? g.Klast : g.K;
   if (bz >= g.nz) return;
@@ -440,10 +516,29 @@ __global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, 
   const int K1 = SEG ? g.K1 : 0;
   const double* A1 = SEG ? g.A1 + zb * g.sA + tab[2] : A;
   const double* B1 = SEG ? g.B1 + zb * g.sB + tab[3] : B;
-  int tm, tn;
-  if (!tile_coords_bounded(second ? bx - nt0 : bx, second ? (int)gridDim.x - nt0 : nt0,
-                           g.tiles_m, g.tiles_n, tm, tn, placed))
+  // slices: the K tail (columns 16 floor(K/16) .. K-1, zero-padded) first when there is one, then the full
+  // slices from k = 0; the tail is loaded in the prologue
+  const int K16 = K / BK * BK, tail = K > K16 ? 1 : 0;
+  const int nk = K16 / BK + tail + K1 / BK;
+  int tm, tn, ka = 0, kb = nk, wg = 0;
+  bool shared = false;  // the workgroup's result is a part of its tile
+  if (TAIL && bx >= g.tail.whole) {
+    const int x = bx - g.tail.whole, per = ((int)gridDim.x - g.tail.whole) / NXCD;
+    wg = x % NXCD * per + x / NXCD;  // neighbours on one XCD
+    if (wg >= g.tail.wgs) return;
+    int t = 0, c = 0, nc = 1;
+    g.tail.part(wg, t, c, nc);
+    shared = nc > 1;
+    ka = (int)((long)nk * c / nc);
+    kb = (int)((long)nk * (c + 1) / nc);
+    g.tail.coords(g.tail.whole + t, tm, tn);
+  } else if (TAIL) {
+    const int per = g.tail.whole / NXCD;
+    g.tail.coords(bx % NXCD * per + bx / NXCD, tm, tn);
+  } else if (!tile_coords_bounded(second ? bx - nt0 : bx, second ? (int)gridDim.x - nt0 : nt0, g.tiles_m, g.tiles_n,
+                                  tm, tn, placed)) {
     return;
+  }
   const int m0 = tm * BM, n0 = tn * BN;
   // A (and n-contiguous B) share: row am, k = 4 kq + u; k-contiguous B share: rows bn, bn + HT, chunk bc
   // (a k-contiguous A, TA, is shared like a k-contiguous B)
@@ -527,10 +622,7 @@ __global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, 
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = dvec4{0, 0, 0, 0};
   const int fr = lane & 15, fk = lane >> 4;
-  // the K tail first (zero-padded, loaded once in the prologue), then the full slices from k = 0
-  const int K16 = K / BK * BK, tail = K > K16 ? 1 : 0;
-  const int nk = K16 / BK + tail + K1 / BK;
-  if (tail) {
+  if (tail && ka == 0) {
     if constexpr (TA) {
 #pragma unroll
       for (int j = 0; j < 2; ++j)
@@ -569,7 +661,7 @@ __global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, 
         }
     }
   } else {
-    load(0);
+    load(ka - tail);
   }
   store(0);
   __syncthreads();
@@ -577,20 +669,20 @@ __global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, 
     d2v bf[2][2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const int r = wn * 32 + j * 16 + fr;
+      const int r = ncol(j) + fr;
       bf[j][0] = *reinterpret_cast<const d2v*>(&Bs[cur][r * BK + 2 * g64_chunk(2 * fk, r)]);
       bf[j][1] = *reinterpret_cast<const d2v*>(&Bs[cur][r * BK + 2 * g64_chunk(2 * fk + 1, r)]);
     }
     d2v a0[2], a1[2];
     {
-      const int r = wm * HT + fr;
+      const int r = mrow(0) + fr;
       a0[0] = *reinterpret_cast<const d2v*>(&As[cur][r * BK + 2 * g64_chunk(2 * fk, r)]);
       a0[1] = *reinterpret_cast<const d2v*>(&As[cur][r * BK + 2 * g64_chunk(2 * fk + 1, r)]);
     }
 #pragma unroll
     for (int i = 0; i < IB; ++i) {
       if (i + 1 < IB) {
-        const int r = wm * HT + (i + 1) * 16 + fr;
+        const int r = mrow(i + 1) + fr;
         a1[0] = *reinterpret_cast<const d2v*>(&As[cur][r * BK + 2 * g64_chunk(2 * fk, r)]);
         a1[1] = *reinterpret_cast<const d2v*>(&As[cur][r * BK + 2 * g64_chunk(2 * fk + 1, r)]);
       }
@@ -604,43 +696,84 @@ __global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, 
     }
   };
   // the last slice is peeled off, so that the loop body is one block without conditions
-  for (int kt = 0; kt + 1 < nk; ++kt) {
-    const int cur = kt & 1;
-    load(kt + 1 - tail);
-    compute(cur);
-    store(cur ^ 1);
-    __syncthreads();
+  // a tile past the edge of M or N: only the blocks that hold results
+  const int ilim = min(IB, (M - m0 - 16 * wm + 31) / 32), jlim = min(2, (N - n0 - 16 * wn + HT - 1) / HT);
+  auto compute_edge = [&](int cur) {
+    if (ilim <= 0 || jlim <= 0) return;
+    d2v bf[2][2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int r = ncol(j) + fr;
+      bf[j][0] = *reinterpret_cast<const d2v*>(&Bs[cur][r * BK + 2 * g64_chunk(2 * fk, r)]);
+      bf[j][1] = *reinterpret_cast<const d2v*>(&Bs[cur][r * BK + 2 * g64_chunk(2 * fk + 1, r)]);
+    }
+#pragma unroll
+    for (int i = 0; i < IB; ++i) {
+      if (i >= ilim) break;
+      const int r = mrow(i) + fr;
+      const d2v a[2] = {*reinterpret_cast<const d2v*>(&As[cur][r * BK + 2 * g64_chunk(2 * fk, r)]),
+                        *reinterpret_cast<const d2v*>(&As[cur][r * BK + 2 * g64_chunk(2 * fk + 1, r)])};
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        if (j < jlim)
+#pragma unroll
+          for (int s2 = 0; s2 < 4; ++s2)
+            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bf[j][s2 >> 1][s2 & 1], a[s2 >> 1][s2 & 1], acc[i][j],
+                                                             0, 0, 0);
+    }
+  };
+  const auto loop = [&](auto slice) {
+    for (int kt = ka; kt + 1 < kb; ++kt) {
+      const int cur = (kt - ka) & 1;
+      load(kt + 1 - tail);
+      slice(cur);
+      store(cur ^ 1);
+      __syncthreads();
+    }
+    slice((kb - 1 - ka) & 1);
+  };
+  if (ilim == IB && jlim == 2) loop(compute);
+  else loop(compute_edge);
+  if (TAIL && shared) {
+    // a partial tile, as the registers hold it, for gemm_tail_kernel
+    double* __restrict__ P = g.part + (long)wg * (BM * BN) + tid;
+#pragma unroll
+    for (int i = 0; i < IB; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) P[((i * 2 + j) * 4 + r) * (4 * BT)] = alpha * acc[i][j][r];
+    return;
   }
-  compute((nk - 1) & 1);
 
   // acc[i][j][r]: C(m, n) with m = lane % 16 of block i, n = lane / 16 + 4 r of block j
   if (beta != 0.0 && m0 + BM <= M && n0 + BN <= N) {
     // interior tile accumulating into C: per 16-row block, the loads before the stores
 #pragma unroll
     for (int i = 0; i < IB; ++i) {
-      const long m = m0 + wm * HT + i * 16 + (lane & 15);
+      const long m = m0 + mrow(i) + (lane & 15);
       double cv[2][4];
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) cv[j][r] = C[m + (long)(n0 + wn * 32 + j * 16 + (lane >> 4) + 4 * r) * ldc];
+        for (int r = 0; r < 4; ++r) cv[j][r] = C[m + (long)(n0 + ncol(j) + (lane >> 4) + 4 * r) * ldc];
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          C[m + (long)(n0 + wn * 32 + j * 16 + (lane >> 4) + 4 * r) * ldc] = alpha * acc[i][j][r] + beta * cv[j][r];
+          C[m + (long)(n0 + ncol(j) + (lane >> 4) + 4 * r) * ldc] = alpha * acc[i][j][r] + beta * cv[j][r];
     }
     return;
   }
 #pragma unroll
   for (int i = 0; i < IB; ++i) {
-    const int m = m0 + wm * HT + i * 16 + (lane & 15);
+    const int m = m0 + mrow(i) + (lane & 15);
     if (m >= M) continue;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int n = n0 + wn * 32 + j * 16 + (lane >> 4) + 4 * r;
+        const int n = n0 + ncol(j) + (lane >> 4) + 4 * r;
         if (n < N) {
           const long off = (long)m + (long)n * ldc;
           double v = alpha * acc[i][j][r];
@@ -791,6 +924,37 @@ __global__ void scale_kernel(T* C, long M, long N, long ldc, T beta) {
 // C = beta*C + sum_s W[s] (fixed order), W[s] is M x N with leading dimension M.  Eight loads are in
 // flight per thread: with one element per thread and a few hundred partial products (a 20 x 20 result
 // of K = 200000) the sum is otherwise a chain of as many memory latencies.
+// C = (sum of the parts of a TAIL launch's tile, in the order of its slabs) + beta C.  blockIdx.x: tile of the
+// tail, blockIdx.y: 1024 of its 128 x 128 results, in the order of the workgroups' registers.
+__global__ __launch_bounds__(256) void gemm_tail_kernel(GemmSide<double> g, double beta) {
+  constexpr int BT = 128;
+  const TailMap& tail = g.tail;
+  int tm, tn, q = 0, t = (int)blockIdx.x;
+  tail.coords(tail.whole + t, tm, tn);
+  long first = 0;  // part 0 of the tile's run
+  while (q < 3 && t >= tail.n[q]) {
+    first += (long)tail.n[q] * tail.s[q];
+    t -= tail.n[q++];
+  }
+  if (tail.s[q] == 1) return;  // written by its workgroup
+  const int q0 = (int)blockIdx.y * 1024 + threadIdx.x;
+  double sum[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int c = 0; c < tail.s[q]; ++c) {
+    const double* P = g.part + (first + (long)c * tail.n[q] + t) * (BT * BT) + q0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) sum[u] += P[256 * u];
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int x = q0 + 256 * u, th = x % 512, e = x / 512, lane = th & 63, wm = (th >> 6) & 1, wn = th >> 7;
+    const int i = e / 8, j = e / 4 % 2, r = e % 4;
+    const int m = tm * BT + (2 * i + wm) * 16 + (lane & 15), n = tn * BT + (4 * j + wn) * 16 + (lane >> 4) + 4 * r;
+    if (m >= g.M || n >= g.N) continue;
+    double* c = g.C + m + (long)n * g.ldc;
+    *c = beta != 0.0 ? sum[u] + beta * *c : sum[u];
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const T* __restrict__ W, int S, long M, long N,
                                                             T* __restrict__ C, long ldc, T beta) {
@@ -1374,6 +1538,7 @@ enum GemmForm { TILE128, TILE64, SHORT, TALL, DIRECT22, DIRECT21, DIRECT12, DIRE
 struct GemmPlan {
   int form = DIRECT22;
   long split = 1;   // chunks of the contraction, each a launch-z entry with its own partial product
+  TailMap tail;     // wgs > 0: a TAIL launch of FP64 128x128 tiles
   double us = 1e300;
 };
 
@@ -1456,6 +1621,50 @@ static double reduce_us(long S, double elems) {
   return S > 1 ? 2.0 + (S + 1) * elems * sizeof(T) / 4.5e6 + 0.18 * S : 0.0;
 }
 
+// The TAIL launch of an M x N x K product with `whole` full tiles to themselves and the others in `chunks` chunks,
+// those past an edge in fewer by the cost of their slabs; wgs = 0 in the result if it is not of use (fewer full tiles,
+// chunks under 8 slabs, parts over 256 MiB).
+static TailMap tail_map(long M, long N, long K, long whole, int chunks) {
+  TailMap t;
+  const long fm = M / 128, fn = N / 128, nk = cdiv(K, 16);
+  const int em = (int)cdiv(M % 128, 16), en = (int)cdiv(N % 128, 16);  // 16-row and 16-column blocks past the edge
+  const long rest = cdiv(M, 128) * cdiv(N, 128) - whole;
+  if (fm * fn < whole || rest < 1 || rest > 2048 || nk < 8L * chunks) return t;
+  t.whole = (int)whole;
+  t.nk = (int)nk;
+  t.full_m = (int)fm;
+  t.full_n = (int)fn;
+  // eighths of a full tile's cost: the blocks that a wavefront has of its 4 (2), at least 3 for the staging
+  const int wm = (int)cdiv(em, 2), wn = (int)cdiv(en, 4);
+  const int n[4] = {(int)(fm * fn - whole), en ? (int)fm : 0, em ? (int)fn : 0, em && en ? 1 : 0};
+  const int w[4] = {8, std::max(3, 4 * wn), std::max(3, 2 * wm), std::max(3, wm * wn)};
+  long wgs = 0;
+  for (int q = 0; q < 4; ++q) {
+    t.n[q] = n[q];
+    t.s[q] = std::max(1, (chunks * w[q] + 4) / 8);
+    wgs += (long)t.n[q] * t.s[q];
+  }
+  if (wgs <= 2048) t.wgs = (int)wgs;
+  return t;
+}
+
+// Estimated time (us) of a TAIL launch: a compute unit's slabs, and 2.5 for each workgroup's start and end, at the
+// rate that a long FP64 launch of 128x128 tiles reaches (1.87 us; 8% more where there is a single workgroup), but at
+// least the 1.64 us of latency of each slab of the longest chunk; and the parts, written and read once.
+static double tail_us(const TailMap& t) {
+  int tiles = 0, least = 1 << 30;
+  for (int q = 0; q < 4; ++q) {
+    tiles += t.n[q];
+    if (t.n[q]) least = std::min(least, t.s[q]);
+  }
+  const int chunks = t.n[0] ? t.s[0] : least;
+  const double rounds = (double)cdiv(t.wgs, 256);
+  const double slabs = t.whole / 256 * (t.nk + 2.5) + rounds * ((double)t.nk / chunks + 2.5);
+  const double latency = 1.64 / 1.87 * (t.nk * (t.whole / 256 + 1.0 / least) + 2.5);
+  const double parts = t.wgs > tiles ? (2.0 * t.wgs + tiles) * 131072.0 / 4.5e6 + 5.0 : 0.0;
+  return 11.0 + 1.87 * std::max(slabs, latency) * (t.whole + t.wgs <= 256 ? 1.08 : 1.0) + parts;
+}
+
 static const long kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128};
 
 // The form and split with the smallest estimated time.  A split product's partial results take at most
@@ -1482,8 +1691,18 @@ static GemmPlan gemm_plan(bool ta, bool tb, long M, long N, long K, long lda, lo
       const long slabs = cdiv(cdiv(K, s), 16);
       const double us = form_us<T>(form, tiles * s * batch, slabs, bytes) + reduce_us<T>(s, (double)M * N) +
                         (copy_a ? 6.0 : 0.0);
-      if (us < best.us) best = GemmPlan{form, s, us};
+      if (us < best.us) best = GemmPlan{form, s, TailMap{}, us};
     }
+  }
+  if (sizeof(T) == 8 && allow_split && batch == 1 && form_ok<T>(TILE128, ta, tb, M, N, K, lda, ldb)) {
+    const long full = (M / 128) * (N / 128) / 256 * 256;
+    for (const long whole : {full, full - 256})
+      for (int chunks = 1; whole >= 0 && chunks <= 32; ++chunks) {
+        const TailMap t = tail_map(M, N, K, whole, chunks);
+        if (!t.wgs || t.wgs == t.n[0] + t.n[1] + t.n[2] + t.n[3]) continue;  // (nothing shared: the plain launch)
+        const double us = tail_us(t);
+        if (us < best.us) best = GemmPlan{TILE128, 1, t, us};
+      }
   }
   return best;
 }
@@ -1508,7 +1727,8 @@ static void tile_launch(jues_ctx* ctx, int form, bool tb, int kind, GemmSide<T> 
   JUES_REQUIRE(total < (1L << 31), "gemm: too many tiles");
   p0.nz = p1.nz = nb;
   if (!two) p1 = p0;
-  const dim3 grid((unsigned)total, 1, grid_z(nb));
+  const bool tail = p0.tail.wgs > 0;
+  const dim3 grid((unsigned)(tail ? p0.tail.whole + cdiv(p0.tail.wgs, NXCD) * NXCD : total), 1, grid_z(nb));
   if constexpr (sizeof(T) == 4) {
 #define JUES_GEMM32(K_, TB_, TA_, SEG_, BT_)                                                                        \
   hipLaunchKernelGGL((gemm32_nn_kernel<K_, TB_, TA_, SEG_, false, BT_>), grid, dim3(NT), 0, ctx->stream, p0, p1,    \
@@ -1533,9 +1753,10 @@ static void tile_launch(jues_ctx* ctx, int form, bool tb, int kind, GemmSide<T> 
 #undef JUES_GEMM32_SHAPES
 #undef JUES_GEMM32
   } else {
-#define JUES_GEMM64(K_, TB_, TA_, SEG_, BT_)                                                                     \
-  hipLaunchKernelGGL((gemm64_kernel<K_, TB_, TA_, SEG_, BT_>), grid, dim3(4 * BT_), 0, ctx->stream, p0, p1, (int)nt0, \
-                     (double)alpha, (double)beta)
+#define JUES_GEMM64(K_, TB_, TA_, SEG_, BT_, ...)                                                                \
+  hipLaunchKernelGGL((gemm64_kernel<K_, TB_, TA_, SEG_, BT_, ##__VA_ARGS__>), grid, dim3(4 * BT_), 0, ctx->stream, \
+                     p0, p1, (int)nt0, (double)alpha, (double)beta)
+#define JUES_GEMM64_TAIL(K_, TB_, TA_) JUES_GEMM64(K_, TB_, TA_, false, 128, true)
 #define JUES_GEMM64_SHAPES(BT_)                      \
   if (seg) {                                         \
     if (tb) JUES_GEMM64(0, true, false, true, BT_);  \
@@ -1544,7 +1765,19 @@ static void tile_launch(jues_ctx* ctx, int form, bool tb, int kind, GemmSide<T> 
     if (tb) JUES_GEMM64(0, true, true, false, BT_);  \
     else JUES_GEMM64(0, false, true, false, BT_);    \
   } else if (tb) JUES_GEMM64(0, true, false, false, BT_)
-    if (form == TILE64) {
+    if (tail) {
+      if (ta && tb) JUES_GEMM64_TAIL(0, true, true);
+      else if (ta) JUES_GEMM64_TAIL(0, false, true);
+      else if (tb) JUES_GEMM64_TAIL(0, true, false);
+      else if (kind == 1) JUES_GEMM64_TAIL(1, false, false);
+      else if (kind == 2) JUES_GEMM64_TAIL(2, false, false);
+      else JUES_GEMM64_TAIL(0, false, false);
+      JUES_HIP(hipGetLastError());
+      int tiles = 0;
+      for (const int n : p0.tail.n) tiles += n;
+      if (p0.tail.wgs > tiles)
+        hipLaunchKernelGGL(gemm_tail_kernel, dim3((unsigned)tiles, 16), dim3(256), 0, ctx->stream, p0, (double)beta);
+    } else if (form == TILE64) {
       JUES_GEMM64_SHAPES(64);
       else JUES_GEMM64(0, false, false, false, 64);
     } else {
@@ -1554,6 +1787,7 @@ static void tile_launch(jues_ctx* ctx, int form, bool tb, int kind, GemmSide<T> 
       else JUES_GEMM64(0, false, false, false, 128);
     }
 #undef JUES_GEMM64_SHAPES
+#undef JUES_GEMM64_TAIL
 #undef JUES_GEMM64
   }
   JUES_HIP(hipGetLastError());
@@ -1676,6 +1910,18 @@ static void gemm_impl(jues_ctx* ctx, bool ta, bool tb, long M, long N, long K, T
     }
     plan = gemm_plan<T>(ta, tb, M, N, K, lda, ldb, sA, sB, batch, false);
   }
+  if (plan.tail.wgs) {
+    T* part = split_work<T>(ctx, 9, (size_t)plan.tail.wgs * 128 * 128);
+    if (part) {
+      KTimer t(ctx, name, 2.0 * M * N * K, (double)sizeof(T) * ((double)M * K + (double)K * N + (double)M * N));
+      GemmSide<T> p = make_side<T>(M, N, K, A, lda, 0, B, ldb, 0, C, ldc, 0);
+      p.tail = plan.tail;
+      p.part = part;
+      tile_launch<T>(ctx, TILE128, tb, kind, p, p, false, 1, alpha, beta, ta);
+      return;
+    }
+    plan = gemm_plan<T>(ta, tb, M, N, K, lda, ldb, sA, sB, batch, false);
+  }
   const double flops = 2.0 * M * N * K * batch;
   const double bytes = (double)sizeof(T) * ((double)M * K + (double)K * N + (beta != T(0) ? 2.0 : 1.0) * M * N) * batch;
   KTimer timer(ctx, name, flops, bytes);
@@ -1740,7 +1986,7 @@ void gemm_pair(jues_ctx* ctx, bool tb, long M0, long N0, long K0, const T* A0, l
           break;
         const double us = form_us<T>(form, tiles * s, cdiv(cdiv(std::max(K0, K1), s), 16), bytes) +
                           (s > 1 ? 2.0 : 0.0) + reduce_us<T>(s, elems);
-        if (us < best.us) best = GemmPlan{form, s, us};
+        if (us < best.us) best = GemmPlan{form, s, TailMap{}, us};
       }
     }
     const double apart = gemm_plan<T>(false, tb, M0, N0, K0, lda0, ldb0, 0, 0, 1, !no_alloc_active()).us +
@@ -1810,7 +2056,7 @@ void gemm_ksum(jues_ctx* ctx, bool tb, long M, long N, long K, const T* A0, cons
     if (!form_ok<T>(form, false, tb, M, N, K, lda, ldb)) continue;
     const long bt = form == TILE128 ? 128 : 64;
     const double us = form_us<T>(form, cdiv(M, bt) * cdiv(N, bt) * batch, 2 * K / 16, 0.0);
-    if (us < best.us) best = GemmPlan{form, 1, us};
+    if (us < best.us) best = GemmPlan{form, 1, TailMap{}, us};
   }
   JUES_REQUIRE(best.us < 1e300, "gemm_ksum: leading dimension too large");
   const char* name = tag ? tag : (sizeof(T) == 8 ? "gemm_f64" : "gemm_f32");
