@@ -217,8 +217,19 @@ jues_status jues_rmp2(jues_ctx* ctx, int prec, const double* Cocc, int o, const 
   if (prec == JUES_FP64) {
     DeviceArray<double> co(ctx, Cocc, (size_t)n * o), cv(ctx, Cvir, (size_t)n * v);
     DevBuf K(total * sizeof(double));
-    tei_transform_dev<double>(ctx, co.p, o, cv.p, v, co.p, o, cv.p, v, K.as<double>());
-    *E = mp2_energy_dev<double>(ctx, K.as<double>(), e.p, o, v);
+    if (!ctx->gao.p && ctx->Bfac.p && o >= LOWER_MIN_O && o <= LOWER_MAX_O) {
+      // K = L L^T is symmetric: its lower triangle is enough
+      const long ov = (long)o * v, naux = ctx->naux;
+      double* L = static_cast<double*>(scratch(ctx, 5, sizeof(double) * (size_t)(ov * naux)));
+      mo_factors_dev<double>(ctx, co.p, o, cv.p, v, L);
+      if (!gemm_lower(ctx, ov, naux, L, ov, K.as<double>(), ov, "xform_factor_gemm"))
+        gemm<double>(ctx, false, true, ov, ov, naux, 1.0, L, ov, 0, L, ov, 0, 0.0, K.as<double>(), ov, 0, 1,
+                     "xform_factor_gemm");
+      *E = mp2_lower_dev(ctx, K.as<double>(), e.p, o, v);
+    } else {
+      tei_transform_dev<double>(ctx, co.p, o, cv.p, v, co.p, o, cv.p, v, K.as<double>());
+      *E = mp2_energy_dev<double>(ctx, K.as<double>(), e.p, o, v);
+    }
   } else {
     DeviceArray<float> co(ctx, Cocc, (size_t)n * o), cv(ctx, Cvir, (size_t)n * v);
     DevBuf K(total * sizeof(float));

@@ -174,6 +174,11 @@ void gemm(jues_ctx* ctx, bool ta, bool tb, long M, long N, long K, T alpha, cons
           long sA, const T* B, long ldb, long sB, T beta, T* C, long ldc, long sC, int batch = 1,
           const char* tag = nullptr);
 
+// C = L L^T (M x M, L M x K) in the tiles of the lower triangle only (what lies above the diagonal's tiles is left
+// as it is); returns false, launching nothing, where the whole square is faster or the kernel does not apply.
+bool gemm_lower(jues_ctx* ctx, long M, long K, const double* L, long ldl, double* C, long ldc,
+                const char* tag = nullptr);
+
 // C = A B in FP32 MFMA work with the FP64 result written directly (NN, beta = 0, one product), on
 // the high-occupancy FP32 kernel; returns false, launching nothing, where that kernel does not apply.
 bool gemm32_out64(jues_ctx* ctx, long M, long N, long K, const float* A, long lda, const float* B, long ldb,
@@ -299,6 +304,12 @@ void mo_factors_dev(jues_ctx* ctx, const T* C1, int d1, const T* C2, int d2, T* 
 // RMP2 energy from K[i,a,j,b] = (ia|jb) (device, o x v x o x v) and eps (device FP64, n)
 template <typename T>
 double mp2_energy_dev(jues_ctx* ctx, const T* K, const double* eps, int o, int v);
+// The same from the lower triangle (rows >= columns) of a symmetric K = (ia|jb); with G non-null also the whole of
+// G[i,a,j,b] = dE/dK = 2 (2 K_iajb - K_ibja) / D and, with r non-null, r[i,a] = the row and column sums of
+// K (2 K - K_ibja) / D^2 (device; work: o v^2 doubles).  For o in [LOWER_MIN_O, LOWER_MAX_O].
+constexpr int LOWER_MIN_O = 16, LOWER_MAX_O = 88;
+double mp2_lower_dev(jues_ctx* ctx, const double* K, const double* eps, int o, int v, double* G = nullptr,
+                     double* r = nullptr, double* work = nullptr);
 // One UMP2 spin block from K[i,a,J,B] = (ia|JB) (oA vA x oB vB) and the two spins' orbital
 // energies (occupied first); same = alpha-alpha or beta-beta (K square, eA == eB).
 template <typename T>

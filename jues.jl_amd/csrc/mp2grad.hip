@@ -108,20 +108,19 @@ __global__ __launch_bounds__(256) void mp2_w_r_kernel(const double* __restrict__
   r[ia] = wcol[ia] + s;
 }
 
-// deps[k] = -sum_a r[k,a] (occupied k), deps[o+c] = sum_i r[i,c] (virtual c)
+// deps[k] = -sum_a r[k,a] (occupied k), deps[o+c] = sum_i r[i,c] (virtual c): a wavefront per orbital (one thread's
+// chain of loads took 60 us at 81 virtual orbitals, 5 this way)
 __global__ __launch_bounds__(256) void mp2_deps_kernel(const double* __restrict__ r, int o, int v,
                                                        double* __restrict__ deps) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
+  const int p = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (p >= o + v) return;
   double s = 0.0;
-  if (p < o) {
-    for (int a = 0; a < v; ++a) s += r[p + (long)o * a];
-    deps[p] = -s;
-  } else {
-    const long c = p - o;
-    for (int i = 0; i < o; ++i) s += r[i + o * c];
-    deps[p] = s;
-  }
+  if (p < o)
+    for (int a = lane; a < v; a += 64) s += r[p + (long)o * a];
+  else
+    for (int i = lane; i < o; i += 64) s += r[i + o * (long)(p - o)];
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+  if (lane == 0) deps[p] = p < o ? -s : s;
 }
 
 // G = dE/dK from K, the energy into *E (host) and, with deps non-null, dE/deps (device, o+v)
@@ -147,7 +146,7 @@ void mp2_g(jues_ctx* ctx, const T* K, const double* eps, int o, int v, T* G, dou
                        ov, chunk, rowpart.as<double>());
     hipLaunchKernelGGL(mp2_w_r_kernel, dim3(gx), dim3(256), 0, ctx->stream, rowpart.as<double>(), (int)nchunk,
                        wcol.as<double>(), ov, r.as<double>());
-    hipLaunchKernelGGL(mp2_deps_kernel, dim3((unsigned)((o + v + 255) / 256)), dim3(256), 0, ctx->stream,
+    hipLaunchKernelGGL(mp2_deps_kernel, dim3((unsigned)((o + v + 3) / 4)), dim3(256), 0, ctx->stream,
                        r.as<double>(), o, v, deps);
     JUES_HIP(hipGetLastError());
     sync(ctx);
@@ -171,8 +170,27 @@ void mp2_grad_factors_dev(jues_ctx* ctx, const T* Co, const T* Cv, int o, int v,
     DevBuf Kb(N * sizeof(T)), Gb(N * sizeof(T));
     T* K = Kb.as<T>();
     T* G = Gb.as<T>();
-    gemm<T>(ctx, false, true, ov, ov, naux, one, L, ov, 0, L, ov, 0, zero, K, ov, 0, 1, "mp2grad_k");
-    mp2_g<T>(ctx, K, eps, o, v, G, E, deps);
+    // in FP64 the lower triangle of the symmetric K is enough
+    bool lower = false, triangle = false;
+    if constexpr (sizeof(T) == 8) {
+      lower = o >= LOWER_MIN_O && o <= LOWER_MAX_O;
+      triangle = lower && gemm_lower(ctx, ov, naux, L, ov, K, ov, "mp2grad_k");
+    }
+    if (!triangle)
+      gemm<T>(ctx, false, true, ov, ov, naux, one, L, ov, 0, L, ov, 0, zero, K, ov, 0, 1, "mp2grad_k");
+    if constexpr (sizeof(T) == 8)
+      if (lower) {
+        DevBuf r(deps ? (size_t)(ov * (v + 1)) * sizeof(double) : 0);
+        *E = mp2_lower_dev(ctx, K, eps, o, v, G, deps ? r.as<double>() + ov * v : nullptr, r.as<double>());
+        if (deps) {
+          KTimer t(ctx, "mp2_grad_eps", 0.0, (double)ov * 16);
+          hipLaunchKernelGGL(mp2_deps_kernel, dim3((unsigned)((o + v + 3) / 4)), dim3(256), 0, ctx->stream,
+                             r.as<double>() + ov * v, o, v, deps);
+          JUES_HIP(hipGetLastError());
+          sync(ctx);
+        }
+      }
+    if (!lower) mp2_g<T>(ctx, K, eps, o, v, G, E, deps);
     Kb.release();
     // dL = (G + G^T) L = 2 G L (G is symmetric: K = L L^T is)
     gemm<T>(ctx, false, false, ov, naux, ov, T(2), G, ov, 0, L, ov, 0, zero, dL, ov, 0, 1, "mp2grad_dl");

@@ -202,6 +202,127 @@ __global__ __launch_bounds__(256) void sum_fixed_kernel(const double* __restrict
   if (threadIdx.x == 0) out[0] = sh[0];
 }
 
+// Energy (and adjoint) from the lower triangle of a symmetric K[(i,a),(j,b)] = (ia|jb).  One workgroup per pair
+// a >= b: its o x o block X[i,j] = K[ia,jb] also holds the exchanged integrals, K_ibja = X[j,i], and all of the pair
+// (b,a)'s, so it is read once into LDS (rows padded to o + 1) and half of K is read in all.  In the blocks a = b,
+// which are symmetric, only i >= j is read.
+// GRAD (a wavefront takes columns j, its lanes i) writes both blocks of G in runs of o and, with rpart non-null, the sums over one occupied index of
+// w = K (2 K - K_ibja) / D^2: rpart[b + v (i + o a)] = sum_j w[ia,jb], and the same with a and b exchanged.
+// Bound by the latency of a pair's loads and by memory: 8640 rows take 132 us (257 as a pass over all of K with the
+// exchanged integrals read from memory), with G and the sums 328 (720 with w stored and summed by passes of its own).
+template <bool GRAD>
+__global__ __launch_bounds__(256) void mp2_lower_kernel(const double* __restrict__ K, const double* __restrict__ eps,
+                                                        int o, int v, double* __restrict__ G,
+                                                        double* __restrict__ rpart, double* __restrict__ part) {
+  extern __shared__ double X[];  // X[i + (o + 1) j], then (GRAD) the wavefronts' sums over j, 4 x o
+  __shared__ double sh[4];
+  const int ld = o + 1, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // pairs in the order of b, then a, a contiguous range of them on each of the 8 XCDs: neighbours, whose runs of o
+  // share cache lines, meet in one L2
+  const long np = (long)v * (v + 1) / 2, per = np / 8, more = np % 8, xcd = blockIdx.x % 8;
+  const long p = np - 1 - (xcd * per + (xcd < more ? xcd : more) + blockIdx.x / 8);
+  int x = (int)((sqrt(8.0 * p + 1.0) - 1.0) / 2.0);
+  while ((long)x * (x + 1) / 2 > p) --x;
+  while ((long)(x + 1) * (x + 2) / 2 <= p) ++x;
+  const int b = v - 1 - x, a = v - 1 - (int)(p - (long)x * (x + 1) / 2);
+  const long ov = (long)o * v, blk = (long)o * a + ov * ((long)o * b), mir = (long)o * b + ov * ((long)o * a);
+  // eight loads of a thread in flight (158 us at 8640 rows with one at a time)
+  for (int q0 = threadIdx.x; q0 < o * o; q0 += 2048) {
+    double x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int q = min(q0 + 256 * u, o * o - 1), i = q % o, j = q / o;
+      x[u] = a == b ? K[blk + max(i, j) + ov * min(i, j)] : K[blk + i + ov * j];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int q = q0 + 256 * u;
+      if (q < o * o) X[q % o + ld * (q / o)] = x[u];
+    }
+  }
+  __syncthreads();
+  const double eab = -eps[o + a] - eps[o + b];
+  double s = 0.0, row[2] = {0.0, 0.0};
+  if (!GRAD)
+    for (int q = threadIdx.x; q < o * o; q += 256) {
+      const int i = q % o, j = q / o;
+      const double x = X[i + ld * j];
+      s += x * ((2.0 * x - X[j + ld * i]) / (eps[i] + eps[j] + eab));
+    }
+  for (int j = wave; GRAD && j < o; j += 4) {
+    double col = 0.0;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int i = lane + 64 * u;
+      if (i >= o) continue;
+      const double x = X[i + ld * j], d = eps[i] + eps[j] + eab, q = (2.0 * x - X[j + ld * i]) / d;
+      s += x * q;
+      G[blk + i + ov * j] = 2.0 * q;
+      if (rpart) {
+        const double w = x * q / d;
+        row[u] += w;
+        col += w;
+      }
+    }
+    if (rpart) {
+      for (int off = 32; off > 0; off >>= 1) col += __shfl_down(col, off, 64);
+      if (lane == 0 && a != b) rpart[a + (long)v * (j + (long)o * b)] = col;
+    }
+  }
+  if constexpr (GRAD) {
+    if (a != b)  // the mirrored block: lanes j
+      for (int i = wave; i < o; i += 4)
+        for (int j = lane; j < o; j += 64)
+          G[mir + j + ov * i] = 2.0 * ((2.0 * X[i + ld * j] - X[j + ld * i]) / (eps[i] + eps[j] + eab));
+    if (rpart) {
+      double* R = X + (long)ld * o;
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        if (lane + 64 * u < o) R[wave * o + lane + 64 * u] = row[u];
+      __syncthreads();
+      for (int i = threadIdx.x; i < o; i += 256)
+        rpart[b + (long)v * (i + (long)o * a)] = (R[i] + R[o + i]) + (R[2 * o + i] + R[3 * o + i]);
+    }
+  }
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+  if (lane == 0) sh[wave] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) part[blockIdx.x] = (a == b ? 1.0 : 2.0) * ((sh[0] + sh[1]) + (sh[2] + sh[3]));
+}
+
+// out = sum of `count` partial sums in a fixed order, four of a thread's loads in flight (with one at a time the
+// 23436 of 216 virtual orbitals took 60 us)
+__global__ __launch_bounds__(1024) void sum_pairs_kernel(const double* __restrict__ part, int count,
+                                                         double* __restrict__ out) {
+  __shared__ double sh[16];
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int i = threadIdx.x; i < count; i += 4096)
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (i + 1024 * u < count) s[u] += part[i + 1024 * u];
+  double t = (s[0] + s[1]) + (s[2] + s[3]);
+  for (int off = 32; off > 0; off >>= 1) t += __shfl_down(t, off, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = t;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double r = 0.0;
+    for (int w = 0; w < 16; ++w) r += sh[w];
+    out[0] = r;
+  }
+}
+
+// r[ia] = 2 sum_b rpart[b, ia] (w is symmetric: its row sums are its column sums), a wavefront per row
+__global__ __launch_bounds__(256) void mp2_lower_r_kernel(const double* __restrict__ rpart, int v, long ov,
+                                                          double* __restrict__ r) {
+  const int lane = threadIdx.x & 63;
+  const long ia = blockIdx.x * 4L + (threadIdx.x >> 6);
+  if (ia >= ov) return;
+  double s = 0.0;
+  for (int b = lane; b < v; b += 64) s += rpart[b + v * ia];
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+  if (lane == 0) r[ia] = 2.0 * s;
+}
+
 // UMP2 blocks (UMP2.jl:30-77).  One block per (J,B) column of K[i,a,J,B] = (ia|JB).
 // same != 0 (alpha-alpha or beta-beta, K square): accumulates (ia|jb)((ia|jb) - (ib|ja)) / D,
 // half of which is the sum over i > j, a > b of <ij||ab>^2 / D; otherwise (ia|JB)^2 / D.
@@ -264,6 +385,31 @@ double mp2_energy_dev(jues_ctx* ctx, const T* K, const double* eps, int o, int v
   }
   double E = 0.0;
   d2h(ctx, &E, part + ov, sizeof(double));
+  return E;
+}
+
+double mp2_lower_dev(jues_ctx* ctx, const double* K, const double* eps, int o, int v, double* G, double* r,
+                     double* work) {
+  JUES_REQUIRE(o >= LOWER_MIN_O && o <= LOWER_MAX_O && (!r || (G && work)), "mp2_lower: bad arguments");
+  const long ov = (long)o * v, pairs = (long)v * (v + 1) / 2;
+  JUES_REQUIRE(pairs < (1L << 31), "mp2_lower: too many pairs");
+  double* part = static_cast<double*>(scratch(ctx, 14, sizeof(double) * (size_t)(pairs + 1)));
+  const size_t lds = sizeof(double) * (size_t)(o * (o + 1) + (r ? 4 * o : 0));
+  {
+    KTimer t(ctx, G ? "mp2_grad_g" : "mp2_energy", 6.0 * ov * ov / 2, (double)ov * ov * (G ? 12.0 : 4.0));
+    if (G)
+      hipLaunchKernelGGL(mp2_lower_kernel<true>, dim3((unsigned)pairs), dim3(256), lds, ctx->stream, K, eps, o, v, G,
+                         r ? work : nullptr, part);
+    else
+      hipLaunchKernelGGL(mp2_lower_kernel<false>, dim3((unsigned)pairs), dim3(256), lds, ctx->stream, K, eps, o, v,
+                         nullptr, nullptr, part);
+    hipLaunchKernelGGL(sum_pairs_kernel, dim3(1), dim3(1024), 0, ctx->stream, part, (int)pairs, part + pairs);
+    if (r)
+      hipLaunchKernelGGL(mp2_lower_r_kernel, dim3((unsigned)((ov + 3) / 4)), dim3(256), 0, ctx->stream, work, v, ov, r);
+    JUES_HIP(hipGetLastError());
+  }
+  double E = 0.0;
+  d2h(ctx, &E, part + pairs, sizeof(double));
   return E;
 }
 
