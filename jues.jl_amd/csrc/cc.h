@@ -25,7 +25,6 @@ struct CCInts {
   // o v^3 terms contract these factors (LovT[a,i,P] = Lov[i,a,P], Lovp[i,P,a] = Lov[i,a,P])
   DevBuf Lov, LovT, Lovp;
   DevBuf Lvv;     // MO factors L[ae,P] (v^2 x naux) when the ladder is recomputed or (ia|bc) factored
-  DevBuf Lvvt;    // the same with a and e exchanged: L[ea,P]
   // off-diagonal Fock blocks of a non-canonical reference (AutoRCCSD.jl:215-232):
   // f_mi at [m,i], f_ae at [a,e] (diagonals zero), f_ia at [i,a]
   DevBuf fOO, fVV, fOV;
@@ -74,7 +73,7 @@ struct CCWork {
 enum SplitSlot {
   SP_UOV, SP_TTOV, SP_WE, SP_WJ, SP_U2, SP_Q, SP_TPT, SP_TMT, SP_TQ, SP_TM, SP_WPT, SP_WMT,
   SP_UOV_T, SP_TTOV_T,
-  SPLIT_CONST = 16, SP_LX = SPLIT_CONST, SP_KX, SP_VP, SP_VM, SP_KPT, SP_KMT, SP_LVVT, SP_LVVTT, SP_WE0, SP_WJ0,
+  SPLIT_CONST = 16, SP_LX = SPLIT_CONST, SP_KX, SP_VP, SP_VM, SP_KPT, SP_KMT, SP_LVVT, SP_WE0, SP_WJ0,
   SP_LOV, SP_LOVT, SP_LOVAT, SPLIT_SLOTS
 };
 struct SplitState {

@@ -56,6 +56,14 @@ void build_pairs(jues_ctx* ctx, CCState& S) {
   S.P.v_lt = S.pair_buf[3].as<int2>();
 }
 
+// Virtual indices f of a slab of (ae|bf): an eighth of them, since a slab's products with e >= f1 are left out (0.56 of
+// the work then; at 190 virtual orbitals 18 ms, 29 in slabs of 2 GB), but 1400 columns (b,f) for the product's sake, and
+// at most 1 GB
+long vvvv_slab(int v, size_t elem) {
+  const long nf = std::max<long>((v + 7) / 8, (1400 + v - 1) / v);
+  return std::max(1L, std::min<long>(std::min<long>(nf, v), (1L << 30) / ((long)v * v * v * (long)elem)));
+}
+
 // chemist (vv|vv) slabs -> packed V+/V- (FP64); dense route transforms the whole block
 void build_vvvv(jues_ctx* ctx, CCState& S, CCInts<double>& I, const double* Cv) {
   const int v = S.v;
@@ -65,33 +73,31 @@ void build_vvvv(jues_ctx* ctx, CCState& S, CCInts<double>& I, const double* Cv) 
   if (ctx->gao.p) {
     DevBuf X((size_t)v2 * v2 * sizeof(double));
     tei_transform_dev<double>(ctx, Cv, v, Cv, v, Cv, v, Cv, v, X.as<double>());
-    pack_v<double, double>(ctx, S.P, X.as<double>(), v, 0, v, Vp, Vm);
+    pack_v<double>(ctx, S.P, X.as<double>(), v2, v, 0, v, Vp, 0, S.P.npv, Vm, 0, std::max(1L, S.P.nmv));
     sync(ctx);
   } else {
     const long naux = ctx->naux;
     DevBuf Lvv((size_t)v2 * naux * sizeof(double));
     mo_factors_dev<double>(ctx, Cv, v, Cv, v, Lvv.as<double>());
-    // slab of nf virtual indices f: X[a,e,b,f] = sum_P Lvv[ae,P] Lvv[bf,P] (~2 GB per slab)
-    long nf = std::max(1L, std::min<long>(v, (2L << 30) / (long)(v2 * v * sizeof(double))));
+    // slabs of nf virtual indices f: X[a,e,b,f] = sum_P Lvv[ae,P] Lvv[bf,P] in the rows e < f1 that the pairs e <= f need
+    const long nf = vvvv_slab(v, sizeof(double));
     DevBuf X((size_t)(v2 * v * nf) * sizeof(double));
     for (int f0 = 0; f0 < v; f0 += (int)nf) {
       const int f1 = (int)std::min<long>(v, f0 + nf);
-      gemm<double>(ctx, false, true, v2, (long)v * (f1 - f0), naux, 1.0, Lvv.as<double>(), v2, 0,
-                   Lvv.as<double>() + (long)v * f0, v2, 0, 0.0, X.as<double>(), v2, 0, 1, "setup_vvvv");
-      pack_v<double, double>(ctx, S.P, X.as<double>(), v, f0, f1, Vp, Vm);
+      const long rows = (long)v * f1;
+      gemm<double>(ctx, false, true, rows, (long)v * (f1 - f0), naux, 1.0, Lvv.as<double>(), v2, 0,
+                   Lvv.as<double>() + (long)v * f0, v2, 0, 0.0, X.as<double>(), rows, 0, 1, "setup_vvvv");
+      pack_v<double>(ctx, S.P, X.as<double>(), rows, v, f0, f1, Vp, 0, S.P.npv, Vm, 0, std::max(1L, S.P.nmv));
     }
     sync(ctx);
   }
 }
 
-// MO factors of the (vv|vv) block for the recomputed ladder: L[ae,P] = (Cv^T B_P Cv)[a,e],
-// and L[ea,P] (no symmetry of B_P in the AO pair is assumed)
+// MO factors of the (vv|vv) block for the recomputed ladder: L[ae,P] = (Cv^T B_P Cv)[a,e]
 void build_lvv(jues_ctx* ctx, CCInts<double>& I, const double* Cv, int v) {
   const long naux = ctx->naux;
   double* L = bufp<double>(I.Lvv, (size_t)v * v * naux);
   mo_factors_dev<double>(ctx, Cv, v, Cv, v, L);
-  double* Lt = bufp<double>(I.Lvvt, (size_t)v * v * naux);
-  permute<double, double>(ctx, L, {v, v, naux}, {1, 0, 2}, Lt, 1.0, 0.0, "setup_vvvv");
 }
 
 // Whether <ab|ef> is rebuilt every iteration.  Auto: when the packed V+/V- (with its FP32
@@ -225,7 +231,6 @@ void cc_make_ints32(jues_ctx* ctx, CCState& S) {
   convert_buf<float>(ctx, a.LovT, b.LovT);
   convert_buf<float>(ctx, a.Lovp, b.Lovp);
   convert_buf<float>(ctx, a.Lvv, b.Lvv);
-  convert_buf<float>(ctx, a.Lvvt, b.Lvvt);
   convert_buf<float>(ctx, a.fOO, b.fOO);
   convert_buf<float>(ctx, a.fVV, b.fVV);
   convert_buf<float>(ctx, a.fOV, b.fOV);
@@ -428,9 +433,10 @@ template void ovvv_z_slab<float>(jues_ctx*, CCState&, int, int, const float*, co
                                  float*, float*);
 
 // The ladder with <ab|ef> rebuilt from the factors every iteration (DF-RCCD.jl:198-215
-// contracts bvv[a,e,Q] bvv[b,f,Q] the same way): for a slab of f, X[e,a,b,f] =
-// sum_P L[ea,P] L[bf,P] = (ae|bf); its rows of V+/V- (pairs e<=f / e<f with f in the slab)
-// are a contiguous K-range of the ladder product, accumulated into Lp / Lm.  V+/V- never exist.
+// contracts bvv[a,e,Q] bvv[b,f,Q] the same way): for a slab of f, X[a,e,b,f] =
+// sum_P L[ae,P] L[bf,P] = (ae|bf), in smaller slabs whose rows with e past them are left out; its rows of V+/V-
+// (pairs e<=f / e<f with f in the slab) are a contiguous K-range of the ladder product, accumulated into Lp / Lm.
+// V+/V- never exist.
 template <typename T>
 static void ladder_recompute_mm(jues_ctx* ctx, CCState& S, const double* amp, const double* t1, T* Tp, T* Tm, T* Lp,
                                 T* Lm) {
@@ -445,11 +451,11 @@ static void ladder_recompute_mm(jues_ctx* ctx, CCState& S, const double* amp, co
   if (const char* env = std::getenv("JUES_LADDER_SLAB_BYTES")) slab_bytes = std::max(1L, std::atol(env));
   const long nf = std::max(1L, std::min<long>(v, slab_bytes / (long)(v2 * v * sizeof(T))));
   const long rows_p = (long)std::min<long>(v, nf) * v;  // bound on the packed rows of one slab
-  T* X = bufp<T>(W.Xs, (size_t)(v2 * v * nf));
+  const long nx = std::min(nf, vvvv_slab(v, sizeof(T)));
+  T* X = bufp<T>(W.Xs, (size_t)(v2 * v * nx));
   T* Vps = bufp<T>(W.Vps, (size_t)(rows_p * P.npv));
   T* Vms = bufp<T>(W.Vms, (size_t)std::max(1L, rows_p * P.nmv));
   const T* L = ints<T>(S).Lvv.template as<T>();
-  const T* Lt = ints<T>(S).Lvvt.template as<T>();
   bool split = false;
   if constexpr (sizeof(T) == 4) split = S.split_on;
   bool first_m = true;
@@ -457,15 +463,27 @@ static void ladder_recompute_mm(jues_ctx* ctx, CCState& S, const double* amp, co
     const int f1 = (int)std::min<long>(v, f0 + nf);
     const long r0p = (long)f0 * (f0 + 1) / 2, nrp = (long)f1 * (f1 + 1) / 2 - r0p;
     const long r0m = (long)f0 * (f0 - 1) / 2, nrm = (long)f1 * (f1 - 1) / 2 - r0m;
-    const long ncol = (long)v * (f1 - f0);
+    for (int g0 = f0; g0 < f1; g0 += (int)nx) {
+      const int g1 = (int)std::min<long>(f1, g0 + nx);
+      const long rows = (long)v * g1, ncol = (long)v * (g1 - g0);
+      bool done = false;
+      if constexpr (sizeof(T) == 4) {
+        if (split) {
+          // from the planes (k = P) of L[ae,P]: the rows and the slab's columns (bf) are columns of them
+          const Split16& lt = split_operand<double>(ctx, S, SP_LVVT, S.i64->Lvv.as<double>(), naux, v2, true);
+          gemm16_tn(ctx, rows, ncol, 1.0f, split16_cols(lt, 0, rows), split16_cols(lt, (long)v * g0, ncol), 0.0f, X,
+                    rows, "cc_vvvv_gen");
+          done = true;
+        }
+      }
+      if (!done)
+        gemm<T>(ctx, false, true, rows, ncol, naux, T(1), L, v2, 0, L + (long)v * g0, v2, 0, T(0), X, rows, 0, 1,
+                "cc_vvvv_gen");
+      pack_v<T>(ctx, P, X, rows, v, g0, g1, Vps, r0p, nrp, Vms, r0m, std::max(1L, nrm));
+    }
     if constexpr (sizeof(T) == 4) {
       if (split) {
         SplitState& Z = split_state(S);
-        // X[(ea),(bf)] from the planes (k = P) of L[ea,P] and of the slab's columns (bf) of L[bf,P]
-        const Split16& lt = split_operand<double>(ctx, S, SP_LVVT, S.i64->Lvv.as<double>(), naux, v2, true);
-        const Split16& ltt = split_operand<double>(ctx, S, SP_LVVTT, S.i64->Lvvt.as<double>(), naux, v2, true);
-        gemm16_tn(ctx, v2, ncol, 1.0f, ltt, split16_cols(lt, (long)v * f0, ncol), 0.0f, X, v2, "cc_vvvv_gen");
-        pack_v_ea<float>(ctx, P, X, v, f0, f1, Vps, Vms);
         split16t<float>(ctx, Tp + r0p * P.npo, nrp, P.npo, P.npo, Z.tpc, "cc_split");
         split16<float>(ctx, Vps, nrp, P.npv, nrp, Z.vps, "cc_split");
         gemm16_tn(ctx, P.npo, P.npv, 1.0f, Z.tpc.s, Z.vps.s, f0 == 0 ? 0.0f : 1.0f, Lp, P.npo, "cc_pp_ladder");
@@ -478,9 +496,6 @@ static void ladder_recompute_mm(jues_ctx* ctx, CCState& S, const double* amp, co
         continue;
       }
     }
-    gemm<T>(ctx, false, true, v2, ncol, naux, T(1), Lt, v2, 0, L + (long)v * f0, v2, 0, T(0), X, v2, 0, 1,
-            "cc_vvvv_gen");
-    pack_v_ea<T>(ctx, P, X, v, f0, f1, Vps, Vms);
     gemm<T>(ctx, false, false, P.npo, P.npv, nrp, T(1), Tp + r0p * P.npo, P.npo, 0, Vps, nrp, 0,
             f0 == 0 ? T(0) : T(1), Lp, P.npo, 0, 1, "cc_pp_ladder");
     if (minus && nrm > 0) {
@@ -1086,7 +1101,7 @@ static void thin_fp64_ints(jues_ctx* ctx, CCState& S) {
   sync(ctx);
   CCInts<double>& I = *S.i64;
   for (DevBuf* b : {&I.Kov, &I.Ktov, &I.Jov, &I.Lx, &I.Ka, &I.oooo, &I.Vp, &I.Vm, &I.KP, &I.KM, &I.ooov_c, &I.ovvv_c,
-                    &I.Lov, &I.LovT, &I.Lovp, &I.Lvv, &I.Lvvt})
+                    &I.Lov, &I.LovT, &I.Lovp, &I.Lvv})
     b->release();
   S.i64_thin = true;
 }

@@ -72,9 +72,10 @@ struct DiisOrder {
 template <typename T>
 void pack_t(jues_ctx* ctx, const PairTables& P, const double* t, int o, int v, T* Tp, T* Tm,
             const double* t1 = nullptr);
-template <typename Ts, typename Td>
-void pack_v(jues_ctx* ctx, const PairTables& P, const Ts* X, int v, int f0, int f1, Td* Vp, Td* Vm,
-            bool slab = false);
+// V+/V- rows (pairs with f in [f0,f1)) from X[a,e,b,f-f0] = (ae|bf), whose rows (a,e) hold e < f1 (at least)
+template <typename T>
+void pack_v(jues_ctx* ctx, const PairTables& P, const T* X, long ldx, int v, int f0, int f1, T* Vp, long rowp0,
+            long ldp, T* Vm, long rowm0, long ldm);
 // hole-hole ladder integrals on pairs: KP[(k<=l),(c<=d)], KM[(k<l),(c<d)] from K[k,l,c,d] = <kl|cd>
 void pack_khh(jues_ctx* ctx, const PairTables& P, const double* K, int o, int v, double* KP, double* KM);
 // W[m,n,i,j] -> WPT[(i<=j),(k<=l)], WMT[(i<j),(k<l)] (the kl-pair sum / difference, transposed)
@@ -92,9 +93,6 @@ void ring_start(jues_ctx* ctx, const T* K, T s, const T* X, const T* Fae, const 
 // Tq = Tp with its (a,a) columns doubled
 template <typename T>
 void pair_diag2(jues_ctx* ctx, const PairTables& P, const T* Tp, T* Tq);
-// slab-local V+/V- rows (pairs with f in [f0,f1)) from X[e,a,b,f-f0] = (ae|bf)
-template <typename T>
-void pack_v_ea(jues_ctx* ctx, const PairTables& P, const T* X, int v, int f0, int f1, T* Vp, T* Vm);
 template <typename TR>
 void t2_update(jues_ctx* ctx, const UpdateArgs<TR>& A);
 // whether the update kernel sums S = H + H^T + Y^x + (Y^x)^T itself: its o x (o + 1) LDS slab

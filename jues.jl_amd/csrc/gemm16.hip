@@ -474,23 +474,16 @@ void Split16Buf::ensure(long rows, long cols) {
 }
 
 template <typename Ti>
-void split16(jues_ctx* ctx, const Ti* X, long rows, long cols, long ldx, Split16Buf& out, const char* tag,
-             const int* sexp_of) {
+void split16(jues_ctx* ctx, const Ti* X, long rows, long cols, long ldx, Split16Buf& out, const char* tag) {
   JUES_REQUIRE(ldx >= rows, "split16: ldx < rows");
   out.ensure(rows, cols);
   const Split16& s = out.s;
   const long n = rows * cols;
-  KTimer t(ctx, tag ? tag : "split16", 0.0, (sexp_of ? 1.0 : 2.0) * sizeof(Ti) * n + 4.0 * s.rows_p * s.cols_p);
-  if (sexp_of) {
-    // the caller vouches that X holds the same values as the operand whose scale this is
-    JUES_HIP(hipMemcpyAsync(s.sexp, sexp_of, sizeof(int), hipMemcpyDeviceToDevice, ctx->stream));
-  } else {
-    double* part = static_cast<double*>(scratch(ctx, 3, MAX_PART * sizeof(double)));
-    const int nb = grid_for(n, MAX_PART);
-    hipLaunchKernelGGL((maxabs_kernel<Ti>), dim3(nb), dim3(256), 0, ctx->stream, X, rows, cols, ldx, aligned16(X),
-                       part);
-    hipLaunchKernelGGL(split_scale_kernel, dim3(1), dim3(256), 0, ctx->stream, part, nb, s.sexp);
-  }
+  KTimer t(ctx, tag ? tag : "split16", 0.0, 2.0 * sizeof(Ti) * n + 4.0 * s.rows_p * s.cols_p);
+  double* part = static_cast<double*>(scratch(ctx, 3, MAX_PART * sizeof(double)));
+  const int nb = grid_for(n, MAX_PART);
+  hipLaunchKernelGGL((maxabs_kernel<Ti>), dim3(nb), dim3(256), 0, ctx->stream, X, rows, cols, ldx, aligned16(X), part);
+  hipLaunchKernelGGL(split_scale_kernel, dim3(1), dim3(256), 0, ctx->stream, part, nb, s.sexp);
   if (s.rows_p / 8 >= 192) {
     const int vec = aligned16(X) && (ldx * (long)sizeof(Ti)) % 16 == 0;
     hipLaunchKernelGGL((split_cols_kernel<Ti>), dim3((unsigned)std::min(s.cols_p, 65536L)), dim3(256), 0, ctx->stream,
@@ -593,8 +586,8 @@ void gemm16_tn(jues_ctx* ctx, long M, long N, float alpha, const Split16& A, con
   }
 }
 
-template void split16<float>(jues_ctx*, const float*, long, long, long, Split16Buf&, const char*, const int*);
-template void split16<double>(jues_ctx*, const double*, long, long, long, Split16Buf&, const char*, const int*);
+template void split16<float>(jues_ctx*, const float*, long, long, long, Split16Buf&, const char*);
+template void split16<double>(jues_ctx*, const double*, long, long, long, Split16Buf&, const char*);
 template void split16t<float>(jues_ctx*, const float*, long, long, long, Split16Buf&, const char*);
 template void split16t<double>(jues_ctx*, const double*, long, long, long, Split16Buf&, const char*);
 
