@@ -1619,10 +1619,10 @@ static double form_us(int form, long tiles, long slabs, double bytes) {
   switch (form) {
     case TILE128: return 8.5 + std::max(hbm, (slabs + 1) * std::max(f == 1.0 ? 2.5 : 1.4, cu * 1.71 * f / 0.86));
     case TILE64: {
-      // twice TILE128's operand traffic: at 7.2 TB/s from the L2s it is what bounds a 6460^3 FP64 product
-      // (9.5 ms; 8.6 with 128x128 tiles)
-      const double cache = (double)tiles * slabs * 2048.0 * sizeof(T) / 7.2e6;
-      return 7.0 + std::max(std::max(hbm, cache), (slabs + 1) * std::max(f == 1.0 ? 0.8 : 0.72, cu * 0.427 * f / 0.8));
+      // twice TILE128's operand traffic: at 8.4 TB/s from the L2s it is what bounds a 6460^3 FP64 product
+      // (9.0 ms; 7.7 with 128x128 tiles)
+      const double cache = (double)tiles * slabs * 2048.0 * sizeof(T) / 8.4e6;
+      return 7.0 + std::max(std::max(hbm, cache), (slabs + 1) * std::max(f == 1.0 ? 0.8 : 0.72, cu * 0.427 * f / (f == 1.0 ? 0.8 : 0.85)));
     }
     case SHORT:
     case TALL: return 8.0 + std::max(hbm, (slabs + 1) * std::max(1.6 * f, cu * 1.28 * f / 0.75));
@@ -1688,7 +1688,7 @@ static double tail_us(const TailMap& t) {
   const double rounds = (double)cdiv(t.wgs, 256);
   const double slabs = t.whole / 256 * (t.nk + 2.5) + rounds * ((double)t.nk / chunks + 2.5);
   const double latency = 1.64 / 1.87 * (t.nk * (t.whole / 256 + 1.0 / least) + 2.5);
-  const double parts = t.wgs > tiles ? (2.0 * t.wgs + tiles) * 131072.0 / 4.5e6 + 5.0 : 0.0;
+  const double parts = t.wgs > tiles ? (2.0 * t.wgs + tiles) * 131072.0 / 6.0e6 + 5.0 : 0.0;
   return 11.0 + 1.87 * std::max(slabs, latency) * (t.whole + t.wgs <= 256 ? 1.08 : 1.0) + parts;
 }
 
