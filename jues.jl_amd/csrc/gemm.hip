@@ -122,10 +122,10 @@ __device__ inline void lower_tile(int p2, int m, int& tm, int& tn) {
 // A TAIL launch of a product: `whole` workgroups have a tile each, and the other tiles' 16-deep k-slabs are shared by
 // several workgroups a tile, whose parts of it gemm_tail_kernel adds.  Tiles are taken full ones first (grouped),
 // then those past the edge of N, of M and of both: four runs of n[] tiles left to the tail, in s[] chunks each.
-// Within a run, workgroups (and their parts) are ordered chunk by chunk: neighbours read the same k-slabs.
+// Within a run, the parts are ordered chunk by chunk: neighbours read the same k-slabs.
 // 256 compute units leave much of a last round of tiles idle otherwise, and split whole products write more parts
-// (and round no better): 3082^3 took 980 us in two chunks, 878 this way, 6460^3 8.6 and 7.7 ms (73 TFLOP/s would be 7.4),
-// 253 x 8911 x 8911 855 and 652 us, 8640 x 768 x 8640 1790 and 1660.
+// (and round no better): FP64 3082^3 took 980 us in two chunks, 890 this way, 6460^3 8.6 and 7.6 ms (73 TFLOP/s would be
+// 7.4), 276 x 9045 x 9045 902 and 792 us, 8640 x 768 x 8640 1790 and 1660; FP32 3082^3 507 and 478.
 struct TailMap {
   int whole = 0, wgs = 0, nk = 0, full_m = 0, full_n = 0;
   int n[4] = {}, s[4] = {};
@@ -139,21 +139,27 @@ struct TailMap {
     else if ((p2 -= n[1]) < n[2]) tm = full_m, tn = p2;
     else tm = full_m, tn = full_n;
   }
-  // tile of the tail and chunk of it (of `chunks`) of workgroup x
-  __device__ void part(int x, int& tile, int& chunk, int& chunks) const {
-    int base = 0;
+  // tile of the tail, chunk of it (of `chunks`) and place of its part, of workgroup x.  The runs past an edge come
+  // first (their few long chunks end last otherwise), and each run is dealt to the XCDs in equal contiguous shares.
+  __device__ void part(int x, int& tile, int& chunk, int& chunks, int& place) const {
+    int at = 0;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (x < n[q] * s[q]) {
-        chunk = x / n[q];
-        tile = base + x - chunk * n[q];
+    for (int k = 1; k <= 4; ++k) {
+      const int q = k & 3, count = n[q] * s[q];
+      if (x < count) {
+        const int per = count / NXCD, more = count % NXCD, xcd = x % NXCD;
+        const int y = xcd * per + min(xcd, more) + x / NXCD;
+        chunk = y / n[q];
+        tile = first_tile(q) + y - chunk * n[q];
         chunks = s[q];
+        place = at + y;
         return;
       }
-      x -= n[q] * s[q];
-      base += n[q];
+      x -= count;
+      at += count;
     }
   }
+  __device__ int first_tile(int q) const { return (q > 0 ? n[0] : 0) + (q > 1 ? n[1] : 0) + (q > 2 ? n[2] : 0); }
 };
 
 // One product of a high-occupancy kernel launch: C = alpha A op(B) + beta C, batched over
@@ -207,7 +213,7 @@ __device__ inline int g32_chunk(int q, int r) { return q ^ ((r >> 2) & 3); }
 // Workgroups [0, nt0) run product p0 (nt0 padded up to a multiple of NXCD when a second
 // product follows), the rest p1.  OUT64: C = alpha A op(B) is written to the FP64 array C64
 // (beta = 0).
-template <int KIND, bool TB, bool TA = false, bool SEG = false, bool OUT64 = false, int BT = 128>
+template <int KIND, bool TB, bool TA = false, bool SEG = false, bool OUT64 = false, int BT = 128, bool TAIL = false>
 __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, GemmSide<float> p1, int nt0,
                                                            float alpha, float beta) {
   constexpr int BM = BT, BN = BT, BK = 16;
@@ -222,7 +228,7 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
   const auto mrow = [&](int i) { return (2 * i + wm) * 16; };
   const auto ncol = [&](int j) { return (2 * j + wn) * 16; };
   int bx, bz;
-  const bool placed = entry_place(bx, bz), second = bx >= nt0;
+  const bool placed = entry_place(bx, bz), second = !TAIL && bx >= nt0;
   const GemmSide<float> g = second ? p1 : p0;
   const int M = g.M, N = g.N, K = bz == g.nz - 1 ? g.Klast : g.K;
   if (bz >= g.nz) return;
@@ -241,10 +247,22 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
   // slices from k = 0; the tail is loaded in the prologue
   const int K16 = K / BK * BK, tail = K > K16 ? 1 : 0;
   const int nk = K16 / BK + tail + K1 / BK;
-  int tm, tn;
-  if (!tile_coords_bounded(second ? bx - nt0 : bx, second ? (int)gridDim.x - nt0 : nt0, g.tiles_m, g.tiles_n, tm, tn,
-                           placed))
+  int tm, tn, ka = 0, kb = nk, wg = 0;
+  bool shared = false;  // the workgroup's result is a part of its tile
+  if (TAIL && bx >= g.tail.whole) {
+    int t = 0, c = 0, nc = 1;
+    g.tail.part(bx - g.tail.whole, t, c, nc, wg);
+    shared = nc > 1;
+    ka = (int)((long)nk * c / nc);
+    kb = (int)((long)nk * (c + 1) / nc);
+    g.tail.coords(g.tail.whole + t, tm, tn);
+  } else if (TAIL) {
+    const int per = g.tail.whole / NXCD;
+    g.tail.coords(bx % NXCD * per + bx / NXCD, tm, tn);
+  } else if (!tile_coords_bounded(second ? bx - nt0 : bx, second ? (int)gridDim.x - nt0 : nt0, g.tiles_m, g.tiles_n,
+                                  tm, tn, placed)) {
     return;
+  }
   const int m0 = tm * BM, n0 = tn * BN;
 
   // A share: row am, 4-k chunks ac0 and ac0 + 2; B share: rows bn and bn + 64, chunk bc
@@ -340,7 +358,7 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
     for (int j = 0; j < NB; ++j) acc[i][j] = fvec4{0, 0, 0, 0};
 
   const int fr = lane & 15, fk = lane >> 4;
-  if (tail) {
+  if (tail && ka == 0) {
     if constexpr (TA) {
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
@@ -378,7 +396,7 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
         rb[j][u] = val;
       }
   } else {
-    load(0);
+    load(ka - tail);
   }
   store(0);
   __syncthreads();
@@ -431,17 +449,28 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
     }
   };
   const auto loop = [&](auto slice) {
-    for (int kt = 0; kt + 1 < nk; ++kt) {
-      const int cur = kt & 1;
+    for (int kt = ka; kt + 1 < kb; ++kt) {
+      const int cur = (kt - ka) & 1;
       load(kt + 1 - tail);
       slice(cur);
       store(cur ^ 1);
       __syncthreads();
     }
-    slice((nk - 1) & 1);
+    slice((kb - 1 - ka) & 1);
   };
   if (ilim == NB && jlim == NB) loop(compute);
   else loop(compute_edge);
+  if (TAIL && shared) {
+    // a partial tile, as the registers hold it, for gemm_tail_kernel
+    float* __restrict__ P = g.part + (long)wg * (BM * BN) + tid;
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) P[((i * NB + j) * 4 + r) * 256] = alpha * acc[i][j][r];
+    return;
+  }
 
   if constexpr (OUT64) {
     double* __restrict__ C64 = g.C64 + (long)bz * g.sC;
@@ -547,11 +576,8 @@ __global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, 
   int tm, tn, ka = 0, kb = nk, wg = 0;
   bool shared = false;  // the workgroup's result is a part of its tile
   if (TAIL && bx >= g.tail.whole) {
-    const int x = bx - g.tail.whole, per = ((int)gridDim.x - g.tail.whole) / NXCD;
-    wg = x % NXCD * per + x / NXCD;  // neighbours on one XCD
-    if (wg >= g.tail.wgs) return;
     int t = 0, c = 0, nc = 1;
-    g.tail.part(wg, t, c, nc);
+    g.tail.part(bx - g.tail.whole, t, c, nc, wg);
     shared = nc > 1;
     ka = (int)((long)nk * c / nc);
     kb = (int)((long)nk * (c + 1) / nc);
@@ -950,32 +976,32 @@ __global__ void scale_kernel(T* C, long M, long N, long ldc, T beta) {
 // of K = 200000) the sum is otherwise a chain of as many memory latencies.
 // C = (sum of the parts of a TAIL launch's tile, in the order of its slabs) + beta C.  blockIdx.x: tile of the
 // tail, blockIdx.y: 1024 of its 128 x 128 results, in the order of the workgroups' registers.
-__global__ __launch_bounds__(256) void gemm_tail_kernel(GemmSide<double> g, double beta) {
-  constexpr int BT = 128;
+template <typename T>
+__global__ __launch_bounds__(256) void gemm_tail_kernel(GemmSide<T> g, T beta) {
+  constexpr int BT = 128, NTH = sizeof(T) == 8 ? 512 : 256, NJ = sizeof(T) == 8 ? 2 : 4;
   const TailMap& tail = g.tail;
-  int tm, tn, q = 0, t = (int)blockIdx.x;
-  tail.coords(tail.whole + t, tm, tn);
-  long first = 0;  // part 0 of the tile's run
-  while (q < 3 && t >= tail.n[q]) {
-    first += (long)tail.n[q] * tail.s[q];
-    t -= tail.n[q++];
-  }
+  int tm, tn, q = 3, first = 0;  // the tile's run and its parts' place
+  tail.coords(tail.whole + (int)blockIdx.x, tm, tn);
+  while (q > 0 && (int)blockIdx.x < tail.first_tile(q)) --q;
   if (tail.s[q] == 1) return;  // written by its workgroup
+  for (int k = 1; k <= 3 && k != q; ++k) first += tail.n[k] * tail.s[k];
+  const int t = (int)blockIdx.x - tail.first_tile(q);
   const int q0 = (int)blockIdx.y * 1024 + threadIdx.x;
-  double sum[4] = {0.0, 0.0, 0.0, 0.0};
+  T sum[4] = {T(0), T(0), T(0), T(0)};
   for (int c = 0; c < tail.s[q]; ++c) {
-    const double* P = g.part + (first + (long)c * tail.n[q] + t) * (BT * BT) + q0;
+    const T* P = g.part + (long)(first + c * tail.n[q] + t) * (BT * BT) + q0;
 #pragma unroll
     for (int u = 0; u < 4; ++u) sum[u] += P[256 * u];
   }
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
-    const int x = q0 + 256 * u, th = x % 512, e = x / 512, lane = th & 63, wm = (th >> 6) & 1, wn = th >> 7;
-    const int i = e / 8, j = e / 4 % 2, r = e % 4;
-    const int m = tm * BT + (2 * i + wm) * 16 + (lane & 15), n = tn * BT + (4 * j + wn) * 16 + (lane >> 4) + 4 * r;
+    const int x = q0 + 256 * u, th = x % NTH, e = x / NTH, lane = th & 63, wm = (th >> 6) & 1, wn = th >> 7;
+    const int i = e / (4 * NJ), j = e / 4 % NJ, r = e % 4, m = tm * BT + (2 * i + wm) * 16 + (lane & 15);
+    const int n = tn * BT + (sizeof(T) == 8 ? (4 * j + wn) * 16 + (lane >> 4) + 4 * r
+                                            : (2 * j + wn) * 16 + 4 * (lane >> 4) + r);
     if (m >= g.M || n >= g.N) continue;
-    double* c = g.C + m + (long)n * g.ldc;
-    *c = beta != 0.0 ? sum[u] + beta * *c : sum[u];
+    T* c = g.C + m + (long)n * g.ldc;
+    *c = beta != T(0) ? sum[u] + beta * *c : sum[u];
   }
 }
 
@@ -1562,7 +1588,7 @@ enum GemmForm { TILE128, TILE64, SHORT, TALL, DIRECT22, DIRECT21, DIRECT12, DIRE
 struct GemmPlan {
   int form = DIRECT22;
   long split = 1;   // chunks of the contraction, each a launch-z entry with its own partial product
-  TailMap tail;     // wgs > 0: a TAIL launch of FP64 128x128 tiles
+  TailMap tail;     // wgs > 0: a TAIL launch of 128x128 tiles
   double us = 1e300;
 };
 
@@ -1676,9 +1702,11 @@ static TailMap tail_map(long M, long N, long K, long whole, int chunks, bool low
 }
 
 // Estimated time (us) of a TAIL launch: a compute unit's slabs, and 2.5 for each workgroup's start and end, at the
-// rate that a long FP64 launch of 128x128 tiles reaches (1.87 us; 8% more where there is a single workgroup), but at
-// least the 1.64 us of latency of each slab of the longest chunk; and the parts, written and read once.
+// rate that a long launch of 128x128 tiles reaches (1.87 us in FP64, 0.92 in FP32; more where few workgroups
+// share a unit), but at least the latency of each slab of the longest chunk; and the parts, written and read once.
+template <typename T>
 static double tail_us(const TailMap& t) {
+  constexpr bool dp = sizeof(T) == 8;
   int tiles = 0, least = 1 << 30;
   for (int q = 0; q < 4; ++q) {
     tiles += t.n[q];
@@ -1687,9 +1715,11 @@ static double tail_us(const TailMap& t) {
   const int chunks = t.n[0] ? t.s[0] : least;
   const double rounds = (double)cdiv(t.wgs, 256);
   const double slabs = t.whole / 256 * (t.nk + 2.5) + rounds * ((double)t.nk / chunks + 2.5);
-  const double latency = 1.64 / 1.87 * (t.nk * (t.whole / 256 + 1.0 / least) + 2.5);
-  const double parts = t.wgs > tiles ? (2.0 * t.wgs + tiles) * 131072.0 / 6.0e6 + 5.0 : 0.0;
-  return 11.0 + 1.87 * std::max(slabs, latency) * (t.whole + t.wgs <= 256 ? 1.08 : 1.0) + parts;
+  const double latency = (dp ? 0.88 : 1.2) * (t.nk * (t.whole / 256 + 1.0 / least) + 2.5);
+  const long each = cdiv(t.whole + t.wgs, 256);
+  const double few = dp ? (each == 1 ? 1.08 : 1.0) : (each == 1 ? 1.3 : each == 2 ? 1.12 : each == 3 ? 1.05 : 1.0);
+  const double parts = t.wgs > tiles ? (2.0 * t.wgs + tiles) * 16384.0 * sizeof(T) / 6.0e6 + 5.0 : 0.0;
+  return 11.0 + (dp ? 1.87 : 0.92) * std::max(slabs, latency) * few + parts;
 }
 
 static const long kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128};
@@ -1721,13 +1751,13 @@ static GemmPlan gemm_plan(bool ta, bool tb, long M, long N, long K, long lda, lo
       if (us < best.us) best = GemmPlan{form, s, TailMap{}, us};
     }
   }
-  if (sizeof(T) == 8 && allow_split && batch == 1 && form_ok<T>(TILE128, ta, tb, M, N, K, lda, ldb)) {
+  if (allow_split && batch == 1 && form_ok<T>(TILE128, ta, tb, M, N, K, lda, ldb)) {
     const long full = (M / 128) * (N / 128) / 256 * 256;
     for (const long whole : {full, full - 256})
       for (int chunks = 1; whole >= 0 && chunks <= 32; ++chunks) {
         const TailMap t = tail_map(M, N, K, whole, chunks);
         if (!t.wgs || t.wgs == t.n[0] + t.n[1] + t.n[2] + t.n[3]) continue;  // (nothing shared: the plain launch)
-        const double us = tail_us(t);
+        const double us = tail_us<T>(t);
         if (us < best.us) best = GemmPlan{TILE128, 1, t, us};
       }
   }
@@ -1755,11 +1785,12 @@ static void tile_launch(jues_ctx* ctx, int form, bool tb, int kind, GemmSide<T> 
   p0.nz = p1.nz = nb;
   if (!two) p1 = p0;
   const bool tail = p0.tail.wgs > 0;
-  const dim3 grid((unsigned)(tail ? p0.tail.whole + cdiv(p0.tail.wgs, NXCD) * NXCD : total), 1, grid_z(nb));
+  const dim3 grid((unsigned)(tail ? p0.tail.whole + p0.tail.wgs : total), 1, grid_z(nb));
   if constexpr (sizeof(T) == 4) {
-#define JUES_GEMM32(K_, TB_, TA_, SEG_, BT_)                                                                        \
-  hipLaunchKernelGGL((gemm32_nn_kernel<K_, TB_, TA_, SEG_, false, BT_>), grid, dim3(NT), 0, ctx->stream, p0, p1,    \
-                     (int)nt0, (float)alpha, (float)beta)
+#define JUES_GEMM32(K_, TB_, TA_, SEG_, BT_, ...)                                                                   \
+  hipLaunchKernelGGL((gemm32_nn_kernel<K_, TB_, TA_, SEG_, false, BT_, ##__VA_ARGS__>), grid, dim3(NT), 0,          \
+                     ctx->stream, p0, p1, (int)nt0, (float)alpha, (float)beta)
+#define JUES_GEMM32_TAIL(K_, TB_, TA_) JUES_GEMM32(K_, TB_, TA_, false, 128, true)
 #define JUES_GEMM32_SHAPES(BT_)                      \
   if (seg) {                                         \
     if (tb) JUES_GEMM32(0, true, false, true, BT_);  \
@@ -1768,7 +1799,14 @@ static void tile_launch(jues_ctx* ctx, int form, bool tb, int kind, GemmSide<T> 
     if (tb) JUES_GEMM32(0, true, true, false, BT_);  \
     else JUES_GEMM32(0, false, true, false, BT_);    \
   } else if (tb) JUES_GEMM32(0, true, false, false, BT_)
-    if (form == TILE64) {
+    if (tail) {
+      if (ta && tb) JUES_GEMM32_TAIL(0, true, true);
+      else if (ta) JUES_GEMM32_TAIL(0, false, true);
+      else if (tb) JUES_GEMM32_TAIL(0, true, false);
+      else if (kind == 1) JUES_GEMM32_TAIL(1, false, false);
+      else if (kind == 2) JUES_GEMM32_TAIL(2, false, false);
+      else JUES_GEMM32_TAIL(0, false, false);
+    } else if (form == TILE64) {
       JUES_GEMM32_SHAPES(64);
       else JUES_GEMM32(0, false, false, false, 64);
     } else {
@@ -1778,6 +1816,7 @@ static void tile_launch(jues_ctx* ctx, int form, bool tb, int kind, GemmSide<T> 
       else JUES_GEMM32(0, false, false, false, 128);
     }
 #undef JUES_GEMM32_SHAPES
+#undef JUES_GEMM32_TAIL
 #undef JUES_GEMM32
   } else {
 #define JUES_GEMM64(K_, TB_, TA_, SEG_, BT_, ...)                                                                \
@@ -1799,11 +1838,6 @@ static void tile_launch(jues_ctx* ctx, int form, bool tb, int kind, GemmSide<T> 
       else if (kind == 1) JUES_GEMM64_TAIL(1, false, false);
       else if (kind == 2) JUES_GEMM64_TAIL(2, false, false);
       else JUES_GEMM64_TAIL(0, false, false);
-      JUES_HIP(hipGetLastError());
-      int tiles = 0;
-      for (const int n : p0.tail.n) tiles += n;
-      if (p0.tail.wgs > tiles)
-        hipLaunchKernelGGL(gemm_tail_kernel, dim3((unsigned)tiles, 16), dim3(256), 0, ctx->stream, p0, (double)beta);
     } else if (form == TILE64) {
       JUES_GEMM64_SHAPES(64);
       else JUES_GEMM64(0, false, false, false, 64);
@@ -1816,6 +1850,13 @@ static void tile_launch(jues_ctx* ctx, int form, bool tb, int kind, GemmSide<T> 
 #undef JUES_GEMM64_SHAPES
 #undef JUES_GEMM64_TAIL
 #undef JUES_GEMM64
+  }
+  if (tail) {
+    JUES_HIP(hipGetLastError());
+    int tiles = 0;
+    for (const int n : p0.tail.n) tiles += n;
+    if (p0.tail.wgs > tiles)
+      hipLaunchKernelGGL((gemm_tail_kernel<T>), dim3((unsigned)tiles, 16), dim3(256), 0, ctx->stream, p0, beta);
   }
   JUES_HIP(hipGetLastError());
 }
@@ -1974,14 +2015,14 @@ bool gemm_lower(jues_ctx* ctx, long M, long K, const double* L, long ldl, double
   TailMap best = tail_map(M, M, K, full, 1, true);  // nothing shared, if there is no workspace
   if (!best.wgs && full >= 256) best = tail_map(M, M, K, full - 256, 1, true);
   if (!best.wgs) return false;
-  double us = tail_us(best);
+  double us = tail_us<double>(best);
   double* part = nullptr;
   if (!no_alloc_active()) {
     TailMap shared;
     for (const long whole : {full, full - 256})
       for (int chunks = 2; whole >= 0 && chunks <= 32; ++chunks) {
         const TailMap t = tail_map(M, M, K, whole, chunks, true);
-        if (t.wgs && tail_us(t) < us) shared = t, us = tail_us(t);
+        if (t.wgs && tail_us<double>(t) < us) shared = t, us = tail_us<double>(t);
       }
     if (shared.wgs && (part = split_work<double>(ctx, 9, (size_t)shared.wgs * 128 * 128))) best = shared;
   }
