@@ -52,8 +52,9 @@ struct CCWork {
   // RCCSD
   DevBuf t1, Fme, X2, Z, Q, n1, U2, Tau, FmiT;
   // RCCSD o v^3 terms through the factors: B1[m,P,e] / Y2[m,e,P] = sum_f t1[m,f] Lvv[e,f,P],
-  // Y3[m,j,P] = sum_f Lov[m,f,P] t1[j,f], W1[i,e,P], g[P]; Zs / Zsp: slabs of (mf|ae)
-  DevBuf B1, Y2, Y3, W1, gP, Zs, Zsp;
+  // Y3[m,j,P] = sum_f Lov[m,f,P] t1[j,f], W1[i,e,P], g[P]; Zs / Zsp: slabs of (mf|ae),
+  // Zpm: Z on packed pairs
+  DevBuf B1, Y2, Y3, W1, gP, Zs, Zsp, Zpm;
   // where the last residual evaluation left H, Y (ov layout) and, when the update kernel does
   // not symmetrise them itself, S = G + G^T of G = H + y_direct Y + Y^x (the buffers may be shared)
   double y_direct = 0.0;
@@ -84,9 +85,7 @@ struct SplitState {
   };
   Entry e[SPLIT_SLOTS];
   Split16Buf vps, vms, tpc, tmc;  // per-slab planes of the recomputed ladder (never cached)
-  Split16Buf tppt, zsp;           // RCCSD's tau^T (once per iteration) and one (ef) x (a m) slab
-  const void* tppt_src = nullptr;
-  long tppt_stamp = -2;
+  Split16Buf zsp;                 // RCCSD's packed (ef) x (a m) slab (never cached)
   Split16Buf y2t, y3t;            // RCCSD's Y2^T (once per iteration, two products) and Y3^T
   const void* y2t_src = nullptr;
   long y2t_stamp = -2;
@@ -185,11 +184,12 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
 template <typename T>
 void rccd_delta_contractions(jues_ctx* ctx, CCState& S, const double* t2);
 // One slab of occupied m (m0 .. m0 + cnt - 1) of RCCSD's Z[(ij),(a,m)] = sum_ef tau[ij,ef] (mf|ae) with
-// (ia|bc) factored: Zs[(f,m'),(a,e)] = sum_P LovT[(f,m),P] Lvv[(ae),P], permuted to Zsp[(e,f),(a,m')],
-// times Tpp = tau [(ij),(ef)] into Z's columns (a,m) of the slab.  Split-FP16 in the split stage.
+// (ia|bc) factored, on the ladder's packed tau: Zs[(f,m'),(a,e)] = sum_P LovT[(f,m),P] Lvv[(ae),P], packed to
+// G+-[(e,f),(a,m')] = ((mf|ae) +- (me|af))/2, and Zp = T+ G+, Zm = T- G- in the slab's columns (a,m):
+// Z[ij] = Zp + Zm, Z[ji] = Zp - Zm (half the work of the product over all (ij) and (ef)).  G: v^2 columns' room.
 template <typename T>
-void ovvv_z_slab(jues_ctx* ctx, CCState& S, int m0, int cnt, const T* LovT, const T* Lvv, const T* Tpp, T* Zs,
-                 T* Zsp, T* Z);
+void ovvv_z_slab(jues_ctx* ctx, CCState& S, int m0, int cnt, const T* LovT, const T* Lvv, const T* Tp, const T* Tm,
+                 T* Zs, T* G, T* Zp, T* Zm);
 // RCCSD's (ia|bc) factor products (split-FP16 in the split stage): W1 = Uov Lov (ov x naux);
 // C += Lov Y2^T (y2_right) or C += Y2 Lov^T (Y2: ov x naux); Q = Y3 Lvv^T (Y3: o^2 x naux)
 template <typename T>

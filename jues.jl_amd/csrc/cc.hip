@@ -330,44 +330,44 @@ template const double* ring_lx<double>(jues_ctx*, CCState&);
 template const float* ring_lx<float>(jues_ctx*, CCState&);
 
 template <typename T>
-void ovvv_z_slab(jues_ctx* ctx, CCState& S, int m0, int cnt, const T* LovT, const T* Lvv, const T* Tpp, T* Zs,
-                 T* Zsp, T* Z) {
-  const int o = S.o, v = S.v;
-  const long ov = (long)o * v, vv = (long)v * v, oo = (long)o * o, naux = ctx->naux, nr = (long)v * cnt;
-  bool split = false;
-  if constexpr (sizeof(T) == 4) split = S.split_on;
+void ovvv_z_slab(jues_ctx* ctx, CCState& S, int m0, int cnt, const T* LovT, const T* Lvv, const T* Tp, const T* Tm,
+                 T* Zs, T* G, T* Zp, T* Zm) {
+  const PairTables& P = S.P;
+  const int v = S.v;
+  const long ov = (long)S.o * v, vv = (long)v * v, naux = ctx->naux, nr = (long)v * cnt, c0 = (long)v * m0;
+  const bool minus = P.nmo > 0 && P.nmv > 0;
+  T *Gp = G, *Gm = G + P.npv * nr;
   if constexpr (sizeof(T) == 4) {
-    if (split) {
-      // Zs = (LovT slab) Lvv^T from the factors' planes (k = P), split once per stage
+    if (S.split_on) {
+      // Zs = (LovT slab) Lvv^T from the factors' planes (k = P), split once per stage; the packed tau's transposed
+      // planes are the ladder's, the slab's planes are split every time
       const Split16& lat = split_operand<double>(ctx, S, SP_LOVAT, S.i64->LovT.as<double>(), naux, ov, true);
       const Split16& lvt = split_operand<double>(ctx, S, SP_LVVT, S.i64->Lvv.as<double>(), naux, vv, true);
-      gemm16_tn(ctx, nr, vv, 1.0f, split16_cols(lat, (long)v * m0, nr), lvt, 0.0f, Zs, nr, "cc_ovvv_gen");
-    }
-  }
-  if (!split)
-    gemm<T>(ctx, false, true, nr, vv, naux, T(1), LovT + (long)v * m0, ov, 0, Lvv, vv, 0, T(0), Zs, nr, 0, 1,
-            "cc_ovvv_gen");
-  permute<T, T>(ctx, Zs, {v, cnt, v, v}, {3, 0, 2, 1}, Zsp, 1.0, 0.0, "cc_ovvv_gen");
-  T* Zc = Z + oo * v * m0;
-  if constexpr (sizeof(T) == 4) {
-    if (split) {
-      // tau's transposed planes (k = (ef)) once per iteration, the slab's planes every slab
-      SplitState& Zt = split_state(S);
-      if (Zt.tppt_src != static_cast<const void*>(Tpp) || Zt.tppt_stamp != (long)S.iter) {
-        split16t<float>(ctx, Tpp, vv, oo, oo, Zt.tppt, "cc_split");
-        Zt.tppt_src = Tpp;
-        Zt.tppt_stamp = S.iter;
+      gemm16_tn(ctx, nr, vv, 1.0f, split16_cols(lat, c0, nr), lvt, 0.0f, Zs, nr, "cc_ovvv_gen");
+      pack_z<T>(ctx, P, Zs, v, cnt, Gp, Gm);
+      SplitState& Z = split_state(S);
+      const Split16& tp = split_operand<float>(ctx, S, SP_TPT, Tp, P.npv, P.npo, true);
+      split16<float>(ctx, Gp, P.npv, nr, P.npv, Z.zsp, "cc_split");
+      gemm16_tn(ctx, P.npo, nr, 1.0f, tp, Z.zsp.s, 0.0f, Zp + P.npo * c0, P.npo, "cc_ovvv");
+      if (minus) {
+        const Split16& tm = split_operand<float>(ctx, S, SP_TMT, Tm, P.nmv, P.nmo, true);
+        split16<float>(ctx, Gm, P.nmv, nr, P.nmv, Z.zsp, "cc_split");
+        gemm16_tn(ctx, P.nmo, nr, 1.0f, tm, Z.zsp.s, 0.0f, Zm + P.nmo * c0, P.nmo, "cc_ovvv");
       }
-      split16<float>(ctx, Zsp, vv, nr, vv, Zt.zsp, "cc_split");
-      gemm16_tn(ctx, oo, nr, 1.0f, Zt.tppt.s, Zt.zsp.s, 0.0f, Zc, oo, "cc_ovvv");
       return;
     }
   }
-  gemm<T>(ctx, false, false, oo, nr, vv, T(1), Tpp, oo, 0, Zsp, vv, 0, T(0), Zc, oo, 0, 1, "cc_ovvv");
+  gemm<T>(ctx, false, true, nr, vv, naux, T(1), LovT + c0, ov, 0, Lvv, vv, 0, T(0), Zs, nr, 0, 1, "cc_ovvv_gen");
+  pack_z<T>(ctx, P, Zs, v, cnt, Gp, Gm);
+  gemm<T>(ctx, false, false, P.npo, nr, P.npv, T(1), Tp, P.npo, 0, Gp, P.npv, 0, T(0), Zp + P.npo * c0, P.npo, 0, 1,
+          "cc_ovvv");
+  if (minus)
+    gemm<T>(ctx, false, false, P.nmo, nr, P.nmv, T(1), Tm, P.nmo, 0, Gm, P.nmv, 0, T(0), Zm + P.nmo * c0, P.nmo, 0, 1,
+            "cc_ovvv");
 }
 
-template void ovvv_z_slab<double>(jues_ctx*, CCState&, int, int, const double*, const double*, const double*,
-                                  double*, double*, double*);
+template void ovvv_z_slab<double>(jues_ctx*, CCState&, int, int, const double*, const double*, const double*, const double*, double*,
+                                 double*, double*, double*);
 
 template <typename T>
 void fac_uov_lov(jues_ctx* ctx, CCState& S, const T* Uov, T* W1) {
@@ -429,8 +429,8 @@ template void fac_lov_y2<double>(jues_ctx*, CCState&, const double*, bool, doubl
 template void fac_lov_y2<float>(jues_ctx*, CCState&, const float*, bool, float*);
 template void fac_y3_lvv<double>(jues_ctx*, CCState&, const double*, double*);
 template void fac_y3_lvv<float>(jues_ctx*, CCState&, const float*, float*);
-template void ovvv_z_slab<float>(jues_ctx*, CCState&, int, int, const float*, const float*, const float*, float*,
-                                 float*, float*);
+template void ovvv_z_slab<float>(jues_ctx*, CCState&, int, int, const float*, const float*, const float*, const float*, float*,
+                                 float*, float*, float*);
 
 // The ladder with <ab|ef> rebuilt from the factors every iteration (DF-RCCD.jl:198-215
 // contracts bvv[a,e,Q] bvv[b,f,Q] the same way): for a slab of f, X[a,e,b,f] =

@@ -95,6 +95,61 @@ __global__ __launch_bounds__(256) void pack_v_kernel(const T* __restrict__ X, lo
   }
 }
 
+// G+-[(e,f),(a,m)] = ((mf|ae) +- (me|af))/2 from X[f,m,a,e] = (mf|ae): as pack_v_kernel, but X is contiguous in f and
+// the column (a,m) is no pair.  A workgroup takes 16 e, 16 f >= e and 8 columns: X[f,e] goes through LDS, X[e,f] is
+// read as it is written.  Bound by memory.
+template <typename T>
+__global__ __launch_bounds__(256) void pack_z_kernel(const T* __restrict__ X, int v, int cnt, long npv,
+                                                     T* __restrict__ Gp, long nmv, T* __restrict__ Gm) {
+  constexpr int TS = 16, LD = TS + 1, NC = 8;
+  __shared__ T P[NC][TS * LD];
+  int tf = (int)((sqrtf(8.0f * blockIdx.x + 1.0f) - 1.0f) / 2.0f);
+  while (tf * (tf + 1) / 2 > (int)blockIdx.x) --tf;
+  while ((tf + 1) * (tf + 2) / 2 <= (int)blockIdx.x) ++tf;
+  const int f0 = tf * TS, e0 = ((int)blockIdx.x - tf * (tf + 1) / 2) * TS;
+  const int lo = threadIdx.x & 15, hi = threadIdx.x >> 4;
+  const long nr = (long)v * cnt, c0 = (long)blockIdx.y * NC;
+  const auto at = [&](int f, int e, long c) {
+    const int a = (int)(c % v), m = (int)(c / v);
+    return X[min(f, v - 1) + (long)v * m + nr * (a + (long)v * min(e, v - 1))];
+  };
+  T x[NC], y[NC];
+#pragma unroll
+  for (int k = 0; k < NC; ++k) x[k] = at(f0 + lo, e0 + hi, min(c0 + k, nr - 1));
+#pragma unroll
+  for (int k = 0; k < NC; ++k) y[k] = e0 == f0 ? x[k] : at(e0 + lo, f0 + hi, min(c0 + k, nr - 1));
+#pragma unroll
+  for (int k = 0; k < NC; ++k) P[k][hi * LD + lo] = x[k];
+  __syncthreads();
+  const int e = e0 + lo, f = f0 + hi;
+  if (f >= v || e > f) return;
+  const long rp = (long)f * (f + 1) / 2 + e, rm = (long)f * (f - 1) / 2 + e;
+#pragma unroll
+  for (int k = 0; k < NC; ++k) {
+    const long c = c0 + k;
+    if (c >= nr) return;
+    const double s = (double)P[k][lo * LD + hi], t = (double)y[k];
+    Gp[rp + npv * c] = (T)(0.5 * (s + t));
+    if (e < f) Gm[rm + nmv * c] = (T)(0.5 * (s - t));
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void unpack_z_kernel(const T* __restrict__ Zp, const T* __restrict__ Zm, int o,
+                                                       long npo, long nmo, long total, T* __restrict__ Z) {
+  const int oo = o * o;
+  for (long x = blockIdx.x * 256L + threadIdx.x; x < total; x += (long)gridDim.x * 256L) {
+    const long c = x / oo;
+    const int ij = (int)(x - c * oo), i = ij % o, j = ij / o, p = min(i, j), q = max(i, j);
+    T z = Zp[tri_le(p, q) + npo * c];
+    if (i != j) {
+      const T w = Zm[tri_lt(p, q) + nmo * c];
+      z += i < j ? w : -w;
+    }
+    Z[x] = z;
+  }
+}
+
 // W[m,n,i,j] (o^4, holding <mn|ij> plus any T1 terms) on packed pairs, transposed:
 // WPT[(i<=j),(k<=l)] = W[klij] + W[lkij] (k<l), W[kkij] (k=l);  WMT[(i<j),(k<l)] = W[klij] - W[lkij]
 template <typename T>
@@ -552,6 +607,30 @@ void rccd_layouts(jues_ctx* ctx, const double* t, int o, int v, T* Tpp, T* Upp, 
   }
   JUES_HIP(hipGetLastError());
 }
+
+template <typename T>
+void pack_z(jues_ctx* ctx, const PairTables& P, const T* X, int v, int cnt, T* Gp, T* Gm) {
+  const int nt = (v + 15) / 16;
+  const long nr = (long)v * cnt;
+  JUES_REQUIRE(nr <= 8L * 65535, "pack_z: too many columns");
+  KTimer k(ctx, "cc_ovvv_gen", 0.0, (double)v * v * nr * 2 * sizeof(T));
+  hipLaunchKernelGGL((pack_z_kernel<T>), dim3((unsigned)(nt * (nt + 1) / 2), (unsigned)((nr + 7) / 8)), dim3(256), 0,
+                     ctx->stream, X, v, cnt, P.npv, Gp, P.nmv, Gm);
+  JUES_HIP(hipGetLastError());
+}
+
+template <typename T>
+void unpack_z(jues_ctx* ctx, const PairTables& P, const T* Zp, const T* Zm, int o, int v, T* Z) {
+  const long n = (long)o * o * o * v;
+  KTimer k(ctx, "cc_ovvv_gen", 0.0, (double)n * 2 * sizeof(T));
+  hipLaunchKernelGGL((unpack_z_kernel<T>), dim3(grid256(n)), dim3(256), 0, ctx->stream, Zp, Zm, o, P.npo, P.nmo, n, Z);
+  JUES_HIP(hipGetLastError());
+}
+
+template void pack_z<double>(jues_ctx*, const PairTables&, const double*, int, int, double*, double*);
+template void pack_z<float>(jues_ctx*, const PairTables&, const float*, int, int, float*, float*);
+template void unpack_z<double>(jues_ctx*, const PairTables&, const double*, const double*, int, int, double*);
+template void unpack_z<float>(jues_ctx*, const PairTables&, const float*, const float*, int, int, float*);
 
 template <typename T>
 void pack_v(jues_ctx* ctx, const PairTables& P, const T* X, long ldx, int v, int f0, int f1, T* Vp, long rowp0,

@@ -40,7 +40,7 @@ struct CcsdLayouts {
     const long oo = (long)o * o, ov = (long)o * v, x = i + (long)o * j + oo * (a + (long)v * b);
     const double tt = t1[i + (long)o * a] * t1[j + (long)o * b], ttx = t1[i + (long)o * b] * t1[j + (long)o * a];
     const long y = i + (long)o * a + ov * (j + (long)o * b), yx = i + (long)o * b + ov * (j + (long)o * a);
-    Tpp[x] = (T)(t2 + tt);
+    if (Tpp) Tpp[x] = (T)(t2 + tt);  // (the factored route takes the packed tau)
     Upp[x] = (T)(2.0 * (t2 + 0.5 * tt) - (t2x + 0.5 * ttx));
     const T u = (T)(2.0 * t2 - t2x);
     Tov[y] = (T)t2;
@@ -184,9 +184,9 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
   {
     const size_t slab = (size_t)o * (o + 1) * sizeof(double);
     const bool staged = slab <= 65536;
-    KTimer k(ctx, "cc_prep", 0.0, (double)N2 * ((staged ? 8.0 : 16.0) + 7.0 * sizeof(T)));
+    KTimer k(ctx, "cc_prep", 0.0, (double)N2 * ((staged ? 8.0 : 16.0) + (fac ? 6.0 : 7.0) * sizeof(T)));
     hipLaunchKernelGGL((ccsd_layouts_kernel<T>), dim3((unsigned)std::min(vv, 1L << 20)), dim3(256),
-                       staged ? slab : 0, ctx->stream, t2, t1_64, CcsdLayouts<T>{o, v, Tpp, Upp, Tov, Ttov, Uov, U2, Q},
+                       staged ? slab : 0, ctx->stream, t2, t1_64, CcsdLayouts<T>{o, v, fac ? nullptr : Tpp, Upp, Tov, Ttov, Uov, U2, Q},
                        staged ? 1 : 0);
     JUES_HIP(hipGetLastError());
   }
@@ -287,17 +287,18 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
   // Wabef's T1 part: X2 = Lz[ijab] = -sum_m t1[mb] Z[ij,ma],  Z = tau . (mf|ae); the update kernel adds
   // Lz[ijab] + Lz[jiba]
   if (fac) {
-    // Z[i,j,a,m] over slabs of m: Zs[(f,m'),(a,e)] = sum_P LovT[(f,m),P] Lvv[(ae),P] = (mf|ae),
-    // Zsp[(e,f),(a,m')] its permutation, Z[(ij),(a,m)] = Tpp[(ij),(ef)] Zsp; then
-    // Lz[(ija),b] = -sum_m Z[(ija),m] t1[m,b]
+    // Z[i,j,a,m] on the packed pairs of tau over slabs of m, then Lz[(ija),b] = -sum_m Z[(ija),m] t1[m,b]
     const long per_m = (long)v * vv;
     const long ms = std::max(1L, std::min<long>(o, (2L << 30) / (per_m * (long)sizeof(T))));
     T* Zs = bufp_t<T>(W.Zs, (size_t)(ms * per_m));
     T* Zsp = bufp_t<T>(W.Zsp, (size_t)(ms * per_m));
+    T* Zp = bufp_t<T>(W.Zpm, (size_t)(oo * ov));
+    T* Zm = Zp + S.P.npo * ov;
     for (int m0 = 0; m0 < o; m0 += (int)ms) {
       const int cnt = (int)std::min<long>(ms, o - m0);
-      ovvv_z_slab<T>(ctx, S, m0, cnt, LovT, Lvv, Tpp, Zs, Zsp, Z);
+      ovvv_z_slab<T>(ctx, S, m0, cnt, LovT, Lvv, Tp, Tm, Zs, Zsp, Zp, Zm);
     }
+    unpack_z<T>(ctx, S.P, Zp, Zm, o, v, Z);
     gemm<T>(ctx, false, false, oo * v, v, o, T(-1), Z, oo * v, 0, t1, o, 0, zero, X2, oo * v, 0, 1, "cc_t1");
   } else {
     contract<T>(ctx, 1.0, TN(Tpp, "ijef"), TN(ovvv, "mfae"), 0.0, TN(Z, "ijma"), "cc_ovvv");

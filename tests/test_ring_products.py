@@ -1,4 +1,5 @@
-"""The four-product form of the ring terms against the six products they are written with, in NumPy."""
+"""The four-product form of the ring terms against the six products they are written with, and RCCSD's o v^3 product
+on packed pairs against the whole one, in NumPy."""
 import numpy as np
 import pytest
 
@@ -32,3 +33,25 @@ def test_four_ring_products_equal_six(o, v, singles):
     got = U @ W + 0.5 * Y + _x(Y, o, v)
     # rounding only: a few products of n terms
     assert np.max(np.abs(got - ref)) < 64 * n * 2.3e-16 * np.max(np.abs(ref) + 10)
+
+
+@pytest.mark.parametrize("o,v", [(1, 1), (1, 3), (2, 1), (3, 4), (4, 6)])
+def test_z_on_packed_pairs(o, v):
+    """Z[ij,am] = sum_ef tau[ij,ef] M[ef,am] with tau[ij,ef] = tau[ji,fe] and any M equals Zp + Zm for i <= j and
+    Zp - Zm for i > j, Zp = T+ G+ and Zm = T- G- over pairs e <= f and e < f."""
+    rng = np.random.default_rng(10 * o + v)
+    t = rng.normal(size=(o, o, v, v))
+    t = t + t.transpose(1, 0, 3, 2)
+    M = rng.normal(size=(v, v, v * o))
+    ref = np.einsum("ijef,efc->ijc", t, M)
+    le = [(e, f) for f in range(v) for e in range(f + 1)]
+    lt = [(e, f) for f in range(v) for e in range(f)]
+    Gp = np.array([0.5 * (M[e, f] + M[f, e]) for e, f in le])
+    Gm = np.array([0.5 * (M[e, f] - M[f, e]) for e, f in lt]).reshape(len(lt), v * o)
+    for i in range(o):
+        for j in range(i, o):
+            Tp = np.array([t[i, j, e, f] + (t[i, j, f, e] if e != f else 0.0) for e, f in le])
+            Tm = np.array([t[i, j, e, f] - t[i, j, f, e] for e, f in lt])
+            zp, zm = Tp @ Gp, Tm @ Gm
+            assert np.allclose(zp + zm, ref[i, j], rtol=1e-13, atol=1e-13)
+            assert np.allclose(zp - zm, ref[j, i], rtol=1e-13, atol=1e-13)
