@@ -86,9 +86,7 @@ struct SplitState {
   Entry e[SPLIT_SLOTS];
   Split16Buf vps, vms, tpc, tmc;  // per-slab planes of the recomputed ladder (never cached)
   Split16Buf zsp;                 // RCCSD's packed (ef) x (a m) slab (never cached)
-  Split16Buf y2t, y3t;            // RCCSD's Y2^T (once per iteration, two products) and Y3^T
-  const void* y2t_src = nullptr;
-  long y2t_stamp = -2;
+  Split16Buf y2t, y3t;            // RCCSD's Y2^T and Y3^T (never cached)
 };
 
 // Defect-correction refinement of RCCD.  An FP64 iteration at the anchor t0 keeps its numerator
@@ -191,11 +189,11 @@ template <typename T>
 void ovvv_z_slab(jues_ctx* ctx, CCState& S, int m0, int cnt, const T* LovT, const T* Lvv, const T* Tp, const T* Tm,
                  T* Zs, T* G, T* Zp, T* Zm);
 // RCCSD's (ia|bc) factor products (split-FP16 in the split stage): W1 = Uov Lov (ov x naux);
-// C += Lov Y2^T (y2_right) or C += Y2 Lov^T (Y2: ov x naux); Q = Y3 Lvv^T (Y3: o^2 x naux)
+// C = Lov Y2^T (Y2: ov x naux); Q = Y3 Lvv^T (Y3: o^2 x naux)
 template <typename T>
 void fac_uov_lov(jues_ctx* ctx, CCState& S, const T* Uov, T* W1);
 template <typename T>
-void fac_lov_y2(jues_ctx* ctx, CCState& S, const T* Y2, bool y2_right, T* C);
+void fac_lov_y2(jues_ctx* ctx, CCState& S, const T* Y2, T* C);
 template <typename T>
 void fac_y3_lvv(jues_ctx* ctx, CCState& S, const T* Y3, T* Q);
 // The split-FP16 stage runs its products on split planes from this ov on, below it in FP32 MFMA, which is the

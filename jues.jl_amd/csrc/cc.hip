@@ -386,25 +386,19 @@ void fac_uov_lov(jues_ctx* ctx, CCState& S, const T* Uov, T* W1) {
 }
 
 template <typename T>
-void fac_lov_y2(jues_ctx* ctx, CCState& S, const T* Y2, bool y2_right, T* C) {
+void fac_lov_y2(jues_ctx* ctx, CCState& S, const T* Y2, T* C) {
   const long ov = (long)S.o * S.v, naux = ctx->naux;
   if constexpr (sizeof(T) == 4) {
     if (S.split_on) {
       SplitState& Z = split_state(S);
-      if (Z.y2t_src != static_cast<const void*>(Y2) || Z.y2t_stamp != (long)S.iter) {
-        split16t<float>(ctx, Y2, naux, ov, ov, Z.y2t, "cc_split");
-        Z.y2t_src = Y2;
-        Z.y2t_stamp = S.iter;
-      }
+      split16t<float>(ctx, Y2, naux, ov, ov, Z.y2t, "cc_split");
       const Split16& lt = split_operand<double>(ctx, S, SP_LOVT, S.i64->Lov.as<double>(), naux, ov, true);
-      if (y2_right) gemm16_tn(ctx, ov, ov, 1.0f, lt, Z.y2t.s, 1.0f, C, ov, "cc_ovvv_fac");
-      else gemm16_tn(ctx, ov, ov, 1.0f, Z.y2t.s, lt, 1.0f, C, ov, "cc_ovvv_fac");
+      gemm16_tn(ctx, ov, ov, 1.0f, lt, Z.y2t.s, 0.0f, C, ov, "cc_ovvv_fac");
       return;
     }
   }
-  const T* L = ints<T>(S).Lov.template as<T>();
-  if (y2_right) gemm<T>(ctx, false, true, ov, ov, naux, T(1), L, ov, 0, Y2, ov, 0, T(1), C, ov, 0, 1, "cc_ovvv_fac");
-  else gemm<T>(ctx, false, true, ov, ov, naux, T(1), Y2, ov, 0, L, ov, 0, T(1), C, ov, 0, 1, "cc_ovvv_fac");
+  gemm<T>(ctx, false, true, ov, ov, naux, T(1), ints<T>(S).Lov.template as<T>(), ov, 0, Y2, ov, 0, T(0), C, ov, 0, 1,
+          "cc_ovvv_fac");
 }
 
 template <typename T>
@@ -425,8 +419,8 @@ void fac_y3_lvv(jues_ctx* ctx, CCState& S, const T* Y3, T* Q) {
 
 template void fac_uov_lov<double>(jues_ctx*, CCState&, const double*, double*);
 template void fac_uov_lov<float>(jues_ctx*, CCState&, const float*, float*);
-template void fac_lov_y2<double>(jues_ctx*, CCState&, const double*, bool, double*);
-template void fac_lov_y2<float>(jues_ctx*, CCState&, const float*, bool, float*);
+template void fac_lov_y2<double>(jues_ctx*, CCState&, const double*, double*);
+template void fac_lov_y2<float>(jues_ctx*, CCState&, const float*, float*);
 template void fac_y3_lvv<double>(jues_ctx*, CCState&, const double*, double*);
 template void fac_y3_lvv<float>(jues_ctx*, CCState&, const float*, float*);
 template void ovvv_z_slab<float>(jues_ctx*, CCState&, int, int, const float*, const float*, const float*, const float*, float*,

@@ -93,9 +93,10 @@ void rccd_layouts(jues_ctx* ctx, const double* t, int o, int v, T* Tpp, T* Upp, 
 // WE[(k,c),(j,b)] += s (delta_kj Fae[b,c] - delta_cb Fmi[k,j]) (ov layout; FmiT[j,k] = Fmi[k,j])
 template <typename T>
 void fock_dress(jues_ctx* ctx, T* WE, const T* Fae, const T* FmiT, int o, int v, T s);
-// WE = s X + D/2 and W = K + WE/2 with D[(k,c),(j,b)] = delta_kj Fae[b,c] - delta_cb Fmi[k,j]; X may be WE
+// WE = s X + D/2 and W = K + WE/2 (+ A) with D[(k,c),(j,b)] = delta_kj Fae[b,c] - delta_cb Fmi[k,j]; X may be WE
 template <typename T>
-void ring_start(jues_ctx* ctx, const T* K, T s, const T* X, const T* Fae, const T* FmiT, int o, int v, T* WE, T* W);
+void ring_start(jues_ctx* ctx, const T* K, T s, const T* X, const T* Fae, const T* FmiT, int o, int v, T* WE, T* W,
+                const T* A = nullptr);
 // Tq = Tp with its (a,a) columns doubled
 template <typename T>
 void pair_diag2(jues_ctx* ctx, const PairTables& P, const T* Tp, T* Tq);

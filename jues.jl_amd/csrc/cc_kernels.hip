@@ -209,12 +209,12 @@ __global__ __launch_bounds__(256) void fock_dress_kernel(T* __restrict__ WE, con
   }
 }
 
-// Start of the ring intermediates: WE = s X + D/2 and W = K + WE/2, D as in fock_dress_kernel (X may be WE).
+// Start of the ring intermediates: WE = s X + D/2 and W = K + WE/2 (+ A), D as in fock_dress_kernel (X may be WE).
 // One pass at the copy rate in place of a copy, a scaled copy and the two dressings.
 template <typename T>
 __global__ __launch_bounds__(256) void ring_start_kernel(const T* __restrict__ K, T s, const T* X,
                                                          const T* __restrict__ Fae, const T* __restrict__ FmiT, int o,
-                                                         int v, T* WE, T* __restrict__ W) {
+                                                         int v, T* WE, T* __restrict__ W, const T* __restrict__ A) {
   const int ov = o * v;
   for (int jb = blockIdx.x; jb < ov; jb += gridDim.x) {
     const int j = jb % o, b = jb / o;
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(256) void ring_start_kernel(const T* __restrict__ K
       if (k == j) w += T(0.5) * Fae[b + (long)v * c];
       if (c == b) w -= T(0.5) * FmiT[j + (long)o * k];
       WE[x] = w;
-      W[x] = K[x] + T(0.5) * w;
+      W[x] = A ? K[x] + T(0.5) * w + A[x] : K[x] + T(0.5) * w;
     }
   }
 }
@@ -582,11 +582,12 @@ void fock_dress(jues_ctx* ctx, T* WE, const T* Fae, const T* FmiT, int o, int v,
 }
 
 template <typename T>
-void ring_start(jues_ctx* ctx, const T* K, T s, const T* X, const T* Fae, const T* FmiT, int o, int v, T* WE, T* W) {
+void ring_start(jues_ctx* ctx, const T* K, T s, const T* X, const T* Fae, const T* FmiT, int o, int v, T* WE, T* W,
+                const T* A) {
   const long n = (long)o * v * o * v;
-  KTimer k(ctx, "cc_prep", 0.0, (double)n * 4.0 * sizeof(T));
+  KTimer k(ctx, "cc_prep", 0.0, (double)n * (A ? 5.0 : 4.0) * sizeof(T));
   hipLaunchKernelGGL((ring_start_kernel<T>), dim3((unsigned)std::min((long)o * v, 1L << 20)), dim3(256), 0, ctx->stream, K, s, X, Fae, FmiT, o, v,
-                     WE, W);
+                     WE, W, A);
   JUES_HIP(hipGetLastError());
 }
 
@@ -695,9 +696,9 @@ void divide_d2(jues_ctx* ctx, double* t, const double* eps, int o, int v, double
 template void fock_dress<double>(jues_ctx*, double*, const double*, const double*, int, int, double);
 template void fock_dress<float>(jues_ctx*, float*, const float*, const float*, int, int, float);
 template void ring_start<double>(jues_ctx*, const double*, double, const double*, const double*, const double*, int,
-                                 int, double*, double*);
+                                 int, double*, double*, const double*);
 template void ring_start<float>(jues_ctx*, const float*, float, const float*, const float*, const float*, int, int,
-                                float*, float*);
+                                float*, float*, const float*);
 template void rccd_layouts<double>(jues_ctx*, const double*, int, int, double*, double*, double*, double*);
 template void rccd_layouts<float>(jues_ctx*, const double*, int, int, float*, float*, float*, float*);
 template void pack_whh<double>(jues_ctx*, const PairTables&, const double*, int, double*, double*);

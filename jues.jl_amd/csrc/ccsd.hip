@@ -232,10 +232,9 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
   // Fmi[m,i] += sum_ne t1[ne] (2(mi|ne) - (ni|me))
   contract<T>(ctx, 2.0, TN(t1, "ne"), TN(ooov, "mine"), 1.0, TN(Fmi, "mi"), "cc_t1");
   contract<T>(ctx, -1.0, TN(t1, "ne"), TN(ooov, "nime"), 1.0, TN(Fmi, "mi"), "cc_t1");
-  // Fme[m,e] = sum_nf t1[nf] (2(me|nf) - (ne|mf)), (ne|mf) = (mf|ne) = Kx[m,e,n,f]
+  // Fme[m,e] = sum_nf t1[nf] (2(me|nf) - (ne|mf)), (ne|mf) = (mf|ne) = Kx[m,e,n,f]: 2 Lx t1
   const T* Kx = I.Ktov.template as<T>();
-  contract<T>(ctx, 2.0, TN(t1, "nf"), TN(Kov, "menf"), 0.0, TN(Fme, "me"), "cc_t1");
-  contract<T>(ctx, -1.0, TN(t1, "nf"), TN(Kx, "menf"), 1.0, TN(Fme, "me"), "cc_t1");
+  contract<T>(ctx, 2.0, TN(t1, "nf"), TN(ring_lx<T>(ctx, S), "menf"), 0.0, TN(Fme, "me"), "cc_t1");
 
   // ---- off-diagonal Fock terms of a non-canonical reference (AutoRCCSD.jl:76-81,127-132):
   // Fae += f_ae - t1[ma] f_me / 2, Fmi += f_mi + t1[ie] f_me / 2, Fme += f_me
@@ -309,39 +308,39 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
   // (as in RCCD, with U2 = 2 T - Q: W = WJ + WE/2 = K - J/2 + (K - Kx/2) U2/2 and the T1 terms of WJ and half of
   // WE's, H = U W + Y/2; every left operand of the ring products is a symmetric (ov) x (ov) matrix)
   permute<T, T>(ctx, Jov, {ov, ov}, {0, 1}, WE, -1.0, 0.0, "cc_prep");
-  // WE[me,jb] -= sum_f t1[jf] (mf|be): with factors, H[(mj),(be)] = sum_P Y3[(mj),P] Lvv[(be),P]
-  // (H is free until the ring products) permuted into WE
+  // WE[me,jb] += sum_n t1[nb] (mj|ne) - sum_f t1[jf] (mf|be).  With factors both are products over [(mj),(be)], the
+  // second sum_P Y3[(mj),P] Lvv[(be),P], formed in H (free until the ring products) and permuted into WE at once
   if (fac) {
     fac_y3_lvv<T>(ctx, S, Y3, H);
+    gemm<T>(ctx, false, false, oo, v, o, T(-1), ooov, oo, oo * o, t1, o, 0, one, H, oo, oo * v, v, "cc_t1");
     permute<T, T>(ctx, H, d4, {0, 3, 1, 2}, WE, -1.0, 1.0, "cc_ovvv_fac");
   } else {
     contract<T>(ctx, -1.0, TN(t1, "jf"), TN(ovvv, "mfbe"), 1.0, TN(WE, "mejb"), "cc_t1");
+    contract<T>(ctx, 1.0, TN(t1, "nb"), TN(ooov, "mjne"), 1.0, TN(WE, "mejb"), "cc_t1", H, N2);
   }
-  contract<T>(ctx, 1.0, TN(t1, "nb"), TN(ooov, "mjne"), 1.0, TN(WE, "mejb"), "cc_t1", H, N2);
   // Fock-like terms with Fb / Fj, carried by WE as in RCCD: WE += D/2 with
   // D[kc,jb] = delta_kj Fb[b,c] - delta_cb Fj[k,j]
   T* FmiT = bufp_t<T>(W.FmiT, oo);
   permute<T, T>(ctx, Fmi, {o, o}, {1, 0}, FmiT, 1.0, 0.0, "cc_fock");
-  ring_start<T>(ctx, Kov, one, WE, Fae, FmiT, o, v, WE, WJ);
-  // WJ's T1 terms: sum_f t1[jf] (me|bf) - sum_n t1[nb] (nj|me)
-  if (fac) fac_lov_y2<T>(ctx, S, Y2, true, WJ);
-  else contract<T>(ctx, 1.0, TN(t1, "jf"), TN(ovvv, "mebf"), 1.0, TN(WJ, "mejb"), "cc_t1");
-  contract<T>(ctx, -1.0, TN(t1, "nb"), TN(ooov, "njme"), 1.0, TN(WJ, "mejb"), "cc_t1", H, N2);
+  // A = sum_f t1[jf] (me|bf) at [me,jb] is one of WJ's T1 terms, and H's term t1[ie] (jb|ae) is its transpose, which
+  // S = G + G^T cannot tell from A: formed once, in H
+  if (fac) fac_lov_y2<T>(ctx, S, Y2, H);
+  else contract<T>(ctx, 1.0, TN(t1, "jf"), TN(ovvv, "mebf"), 0.0, TN(H, "mejb"), "cc_t1");
+  ring_start<T>(ctx, Kov, one, WE, Fae, FmiT, o, v, WE, WJ, H);
+  // WJ's other T1 term, through Y (free until Tx WE)
+  contract<T>(ctx, -1.0, TN(t1, "nb"), TN(ooov, "njme"), 1.0, TN(WJ, "mejb"), "cc_t1", Y, N2);
   ring_mm<T>(ctx, S, half, ring_lx<T>(ctx, S), SP_LX, U2, SP_U2, one, WJ);
   ring_mm<T>(ctx, S, half, Kx, SP_KX, Q, SP_Q, one, WE);
-  ring_mm<T>(ctx, S, one, Uov, SP_UOV, WJ, SP_WJ, zero, H);
+  ring_mm<T>(ctx, S, one, Uov, SP_UOV, WJ, SP_WJ, one, H);
   // exchange ring term t[m,i,b,e] WmBEj[m,a,e,j] = (Tx WE)[ib,ja], and half the direct one
   ring_mm<T>(ctx, S, one, Ttov, SP_TTOV, WE, SP_WE, zero, Y);
-  // T1^2 terms: -t1[ie] t1[ma] (me|jb) and -t1[ie] t1[mb] (mj|ae); (me|jb) = K[j,b,m,e] is read
-  // in place, and the products permuted into H go through U2, free once WJ is built
-  contract<T>(ctx, 1.0, TN(t1, "ie"), TN(Kov, "jbme"), 0.0, TN(Q, "imjb"), "cc_t1");
-  contract<T>(ctx, -1.0, TN(t1, "ma"), TN(Q, "imjb"), 1.0, TN(H, "iajb"), "cc_t1", U2, N2);
-  contract<T>(ctx, 1.0, TN(t1, "ie"), TN(Jov, "maje"), 0.0, TN(Q, "imaj"), "cc_t1");
-  contract<T>(ctx, -1.0, TN(t1, "mb"), TN(Q, "imaj"), 1.0, TN(H, "iajb"), "cc_t1", U2, N2);
-  // T1-linear terms: t1[ie] (jb|ae) - t1[ma] (mi|jb); with factors the first is Y2[(ia),P] Lov[(jb),P]
-  if (fac) fac_lov_y2<T>(ctx, S, Y2, false, H);
-  else contract<T>(ctx, 1.0, TN(t1, "ie"), TN(ovvv, "jbae"), 1.0, TN(H, "iajb"), "cc_t1");
-  contract<T>(ctx, -1.0, TN(t1, "ma"), TN(ooov, "mijb"), 1.0, TN(H, "iajb"), "cc_t1", U2, N2);
+  // T1^2 terms -t1[ie] t1[ma] (me|jb) and -t1[ie] t1[mb] (mj|ae), T1-linear term -t1[ma] (mi|jb): with the second
+  // transposed (S = G + G^T) all are -t1[ma] Q[mi,jb], Q = (mi|jb) + t1[ie] (me|jb) + t1[je] (mi|be); the
+  // product permuted into H goes through U2, free once WJ is built
+  JUES_HIP(hipMemcpyAsync(Q, ooov, (size_t)(oo * ov) * sizeof(T), hipMemcpyDeviceToDevice, ctx->stream));
+  contract<T>(ctx, 1.0, TN(t1, "ie"), TN(Kov, "jbme"), 1.0, TN(Q, "mijb"), "cc_t1");
+  contract<T>(ctx, 1.0, TN(t1, "je"), TN(Jov, "mbie"), 1.0, TN(Q, "mijb"), "cc_t1");
+  contract<T>(ctx, -1.0, TN(t1, "ma"), TN(Q, "mijb"), 1.0, TN(H, "iajb"), "cc_t1", U2, N2);
   // S = G + G^T, G = H + Y/2 + Y^x: summed by the update kernel, or here (into WJ) when its LDS slab
   // would not fit
   if (!fused_sym(o, sizeof(T))) {

@@ -55,3 +55,21 @@ def test_z_on_packed_pairs(o, v):
             zp, zm = Tp @ Gp, Tm @ Gm
             assert np.allclose(zp + zm, ref[i, j], rtol=1e-13, atol=1e-13)
             assert np.allclose(zp - zm, ref[j, i], rtol=1e-13, atol=1e-13)
+
+
+@pytest.mark.parametrize("o,v", [(1, 1), (2, 3), (3, 5)])
+def test_merged_singles_terms(o, v):
+    """S = H + H^T does not tell H's terms from their transposes: the term t1[ie] (jb|ae) taken as A[ia,jb] =
+    sum_f t1[jf] (ia|bf), and the T1^2 and T1-linear terms as one product -t1[ma] Q[mi,jb], give the same S."""
+    rng = np.random.default_rng(5 * o + v)
+    es = np.einsum
+    t1 = rng.normal(size=(o, v))
+    ovvv, ooov = rng.normal(size=(o, v, v, v)), rng.normal(size=(o, o, o, v))
+    ovvv = ovvv + ovvv.transpose(0, 1, 3, 2)                         # (ia|bc) = (ia|cb)
+    K, J = rng.normal(size=(o, v, o, v)), rng.normal(size=(o, v, o, v))
+    K = K + K.transpose(2, 3, 0, 1)
+    H = -es("ma,imjb->iajb", t1, es("ie,mejb->imjb", t1, K)) - es("mb,imaj->iajb", t1, es("ie,maje->imaj", t1, J))
+    H = H + es("ie,jbae->iajb", t1, ovvv) - es("ma,mijb->iajb", t1, ooov)
+    Q = ooov + es("ie,jbme->mijb", t1, K) + es("je,mbie->mijb", t1, J)
+    G = es("jf,iabf->iajb", t1, ovvv) - es("ma,mijb->iajb", t1, Q)
+    assert np.allclose(G + G.transpose(2, 3, 0, 1), H + H.transpose(2, 3, 0, 1), rtol=1e-12, atol=1e-12)
