@@ -50,7 +50,7 @@ struct CCWork {
   DevBuf Wpt, Wmt, Tq;  // hole-hole ladder on packed pairs
   DevBuf Xs, Vps, Vms;  // recomputed ladder: (ae|bf) slab and its packed V+/V- rows
   // RCCSD
-  DevBuf t1, Fme, X2, Z, Q, n1, U2, Tau, FmiT;
+  DevBuf t1, Fme, X2, Z, Q, n1, U2, FmiT, KT, JT;
   // RCCSD o v^3 terms through the factors: B1[m,P,e] / Y2[m,e,P] = sum_f t1[m,f] Lvv[e,f,P],
   // Y3[m,j,P] = sum_f Lov[m,f,P] t1[j,f], W1[i,e,P], g[P]; Zs / Zsp: slabs of (mf|ae),
   // Zpm: Z on packed pairs

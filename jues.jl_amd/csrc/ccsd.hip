@@ -40,10 +40,10 @@ struct CcsdLayouts {
     const long oo = (long)o * o, ov = (long)o * v, x = i + (long)o * j + oo * (a + (long)v * b);
     const double tt = t1[i + (long)o * a] * t1[j + (long)o * b], ttx = t1[i + (long)o * b] * t1[j + (long)o * a];
     const long y = i + (long)o * a + ov * (j + (long)o * b), yx = i + (long)o * b + ov * (j + (long)o * a);
-    if (Tpp) Tpp[x] = (T)(t2 + tt);  // (the factored route takes the packed tau)
+    if (Tpp) Tpp[x] = (T)(t2 + tt);  // (the factored route takes the packed tau, and U for T)
     Upp[x] = (T)(2.0 * (t2 + 0.5 * tt) - (t2x + 0.5 * ttx));
     const T u = (T)(2.0 * t2 - t2x);
-    Tov[y] = (T)t2;
+    if (Tov) Tov[y] = (T)t2;
     Uov[y] = u;
     U2[y] = (T)((double)u - 2.0 * (double)(T)ttx);
     Ttov[yx] = (T)t2;                                  // Ttov[i,b,j,a] = t2[i,j,a,b]
@@ -75,6 +75,20 @@ __global__ __launch_bounds__(256) void ccsd_layouts_kernel(const double* __restr
       L.put(t1, i, j, a, b, staged ? slab[i + ld * j] : src[q], staged ? slab[j + ld * i] : src[j + (long)o * i]);
     }
   }
+}
+
+// n1[i,a] += 2 sum_m KT[i,a,m,m] - sum_m JT[m,a,i,m] (KT o x v x o x o, JT o x v x o x o): takes the place of two products
+// of t1 with all of (ia|me) and (mi|ae), and of a permuted copy of the latter, 60 us at ov = 2000
+template <typename T>
+__global__ __launch_bounds__(256) void singles_trace_kernel(const T* __restrict__ KT, const T* __restrict__ JT, int o,
+                                                            int v, T* __restrict__ n1) {
+  const int x = blockIdx.x * 256 + threadIdx.x;
+  if (x >= o * v) return;
+  const long ov = (long)o * v, i = x % o, a = x / o;
+  double s = 0.0;
+  for (int m = 0; m < o; ++m)
+    s += 2.0 * (double)KT[x + ov * m + ov * o * m] - (double)JT[m + o * a + ov * i + ov * o * m];
+  n1[x] = (T)((double)n1[x] + s);
 }
 
 // per (a,b): sum_ij Lener[i,j,a,b] t1[i,a] t1[j,b]
@@ -151,7 +165,7 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
   const bool fac = S.ovvv_factored;
   T* Tpp = bufp_t<T>(W.Tpp, N2);   // tau
   T* Upp = bufp_t<T>(W.Upp, N2);   // 2 tau' - tau'^(ij)
-  T* Tov = bufp_t<T>(W.Tov, N2);   // t2 [i,a,j,b]
+  T* Tov = fac ? nullptr : bufp_t<T>(W.Tov, N2);   // t2 [i,a,j,b]
   T* Ttov = bufp_t<T>(W.Ttov, N2); // t2[i,j,b,a] at [i,a,j,b]
   T* Uov = bufp_t<T>(W.Uov, N2);   // 2 t2 - t2^x (ov)
   T* Ua = bufp_t<T>(W.Ua, N2);
@@ -171,6 +185,8 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
   T* U2 = bufp_t<T>(W.U2, N2);
   T* Q = bufp_t<T>(W.Q, std::max(N2, oo * ov));
   T* Z = bufp_t<T>(W.Z, oo * ov);
+  T* KT = bufp_t<T>(W.KT, oo * ov);
+  T* JT = bufp_t<T>(W.JT, oo * ov);
   T* Tp = bufp_t<T>(W.Tp, S.P.npo * S.P.npv);
   T* Tm = bufp_t<T>(W.Tm, std::max(1L, S.P.nmo * S.P.nmv));
   T* Lp = bufp_t<T>(W.Lp, S.P.npo * S.P.npv);
@@ -184,9 +200,10 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
   {
     const size_t slab = (size_t)o * (o + 1) * sizeof(double);
     const bool staged = slab <= 65536;
-    KTimer k(ctx, "cc_prep", 0.0, (double)N2 * ((staged ? 8.0 : 16.0) + (fac ? 6.0 : 7.0) * sizeof(T)));
+    KTimer k(ctx, "cc_prep", 0.0, (double)N2 * ((staged ? 8.0 : 16.0) + (fac ? 5.0 : 7.0) * sizeof(T)));
     hipLaunchKernelGGL((ccsd_layouts_kernel<T>), dim3((unsigned)std::min(vv, 1L << 20)), dim3(256),
-                       staged ? slab : 0, ctx->stream, t2, t1_64, CcsdLayouts<T>{o, v, fac ? nullptr : Tpp, Upp, Tov, Ttov, Uov, U2, Q},
+                       staged ? slab : 0, ctx->stream, t2, t1_64,
+                       CcsdLayouts<T>{o, v, fac ? nullptr : Tpp, Upp, Tov, Ttov, Uov, U2, Q},
                        staged ? 1 : 0);
     JUES_HIP(hipGetLastError());
   }
@@ -250,15 +267,21 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
   }
 
   // ---- T1 residual (mRCCSD.jl:202-212) ----------------------------------------------
-  // (Ua is free from the Fae product until WE is built: the permuted copy of (mi|ae) goes
-  // there; t2[m,n,a,e] = t2[n,m,e,a] is read as Tov[n,e,m,a], no copy)
   contract<T>(ctx, 1.0, TN(t1, "ie"), TN(Fae, "ae"), 0.0, TN(n1, "ia"), "cc_t1");
   contract<T>(ctx, -1.0, TN(t1, "ma"), TN(Fmi, "mi"), 1.0, TN(n1, "ia"), "cc_t1");
   contract<T>(ctx, 1.0, TN(Fme, "me"), TN(Uov, "iame"), 1.0, TN(n1, "ia"), "cc_t1");
-  contract<T>(ctx, 2.0, TN(t1, "me"), TN(Kov, "iame"), 1.0, TN(n1, "ia"), "cc_t1");
-  contract<T>(ctx, -1.0, TN(t1, "me"), TN(Jov, "maie"), 1.0, TN(n1, "ia"), "cc_t1", Ua, N2);
-  contract<T>(ctx, -2.0, TN(Tov, "nema"), TN(ooov, "mine"), 1.0, TN(n1, "ia"), "cc_t1");
-  contract<T>(ctx, 1.0, TN(Tov, "nema"), TN(ooov, "nime"), 1.0, TN(n1, "ia"), "cc_t1");
+  // t1[ie] (jb|me) at [j,b,m,i] and t1[je] (mi|be) at [m,b,i,j], which the ring's T1^2 terms take too; their traces over
+  // the two m are the terms 2 t1[me] (ia|me) - t1[me] (mi|ae)
+  contract<T>(ctx, 1.0, TN(t1, "ie"), TN(Kov, "jbme"), 0.0, TN(KT, "jbmi"), "cc_t1");
+  contract<T>(ctx, 1.0, TN(t1, "je"), TN(Jov, "mbie"), 0.0, TN(JT, "mbij"), "cc_t1");
+  {
+    KTimer k(ctx, "cc_t1", 0.0, 2.0 * oo * v * sizeof(T));
+    hipLaunchKernelGGL((singles_trace_kernel<T>), dim3((unsigned)((ov + 255) / 256)), dim3(256), 0, ctx->stream, KT, JT,
+                       o, v, n1);
+    JUES_HIP(hipGetLastError());
+  }
+  // -sum_nme (2 T[ne,ma] - T[me,na]) (mi|ne) = -sum U[ne,ma] (mi|ne)
+  contract<T>(ctx, -1.0, TN(Uov, "nema"), TN(ooov, "mine"), 1.0, TN(n1, "ia"), "cc_t1");
   if (fac) {
     // sum_emf (2 T[ie,mf] - T[me,if]) (mf|ae) = sum_(eP) W1[i,(eP)] Lvv[a,(eP)] with
     // W1[(ie),P] = sum_(mf) U[(ie),(mf)] Lov[(mf),P], U = 2 T - T^x: both terms in one (ov)^2 naux product
@@ -338,8 +361,8 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
   // transposed (S = G + G^T) all are -t1[ma] Q[mi,jb], Q = (mi|jb) + t1[ie] (me|jb) + t1[je] (mi|be); the
   // product permuted into H goes through U2, free once WJ is built
   JUES_HIP(hipMemcpyAsync(Q, ooov, (size_t)(oo * ov) * sizeof(T), hipMemcpyDeviceToDevice, ctx->stream));
-  contract<T>(ctx, 1.0, TN(t1, "ie"), TN(Kov, "jbme"), 1.0, TN(Q, "mijb"), "cc_t1");
-  contract<T>(ctx, 1.0, TN(t1, "je"), TN(Jov, "mbie"), 1.0, TN(Q, "mijb"), "cc_t1");
+  permute<T, T>(ctx, KT, {o, v, o, o}, {2, 3, 0, 1}, Q, 1.0, 1.0, "cc_t1");
+  permute<T, T>(ctx, JT, {o, v, o, o}, {0, 2, 3, 1}, Q, 1.0, 1.0, "cc_t1");
   contract<T>(ctx, -1.0, TN(t1, "ma"), TN(Q, "mijb"), 1.0, TN(H, "iajb"), "cc_t1", U2, N2);
   // S = G + G^T, G = H + Y/2 + Y^x: summed by the update kernel, or here (into WJ) when its LDS slab
   // would not fit

@@ -73,3 +73,23 @@ def test_merged_singles_terms(o, v):
     Q = ooov + es("ie,jbme->mijb", t1, K) + es("je,mbie->mijb", t1, J)
     G = es("jf,iabf->iajb", t1, ovvv) - es("ma,mijb->iajb", t1, Q)
     assert np.allclose(G + G.transpose(2, 3, 0, 1), H + H.transpose(2, 3, 0, 1), rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("o,v", [(1, 1), (2, 3), (3, 5)])
+def test_singles_residual_terms(o, v):
+    """The T1 residual's terms 2 t1[me] (ia|me) - t1[me] (mi|ae) as traces of the ring's T1 products, and its two
+    products of T2 with (mi|ne) as one with U = 2T - Tx."""
+    rng = np.random.default_rng(7 * o + v)
+    es = np.einsum
+    t1 = rng.normal(size=(o, v))
+    K, J, ooov = rng.normal(size=(o, v, o, v)), rng.normal(size=(o, v, o, v)), rng.normal(size=(o, o, o, v))
+    K = K + K.transpose(2, 3, 0, 1)
+    KT, JT = es("ie,jbme->jbmi", t1, K), es("je,mbie->mbij", t1, J)
+    ref = 2 * es("me,iame->ia", t1, K) - es("me,maie->ia", t1, J)
+    assert np.allclose(2 * es("iamm->ia", KT) - es("maim->ia", JT), ref, rtol=1e-12, atol=1e-12)
+    t2 = rng.normal(size=(o, o, v, v))
+    t2 = t2 + t2.transpose(1, 0, 3, 2)
+    T = t2.transpose(0, 2, 1, 3)
+    U = 2 * T - es("ijba->iajb", t2)
+    ref = -2 * es("nema,mine->ia", T, ooov) + es("nema,nime->ia", T, ooov)
+    assert np.allclose(-es("nema,mine->ia", U, ooov), ref, rtol=1e-12, atol=1e-12)
