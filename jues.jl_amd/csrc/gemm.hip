@@ -9,6 +9,7 @@
 //
 // Workgroup ids are remapped so that each of the 8 XCDs (each with its own L2) receives a contiguous
 // range of tiles, and tiles are walked in groups of 8 tile-rows to reuse B columns within an L2.
+#include "gemm_tail.h"
 #include "jues_internal.h"
 
 #include <algorithm>
@@ -70,17 +71,6 @@ __device__ inline bool entry_place(int& x, int& z) {
   return true;
 }
 
-// Tile p2 of tiles_m x tiles_n in grouped order: GROUP_M tile-rows share each sweep over tile-columns
-__device__ inline void grouped_tile(int p2, int tiles_m, int tiles_n, int& tm, int& tn) {
-  const int group_size = GROUP_M * tiles_n;
-  const int gid = p2 / group_size;
-  const int first_m = gid * GROUP_M;
-  const int gsz = min(tiles_m - first_m, GROUP_M);
-  const int r = p2 - gid * group_size;
-  tm = first_m + r % gsz;
-  tn = r / gsz;
-}
-
 // Tile of workgroup pid of nwg, of which only the first tiles_m * tiles_n carry a tile (a launch
 // padded to a multiple of NXCD); false for the padding ids.  plain: the workgroups are on one XCD already.
 __device__ inline bool tile_coords_bounded(int pid, int nwg, int tiles_m, int tiles_n, int& tm, int& tn,
@@ -96,71 +86,6 @@ __device__ inline bool tile_coords_bounded(int pid, int nwg, int tiles_m, int ti
   grouped_tile(p2, tiles_m, tiles_n, tm, tn);
   return true;
 }
-
-// Tile p2 of the lower triangle of m x m tiles (tm >= tn), in bands of GROUP_M tile-rows that sweep the tile-columns
-// up to the diagonal
-__device__ inline void lower_tile(int p2, int m, int& tm, int& tn) {
-  constexpr int G = GROUP_M;  // band g starts after G^2 g (g - 1) / 2 + G (G + 1) / 2 g tiles
-  const auto before = [](int g) { return G * G * (g * (g - 1) / 2) + G * (G + 1) / 2 * g; };
-  int g = (int)(sqrtf(2.0f * (float)p2) / (float)G);
-  while (before(g) > p2) --g;
-  while (before(g + 1) <= p2) ++g;
-  int r = p2 - before(g);
-  const int h = min(G, m - G * g);
-  if (r < h * G * g) {
-    tm = G * g + r % h;
-    tn = r / h;
-    return;
-  }
-  r -= h * G * g;
-  int c = 0;
-  while (r >= h - c) r -= h - c++;
-  tm = G * g + c + r;
-  tn = G * g + c;
-}
-
-// A TAIL launch of a product: `whole` workgroups have a tile each, and the other tiles' 16-deep k-slabs are shared by
-// several workgroups a tile, whose parts of it gemm_tail_kernel adds.  Tiles are taken full ones first (grouped),
-// then those past the edge of N, of M and of both: four runs of n[] tiles left to the tail, in s[] chunks each.
-// Within a run, the parts are ordered chunk by chunk: neighbours read the same k-slabs.
-// 256 compute units leave much of a last round of tiles idle otherwise, and split whole products write more parts
-// (and round no better): FP64 3082^3 took 980 us in two chunks, 890 this way, 6460^3 8.6 and 7.6 ms (73 TFLOP/s would be
-// 7.4), 276 x 9045 x 9045 902 and 792 us, 8640 x 768 x 8640 1790 and 1660; FP32 3082^3 507 and 478.
-struct TailMap {
-  int whole = 0, wgs = 0, nk = 0, full_m = 0, full_n = 0;
-  int n[4] = {}, s[4] = {};
-  bool lower = false;  // a square result of which only the tiles tm >= tn are formed
-
-  __device__ void coords(int p2, int& tm, int& tn) const {
-    const int full = lower ? full_m * (full_m + 1) / 2 : full_m * full_n;
-    if (p2 < full && lower) lower_tile(p2, full_m, tm, tn);
-    else if (p2 < full) grouped_tile(p2, full_m, full_n, tm, tn);
-    else if ((p2 -= full) < n[1]) tm = p2, tn = full_n;
-    else if ((p2 -= n[1]) < n[2]) tm = full_m, tn = p2;
-    else tm = full_m, tn = full_n;
-  }
-  // tile of the tail, chunk of it (of `chunks`) and place of its part, of workgroup x.  The runs past an edge come
-  // first (their few long chunks end last otherwise), and each run is dealt to the XCDs in equal contiguous shares.
-  __device__ void part(int x, int& tile, int& chunk, int& chunks, int& place) const {
-    int at = 0;
-#pragma unroll
-    for (int k = 1; k <= 4; ++k) {
-      const int q = k & 3, count = n[q] * s[q];
-      if (x < count) {
-        const int per = count / NXCD, more = count % NXCD, xcd = x % NXCD;
-        const int y = xcd * per + min(xcd, more) + x / NXCD;
-        chunk = y / n[q];
-        tile = first_tile(q) + y - chunk * n[q];
-        chunks = s[q];
-        place = at + y;
-        return;
-      }
-      x -= count;
-      at += count;
-    }
-  }
-  __device__ int first_tile(int q) const { return (q > 0 ? n[0] : 0) + (q > 1 ? n[1] : 0) + (q > 2 ? n[2] : 0); }
-};
 
 // One product of a high-occupancy kernel launch: C = alpha A op(B) + beta C, batched over
 // blockIdx.z with strides sA, sB, sC.  A launch carries one or two of them (two
@@ -1671,35 +1596,9 @@ static double reduce_us(long S, double elems) {
   return S > 1 ? 2.0 + (S + 1) * elems * sizeof(T) / 4.5e6 + 0.18 * S : 0.0;
 }
 
-// The TAIL launch of an M x N x K product with `whole` full tiles to themselves and the others in `chunks` chunks,
-// those past an edge in fewer by the cost of their slabs; wgs = 0 in the result if it is not of use (fewer full tiles,
-// chunks under 8 slabs, parts over 256 MiB).
-// lower: the lower triangle of tiles of a square result.
-static TailMap tail_map(long M, long N, long K, long whole, int chunks, bool lower = false) {
-  TailMap t;
-  const long fm = M / 128, fn = N / 128, nk = cdiv(K, 16);
-  const int em = (int)cdiv(M % 128, 16), en = (int)cdiv(N % 128, 16);  // 16-row and 16-column blocks past the edge
-  const long full = lower ? fm * (fm + 1) / 2 : fm * fn;
-  const long rest = (lower ? full + (em ? fm + 1 : 0) : cdiv(M, 128) * cdiv(N, 128)) - whole;
-  if (full < whole || rest < 1 || rest > 2048 || (chunks > 1 && nk < 8L * chunks)) return t;
-  t.lower = lower;
-  t.whole = (int)whole;
-  t.nk = (int)nk;
-  t.full_m = (int)fm;
-  t.full_n = (int)fn;
-  // eighths of a full tile's cost: the blocks that a wavefront has of its 4 (2), at least 3 for the staging
-  const int wm = (int)cdiv(em, 2), wn = (int)cdiv(en, 4);
-  const int n[4] = {(int)(full - whole), en && !lower ? (int)fm : 0, em ? (int)fn : 0, em && en ? 1 : 0};
-  const int w[4] = {8, std::max(3, 4 * wn), std::max(3, 2 * wm), std::max(3, wm * wn)};
-  long wgs = 0;
-  for (int q = 0; q < 4; ++q) {
-    t.n[q] = n[q];
-    t.s[q] = std::max(1, (chunks * w[q] + 4) / 8);
-    wgs += (long)t.n[q] * t.s[q];
-  }
-  if (wgs <= 2048) t.wgs = (int)wgs;
-  return t;
-}
+// 128x128 tiles: 2 x 4 wavefronts of 64x32 in FP64, 2 x 2 of 64x64 in FP32
+template <typename T>
+constexpr TailShape kTail{128, 128, 2, sizeof(T) == 8 ? 4 : 2, 16, 0.375, 8};
 
 // Estimated time (us) of a TAIL launch: a compute unit's slabs, and 2.5 for each workgroup's start and end, at the
 // rate that a long launch of 128x128 tiles reaches (1.87 us in FP64, 0.92 in FP32; more where few workgroups
@@ -1755,7 +1654,7 @@ static GemmPlan gemm_plan(bool ta, bool tb, long M, long N, long K, long lda, lo
     const long full = (M / 128) * (N / 128) / 256 * 256;
     for (const long whole : {full, full - 256})
       for (int chunks = 1; whole >= 0 && chunks <= 32; ++chunks) {
-        const TailMap t = tail_map(M, N, K, whole, chunks);
+        const TailMap t = tail_map(kTail<T>, M, N, K, whole, chunks);
         if (!t.wgs || t.wgs == t.n[0] + t.n[1] + t.n[2] + t.n[3]) continue;  // (nothing shared: the plain launch)
         const double us = tail_us<T>(t);
         if (us < best.us) best = GemmPlan{TILE128, 1, t, us};
@@ -2012,8 +1911,8 @@ bool gemm_lower(jues_ctx* ctx, long M, long K, const double* L, long ldl, double
     return false;
   JUES_REQUIRE(ldl >= M && ldc >= M, "gemm_lower: leading dimension too small");
   const long fm = M / 128, full = fm * (fm + 1) / 2 / 256 * 256;
-  TailMap best = tail_map(M, M, K, full, 1, true);  // nothing shared, if there is no workspace
-  if (!best.wgs && full >= 256) best = tail_map(M, M, K, full - 256, 1, true);
+  TailMap best = tail_map(kTail<double>, M, M, K, full, 1, true);  // nothing shared, if there is no workspace
+  if (!best.wgs && full >= 256) best = tail_map(kTail<double>, M, M, K, full - 256, 1, true);
   if (!best.wgs) return false;
   double us = tail_us<double>(best);
   double* part = nullptr;
@@ -2021,7 +1920,7 @@ bool gemm_lower(jues_ctx* ctx, long M, long K, const double* L, long ldl, double
     TailMap shared;
     for (const long whole : {full, full - 256})
       for (int chunks = 2; whole >= 0 && chunks <= 32; ++chunks) {
-        const TailMap t = tail_map(M, M, K, whole, chunks, true);
+        const TailMap t = tail_map(kTail<double>, M, M, K, whole, chunks, true);
         if (t.wgs && tail_us<double>(t) < us) shared = t, us = tail_us<double>(t);
       }
     if (shared.wgs && (part = split_work<double>(ctx, 9, (size_t)shared.wgs * 128 * 128))) best = shared;

@@ -28,6 +28,7 @@
 // 128x128/4-wave, 256x128/4-wave, 128x256, 256x256, 32x32x16 MFMA, LDS-DMA with
 // three LDS stages and split (non-interleaved) planes, this was fastest on the
 // ring (20400^3) and ladder (1830 x 57970 x 57970) products.
+#include "gemm_tail.h"
 #include "jues_internal.h"
 
 #include <algorithm>
@@ -42,7 +43,8 @@ typedef float fvec4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 
 // Workgroup tile BM x BN over WM x WN wavefronts (each (BM/WM) x (BN/WN)), k-slices of 32.
-constexpr int BM = 256, BN = 128, WM = 4, WN = 2, NT = 64 * WM * WN, BK = 32, NXCD = 8, GROUP_M = 8;
+constexpr int BM = 256, BN = 128, WM = 4, WN = 2, NT = 64 * WM * WN, BK = 32, NXCD = TAIL_XCD;
+constexpr TailShape kTail16{BM, BN, WM, WN, BK, 0.5, 16};  // (one workgroup a compute unit: a slice's latency is its time)
 constexpr int PAD_C = 256;  // column padding of every plane (>= BM, BN)
 constexpr int kBufferDword3 = 0x00020000;  // gfx9-family raw buffer descriptor word 3
 
@@ -61,36 +63,51 @@ __device__ inline void tile_coords(int pid, int nwg, int tiles_m, int tiles_n, i
   if (tall == 0) tall = NXCD;
   const int xcd = pid % NXCD, loc = pid / NXCD;
   const int p2 = xcd < tall ? xcd * per + loc : tall * per + (xcd - tall) * (per - 1) + loc;
-  const int group_size = GROUP_M * tiles_n;
-  const int gid = p2 / group_size;
-  const int first_m = gid * GROUP_M;
-  const int gsz = min(tiles_m - first_m, GROUP_M);
-  const int r = p2 - gid * group_size;
-  tm = first_m + r % gsz;
-  tn = r / gsz;
+  grouped_tile(p2, tiles_m, tiles_n, tm, tn);
 }
 
 // KIND separates kernel symbols for profiles (0 generic, 1 CC ring, 2 CC pp-ladder, 3 CC hole-hole).
 // blockIdx.z selects a chunk of kchunk rows of K (a multiple of BK; the last chunk may be
-// shorter) whose product goes to C + z sC: a split-K launch writes partial products.
-template <int KIND>
+// shorter) whose product goes to C + z sC: a split-K launch writes partial products.  TAIL: `tail` deals the tiles
+// and their slices to the workgroups; the parts of a shared tile go to `part` for gemm16_tail_kernel.
+// A wavefront's 16-row (16-column) blocks alternate with its neighbours', so that a tile past the edge of M or N keeps
+// all of them at work on the blocks it has; the others are skipped.
+template <int KIND, bool TAIL>
 __global__ __launch_bounds__(NT, 1) void gemm16_kernel(int M, int N, int Kp, float alpha,
                                                        const _Float16* __restrict__ A, long lda2,
                                                        const int* __restrict__ ea,
                                                        const _Float16* __restrict__ B, long ldb2,
                                                        const int* __restrict__ eb, float beta,
                                                        float* __restrict__ C, long ldc, int tiles_m, int tiles_n,
-                                                       int kchunk, long sC) {
+                                                       int kchunk, long sC, TailMap tail,
+                                                       float* __restrict__ part) {
   constexpr int PA = BM * 128, PB = BN * 128;         // bytes of one slice of each operand
   constexpr int CA = BM * 8 / NT, CB = BN * 8 / NT;   // 16-byte chunks per thread per slice
   constexpr int IM = BM / WM / 16, JN = BN / WN / 16;
   static_assert(CA * NT == BM * 8 && CB * NT == BN * 8, "tile does not divide into chunks");
   __shared__ __attribute__((aligned(16))) char lds[2][PA + PB];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % WM, wn = wave / WM;
-  int tm, tn;
-  tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
+  const auto mrow = [&](int i) { return (WM * i + wm) * 16; };
+  const auto ncol = [&](int j) { return (WN * j + wn) * 16; };
+  int tm, tn, wg = 0;
+  // this workgroup's k-range: kz0 .. kz0 + 32 nk
+  int kz0 = (int)blockIdx.z * kchunk, nk = min(kchunk, Kp - kz0) / BK;
+  bool shared = false;
+  if (TAIL && (int)blockIdx.x >= tail.whole) {
+    int t = 0, c = 0, nc = 1;
+    tail.part((int)blockIdx.x - tail.whole, t, c, nc, wg);
+    shared = nc > 1;
+    const int ka = (int)((long)tail.nk * c / nc);
+    nk = (int)((long)tail.nk * (c + 1) / nc) - ka;
+    kz0 = ka * BK;
+    tail.coords(tail.whole + t, tm, tn);
+  } else if (TAIL) {
+    tail.coords((int)blockIdx.x % NXCD * (tail.whole / NXCD) + (int)blockIdx.x / NXCD, tm, tn);
+  } else {
+    tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
+  }
   const int m0 = tm * BM, n0 = tn * BN;
 
   // chunk q = tid + NT p of a slice is tile column q/8, chunk q%8 of its 128-byte line
@@ -107,8 +124,7 @@ __global__ __launch_bounds__(NT, 1) void gemm16_kernel(int M, int N, int Kp, flo
     voffB[p] = (int)(2 * ((q & 7) * 8 + (long)(q >> 3) * ldb2));
     loffB[p] = PA + lds_off(q >> 3, q & 7);
   }
-  // this chunk's k-range starts 2 kz0 halves into every column (k-blocks of 32 hi + 32 lo)
-  const int kz0 = (int)blockIdx.z * kchunk;
+  // the k-range starts 2 kz0 halves into every column (k-blocks of 32 hi + 32 lo)
   const _Float16* aT = A + (long)m0 * lda2 + 2L * kz0;
   const _Float16* bT = B + (long)n0 * ldb2 + 2L * kz0;
   C += (long)blockIdx.z * sC;
@@ -118,7 +134,6 @@ __global__ __launch_bounds__(NT, 1) void gemm16_kernel(int M, int N, int Kp, flo
   // re-read the last slice (in bounds, never used), which keeps the body free of
   // branches so the scheduler can interleave loads, LDS traffic and MFMAs.  (Macros,
   // not lambdas: lambdas over the register arrays cost spills.)
-  const int nk = min(kchunk, Kp - kz0) / BK;
   u4 sa0[CA], sb0[CB], sa1[CA], sb1[CB];
 #define GLOAD(SA, SB, KT)                                                                                 \
   {                                                                                                       \
@@ -145,9 +160,9 @@ __global__ __launch_bounds__(NT, 1) void gemm16_kernel(int M, int N, int Kp, flo
   const int fr = lane & 15, fc = lane >> 4;
   int aoff[IM], boff[JN];
 #pragma unroll
-  for (int i = 0; i < IM; ++i) aoff[i] = lds_off(wm * (BM / WM) + i * 16 + fr, fc);
+  for (int i = 0; i < IM; ++i) aoff[i] = lds_off(mrow(i) + fr, fc);
 #pragma unroll
-  for (int j = 0; j < JN; ++j) boff[j] = PA + lds_off(wn * (BN / WN) + j * 16 + fr, fc);
+  for (int j = 0; j < JN; ++j) boff[j] = PA + lds_off(ncol(j) + fr, fc);
   // the lo chunk of a fragment is its hi chunk's slot with bit 2 flipped: offset ^ 64
 #define COMPUTE(BUF)                                                                                      \
   {                                                                                                       \
@@ -162,6 +177,27 @@ __global__ __launch_bounds__(NT, 1) void gemm16_kernel(int M, int N, int Kp, flo
     _Pragma("unroll") for (int i = 0; i < IM; ++i) _Pragma("unroll") for (int j = 0; j < JN; ++j) {      \
       acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bl[j], ah[i], acc[i][j], 0, 0, 0);               \
       acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bh[j], al[i], acc[i][j], 0, 0, 0);               \
+    }                                                                                                     \
+  }
+  // a tile past the edge of M or N: only the blocks that hold results
+  const int ilim = min(IM, (M - m0 - 16 * wm + 16 * WM - 1) / (16 * WM));
+  const int jlim = min(JN, (N - n0 - 16 * wn + 16 * WN - 1) / (16 * WN));
+#define COMPUTE_EDGE(BUF)                                                                                 \
+  if (ilim > 0 && jlim > 0) {                                                                             \
+    h8 bh[JN], bl[JN];                                                                                    \
+    _Pragma("unroll") for (int j = 0; j < JN; ++j) {                                                     \
+      bh[j] = *reinterpret_cast<const h8*>(&lds[BUF][boff[j]]);                                           \
+      bl[j] = *reinterpret_cast<const h8*>(&lds[BUF][boff[j] ^ 64]);                                      \
+    }                                                                                                     \
+    _Pragma("unroll") for (int i = 0; i < IM; ++i) {                                                     \
+      if (i >= ilim) break;                                                                               \
+      const h8 ah = *reinterpret_cast<const h8*>(&lds[BUF][aoff[i]]);                                     \
+      const h8 al = *reinterpret_cast<const h8*>(&lds[BUF][aoff[i] ^ 64]);                                \
+      _Pragma("unroll") for (int j = 0; j < JN; ++j) if (j < jlim) {                                     \
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bh[j], ah, acc[i][j], 0, 0, 0);                \
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bl[j], ah, acc[i][j], 0, 0, 0);                \
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bh[j], al, acc[i][j], 0, 0, 0);                \
+      }                                                                                                   \
     }                                                                                                     \
   }
   // Schedule of one half-iteration: all fragment reads first, then the MFMAs with the
@@ -187,22 +223,36 @@ __global__ __launch_bounds__(NT, 1) void gemm16_kernel(int M, int N, int Kp, flo
   GLOAD(sa1, sb1, 1);
   GLOAD(sa0, sb0, 2);
   __syncthreads();
-  for (int kt = 0; kt < nk; kt += 2) {
-    // buffer 0 holds slice kt; slot 1 holds kt+1, slot 0 holds kt+2
-    COMPUTE(0);
-    LSTORE(1, sa1, sb1);
-    GLOAD(sa1, sb1, kt + 3);
-    SCHEDULE();
-    __syncthreads();
-    if (kt + 1 >= nk) break;
-    COMPUTE(1);
-    LSTORE(0, sa0, sb0);
-    GLOAD(sa0, sb0, kt + 4);
-    SCHEDULE();
-    __syncthreads();
+#define LOOP(COMPUTE_, SCHEDULE_)                                                                         \
+  for (int kt = 0; kt < nk; kt += 2) {                                                                    \
+    /* buffer 0 holds slice kt; slot 1 holds kt+1, slot 0 holds kt+2 */                                   \
+    COMPUTE_(0);                                                                                          \
+    LSTORE(1, sa1, sb1);                                                                                  \
+    GLOAD(sa1, sb1, kt + 3);                                                                              \
+    SCHEDULE_();                                                                                          \
+    __syncthreads();                                                                                      \
+    if (kt + 1 >= nk) break;                                                                              \
+    COMPUTE_(1);                                                                                          \
+    LSTORE(0, sa0, sb0);                                                                                  \
+    GLOAD(sa0, sb0, kt + 4);                                                                              \
+    SCHEDULE_();                                                                                          \
+    __syncthreads();                                                                                      \
   }
+#define NO_SCHEDULE()
+  if (ilim == IM && jlim == JN) LOOP(COMPUTE, SCHEDULE)
+  else LOOP(COMPUTE_EDGE, NO_SCHEDULE)
 
   const int descale = -(ea[0] + eb[0]);
+  if (TAIL && shared) {
+    float* __restrict__ P = part + (long)wg * (BM * BN) + tid;
+#pragma unroll
+    for (int i = 0; i < IM; ++i)
+#pragma unroll
+      for (int j = 0; j < JN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) P[((i * JN + j) * 4 + r) * NT] = alpha * ldexpf(acc[i][j][r], descale);
+    return;
+  }
   // acc[i][j][r] is C(m, n) with m = lane%16 of block i, n = 4(lane/16) + r of block j
   if (beta != 0.0f && m0 + BM <= M && n0 + BN <= N) {
     // interior tile accumulating into C: all of the lane's C loads first, then the updates
@@ -214,27 +264,27 @@ __global__ __launch_bounds__(NT, 1) void gemm16_kernel(int M, int N, int Kp, flo
       for (int j = 0; j < JN; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          cv[i][j][r] = C[(long)(m0 + wm * (BM / WM) + i * 16 + fr) +
-                          (long)(n0 + wn * (BN / WN) + j * 16 + 4 * fc + r) * ldc];
+          cv[i][j][r] = C[(long)(m0 + mrow(i) + fr) +
+                          (long)(n0 + ncol(j) + 4 * fc + r) * ldc];
 #pragma unroll
     for (int i = 0; i < IM; ++i)
 #pragma unroll
       for (int j = 0; j < JN; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          C[(long)(m0 + wm * (BM / WM) + i * 16 + fr) + (long)(n0 + wn * (BN / WN) + j * 16 + 4 * fc + r) * ldc] =
+          C[(long)(m0 + mrow(i) + fr) + (long)(n0 + ncol(j) + 4 * fc + r) * ldc] =
               alpha * ldexpf(acc[i][j][r], descale) + beta * cv[i][j][r];
     return;
   }
 #pragma unroll
   for (int i = 0; i < IM; ++i) {
-    const int m = m0 + wm * (BM / WM) + i * 16 + fr;
+    const int m = m0 + mrow(i) + fr;
     if (m >= M) continue;
 #pragma unroll
     for (int j = 0; j < JN; ++j) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int n = n0 + wn * (BN / WN) + j * 16 + 4 * fc + r;
+        const int n = n0 + ncol(j) + 4 * fc + r;
         if (n < N) {
           const long off = (long)m + (long)n * ldc;
           float v = alpha * ldexpf(acc[i][j][r], descale);
@@ -250,6 +300,37 @@ __global__ __launch_bounds__(NT, 1) void gemm16_kernel(int M, int N, int Kp, flo
 #undef LSTORE
 #undef COMPUTE
 #undef SCHEDULE
+#undef COMPUTE_EDGE
+#undef LOOP
+#undef NO_SCHEDULE
+
+// C = (sum of the parts of a TAIL launch's tile, in the order of its slices) + beta C.  blockIdx.x: tile of the tail,
+// blockIdx.y: 1024 of its results, in the order of the workgroups' registers.
+__global__ __launch_bounds__(256) void gemm16_tail_kernel(TailMap tail, const float* __restrict__ part, int M, int N,
+                                                          float* __restrict__ C, long ldc, float beta) {
+  constexpr int JN = BN / WN / 16;
+  int tm, tn, q = 3, first = 0;
+  tail.coords(tail.whole + (int)blockIdx.x, tm, tn);
+  while (q > 0 && (int)blockIdx.x < tail.first_tile(q)) --q;
+  if (tail.s[q] == 1) return;  // written by its workgroup
+  for (int k = 1; k <= 3 && k != q; ++k) first += tail.n[k] * tail.s[k];
+  const int t = (int)blockIdx.x - tail.first_tile(q), q0 = (int)blockIdx.y * 1024 + threadIdx.x;
+  float sum[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c < tail.s[q]; ++c) {
+    const float* P = part + (long)(first + c * tail.n[q] + t) * (BM * BN) + q0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) sum[u] += P[256 * u];
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int x = q0 + 256 * u, th = x % NT, e = x / NT, lane = th & 63, wm = (th >> 6) % WM, wn = (th >> 6) / WM;
+    const int i = e / (4 * JN), j = e / 4 % JN, r = e % 4;
+    const int m = tm * BM + (WM * i + wm) * 16 + (lane & 15), n = tn * BN + (WN * j + wn) * 16 + 4 * (lane >> 4) + r;
+    if (m >= M || n >= N) continue;
+    float* c = C + m + (long)n * ldc;
+    *c = beta != 0.f ? sum[u] + beta * *c : sum[u];
+  }
+}
 
 // C = beta C + sum_s W[s] (fixed order), W[s] is M x N with leading dimension M
 __global__ __launch_bounds__(256) void splitk16_reduce_kernel(const float* __restrict__ W, int S, long M, long N,
@@ -555,6 +636,37 @@ void gemm16_tn(jues_ctx* ctx, long M, long N, float alpha, const Split16& A, con
   } else {
     S = 1;
   }
+  // or the last round of tiles shared: at 6460^3 (26 x 51 tiles, 5.2 rounds of 256) 1.40 ms, 1.56 as six rounds
+  // (estimates in us: 1.3 for a slice of a whole tile, the parts and partial products at 6 and 4.5 TB/s)
+  TailMap tail;
+  double us = 1.3 * ((double)(kchunk / BK) + 2.0) * (double)((tiles * S + 255) / 256) +
+              (S > 1 ? 4.0 * (S + 1) * M * N / 4.5e6 + 5.0 : 0.0);
+  if (!no_alloc_active()) {
+    const long full = (M / BM) * (N / BN) / 256 * 256;
+    for (const long whole : {full, full - 256})
+      for (int chunks = 2; whole >= 0 && chunks <= 32; ++chunks) {
+        const TailMap t = tail_map(kTail16, M, N, Kp, whole, chunks);
+        if (!t.wgs) continue;
+        int least = chunks;
+        for (int q = 0; q < 4; ++q)
+          if (t.n[q]) least = std::min(least, t.s[q]);
+        const double slices = (double)(whole / 256) * (t.nk + 2.0) +
+                              (double)((t.wgs + 255) / 256) * ((double)t.nk / (t.n[0] ? chunks : least) + 2.0);
+        const double now = 1.3 * std::max(slices, 0.5 * (t.nk * ((double)(whole / 256) + 1.0 / least))) +
+                           2.0 * 4.0 * BM * BN * t.wgs / 6.0e6 + 5.0;
+        if (now < us) us = now, tail = t;
+      }
+  }
+  float* part = nullptr;
+  if (tail.wgs) {
+    try {
+      part = static_cast<float*>(scratch(ctx, 17, sizeof(float) * (size_t)tail.wgs * BM * BN));
+    } catch (const Error& e) {
+      if (e.st != JUES_OOM) throw;
+      tail = TailMap{};  // no room: the plain launch needs none
+    }
+  }
+  if (tail.wgs) S = 1, kchunk = Kp;
   float* Cw = C;
   long ldw = ldc, sW = 0;
   float bw = beta;
@@ -566,17 +678,27 @@ void gemm16_tn(jues_ctx* ctx, long M, long N, float alpha, const Split16& A, con
   }
   {
     KTimer timer(ctx, name, flops, bytes);
-    dim3 grid((unsigned)tiles, 1, (unsigned)S);
-#define JUES_G16(K_)                                                                                             \
-  hipLaunchKernelGGL((gemm16_kernel<K_>), grid, dim3(NT), 0, ctx->stream, (int)M, (int)N, (int)Kp, alpha, A.p,    \
-                     2 * A.rows_p, A.sexp, B.p, 2 * B.rows_p, B.sexp, bw, Cw, ldw, (int)tiles_m, (int)tiles_n,     \
-                     (int)kchunk, sW)
+    const dim3 grid((unsigned)(tail.wgs ? tail.whole + tail.wgs : tiles), 1, (unsigned)S);
+#define JUES_G16_(K_, TAIL_)                                                                                      \
+  hipLaunchKernelGGL((gemm16_kernel<K_, TAIL_>), grid, dim3(NT), 0, ctx->stream, (int)M, (int)N, (int)Kp, alpha,  \
+                     A.p, 2 * A.rows_p, A.sexp, B.p, 2 * B.rows_p, B.sexp, bw, Cw, ldw, (int)tiles_m,             \
+                     (int)tiles_n, (int)kchunk, sW, tail, part)
+#define JUES_G16(K_) \
+  do { if (tail.wgs) JUES_G16_(K_, true); else JUES_G16_(K_, false); } while (0)
     if (kind == 1) JUES_G16(1);
     else if (kind == 2) JUES_G16(2);
     else if (kind == 3) JUES_G16(3);
     else JUES_G16(0);
 #undef JUES_G16
+#undef JUES_G16_
     JUES_HIP(hipGetLastError());
+    if (tail.wgs) {
+      int shared = 0;
+      for (const int n : tail.n) shared += n;
+      hipLaunchKernelGGL(gemm16_tail_kernel, dim3((unsigned)shared, BM * BN / 1024), dim3(256), 0, ctx->stream, tail,
+                         part, (int)M, (int)N, C, ldc, beta);
+      JUES_HIP(hipGetLastError());
+    }
   }
   if (S > 1) {
     KTimer t(ctx, name, 0.0, 4.0 * (S + (beta != 0.0f ? 2 : 1)) * M * N);
