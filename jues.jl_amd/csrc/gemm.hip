@@ -39,7 +39,7 @@ template <> struct Mfma<float> {
   }
 };
 
-constexpr int NT = 256, NXCD = 8, GROUP_M = 8;
+constexpr int NT = 256, NXCD = TAIL_XCD;
 
 // Raw buffer loads: the 64-bit base lives in a scalar resource descriptor, the
 // per-lane part is one 32-bit byte offset and the per-element part a scalar
@@ -461,6 +461,8 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
 // step s = 0..3 for both operands (two 16-byte fragment reads per 16-row block).  B's two
 // blocks are held for the slice and A's four streamed one ahead.  Rows past M or N load a
 // clamped row and are not stored; a K tail is the first slice, zero-padded, loaded in the prologue.
+// BT = 64: 64x64 tiles over 4 wavefronts of 32x32, twice the operand traffic for four times the workgroups: 1125^3 takes
+// 85 us (148 with 128x128 tiles), 66 in three chunks of K (71).
 typedef double d2v __attribute__((ext_vector_type(2)));
 
 __device__ inline int g64_chunk(int q, int r) { return q ^ (r & 7); }
@@ -769,6 +771,9 @@ __global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, 
 // k = 4 (l / 16) + s at MFMA step s, so a k-contiguous operand is read 4 consecutive k per lane and an
 // m-contiguous one in runs of 16 rows.  Rows past M or N load a clamped row and are not stored; the K
 // tail is a predicated slab after the full ones.
+// Bound by the latency of a wavefront's loads (two slabs in flight), and from a few thousand tiles on by the L2s, since
+// operands are read once a tile.  FP64, 128-row tiles before: 1 x 2000 x 2000 275 us and 17 here, 5 x 5 x 1805 251 and 6,
+// 20 x 20 x 200000 about 130 and 26.
 template <typename T, bool TA, bool TB, int NW, int IM, int JN>
 __global__ __launch_bounds__(64 * NW) void gemm_direct_kernel(GemmSide<T> g, T alpha, T beta) {
   constexpr int BM = 16 * IM, BN = 16 * JN;
