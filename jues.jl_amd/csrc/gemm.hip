@@ -146,7 +146,7 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
   constexpr int NJ = BT / 64, NB = BT / 32;
   __shared__ __attribute__((aligned(16))) float As[2][BM * BK];
   __shared__ __attribute__((aligned(16))) float Bs[2][BN * BK];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
   // a wavefront's 16-row and 16-column blocks alternate with its neighbour's, so that a tile at the edge of M
   // or N keeps all of them at work on the blocks it has
@@ -351,7 +351,8 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
   // the last slice is peeled off, so that the loop body is one block without conditions (a schedule
   // that keeps the matrix pipe about 5% busier on the ring products than the conditional form)
   // a tile past the edge of M or N: only the blocks that hold results
-  const int ilim = min(NB, (M - m0 - 16 * wm + 31) / 32), jlim = min(NB, (N - n0 - 16 * wn + 31) / 32);
+  const int ilim = __builtin_amdgcn_readfirstlane(min(NB, (M - m0 - 16 * wm + 31) / 32));
+  const int jlim = __builtin_amdgcn_readfirstlane(min(NB, (N - n0 - 16 * wn + 31) / 32));
   auto compute_edge = [&](int cur) {
     if (ilim <= 0 || jlim <= 0) return;
     f4v bf[NB];
@@ -383,8 +384,13 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
     }
     slice((kb - 1 - ka) & 1);
   };
-  if (ilim == NB && jlim == NB) loop(compute);
-  else loop(compute_edge);
+  // (in the two-segment and FP64-output instantiations the second loop costs spills)
+  if constexpr (SEG || OUT64) {
+    loop(compute);
+  } else {
+    if (ilim == NB && jlim == NB) loop(compute);
+    else loop(compute_edge);
+  }
   if (TAIL && shared) {
     // a partial tile, as the registers hold it, for gemm_tail_kernel
     float* __restrict__ P = g.part + (long)wg * (BM * BN) + tid;
@@ -474,12 +480,8 @@ __global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, 
   constexpr int HT = BT / 2, IB = BT / 32;  // half tile; 16-row MFMA blocks of a wavefront (HT rows)
   __shared__ __attribute__((aligned(16))) double As[2][BM * BK];
   __shared__ __attribute__((aligned(16))) double Bs[2][BN * BK];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x, lane = tid & 63, wave = BT == 64 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;  // 2 x (BT / 32) wavefronts of HT x 32
-  // a wavefront's 16-row and 16-column blocks alternate with its neighbours', so that a tile at the edge of M
-  // or N keeps all of them at work on the blocks it has
-  const auto mrow = [&](int i) { return (2 * i + wm) * 16; };
-  const auto ncol = [&](int j) { return (BT / 32 * j + wn) * 16; };
   int bx, bz;
   const bool placed = entry_place(bx, bz), second = !TAIL && bx >= nt0;
   const GemmSide<double> g = second ? p1 : p0;
@@ -642,24 +644,32 @@ __global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, 
   }
   store(0);
   __syncthreads();
+  // the 16-row and 16-column blocks of a wavefront: in turn with its neighbours' (erow, ecol) in 64x64 tiles, one piece in
+  // whole 128x128 tiles, where turns cost a 20400^3 product 6%, and in turn in those with blocks past the edge of M or N,
+  // so that all wavefronts have some of the others
+  constexpr bool TURN = BT == 64;
+  const auto erow = [&](int i) { return (2 * i + wm) * 16; };
+  const auto ecol = [&](int j) { return (BT / 32 * j + wn) * 16; };
+  const auto frow = [&](int i) { return TURN ? erow(i) : wm * HT + i * 16; };
+  const auto fcol = [&](int j) { return TURN ? ecol(j) : wn * 32 + j * 16; };
   auto compute = [&](int cur) {
     d2v bf[2][2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const int r = ncol(j) + fr;
+      const int r = fcol(j) + fr;
       bf[j][0] = *reinterpret_cast<const d2v*>(&Bs[cur][r * BK + 2 * g64_chunk(2 * fk, r)]);
       bf[j][1] = *reinterpret_cast<const d2v*>(&Bs[cur][r * BK + 2 * g64_chunk(2 * fk + 1, r)]);
     }
     d2v a0[2], a1[2];
     {
-      const int r = mrow(0) + fr;
+      const int r = frow(0) + fr;
       a0[0] = *reinterpret_cast<const d2v*>(&As[cur][r * BK + 2 * g64_chunk(2 * fk, r)]);
       a0[1] = *reinterpret_cast<const d2v*>(&As[cur][r * BK + 2 * g64_chunk(2 * fk + 1, r)]);
     }
 #pragma unroll
     for (int i = 0; i < IB; ++i) {
       if (i + 1 < IB) {
-        const int r = mrow(i + 1) + fr;
+        const int r = frow(i + 1) + fr;
         a1[0] = *reinterpret_cast<const d2v*>(&As[cur][r * BK + 2 * g64_chunk(2 * fk, r)]);
         a1[1] = *reinterpret_cast<const d2v*>(&As[cur][r * BK + 2 * g64_chunk(2 * fk + 1, r)]);
       }
@@ -673,21 +683,23 @@ __global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, 
     }
   };
   // the last slice is peeled off, so that the loop body is one block without conditions
-  // a tile past the edge of M or N: only the blocks that hold results
-  const int ilim = min(IB, (M - m0 - 16 * wm + 31) / 32), jlim = min(2, (N - n0 - 16 * wn + HT - 1) / HT);
+  const int ilim = __builtin_amdgcn_readfirstlane(min(IB, (M - m0 - 16 * wm + 31) / 32));
+  const int jlim = __builtin_amdgcn_readfirstlane(min(2, (N - n0 - 16 * wn + HT - 1) / HT));
+  const bool edge = TURN ? ilim < IB || jlim < 2 : M - m0 <= BM - 16 || N - n0 <= BN - 16;
+  // only the blocks that hold results
   auto compute_edge = [&](int cur) {
     if (ilim <= 0 || jlim <= 0) return;
     d2v bf[2][2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const int r = ncol(j) + fr;
+      const int r = ecol(j) + fr;
       bf[j][0] = *reinterpret_cast<const d2v*>(&Bs[cur][r * BK + 2 * g64_chunk(2 * fk, r)]);
       bf[j][1] = *reinterpret_cast<const d2v*>(&Bs[cur][r * BK + 2 * g64_chunk(2 * fk + 1, r)]);
     }
 #pragma unroll
     for (int i = 0; i < IB; ++i) {
       if (i >= ilim) break;
-      const int r = mrow(i) + fr;
+      const int r = erow(i) + fr;
       const d2v a[2] = {*reinterpret_cast<const d2v*>(&As[cur][r * BK + 2 * g64_chunk(2 * fk, r)]),
                         *reinterpret_cast<const d2v*>(&As[cur][r * BK + 2 * g64_chunk(2 * fk + 1, r)])};
 #pragma unroll
@@ -709,8 +721,10 @@ __global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, 
     }
     slice((kb - 1 - ka) & 1);
   };
-  if (ilim == IB && jlim == 2) loop(compute);
-  else loop(compute_edge);
+  if (edge) loop(compute_edge);
+  else loop(compute);
+  const auto mrow = [&](int i) { return edge ? erow(i) : frow(i); };
+  const auto ncol = [&](int j) { return edge ? ecol(j) : fcol(j); };
   if (TAIL && shared) {
     // a partial tile, as the registers hold it, for gemm_tail_kernel
     double* __restrict__ P = g.part + (long)wg * (BM * BN) + tid;
@@ -926,8 +940,11 @@ __global__ __launch_bounds__(256) void gemm_tail_kernel(GemmSide<T> g, T beta) {
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int x = q0 + 256 * u, th = x % NTH, e = x / NTH, lane = th & 63, wm = (th >> 6) & 1, wn = th >> 7;
-    const int i = e / (4 * NJ), j = e / 4 % NJ, r = e % 4, m = tm * BT + (2 * i + wm) * 16 + (lane & 15);
-    const int n = tn * BT + (sizeof(T) == 8 ? (4 * j + wn) * 16 + (lane >> 4) + 4 * r
+    const int i = e / (4 * NJ), j = e / 4 % NJ, r = e % 4;
+    // (the wavefronts' blocks as in the kernels: in turn in FP32 and, in FP64, in tiles that some are missing from)
+    const bool turn = sizeof(T) == 4 || g.M - tm * BT <= BT - 16 || g.N - tn * BT <= BT - 16;
+    const int m = tm * BT + (turn ? (2 * i + wm) * 16 : wm * 64 + i * 16) + (lane & 15);
+    const int n = tn * BT + (sizeof(T) == 8 ? (turn ? (4 * j + wn) * 16 : wn * 32 + j * 16) + (lane >> 4) + 4 * r
                                             : (2 * j + wn) * 16 + 4 * (lane >> 4) + r);
     if (m >= g.M || n >= g.N) continue;
     T* c = g.C + m + (long)n * g.ldc;
@@ -1606,7 +1623,7 @@ template <typename T>
 constexpr TailShape kTail{128, 128, 2, sizeof(T) == 8 ? 4 : 2, 16, 0.375, 8};
 
 // Estimated time (us) of a TAIL launch: a compute unit's slabs, and 2.5 for each workgroup's start and end, at the
-// rate that a long launch of 128x128 tiles reaches (1.87 us in FP64, 0.92 in FP32; more where few workgroups
+// rate that a long launch of 128x128 tiles reaches (1.87 us in FP64, 0.94 in FP32; more where few workgroups
 // share a unit), but at least the latency of each slab of the longest chunk; and the parts, written and read once.
 template <typename T>
 static double tail_us(const TailMap& t) {
@@ -1619,11 +1636,12 @@ static double tail_us(const TailMap& t) {
   const int chunks = t.n[0] ? t.s[0] : least;
   const double rounds = (double)cdiv(t.wgs, 256);
   const double slabs = t.whole / 256 * (t.nk + 2.5) + rounds * ((double)t.nk / chunks + 2.5);
-  const double latency = (dp ? 0.88 : 1.2) * (t.nk * (t.whole / 256 + 1.0 / least) + 2.5);
+  // (an FP32 unit holds four workgroups)
+  const double latency = (dp ? 0.88 : 1.2) * (t.nk * (t.whole / (dp ? 256 : 1024) + 1.0 / least) + 2.5);
   const long each = cdiv(t.whole + t.wgs, 256);
   const double few = dp ? (each == 1 ? 1.08 : 1.0) : (each == 1 ? 1.3 : each == 2 ? 1.12 : each == 3 ? 1.05 : 1.0);
   const double parts = t.wgs > tiles ? (2.0 * t.wgs + tiles) * 16384.0 * sizeof(T) / 6.0e6 + 5.0 : 0.0;
-  return 11.0 + (dp ? 1.87 : 0.92) * std::max(slabs, latency) * few + parts;
+  return 11.0 + (dp ? 1.87 : 0.94) * std::max(slabs, latency) * few + parts;
 }
 
 static const long kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128};
