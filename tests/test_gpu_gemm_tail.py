@@ -24,3 +24,22 @@ def test_gemm_tail(ctx, trans, M, N, K):
     # the rounding of a K-term sum of independent terms grows as sqrt(K) at most
     assert rel_err(out, ref) < 1e-13 * max(1.0, np.sqrt(K) / 4)
     assert np.array_equal(out, ctx.gemm_test(0, trans[0], trans[1], 0.7, A, B, -1.3, C0))  # fixed order
+
+
+@pytest.mark.parametrize("prec,tol", [(0, 1e-13), (1, 2e-5)])
+@pytest.mark.parametrize("M,N,K", [(400, 2000, 10000), (2500, 2490, 1999)])
+def test_gemm_tail_leading_dimensions(ctx, prec, tol, M, N, K):
+    """Odd leading dimensions above the sizes; what lies past M in C's columns is left alone."""
+    from jues._lib import ptr
+    rng = np.random.default_rng(M + N)
+    A = np.asfortranarray(rng.normal(size=(M + 3, K)))
+    B = np.asfortranarray(rng.normal(size=(K + 5, N)))
+    C = np.asfortranarray(rng.normal(size=(M + 7, N)))
+    C0 = C.copy()
+    ctx.check(ctx.lib.jues_gemm_test(ctx.h, prec, b"N", b"N", M, N, K, 0.7, ptr(A), M + 3, ptr(B), K + 5, -1.3, ptr(C),
+                                     M + 7))
+    ref = 0.7 * (A[:M] @ B[:K]) - 1.3 * C0[:M]
+    # as above and as in the FP32 test: inputs rounded once, a sum's rounding grows as sqrt(K) at most
+    assert rel_err(C[:M], ref) < tol * max(1.0, np.sqrt(K) / 4)
+    left = C0[M:] if prec == 0 else C0[M:].astype(np.float32)  # an FP32 product returns its FP32 copy of C
+    assert np.array_equal(C[M:], left)
