@@ -218,7 +218,9 @@ jues_status jues_rmp2_grad(jues_ctx* ctx, int prec, const double* C, int o, int 
 /* ---- CoupledCluster.{RCCD,mRCCD}.do_rccd (RCCD.jl:33-83, mRCCD.jl:38-118) ------
  * Converges the closed-shell CCD equations of RCCD.jl:134-303.  T2_inout (o x o x v x v,
  * Julia order) may be NULL; when given it receives the final amplitudes, and with
- * guess == JUES_GUESS_USER it also supplies the starting amplitudes. */
+ * guess == JUES_GUESS_USER it also supplies the starting amplitudes.  These have
+ * t[i,j,a,b] = t[j,i,b,a], as every iterate has: the packed ladders read one of the two
+ * and the ring terms their half-sum. */
 jues_status jues_rccd(jues_ctx* ctx, int prec, const jues_cc_opts* opts,
                       const double* Cocc, int o, const double* Cvir, int v, int n,
                       const double* eps, double* E, double* T2_inout,
