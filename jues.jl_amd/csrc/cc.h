@@ -205,7 +205,11 @@ constexpr long SPLIT_MIN_OV = 1900;
 // Whether the residual may be evaluated by the small system's launches (cc_small.hip), where they are faster than
 // the general form's in every precision.  FP64 iterations, general / small form: RCCD 111 / 67 us at ov = 192,
 // 136 / 128 at 336, 169 / 186 at 400; RCCSD 333 / 102 at 192, 387 / 176 at 336, 470 / 372 at 504.
-inline bool small_system(const CCState& S) { return (long)S.o * S.v <= (S.method == 1 ? 504 : 336); }
+// They leave the symmetrisation of the ring terms to the update kernel (no out_S), which does it in every precision up
+// to 77 occupied orbitals (fused_sym).
+inline bool small_system(const CCState& S) {
+  return (long)S.o * S.v <= (S.method == 1 ? 504 : 336) && fused_sym(S.o, sizeof(double));
+}
 // the residual of the resident amplitudes through the small system's launches (out_H, out_Y, out_X, Lp, Lm, R1)
 template <typename T>
 void small_contractions(jues_ctx* ctx, CCState& S);

@@ -653,6 +653,7 @@ void t2_update(jues_ctx* ctx, const UpdateArgs<TR>& A) {
   // S (or H and Y, each read twice), Lp, Lm and extra in the residual's compute type
   KTimer k(ctx, "cc_update", 0.0, (double)n2 * (8.0 * (5 + A.nold + (A.R_out ? 1 : 0)) + (A.H ? 7 : 4) * sizeof(TR)));
   size_t lds = 0;
+  JUES_REQUIRE(A.H || A.S, "t2_update: no ring terms");
   if (A.H) {
     JUES_REQUIRE(A.Y && !A.S && fused_sym(A.o, sizeof(TR)), "t2_update: fused symmetrisation misconfigured");
     lds = (size_t)A.o * (A.o + 1) * sizeof(TR);
