@@ -206,9 +206,10 @@ constexpr long SPLIT_MIN_OV = 1900;
 // the general form's in every precision.  FP64 iterations, general / small form: RCCD 111 / 67 us at ov = 192,
 // 136 / 128 at 336, 169 / 186 at 400; RCCSD 333 / 102 at 192, 387 / 176 at 336, 470 / 372 at 504.
 // They leave the symmetrisation of the ring terms to the update kernel (no out_S), which does it in every precision up
-// to 77 occupied orbitals (fused_sym).
+// to 77 occupied orbitals (fused_sym), and index every tensor with 32 bits, V+ of v (v + 1) / 2 rows and columns being
+// the largest (up to v = 303, which matters at o = 1).
 inline bool small_system(const CCState& S) {
-  return (long)S.o * S.v <= (S.method == 1 ? 504 : 336) && fused_sym(S.o, sizeof(double));
+  return (long)S.o * S.v <= (S.method == 1 ? 504 : 336) && fused_sym(S.o, sizeof(double)) && S.v <= 303;
 }
 // the residual of the resident amplitudes through the small system's launches (out_H, out_Y, out_X, Lp, Lm, R1)
 template <typename T>

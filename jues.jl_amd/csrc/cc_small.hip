@@ -346,13 +346,15 @@ class Builder {
     if (c >= 'w') return extra_[c - 'w'];
     return c >= 'i' && c <= 'n' ? o_ : v_;
   }
+  // elements between neighbours in the letter c (0 without it); the kernel's offsets have 32 bits
   int stride(const char* idx, char c) const {
-    long s = 1;
+    long s = 1, at = 0;
     for (; *idx; ++idx) {
-      if (*idx == c) return (int)s;
+      if (*idx == c) at = s;
       s *= size(*idx);
     }
-    return 0;
+    JUES_REQUIRE(s < (1L << 31), "small contraction: tensor too large");
+    return (int)at;
   }
   int o_, v_, first_ = 0;
   long extra_[4] = {1, 1, 1, 1};
@@ -548,9 +550,10 @@ void small_contractions(jues_ctx* ctx, CCState& S) {
       convert<double, float>(ctx, S.i64->Vm.as<double>(), b.Vm.as<float>(), (long)(S.i64->Vm.bytes / sizeof(double)));
     }
   }
-  if (!W.small) {
-    W.small.reset(new SmallPlan<T>());
-    W.small->build(ctx, S);
+  if (!W.small) {  // (kept only when it is whole: building it allocates)
+    std::unique_ptr<SmallPlan<T>> p(new SmallPlan<T>());
+    p->build(ctx, S);
+    W.small = std::move(p);
   }
   const SmallPlan<T>& plan = *W.small;
   const PairTables& P = S.P;
