@@ -79,7 +79,7 @@ void pack_v(jues_ctx* ctx, const PairTables& P, const T* X, long ldx, int v, int
 // G+-[(e,f),(a,m)] = ((mf|ae) +- (me|af))/2 (pairs e<=f / e<f; columns a + v m) from X[f,m,a,e] = (mf|ae), cnt values of m
 template <typename T>
 void pack_z(jues_ctx* ctx, const PairTables& P, const T* X, int v, int cnt, T* Gp, T* Gm);
-// Z[i,j,a,m] from Zp[(i<=j),(a,m)] and Zm[(i<j),(a,m)]: their sum for i < j, their difference for i > j
+// Z[i,j,a,m] from Zp[(i<=j),(a,m)] and Zm[(i<j),(a,m)] (null: zero): their sum for i < j, their difference for i > j
 template <typename T>
 void unpack_z(jues_ctx* ctx, const PairTables& P, const T* Zp, const T* Zm, int o, int v, T* Z);
 // hole-hole ladder integrals on pairs: KP[(k<=l),(c<=d)], KM[(k<l),(c<d)] from K[k,l,c,d] = <kl|cd>

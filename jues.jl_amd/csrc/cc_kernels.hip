@@ -142,7 +142,7 @@ __global__ __launch_bounds__(256) void unpack_z_kernel(const T* __restrict__ Zp,
     const long c = x / oo;
     const int ij = (int)(x - c * oo), i = ij % o, j = ij / o, p = min(i, j), q = max(i, j);
     T z = Zp[tri_le(p, q) + npo * c];
-    if (i != j) {
+    if (Zm && i != j) {
       const T w = Zm[tri_lt(p, q) + nmo * c];
       z += i < j ? w : -w;
     }

@@ -320,7 +320,8 @@ void rccsd_contractions(jues_ctx* ctx, CCState& S, const double* t2, const doubl
       const int cnt = (int)std::min<long>(ms, o - m0);
       ovvv_z_slab<T>(ctx, S, m0, cnt, LovT, Lvv, Tp, Tm, Zs, Zsp, Zp, Zm);
     }
-    unpack_z<T>(ctx, S.P, Zp, Zm, o, v, Z);
+    // (without pairs e < f the products leave Zm unwritten)
+    unpack_z<T>(ctx, S.P, Zp, S.P.nmv > 0 ? Zm : nullptr, o, v, Z);
     gemm<T>(ctx, false, false, oo * v, v, o, T(-1), Z, oo * v, 0, t1, o, 0, zero, X2, oo * v, 0, 1, "cc_t1");
   } else {
     contract<T>(ctx, 1.0, TN(Tpp, "ijef"), TN(ovvv, "mfae"), 0.0, TN(Z, "ijma"), "cc_ovvv");

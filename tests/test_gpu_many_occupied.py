@@ -39,3 +39,11 @@ def check_one_update(o, v, dense):
 @pytest.mark.parametrize("o,v,dense", SIZES)
 def test_one_update(o, v, dense):
     check_one_update(o, v, dense)
+
+
+@pytest.mark.parametrize("o", [78, 111])
+def test_one_virtual_orbital(o):
+    """No pairs a < b: the antisymmetric part of Z = tau (mf|ae) is empty.  Twice, so that the second run's buffers are
+    the first one's blocks with what they were left with."""
+    for _ in range(2):
+        check_one_update(o, 1, False)
