@@ -781,7 +781,7 @@ __global__ __launch_bounds__(4 * BT, 4) void gemm64_kernel(GemmSide<double> p0, 
 // wavefronts share the contraction instead of the tile.  Wavefront w takes the 16-deep k-slabs w, w + NW,
 // ...: it loads their fragments from global memory straight into registers (nothing is shared between
 // wavefronts, so nothing is staged in LDS and the loop has no barrier), two slabs in flight, and the
-// NW partial tiles are added in a fixed order through LDS at the end.  Lane l supplies
+// NW partial tiles are added in a fixed order through LDS at the end, in FP64 as every sum of partial results here.  Lane l supplies
 // k = 4 (l / 16) + s at MFMA step s, so a k-contiguous operand is read 4 consecutive k per lane and an
 // m-contiguous one in runs of 16 rows.  Rows past M or N load a clamped row and are not stored; the K
 // tail is a predicated slab after the full ones.
@@ -893,15 +893,15 @@ __global__ __launch_bounds__(64 * NW) void gemm_direct_kernel(GemmSide<T> g, T a
         red[wave][(16 * j + Mfma<T>::row(lane, r)) * BM + 16 * i + fr] = acc[i][j][r];
   __syncthreads();
   for (int e = tid; e < BM * BN; e += 64 * NW) {
-    T v = red[0][e];
+    double v = (double)red[0][e];
 #pragma unroll
-    for (int w = 1; w < NW; ++w) v += red[w][e];
+    for (int w = 1; w < NW; ++w) v += (double)red[w][e];
     const int m = m0 + e % BM, n = n0 + e / BM;
     if (m < M && n < N) {
       const long off = (long)m + (long)n * g.ldc;
-      v *= alpha;
-      if (beta != T(0)) v += beta * C[off];
-      C[off] = v;
+      v *= (double)alpha;
+      if (beta != T(0)) v += (double)beta * (double)C[off];
+      C[off] = (T)v;
     }
   }
 }
@@ -915,11 +915,9 @@ __global__ void scale_kernel(T* C, long M, long N, long ldc, T beta) {
   }
 }
 
-// C = beta*C + sum_s W[s] (fixed order), W[s] is M x N with leading dimension M.  Eight loads are in
-// flight per thread: with one element per thread and a few hundred partial products (a 20 x 20 result
-// of K = 200000) the sum is otherwise a chain of as many memory latencies.
-// C = (sum of the parts of a TAIL launch's tile, in the order of its slabs) + beta C.  blockIdx.x: tile of the
-// tail, blockIdx.y: 1024 of its 128 x 128 results, in the order of the workgroups' registers.
+// C = (sum of the parts of a TAIL launch's tile, in FP64 and in the order of its slabs) + beta C.  blockIdx.x: tile
+// of the tail, blockIdx.y: 1024 of its 128 x 128 results, in the order of the workgroups' registers.  Bound by reading
+// the parts.
 template <typename T>
 __global__ __launch_bounds__(256) void gemm_tail_kernel(GemmSide<T> g, T beta) {
   constexpr int BT = 128, NTH = sizeof(T) == 8 ? 512 : 256, NJ = sizeof(T) == 8 ? 2 : 4;
@@ -931,11 +929,11 @@ __global__ __launch_bounds__(256) void gemm_tail_kernel(GemmSide<T> g, T beta) {
   for (int k = 1; k <= 3 && k != q; ++k) first += tail.n[k] * tail.s[k];
   const int t = (int)blockIdx.x - tail.first_tile(q);
   const int q0 = (int)blockIdx.y * 1024 + threadIdx.x;
-  T sum[4] = {T(0), T(0), T(0), T(0)};
+  double sum[4] = {0.0, 0.0, 0.0, 0.0};
   for (int c = 0; c < tail.s[q]; ++c) {
     const T* P = g.part + (long)(first + c * tail.n[q] + t) * (BT * BT) + q0;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) sum[u] += P[256 * u];
+    for (int u = 0; u < 4; ++u) sum[u] += (double)P[256 * u];
   }
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
@@ -948,10 +946,13 @@ __global__ __launch_bounds__(256) void gemm_tail_kernel(GemmSide<T> g, T beta) {
                                             : (2 * j + wn) * 16 + 4 * (lane >> 4) + r);
     if (m >= g.M || n >= g.N) continue;
     T* c = g.C + m + (long)n * g.ldc;
-    *c = beta != T(0) ? sum[u] + beta * *c : sum[u];
+    *c = (T)(beta != T(0) ? sum[u] + (double)beta * (double)*c : sum[u]);
   }
 }
 
+// C = beta*C + sum_s W[s] (in FP64, fixed order), W[s] is M x N with leading dimension M.  Eight loads are in
+// flight per thread: with one element per thread and a few hundred partial products (a 20 x 20 result
+// of K = 200000) the sum is otherwise a chain of as many memory latencies.
 template <typename T>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const T* __restrict__ W, int S, long M, long N,
                                                             T* __restrict__ C, long ldc, T beta) {
