@@ -141,9 +141,9 @@ __global__ __launch_bounds__(64 * SW) void small_contract_kernel(const SmallOut<
   const int em = 16 * tm + tid % 16, en = 16 * tn + tid / 16;
   if (tid >= 256 || em >= M || en >= N) return;
   const int i[4] = {em % O.d[0], em / O.d[0], en % O.d[2], en / O.d[2]};
-  T val = red[0][tid];
+  double val = (double)red[0][tid];  // (the sums of partial results are in FP64 and rounded once)
 #pragma unroll
-  for (int w = 1; w < SW; ++w) val += red[w][tid];
+  for (int w = 1; w < SW; ++w) val += (double)red[w][tid];
   for (int q = O.p0; q < O.p1; ++q) {
     const SmallPoint<T>& p = points[q];
     const T* A = p.A + i[0] * p.a[0] + i[1] * p.a[1] + i[2] * p.a[2] + i[3] * p.a[3];
@@ -151,17 +151,17 @@ __global__ __launch_bounds__(64 * SW) void small_contract_kernel(const SmallOut<
     T s = 0;
 #pragma unroll 8
     for (int k = 0; k < p.K; ++k) s += A[k * p.ka] * B[k * p.kb];
-    val += p.alpha * s;
+    val += (double)(p.alpha * s);
   }
   if (O.D) {
     const T* D = O.D + i[0] * O.e[0] + i[1] * O.e[1] + i[2] * O.e[2] + i[3] * O.e[3];
-    T s = 0;
-    for (int q = 0; q < O.nd; ++q) s += D[(long)q * O.dstep];
-    val += O.beta * s;
+    double s = 0;
+    for (int q = 0; q < O.nd; ++q) s += (double)D[(long)q * O.dstep];
+    val += (double)O.beta * s;
   }
   const int at = i[0] * O.c[0] + i[1] * O.c[1] + i[2] * O.c[2] + i[3] * O.c[3];
-  if (O.C64) O.C64[at] = (double)val;
-  else O.C[at] = val;
+  if (O.C64) O.C64[at] = val;
+  else O.C[at] = (T)val;
 }
 
 // What the contractions read of the amplitudes, in the compute type: t2 and t1 themselves (FP32 only), with t1 also
