@@ -313,15 +313,16 @@ void ring_mm<float>(jues_ctx* ctx, CCState& S, float alpha, const float* A, int 
   gemm16_tn(ctx, ov, ov, alpha, a, b, beta, C, ov, "cc_ring");
 }
 
-// Lx = K - Kx/2 of the ring products, made by their first use (a small system's launches do without)
+// Lx = K - Kx/2 of the ring products, made by their first use (a small system's launches do without) from the
+// FP64 blocks, which a fast stage still has in its first iteration: rounded once
 template <typename T>
 const T* ring_lx(jues_ctx* ctx, CCState& S) {
   CCInts<T>& I = ints<T>(S);
   const long ov = (long)S.o * S.v, N2 = ov * ov;
   if (!I.Lx.p) {
+    JUES_REQUIRE(S.i64->Kov.p && S.i64->Ktov.p, "ring_lx: the FP64 blocks were released");
     T* L = bufp<T>(I.Lx, N2);
-    JUES_HIP(hipMemcpyAsync(L, I.Kov.template as<T>(), N2 * sizeof(T), hipMemcpyDeviceToDevice, ctx->stream));
-    axpby<T>(ctx, N2, -0.5, I.Ktov.template as<T>(), 1.0, L);
+    axpby2<T>(ctx, N2, 1.0, S.i64->Kov.as<double>(), -0.5, S.i64->Ktov.as<double>(), L);
   }
   return I.Lx.template as<T>();
 }

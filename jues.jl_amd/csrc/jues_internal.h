@@ -257,6 +257,9 @@ void fill(jues_ctx* ctx, T* out, long n, double value);
 // y = a*x + b*y
 template <typename T>
 void axpby(jues_ctx* ctx, long n, double a, const T* x, double b, T* y);
+// z = a*x + b*y, formed in FP64 and rounded once to T
+template <typename T>
+void axpby2(jues_ctx* ctx, long n, double a, const double* x, double b, const double* y, T* z);
 // deterministic FP64 dot of two vectors (any element types)
 template <typename Ta, typename Tb>
 double dot(jues_ctx* ctx, const Ta* x, const Tb* y, long n);

@@ -97,6 +97,14 @@ __global__ void axpby_kernel(long n, double a, const T* __restrict__ x, double b
     y[e] = (T)(a * (double)x[e] + (b == 0.0 ? 0.0 : b * (double)y[e]));
 }
 
+// z = a x + b y, rounded once
+template <typename T>
+__global__ void axpby2_kernel(long n, double a, const double* __restrict__ x, double b, const double* __restrict__ y,
+                              T* __restrict__ z) {
+  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x)
+    z[e] = (T)(a * x[e] + b * y[e]);
+}
+
 constexpr int RED_BLOCKS = 1024;
 
 __device__ inline double block_sum(double v, double* sh) {
@@ -218,6 +226,14 @@ void axpby(jues_ctx* ctx, long n, double a, const T* x, double b, T* y) {
   JUES_HIP(hipGetLastError());
 }
 
+template <typename T>
+void axpby2(jues_ctx* ctx, long n, double a, const double* x, double b, const double* y, T* z) {
+  if (n <= 0) return;
+  KTimer t(ctx, "axpby", 0.0, (double)n * (16.0 + sizeof(T)));
+  hipLaunchKernelGGL((axpby2_kernel<T>), dim3(grid_for(n)), dim3(256), 0, ctx->stream, n, a, x, b, y, z);
+  JUES_HIP(hipGetLastError());
+}
+
 template <typename Ta, typename Tb>
 double dot(jues_ctx* ctx, const Ta* x, const Tb* y, long n) {
   double* part = static_cast<double*>(scratch(ctx, 15, (RED_BLOCKS + 1) * sizeof(double)));
@@ -255,6 +271,8 @@ template void fill<double>(jues_ctx*, double*, long, double);
 template void fill<float>(jues_ctx*, float*, long, double);
 template void axpby<double>(jues_ctx*, long, double, const double*, double, double*);
 template void axpby<float>(jues_ctx*, long, double, const float*, double, float*);
+template void axpby2<double>(jues_ctx*, long, double, const double*, double, const double*, double*);
+template void axpby2<float>(jues_ctx*, long, double, const double*, double, const double*, float*);
 template double dot<double, double>(jues_ctx*, const double*, const double*, long);
 template double dot<float, float>(jues_ctx*, const float*, const float*, long);
 template double dot<double, float>(jues_ctx*, const double*, const float*, long);
