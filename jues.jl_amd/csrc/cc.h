@@ -136,6 +136,7 @@ struct CCState {
   bool fast16 = false;    // the fast stage is the split-FP16 one
   bool split_on = false;  // ... and its ring / pp-ladder products run on split-FP16 MFMA
   bool ladder_recompute = false;  // <ab|ef> rebuilt from factors every iteration instead of stored
+  long small_ov = 0, split_ov = 0;  // the forms' limits in ov: small_system, split_products
   hipEvent_t ev[2] = {nullptr, nullptr};
   double lambda = 1.0;  // coupling of the equations being iterated
   double E_prev = 0;
@@ -200,7 +201,12 @@ void fac_y3_lvv(jues_ctx* ctx, CCState& S, const T* Y3, T* Q);
 // more precise form: a product's operands have to be scaled and split first (a dozen extra launches and
 // 256-column padding).  Iterations, FP32 / split: RCCD 519 / 1005 us at ov = 1200, 1270 / 1197 at 1920,
 // 2837 / 1864 at 2700; RCCSD 1011 / 1662, 2071 / 2111, 4347 / 3196.
+// (JUES_SPLIT_MIN_OV and JUES_SMALL_MAX_OV, read by cc_setup, take the place of this and the next limit, e.g. to test
+// the forms at sizes that are not theirs.)
 constexpr long SPLIT_MIN_OV = 1900;
+inline bool split_products(const CCState& S, int prec) {
+  return prec == JUES_FP16X3_MIXED && (long)S.o * S.v >= S.split_ov;
+}
 
 // Whether the residual may be evaluated by the small system's launches (cc_small.hip), where they are faster than
 // the general form's in every precision.  FP64 iterations, general / small form: RCCD 111 / 67 us at ov = 192,
@@ -208,8 +214,9 @@ constexpr long SPLIT_MIN_OV = 1900;
 // They leave the symmetrisation of the ring terms to the update kernel (no out_S), which does it in every precision up
 // to 77 occupied orbitals (fused_sym), and index every tensor with 32 bits, V+ of v (v + 1) / 2 rows and columns being
 // the largest (up to v = 303, which matters at o = 1).
+constexpr long SMALL_MAX_OV_CCD = 336, SMALL_MAX_OV_CCSD = 504;
 inline bool small_system(const CCState& S) {
-  return (long)S.o * S.v <= (S.method == 1 ? 504 : 336) && fused_sym(S.o, sizeof(double)) && S.v <= 303;
+  return (long)S.o * S.v <= S.small_ov && fused_sym(S.o, sizeof(double)) && S.v <= 303;
 }
 // the residual of the resident amplitudes through the small system's launches (out_H, out_Y, out_X, Lp, Lm, R1)
 template <typename T>

@@ -1000,6 +1000,12 @@ void cc_setup(jues_ctx* ctx, int method, int prec, const jues_cc_opts* opts_in, 
   const int oo_ = S.o;
   const long N2 = (long)oo_ * oo_ * v * v, N1 = (long)oo_ * v;
   S.Nd = N2 + (method == 1 ? N1 : 0);
+  const auto limit = [](const char* name, long by_default) {
+    const char* env = std::getenv(name);
+    return env ? std::atol(env) : by_default;
+  };
+  S.small_ov = limit("JUES_SMALL_MAX_OV", method == 1 ? SMALL_MAX_OV_CCSD : SMALL_MAX_OV_CCD);
+  S.split_ov = limit("JUES_SPLIT_MIN_OV", SPLIT_MIN_OV);
   for (auto& e : S.ev) JUES_HIP(hipEventCreate(&e));
   // orbital data (frozen core dropped)
   DeviceArray<double> co(ctx, Cocc + (size_t)fc * n, (size_t)n * oo_), cv(ctx, Cvir, (size_t)n * v);
@@ -1132,7 +1138,7 @@ void cc_run(jues_ctx* ctx, CCState& S, int stage_prec, int nsteps, bool stop_on_
   S.last_stage = stage_prec;
   if (stage_prec != JUES_FP64) cc_make_ints32(ctx, S);
   S.fast16 = stage_prec == JUES_FP16X3_MIXED;
-  S.split_on = S.fast16 && (long)S.o * S.v >= SPLIT_MIN_OV;
+  S.split_on = split_products(S, stage_prec);
   int stall = 0;
   double best = 1e300;
   static const char* stage_name[3] = {"fp64", "fp32", "fp16x3"};
