@@ -44,7 +44,8 @@ typedef enum {
     JUES_FP16X3_MIXED = 2 /* as FP32_MIXED, but the ring, particle-particle ladder and
                              hole-hole GEMMs run on FP16 MFMA with each FP32 operand split
                              into hi + lo halves under a power-of-two scale (three products,
-                             FP32 accumulate; ~2^-21 relative per product) */
+                             FP32 accumulate; ~2^-21 relative per product).  Below o v = 1900 they
+                             run in FP32 MFMA, which is faster there and more precise */
 } jues_prec;
 
 /* Which reference RCCSD equations to follow.  They differ only in the T1 exchange
@@ -115,7 +116,7 @@ typedef struct {
 /* Per-iteration record passed to the optional callback. */
 typedef struct {
     int32_t iter;             /* 1-based */
-    int32_t stage;            /* 0 = FP64, 1 = FP32 (FP32_MIXED), 2 = split-FP16 (FP16X3_MIXED) */
+    int32_t stage;            /* 0 = FP64, 1 = the fast stage of FP32_MIXED, 2 = that of FP16X3_MIXED */
     double energy;            /* correlation energy of the Jacobi update t_new */
     double delta_e;           /* energy - previous energy */
     double rnorm;             /* ||t_new - t_old||_2 (T1 and T2 together for CCSD) */

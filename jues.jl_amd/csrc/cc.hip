@@ -1179,8 +1179,9 @@ void cc_reset_diis(CCState& S) { S.active.clear(); }
 // inner_prec (with DIIS) until its step is below max(r_conv / 10, kappa ||dt||_anchor) or stalls,
 // and the next FP64 iteration starts from that solution.  Each anchor's step measures the FP64
 // residual itself.  kappa is about the factor by which one anchor can shrink the error, set by the
-// inner products' rounding (relative to |d|): 1e-5 for FP32 MFMA, 1e-3 for split-FP16, whose
-// products err by up to ~30x more; iterating the inner equation below that buys nothing.
+// inner products' rounding (relative to |d|): 1e-5 for FP32 MFMA (the split-FP16 form's own products below its limit
+// in ov are that too), 1e-3 for split-FP16, whose products err by up to ~30x more; iterating the inner equation below
+// that buys nothing.
 // Returns the number of FP64 iterations run.
 int cc_refine_dc(jues_ctx* ctx, CCState& S, int inner_prec, int max_anchors, int inner_maxit,
                  jues_iter_info* last, bool* converged, jues_iter_cb cb, void* user) {
@@ -1198,7 +1199,7 @@ int cc_refine_dc(jues_ctx* ctx, CCState& S, int inner_prec, int max_anchors, int
       if (S.dc) S.dc->capture = S.dc->on = false;
     }
   } clear{S};
-  const double kappa = inner_prec == JUES_FP16X3_MIXED ? 1e-3 : (inner_prec == JUES_FP32_MIXED ? 1e-5 : 0.0);
+  const double kappa = split_products(S, inner_prec) ? 1e-3 : (inner_prec != JUES_FP64 ? 1e-5 : 0.0);
   int k = 0;
   while (k < max_anchors) {
     cc_reset_diis(S);
