@@ -443,6 +443,12 @@ __global__ __launch_bounds__(256) void diis_solve_kernel(double* small, DiisOrde
   for (int e = t; e < MAX_DIIS * MAX_DIIS; e += blockDim.x) B[e / MAX_DIIS][e % MAX_DIIS] = small[SMALL_B + e];
   __syncthreads();
   if (t >= 64) return;
+  // the rest is the first wavefront's: its lanes' accesses to LDS are in order, so between them only the compiler has to
+  // keep that order (a workgroup barrier would have to be reached by the wavefronts that are done, too)
+  const auto wave_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+  };
   const int s = ord.newest;
   if (t <= ord.nold) {
     const int sk = t < ord.nold ? ord.old_slots[t] : s;
@@ -456,7 +462,7 @@ __global__ __launch_bounds__(256) void diis_solve_kernel(double* small, DiisOrde
     if (t == 0) { c[0] = 1.0; small[SMALL_FLAG] = 0.0; }
     return;
   }
-  __syncthreads();
+  wave_sync();
   double mx = t < m * m ? fabs(B[ord.slots[t / m]][ord.slots[t % m]]) : 0.0;  // m * m <= 64
   for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
   if (!(mx > 0.0)) mx = 1.0;
@@ -468,7 +474,7 @@ __global__ __launch_bounds__(256) void diis_solve_kernel(double* small, DiisOrde
     else val = p == m && q == m ? 0.0 : -1.0;
     M[p][q] = val;
   }
-  __syncthreads();
+  wave_sync();
   bool ok = true;
   for (int k = 0; k < N; ++k) {
     // the first row of the largest |M[p][k]|, p >= k
@@ -483,7 +489,7 @@ __global__ __launch_bounds__(256) void diis_solve_kernel(double* small, DiisOrde
     piv = __shfl(piv, 0, 64);
     if (!(best > 1e-300)) { ok = false; break; }
     if (piv != k && t <= N) { const double tmp = M[k][t]; M[k][t] = M[piv][t]; M[piv][t] = tmp; }
-    __syncthreads();
+    wave_sync();
     // rows below k; column k itself is not read again
     const int rows = N - 1 - k, cols = N - k;
     for (int e = t; e < rows * cols; e += 64) {
@@ -491,15 +497,15 @@ __global__ __launch_bounds__(256) void diis_solve_kernel(double* small, DiisOrde
       const double f = M[p][k] / M[k][k];
       M[p][q] -= f * M[k][q];
     }
-    __syncthreads();
+    wave_sync();
   }
   if (ok) {
     for (int k = N - 1; k >= 0; --k) {
       const double xk = M[k][N] / M[k][k];
-      __syncthreads();
+      wave_sync();
       if (t < k) M[t][N] -= M[t][k] * xk;
       else if (t == k) M[k][N] = xk;
-      __syncthreads();
+      wave_sync();
     }
     for (int p = 0; p < m; ++p) ok = ok && isfinite(M[p][N]);
   }
