@@ -136,7 +136,7 @@ struct CCState {
   bool fast16 = false;    // the fast stage is the split-FP16 one
   bool split_on = false;  // ... and its ring / pp-ladder products run on split-FP16 MFMA
   bool ladder_recompute = false;  // <ab|ef> rebuilt from factors every iteration instead of stored
-  long small_ov = 0, split_ov = 0;  // the forms' limits in ov: small_system, split_products
+  long small_ov = -1, split_ov = 0;  // limits in ov: small_system (-1: its own rule), split_products
   hipEvent_t ev[2] = {nullptr, nullptr};
   double lambda = 1.0;  // coupling of the equations being iterated
   double E_prev = 0;
@@ -199,24 +199,33 @@ template <typename T>
 void fac_y3_lvv(jues_ctx* ctx, CCState& S, const T* Y3, T* Q);
 // The split-FP16 stage runs its products on split planes from this ov on, below it in FP32 MFMA, which is the
 // more precise form: a product's operands have to be scaled and split first (a dozen extra launches and
-// 256-column padding).  Iterations, FP32 / split: RCCD 519 / 1005 us at ov = 1200, 1270 / 1197 at 1920,
-// 2837 / 1864 at 2700; RCCSD 1011 / 1662, 2071 / 2111, 4347 / 3196.
-// (JUES_SPLIT_MIN_OV and JUES_SMALL_MAX_OV, read by cc_setup, take the place of this and the next limit, e.g. to test
-// the forms at sizes that are not theirs.)
+// 256-column padding).  Iterations in us, FP32 / split: RCCD 519 / 1005 at ov = 1200, 719 / 714 at 1600, 961 / 832 at
+// 1800, 1040 / 910 at 1900, 1157 / 865 at 1995; RCCSD 1011 / 1662, 1277 / 1339, 1651 / 1576, 1774 / 1677, 1911 / 1658.
+// The two cross between 1600 and 1800; up to 1900, where the split form gains little, the more precise one is kept.
+// (JUES_SPLIT_MIN_OV and JUES_SMALL_MAX_OV, read by cc_setup, take the place of this limit and of the next rule by size,
+// e.g. to test the forms at sizes that are not theirs.)
 constexpr long SPLIT_MIN_OV = 1900;
 inline bool split_products(const CCState& S, int prec) {
   return prec == JUES_FP16X3_MIXED && (long)S.o * S.v >= S.split_ov;
 }
 
-// Whether the residual may be evaluated by the small system's launches (cc_small.hip), where they are faster than
-// the general form's in every precision.  FP64 iterations, general / small form: RCCD 111 / 67 us at ov = 192,
-// 136 / 128 at 336, 169 / 186 at 400; RCCSD 333 / 102 at 192, 387 / 176 at 336, 470 / 372 at 504.
-// They leave the symmetrisation of the ring terms to the update kernel (no out_S), which does it in every precision up
-// to 77 occupied orbitals (fused_sym), and index every tensor with 32 bits, V+ of v (v + 1) / 2 rows and columns being
-// the largest (up to v = 303, which matters at o = 1).
-constexpr long SMALL_MAX_OV_CCD = 336, SMALL_MAX_OV_CCSD = 504;
+// Whether the residual may be evaluated by the small system's launches (cc_small.hip): as long as they are not slower
+// than the general form's.  They form the hole-hole terms, o^4 v^2 work, without packing the pairs, and the packed ladder
+// in 16 x 16 tiles that walk v^2 / 2 each, so many occupied or virtual orbitals cost them more than their ov does.
+// FP64 iterations in us, general / small form (o x v): RCCD 115 / 114 at 12 x 28, 119 / 117 at 20 x 16, 132 / 126 at
+// 8 x 42, 134 / 132 at 4 x 60, 106 / 95 at 30 x 7, 105 / 103 at 40 x 1; 135 / 173 at 10 x 40, 118 / 159 at 30 x 11,
+// 202 / 212 at 50 x 2, 152 / 171 at 5 x 66, 140 / 205 at 1 x 100.  RCCSD 407 / 359 at 12 x 42, 384 / 311 at 30 x 12,
+// 451 / 383 at 40 x 8, 749 / 647 at 60 x 2, 505 / 443 at 4 x 90, 353 / 312 at 1 x 100; 456 / 507 at 14 x 40, 453 / 507 at
+// 30 x 16, 568 / 604 at 50 x 6, 768 / 931 at 3 x 120.  (FP32 crosses at the same sizes.)
+// By itself the form can take up to the 77 occupied orbitals for which the update kernel symmetrises the ring terms in
+// every precision (fused_sym; there is no out_S), and 32-bit offsets, V+ of v (v + 1) / 2 rows and columns being the
+// largest tensor at few occupied orbitals (up to v = 303).
 inline bool small_system(const CCState& S) {
-  return (long)S.o * S.v <= S.small_ov && fused_sym(S.o, sizeof(double)) && S.v <= 303;
+  const long o = S.o, v = S.v, ov = o * v;
+  if (!fused_sym(S.o, sizeof(double)) || v > 303) return false;
+  if (S.small_ov >= 0) return ov <= S.small_ov;
+  return S.method == 1 ? ov <= 504 && o <= 60 && v <= 100 && o * ov <= 13000
+                       : ov <= 336 && o <= 40 && v <= 60 && o * ov <= 6400;
 }
 // the residual of the resident amplitudes through the small system's launches (out_H, out_Y, out_X, Lp, Lm, R1)
 template <typename T>

@@ -1004,7 +1004,7 @@ void cc_setup(jues_ctx* ctx, int method, int prec, const jues_cc_opts* opts_in, 
     const char* env = std::getenv(name);
     return env ? std::atol(env) : by_default;
   };
-  S.small_ov = limit("JUES_SMALL_MAX_OV", method == 1 ? SMALL_MAX_OV_CCSD : SMALL_MAX_OV_CCD);
+  S.small_ov = limit("JUES_SMALL_MAX_OV", -1);
   S.split_ov = limit("JUES_SPLIT_MIN_OV", SPLIT_MIN_OV);
   for (auto& e : S.ev) JUES_HIP(hipEventCreate(&e));
   // orbital data (frozen core dropped)

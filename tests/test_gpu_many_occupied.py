@@ -1,6 +1,7 @@
 """One CCD / CCSD update of random amplitudes with many occupied and few virtual orbitals, against the oracle's
 restatements: below and past the 77 (FP64) and 110 (FP32) occupied orbitals up to which the update kernel symmetrises
-the ring terms itself, at products o v where a system of fewer occupied orbitals takes the small system's launches."""
+the ring terms itself, at products o v where a system of fewer occupied orbitals takes the small system's launches, by
+default (up to 40 and 60) or forced (JUES_SMALL_MAX_OV)."""
 import numpy as np
 import pytest
 
@@ -36,8 +37,14 @@ def check_one_update(o, v, dense):
             assert err <= bound, (name, prec)
 
 
-@pytest.mark.parametrize("o,v,dense", SIZES)
+@pytest.mark.parametrize("o,v,dense", SIZES + [(40, 4, False), (41, 4, False), (60, 3, False), (60, 4, True), (61, 3, False)])
 def test_one_update(o, v, dense):
+    check_one_update(o, v, dense)
+
+
+@pytest.mark.parametrize("o,v,dense", SIZES)
+def test_one_update_forced(o, v, dense, monkeypatch):
+    monkeypatch.setenv("JUES_SMALL_MAX_OV", "504")
     check_one_update(o, v, dense)
 
 

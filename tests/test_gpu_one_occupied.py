@@ -1,6 +1,6 @@
-"""One occupied orbital and as many virtual ones as the small system's launches index V+ with 32 bits for (303), and
-one more: the stored ladder, whose V+ has 46056 and 46360 rows and columns there, against the recomputed one, which
-has no V+."""
+"""One occupied orbital and as many virtual ones as the small system's launches (forced here) index V+ with 32 bits for
+(303), and one more: the stored ladder, whose V+ has 46056 and 46360 rows and columns there, against the recomputed one,
+which has no V+."""
 import numpy as np
 import pytest
 
@@ -9,7 +9,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("method", ["rccd", "rccsd"])
 @pytest.mark.parametrize("v", [303, 304])
-def test_stored_ladder_equals_recomputed(v, method):
+def test_stored_ladder_equals_recomputed(v, method, monkeypatch):
+    monkeypatch.setenv("JUES_SMALL_MAX_OV", "504")
     from jues import synthetic
     from jues.CoupledCluster import Solver
     from jues.Wavefunction import Wfn, FactoredERI
