@@ -71,6 +71,14 @@ __device__ inline bool entry_place(int& x, int& z) {
   return true;
 }
 
+// A value that is the same in all lanes, in scalar registers: the operand offsets that a two-segment launch reads from its
+// table.  In vector registers they had gemm32_nn_kernel spill in its loop: the FP32 W products of the triples at v = 340
+// reach 94 TFLOP/s that way, 101 this way.
+__device__ inline long uniform(long x) {
+  return (long)((unsigned long)(unsigned)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32 |
+                (unsigned)__builtin_amdgcn_readfirstlane((int)x));
+}
+
 // Tile of workgroup pid of nwg, of which only the first tiles_m * tiles_n carry a tile (a launch
 // padded to a multiple of NXCD); false for the padding ids.  plain: the workgroups are on one XCD already.
 __device__ inline bool tile_coords_bounded(int pid, int nwg, int tiles_m, int tiles_n, int& tm, int& tn,
@@ -158,16 +166,16 @@ __global__ __launch_bounds__(256, 4) void gemm32_nn_kernel(GemmSide<float> p0, G
   const int M = g.M, N = g.N, K = bz == g.nz - 1 ? g.Klast : g.K;
   if (bz >= g.nz) return;
   const long lda = g.lda, ldb = g.ldb, ldc = g.ldc;
-  const int grp = SEG ? bz / g.inner : 0;  // the table only in the SEG instantiations
+  const int grp = SEG ? __builtin_amdgcn_readfirstlane(bz / g.inner) : 0;  // the table only in the SEG instantiations
   const long zb = (long)bz - (SEG ? (long)grp * g.inner : 0L);
   const long* tab = SEG ? g.tab + 4L * grp : nullptr;
-  const float* __restrict__ A = g.A + zb * g.sA + (SEG ? tab[0] : 0L);
-  const float* __restrict__ B = g.B + zb * g.sB + (SEG ? tab[1] : 0L);
+  const float* __restrict__ A = g.A + zb * g.sA + (SEG ? uniform(tab[0]) : 0L);
+  const float* __restrict__ B = g.B + zb * g.sB + (SEG ? uniform(tab[1]) : 0L);
   float* __restrict__ C = OUT64 ? nullptr : g.C + zb * g.sC + (SEG ? grp * g.sG : 0L);
   // a second contraction segment (A1, B1 over K1 columns) only in the SEG instantiations
   const int K1 = SEG ? g.K1 : 0;
-  const float* A1 = SEG ? g.A1 + zb * g.sA + tab[2] : A;
-  const float* B1 = SEG ? g.B1 + zb * g.sB + tab[3] : B;
+  const float* A1 = SEG ? g.A1 + zb * g.sA + uniform(tab[2]) : A;
+  const float* B1 = SEG ? g.B1 + zb * g.sB + uniform(tab[3]) : B;
   // slices: the K tail (columns 16 floor(K/16) .. K-1, zero-padded) first when there is one, then the full
   // slices from k = 0; the tail is loaded in the prologue
   const int K16 = K / BK * BK, tail = K > K16 ? 1 : 0;
