@@ -1546,12 +1546,20 @@ struct GemmPlan {
   long split = 1;   // chunks of the contraction, each a launch-z entry with its own partial product
   TailMap tail;     // wgs > 0: a TAIL launch of 128x128 tiles
   double us = 1e300;
+  long chain = 0;   // the longest sum over k in one accumulator
 };
 
 static inline long cdiv(long a, long b) { return (a + b - 1) / b; }
 
-// gridDim.z of a launch of nz entries (entry_place); at most 65528 entries
-static inline unsigned grid_z(int nz) { return (unsigned)(nz >= NXCD ? cdiv(nz, NXCD) * NXCD : nz); }
+// gridDim.z of a launch of nz entries of `tiles` workgroups (entry_place); at most 65528 entries.  Not padded where the
+// XCDs' shares would differ too much: in FP32, 17 chunks of 600 x 1500 x 20000 take 483 us in three entries for some XCDs
+// and two for others, 361 dealt tile by tile; 15 chunks of 2800 x 1500 x 33600, each more than an XCD holds at once, 2.77
+// and 2.57 ms.
+static inline unsigned grid_z(int nz, long tiles) {
+  const long padded = cdiv(nz, NXCD) * NXCD;
+  const bool even = 3 * padded <= 4L * nz && (tiles <= 128 || 16 * padded <= 17L * nz);
+  return (unsigned)(nz >= NXCD && even ? padded : nz);
+}
 
 static void form_tile(int form, long M, long N, long& bm, long& bn) {
   switch (form) {
@@ -1655,12 +1663,34 @@ static double tail_us(const TailMap& t) {
 
 static const long kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128};
 
-// The form and split with the smallest estimated time.  A split product's partial results take at most
-// 256 MiB of workspace, 2 GiB when K >= 32768 (RCCSD's o^2 x v.m x v^2 products over (ia|bc)).
+// The longest sum over k that an accumulator of an FP32 product may form before it is added to others in FP64: the error
+// of a long product is that of its accumulators' FP32 sums (it grows as the root of their length: 5.7e-7 of sqrt(K) at
+// 1024, 2.5e-6 at 20000), so a form that is faster without splitting K does not give this up.  Products of few 128x128
+// tiles get chunks of 1024 and longer ones that make a round of four workgroups a compute unit; long ones of more tiles
+// the fewest chunks that fill the rounds; others may sum all of K.
+static long chain_limit(long M, long N, long K) {
+  if (K < 4096) return K;
+  const bool wide = M <= 64 && N >= 8192, tall = N <= 64 && M >= 8192;
+  const long tiles = cdiv(M, wide ? 64 : tall ? 256 : 128) * cdiv(N, wide ? 256 : tall ? 64 : 128);
+  long S = 1;
+  if (tiles < 128) {
+    S = std::max(2L, std::min(K / 1024, 1024 / tiles));
+  } else if (!wide && !tall && K >= 32768) {
+    const auto fill = [&](long s) { return (double)(tiles * s) / (double)(cdiv(tiles * s, 1024) * 1024); };
+    for (long s = 2; s <= 16 && fill(1) < 0.8; ++s)
+      if (fill(s) > fill(S) + 0.02 && 4.0 * s * M * N <= 2147483648.0) S = s;
+  }
+  return cdiv(cdiv(K, S), 32) * 32;
+}
+
+// The form and split with the smallest estimated time, in FP32 within chain_limit where the splits allow it.  A
+// split product's partial results take at most 256 MiB of workspace, 2 GiB when K >= 32768 (RCCSD's o^2 x v.m x v^2
+// products over (ia|bc)).
 template <typename T>
 static GemmPlan gemm_plan(bool ta, bool tb, long M, long N, long K, long lda, long ldb, long sA, long sB, int batch,
-                          bool allow_split) {
+                          bool allow_split, bool limited = true) {
   GemmPlan best;
+  const long limit = sizeof(T) == 4 && limited && allow_split && batch == 1 ? chain_limit(M, N, K) : K;
   const double bytes = (double)sizeof(T) * ((double)M * K * (sA || batch == 1 ? batch : 1) +
                                             (double)N * K * (sB || batch == 1 ? batch : 1) + (double)M * N * batch);
   const double room = K >= 32768 ? 2147483648.0 : 268435456.0;
@@ -1672,14 +1702,22 @@ static GemmPlan gemm_plan(bool ta, bool tb, long M, long N, long K, long lda, lo
     form_tile(form, M, N, bm, bn);
     const long tiles = cdiv(M, bm) * cdiv(N, bn);
     if (tiles >= (1L << 31)) continue;
-    for (const long s : kSplits) {
+    // (operands past the caches' sizes: 4200 x 1500 x 33600 in five chunks takes 4.26 ms with 64x64 tiles, 3.89 with 128x128)
+    if (form == TILE64 && limit < K && K >= 32768 && tiles >= 512) continue;
+    const long parts = limit < K ? cdiv(K, limit) : 1;  // the split that the limit comes from, too
+    for (int q = parts > 1 ? -1 : 0; q < (int)(sizeof(kSplits) / sizeof(kSplits[0])); ++q) {
+      const long s = q < 0 ? parts : kSplits[q];
       if (s > 1 && (!allow_split || batch > 1 || K < 64 * s || tiles * s > 8192 || form == SHORT || form == TALL ||
-                    (double)s * M * N * sizeof(T) > room))
+                    (double)s * M * N * sizeof(T) > room)) {
+        if (q < 0) continue;
         break;
+      }
       const long slabs = cdiv(cdiv(K, s), 16);
+      const long chain = 16 * (form < DIRECT22 ? slabs : cdiv(slabs, form == DIRECT11 ? 8 : 4));
+      if (limit < K && chain > limit) continue;
       const double us = form_us<T>(form, tiles * s * batch, slabs, bytes) + reduce_us<T>(s, (double)M * N) +
                         (copy_a ? 6.0 : 0.0);
-      if (us < best.us) best = GemmPlan{form, s, TailMap{}, us};
+      if (us < best.us) best = GemmPlan{form, s, TailMap{}, us, chain};
     }
   }
   if (allow_split && batch == 1 && form_ok<T>(TILE128, ta, tb, M, N, K, lda, ldb)) {
@@ -1688,10 +1726,13 @@ static GemmPlan gemm_plan(bool ta, bool tb, long M, long N, long K, long lda, lo
       for (int chunks = 1; whole >= 0 && chunks <= 32; ++chunks) {
         const TailMap t = tail_map(kTail<T>, M, N, K, whole, chunks);
         if (!t.wgs || t.wgs == t.n[0] + t.n[1] + t.n[2] + t.n[3]) continue;  // (nothing shared: the plain launch)
+        const long chain = tail_chain(t, 16);
+        if (limit < K && chain > limit) continue;
         const double us = tail_us<T>(t);
-        if (us < best.us) best = GemmPlan{TILE128, 1, t, us};
+        if (us < best.us) best = GemmPlan{TILE128, 1, t, us, chain};
       }
   }
+  if (best.us >= 1e300) return gemm_plan<T>(ta, tb, M, N, K, lda, ldb, sA, sB, batch, allow_split, false);
   return best;
 }
 
@@ -1716,7 +1757,7 @@ static void tile_launch(jues_ctx* ctx, int form, bool tb, int kind, GemmSide<T> 
   p0.nz = p1.nz = nb;
   if (!two) p1 = p0;
   const bool tail = p0.tail.wgs > 0;
-  const dim3 grid((unsigned)(tail ? p0.tail.whole + p0.tail.wgs : total), 1, grid_z(nb));
+  const dim3 grid((unsigned)(tail ? p0.tail.whole + p0.tail.wgs : total), 1, grid_z(nb, total));
   if constexpr (sizeof(T) == 4) {
 #define JUES_GEMM32(K_, TB_, TA_, SEG_, BT_, ...)                                                                   \
   hipLaunchKernelGGL((gemm32_nn_kernel<K_, TB_, TA_, SEG_, false, BT_, ##__VA_ARGS__>), grid, dim3(NT), 0,          \
@@ -1815,7 +1856,8 @@ static void short_launch(jues_ctx* ctx, bool tall, GemmSide<T> p, int nb, T alph
 template <typename T, bool TA, bool TB>
 static void direct_launch_ab(jues_ctx* ctx, int form, GemmSide<T> p, int nb, T alpha, T beta) {
   p.nz = nb;
-  const dim3 grid((unsigned)((long)p.tiles_m * p.tiles_n), 1, grid_z(nb));
+  const long tiles = (long)p.tiles_m * p.tiles_n;
+  const dim3 grid((unsigned)tiles, 1, grid_z(nb, tiles));
 #define JUES_DIRECT(NW_, IM_, JN_)                                                                            \
   hipLaunchKernelGGL((gemm_direct_kernel<T, TA, TB, NW_, IM_, JN_>), grid, dim3(64 * NW_), 0, ctx->stream, p, \
                      alpha, beta)
@@ -2001,8 +2043,15 @@ void gemm_pair(jues_ctx* ctx, bool tb, long M0, long N0, long K0, const T* A0, l
   const bool empty0 = M0 <= 0 || N0 <= 0, empty1 = M1 <= 0 || N1 <= 0;
   // One launch of 64x64 or 128x128 tiles, its contractions split over S chunks, against two planned
   // products, by the same estimate.
+  // In FP32 both keep to sums over k as long as those of 1024 workgroups, each with at least 1024 of k (chain_limit).
   GemmPlan best;
   if (!empty0 && !empty1 && K0 >= 16 && K1 >= 16) {
+    long limit = std::max(K0, K1);
+    if (sizeof(T) == 4 && !no_alloc_active()) {
+      const long t = cdiv(M0, 128) * cdiv(N0, 128) + cdiv(M1, 128) * cdiv(N1, 128);
+      const long S = t < 1024 ? std::min(std::min(K0, K1) / 1024, cdiv(2048, t)) : 1;
+      if (S > 1) limit = cdiv(limit, S);
+    }
     const double bytes = (double)sizeof(T) * ((double)M0 * K0 + (double)K0 * N0 + (double)M0 * N0 + (double)M1 * K1 +
                                               (double)K1 * N1 + (double)M1 * N1);
     for (const int form : {(int)TILE128, (int)TILE64}) {
@@ -2015,14 +2064,16 @@ void gemm_pair(jues_ctx* ctx, bool tb, long M0, long N0, long K0, const T* A0, l
         if (s > 1 && (no_alloc_active() || s > 16 || std::min(K0, K1) < 64 * s || tiles * s > 8192 ||
                       (double)s * elems * sizeof(T) > 268435456.0))
           break;
+        if (cdiv(std::max(K0, K1), s) > limit) continue;
         const double us = form_us<T>(form, tiles * s, cdiv(cdiv(std::max(K0, K1), s), 16), bytes) +
                           (s > 1 ? 2.0 : 0.0) + reduce_us<T>(s, elems);
         if (us < best.us) best = GemmPlan{form, s, TailMap{}, us};
       }
     }
-    const double apart = gemm_plan<T>(false, tb, M0, N0, K0, lda0, ldb0, 0, 0, 1, !no_alloc_active()).us +
-                         gemm_plan<T>(false, tb, M1, N1, K1, lda1, ldb1, 0, 0, 1, !no_alloc_active()).us;
-    if (apart <= best.us) best.us = 1e300;
+    const GemmPlan a0 = gemm_plan<T>(false, tb, M0, N0, K0, lda0, ldb0, 0, 0, 1, !no_alloc_active()),
+                   a1 = gemm_plan<T>(false, tb, M1, N1, K1, lda1, ldb1, 0, 0, 1, !no_alloc_active());
+    const bool within = limit == std::max(K0, K1) || std::max(a0.chain, a1.chain) <= cdiv(limit, 16) * 16;
+    if (a0.us + a1.us <= best.us && (within || best.us >= 1e300)) best.us = 1e300;
   }
   T* Wk = nullptr;
   long S = best.split;

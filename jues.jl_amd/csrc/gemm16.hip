@@ -646,7 +646,7 @@ void gemm16_tn(jues_ctx* ctx, long M, long N, float alpha, const Split16& A, con
     for (const long whole : {full, full - 256})
       for (int chunks = 2; whole >= 0 && chunks <= 32; ++chunks) {
         const TailMap t = tail_map(kTail16, M, N, Kp, whole, chunks);
-        if (!t.wgs) continue;
+        if (!t.wgs || (S > 1 && tail_chain(t, BK) > kchunk)) continue;  // (no longer FP32 sums than the chunks')
         int least = chunks;
         for (int q = 0; q < 4; ++q)
           if (t.n[q]) least = std::min(least, t.s[q]);

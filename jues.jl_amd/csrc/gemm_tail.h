@@ -96,7 +96,7 @@ struct TailShape {
 
 // The TAIL launch of an M x N x K product with `whole` full tiles to themselves and the others in `chunks` chunks,
 // those past an edge in fewer by the cost of their slabs; wgs = 0 in the result if it is not of use (fewer full tiles,
-// chunks under 8 slabs, parts over 256 MiB).
+// chunks under least_slabs, parts over 256 MiB).
 // lower: the lower triangle of tiles of a square result.
 inline TailMap tail_map(const TailShape& g, long M, long N, long K, long whole, int chunks, bool lower = false) {
   const auto cdiv = [](long a, long b) { return (a + b - 1) / b; };
@@ -123,6 +123,14 @@ inline TailMap tail_map(const TailShape& g, long M, long N, long K, long whole, 
   }
   if (wgs <= 2048) t.wgs = (int)wgs;
   return t;
+}
+
+// The longest sum over k in one accumulator of a TAIL launch, slab_k of it a slab
+inline long tail_chain(const TailMap& t, long slab_k) {
+  int least = t.whole ? 1 : 1 << 30;
+  for (int q = 0; q < 4; ++q)
+    if (t.n[q]) least = std::min(least, t.s[q]);
+  return (t.nk + least - 1) / least * slab_k;
 }
 
 }  // namespace
