@@ -127,8 +127,8 @@ struct GemmSide {
 // n-contiguous (NT), 128x128 tile, 4 wavefronts of 64x64.
 // The K slice is 16 deep, so a workgroup needs 32 KB of LDS and at most 128 VGPRs per
 // lane: four workgroups (16 wavefronts) share a CU and cover each other's load and
-// barrier latency (two workgroups of 32-deep slices reach 73% MFMA-busy, this form ~93% with the
-// last slice peeled off the main loop, ~89% with a conditional loop body).
+// barrier latency (two workgroups of 32-deep slices reach 73% MFMA-busy, this form 91% with the
+// last slice peeled off the main loop and the last round of tiles shared, ~89% with a conditional loop body).
 // LDS holds each slice as 64-byte rows of 16 k-values per m (A) or n (B); the 16-byte
 // chunk q of row r sits at chunk q ^ ((r >> 2) & 3), so slices are written with 16-byte
 // stores and fragments read with 16-byte loads.  Lane l of a 16x16x4 MFMA supplies
