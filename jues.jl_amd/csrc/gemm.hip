@@ -1703,7 +1703,7 @@ static GemmPlan gemm_plan(bool ta, bool tb, long M, long N, long K, long lda, lo
     const long tiles = cdiv(M, bm) * cdiv(N, bn);
     if (tiles >= (1L << 31)) continue;
     // (operands past the caches' sizes: 4200 x 1500 x 33600 in five chunks takes 4.26 ms with 64x64 tiles, 3.89 with 128x128)
-    if (form == TILE64 && limit < K && K >= 32768 && tiles >= 512) continue;
+    if (form == TILE64 && limit < K && K >= 32768 && tiles >= 512 && form_ok<T>(TILE128, ta, tb, M, N, K, lda, ldb)) continue;
     const long parts = limit < K ? cdiv(K, limit) : 1;  // the split that the limit comes from, too
     for (int q = parts > 1 ? -1 : 0; q < (int)(sizeof(kSplits) / sizeof(kSplits[0])); ++q) {
       const long s = q < 0 ? parts : kSplits[q];
@@ -1732,7 +1732,8 @@ static GemmPlan gemm_plan(bool ta, bool tb, long M, long N, long K, long lda, lo
         if (us < best.us) best = GemmPlan{TILE128, 1, t, us, chain};
       }
   }
-  if (best.us >= 1e300) return gemm_plan<T>(ta, tb, M, N, K, lda, ldb, sA, sB, batch, allow_split, false);
+  if (best.us >= 1e300 && limit < K)
+    return gemm_plan<T>(ta, tb, M, N, K, lda, ldb, sA, sB, batch, allow_split, false);
   return best;
 }
 
